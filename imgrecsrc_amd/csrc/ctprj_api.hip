@@ -145,6 +145,8 @@ void Tables::release()
     free_ptr(d_rays);
     free_ptr(d_symtab);
     free_ptr(d_tr_items);
+    free_ptr(d_orb_items);
+    free_ptr(d_os_items);
     free_ptr(d_fwd_items);
     free_ptr(d_symf_items);
     free_ptr(d_adj_items);
@@ -159,8 +161,15 @@ void Tables::swap_geometry(Tables& o)
     std::swap(d_symtab, o.d_symtab);
     std::swap(d_tr_items, o.d_tr_items);
     std::swap(n_tr_items, o.n_tr_items);
+    std::swap(d_orb_items, o.d_orb_items);
+    std::swap(d_os_items, o.d_os_items);
     std::swap(n_sym, o.n_sym);
+    std::swap(orb_floats, o.orb_floats);
+    std::swap(os_floats, o.os_floats);
     slice_sym.swap(o.slice_sym);
+    slice_chunk.swap(o.slice_chunk);
+    orb_start.swap(o.orb_start);
+    os_start.swap(o.os_start);
 }
 
 void Tables::swap_fwd(Tables& o)
@@ -169,10 +178,7 @@ void Tables::swap_fwd(Tables& o)
     std::swap(d_symf_items, o.d_symf_items);
     std::swap(n_fwd_items, o.n_fwd_items);
     std::swap(n_symf_items, o.n_symf_items);
-    for (int g = 0; g < 4; ++g) {
-        std::swap(symf_start[g], o.symf_start[g]);
-        std::swap(symf_count[g], o.symf_count[g]);
-    }
+    symf.swap(o.symf);
 }
 
 void Tables::swap_adj(Tables& o)
@@ -181,21 +187,19 @@ void Tables::swap_adj(Tables& o)
     std::swap(d_syma_items, o.d_syma_items);
     std::swap(n_adj_items, o.n_adj_items);
     std::swap(n_syma_items, o.n_syma_items);
-    for (int g = 0; g < 4; ++g) {
-        std::swap(syma_start[g], o.syma_start[g]);
-        std::swap(syma_count[g], o.syma_count[g]);
-    }
+    syma.swap(o.syma);
 }
 
 Plan::~Plan()
 {
     free_ptr(d_fbp_items);
-    free_ptr(d_zero_row);
     free_ptr(d_fbp_kern);
     free_ptr(d_fbp_kern_off);
     free_ptr(d_fbp_prew);
     free_ptr(d_fbp_prew_off);
     free_ptr(d_imgT);
+    free_ptr(d_orb);
+    free_ptr(d_os);
     free_ptr(d_sino_ws);
     free_ptr(d_red);
     free_ptr(d_red_out);
@@ -239,17 +243,32 @@ static int dev_alloc(void** p, size_t bytes, const char* what)
     return 0;
 }
 
+// A workspace of at least `floats` floats in *p (of *cap floats): a larger one replaces it.
+static int grow(float** p, long long* cap, long long floats, const char* what)
+{
+    if (floats <= *cap) return 0;
+    float* q = nullptr;
+    const int rc = dev_alloc((void**)&q, sizeof(float) * (size_t)floats, what);
+    if (rc) return rc;
+    free_ptr(*p);
+    *p = q;
+    *cap = floats;
+    return 0;
+}
+
 // Batch order.  The hardware hands work-group i to XCD i % 8, so the list is built as
 // eight per-XCD queues interleaved (queue k at positions k, k + 8, ...).  Slices go to
 // queues heaviest first (work n^2 np).  `spread` (the default, tune flag bit 3 clear):
-// every slice is split into contiguous eighths, one per queue, which balances the XCDs
-// whatever the per-slice cost.  Otherwise only slices above a quarter of one XCD's
+// every slice is split over the queues, in contiguous eighths (adjoint tiles, which cost
+// the same and share bins with their neighbours) or dealt one by one with a turn per round
+// (`deal`: forward items, in view order, whose cost grows with the view's steepness and
+// falls towards the detector's ends), which balances the XCDs whatever the per-slice cost.  Otherwise only slices above a quarter of one XCD's
 // share are split and the others go whole to the least loaded queue, so each XCD's L2
 // serves whole slices (uniform stacks).  Shorter queues are padded with empty items
 // (slice = -1).
 template <class Item>
 static std::vector<Item> batch_order(const std::vector<Item>& in,
-                                     const std::vector<ctprj_geom>& geoms, bool spread)
+                                     const std::vector<ctprj_geom>& geoms, bool spread, bool deal)
 {
     std::vector<std::vector<Item>> per(geoms.size());
     for (const Item& it : in) per[it.slice].push_back(it);
@@ -264,9 +283,14 @@ static std::vector<Item> batch_order(const std::vector<Item>& in,
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work(a) > work(b); });
     std::vector<Item> q[8];
     double load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    size_t first = 0;  // queue of a dealt slice's first item
     for (int s : order) {
         const std::vector<Item>& its = per[s];
-        if (spread || work(s) > total / 32.0) {
+        if ((spread || work(s) > total / 32.0) && deal) {
+            for (size_t j = 0; j < its.size(); ++j) q[(first + j + j / 8) % 8].push_back(its[j]);
+            first += its.size();
+            for (int k = 0; k < 8; ++k) load[k] += work(s) / 8.0;
+        } else if (spread || work(s) > total / 32.0) {
             const size_t chunk = (its.size() + 7) / 8;
             for (int k = 0; k < 8; ++k) {
                 const size_t a = std::min(its.size(), k * chunk), b = std::min(its.size(), a + chunk);
@@ -340,7 +364,7 @@ static int choose_group(const ctprj_geom& g, int flags, bool* fold, std::vector<
         if (grp == kGrpV4 && (P % 2 || (flags & 4))) continue;
         const bool fo = !fan && grp != kGrpZ2 && 2 * g.np <= P;
         std::vector<int> c;
-        // the symmetric adjoint addresses a fan slice's ray table with 32-bit byte offsets
+        // fan slices with ray tables of 2 GiB and more stay on the general kernels
         if (fan && g.prjWidth * (double)sizeof(Ray) * (P / 2 + 2) >= 2147483648.0) break;
         if (symmetric_views(g, grp, fo, &c) >= 0.5) {
             *fold = fo;
@@ -373,8 +397,14 @@ int Plan::build_geometry(int flags, Tables& G) const
     std::vector<float4> views, bins;
     std::vector<long long> bin_off(nslices), ray_prefix(nslices + 1, 0);
     std::vector<int> symtab;
-    long long nview = 0, nray = 0;
+    std::vector<AdjItem> orbi;
+    std::vector<int2> osi;
+    long long nview = 0, nray = 0, orb_used = 0, os_used = 0;
     G.slice_sym.assign(nslices, 0);
+    G.slice_chunk.assign(nslices, 0);
+    G.orb_start.assign(1, 0);
+    G.os_start.assign(1, 0);
+    G.orb_floats = G.os_floats = 0;
     G.n_sym = 0;
     for (int s = 0; s < nslices; ++s) {
         const ctprj_geom& g = geoms[s];
@@ -394,7 +424,7 @@ int Plan::build_geometry(int flags, Tables& G) const
         D.d = D.fan ? g.d : 0.0f;
         D.invd = D.fan ? 1.0f / g.d : 0.0f;
         D.hbd = 0.5f * (g.dSize * g.effectiveRate);
-        D.er = g.effectiveRate;
+        D.inver = 1.0f / g.effectiveRate;
         D.fbp_scale = kRefPi / (float)g.np / g.dSize / g.dSize;
         D.img_off = img_offsets[s];
         D.sino_off = sino_offsets[s];
@@ -410,27 +440,43 @@ int Plan::build_geometry(int flags, Tables& G) const
             D.P = g.prjFull;
             D.ncanon = (int)canon.size();
             D.tab_off = (long long)symtab.size();
-            const unsigned all = group_masks(grp).all;
-            for (int a0 : canon)
-                for (int e2 = 0; e2 < 8; ++e2)
-                    for (int h = 0; h < 8; ++h) {
-                        if (!(all >> e2 & 1u) || !(all >> h & 1u)) {
-                            symtab.push_back(kRowNone);
-                            continue;
-                        }
-                        const int k1 = h & 3, m1 = h >> 2, k2 = e2 & 3, m2 = e2 >> 2;
-                        bool flip = false;
-                        const int v = host_map_view(g.prjFull, fold, k1 + (m1 ? -k2 : k2),
-                                                    m1 ^ m2, a0, &flip);
-                        // the kernels take the reflection of off-mirror views from
-                        // elem_flip() at compile time
-                        const bool mirror = a0 == 0 || group_masks(grp).q * a0 == g.prjFull;
-                        if (!mirror && flip != elem_flip(h, e2, fold))
-                            return fail(CTPRJ_EINVAL, "internal: reflection table mismatch "
-                                        "(slice %d, view %d, elements %d/%d)", s, a0, e2, h);
-                        symtab.push_back(v < g.np ? v * g.prjWidth * 4 + (flip ? kRowFlip : 0)
-                                                  : kRowNone);
-                    }
+            const GroupMasks M = group_masks(grp);
+            for (int a0 : canon) {
+                const bool mirror = a0 == 0 || M.q * a0 == g.prjFull;
+                for (int e = 0; e < 8; ++e) {
+                    bool flip = false;
+                    const int v = host_map_view(g.prjFull, fold, e & 3, e >> 2, a0, &flip);
+                    const bool read = ((mirror ? M.rot : M.all) >> e & 1u) && v < g.np;
+                    symtab.push_back(read ? v * g.prjWidth * 4 + (flip ? kRowFlip : 0) : kRowNone);
+                }
+            }
+            // orbit workspaces: 16-byte aligned rows, 4 n^2 floats (Z2: 3 n^2) of image and
+            // ncanon rows of bins
+            const long long edge = 2 * D.H + 1;
+            D.orb_pitch = (int)((edge + 3) & ~3LL);
+            D.os_pitch = (g.prjWidth + 3) & ~3;
+            const long long orb_rows = grp == kGrpD4   ? D.H + 1
+                                       : grp == kGrpV4 ? 2 * (D.H + 1)
+                                                       : edge + D.H + 1;
+            const long long orb = orb_rows * M.order * D.orb_pitch;
+            const long long os = (long long)D.ncanon * M.order * D.os_pitch;
+            if (orb_used > 0 && (orb_used + orb > kOrbitChunkFloats || os_used + os > kOrbitChunkFloats)) {
+                orb_used = os_used = 0;  // a new chunk
+                G.orb_start.push_back((int)orbi.size());
+                G.os_start.push_back((int)osi.size());
+            }
+            D.orb_off = orb_used;
+            D.os_off = os_used;
+            orb_used += orb;
+            os_used += os;
+            G.orb_floats = std::max(G.orb_floats, orb_used);
+            G.os_floats = std::max(G.os_floats, os_used);
+            for (int mode = 0; mode < (grp == kGrpD4 ? 1 : 2); ++mode) {
+                const int rows = grp == kGrpZ2 && mode == 0 ? (int)edge : D.H + 1;
+                for (int r = 0; r < rows; r += 32)
+                    for (int c = 0; c < edge; c += 32) orbi.push_back(AdjItem{s, r, c, mode});
+            }
+            for (int i = 0; i < D.ncanon; ++i) osi.push_back(make_int2(s, i));
             for (int a0 : canon) {
                 float c, si;
                 view_trig(a0, g.prjFull, &c, &si);
@@ -439,6 +485,7 @@ int Plan::build_geometry(int flags, Tables& G) const
                 views.push_back(make_float4(c, si, tag, 0.0f));
             }
             G.slice_sym[s] = grp;
+            G.slice_chunk[s] = (int)G.orb_start.size() - 1;
             ++G.n_sym;
         } else {
             for (int a = 0; a < g.np; ++a) {
@@ -462,10 +509,12 @@ int Plan::build_geometry(int flags, Tables& G) const
         }
         ray_prefix[s + 1] = nray;
     }
-    // the transposed image serves the general forward's steep views, D4's odd rotations
-    // and the column walks of V4 / Z2 canonical views beyond 45 degrees
+    G.orb_start.push_back((int)orbi.size());
+    G.os_start.push_back((int)osi.size());
+    // the transposed image serves the general forward's steep views
     std::vector<AdjItem> tr;
     for (int s = 0; s < nslices; ++s) {
+        if (G.slice_sym[s]) continue;
         for (int r = 0; r < geoms[s].n; r += 32)
             for (int c = 0; c < geoms[s].n; c += 32) tr.push_back(AdjItem{s, r, c, 0});
     }
@@ -479,6 +528,8 @@ int Plan::build_geometry(int flags, Tables& G) const
         (rc = upload(&d_ray_prefix, ray_prefix, "ray offsets")) ||
         (rc = upload(&G.d_symtab, symtab, "symmetric view-row table")) ||
         (rc = upload(&G.d_tr_items, tr, "transpose work list")) ||
+        (rc = upload(&G.d_orb_items, orbi, "orbit image work list")) ||
+        (rc = upload(&G.d_os_items, osi, "orbit sinogram work list")) ||
         (rc = dev_alloc((void**)&G.d_rays, sizeof(Ray) * (size_t)nray, "ray table"))) {
         free_dev(d_bins);
         free_dev(d_bin_off);
@@ -496,19 +547,25 @@ int Plan::build_geometry(int flags, Tables& G) const
     return 0;
 }
 
-// Concatenates per-group lists (each in batch order) and records the segments.
+// Concatenates the lists of every chunk and group (each in batch order) and records the
+// segments.
 template <class Item>
-static std::vector<Item> group_segments(std::vector<Item> (&by)[4],
+static std::vector<Item> group_segments(const std::vector<Item> (&by)[4], const Tables& G,
                                         const std::vector<ctprj_geom>& geoms, bool spread,
-                                        int* start, int* count)
+                                        bool deal, std::vector<Tables::Segments>* segs)
 {
     std::vector<Item> out;
-    for (int g = 1; g < 4; ++g) {
-        std::vector<Item> seg = batch_order(by[g], geoms, spread);
-        start[g] = (int)out.size();
-        count[g] = (int)seg.size();
-        out.insert(out.end(), seg.begin(), seg.end());
-    }
+    segs->assign(G.chunks(), Tables::Segments{});
+    for (int c = 0; c < G.chunks(); ++c)
+        for (int g = 1; g < 4; ++g) {
+            std::vector<Item> in;
+            for (const Item& it : by[g])
+                if (G.slice_chunk[it.slice] == c) in.push_back(it);
+            const std::vector<Item> seg = batch_order(in, geoms, spread, deal);
+            (*segs)[c].start[g] = (int)out.size();
+            (*segs)[c].count[g] = (int)seg.size();
+            out.insert(out.end(), seg.begin(), seg.end());
+        }
     return out;
 }
 
@@ -533,8 +590,8 @@ int Plan::build_fwd_items(const ctprj_tune& t, Tables& G) const
         }
     }
     const bool spread = !(t.flags & 8);
-    items = batch_order(items, geoms, spread);
-    std::vector<FwdItem> sym = group_segments(by, geoms, spread, G.symf_start, G.symf_count);
+    items = batch_order(items, geoms, spread, true);
+    std::vector<FwdItem> sym = group_segments(by, G, geoms, spread, true, &G.symf);
     G.n_fwd_items = (int)items.size();
     G.n_symf_items = (int)sym.size();
     int rc = upload(&G.d_fwd_items, items, "forward work list");
@@ -571,8 +628,8 @@ int Plan::build_adj_items(const ctprj_tune& t, Tables& G) const
         }
     }
     const bool spread = !(t.flags & 8);
-    items = batch_order(items, geoms, spread);
-    std::vector<AdjItem> sym = group_segments(by, geoms, spread, G.syma_start, G.syma_count);
+    items = batch_order(items, geoms, spread, false);
+    std::vector<AdjItem> sym = group_segments(by, G, geoms, spread, false, &G.syma);
     G.n_adj_items = (int)items.size();
     G.n_syma_items = (int)sym.size();
     int rc = upload(&G.d_adj_items, items, "adjoint work list");
@@ -654,15 +711,12 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
     for (int s = 0; s < nslices; ++s)
         for (int a = 0; a < geoms[s].np; ++a) fbpi.push_back(make_int2(s, a));
     p->n_fbp_items = (int)fbpi.size();
-    std::vector<float> zeros((size_t)max_W + 1, 0.0f);
     p->red_cap = bhc_red_doubles(sino);
     if ((rc = upload(&p->d_fbp_items, fbpi, "fbp work list")) ||
         (rc = upload(&p->d_fbp_kern, kern, "fbp taps")) ||
         (rc = upload(&p->d_fbp_kern_off, kern_off, "fbp tap offsets")) ||
         (rc = upload(&p->d_fbp_prew, prew, "fbp preweights")) ||
         (rc = upload(&p->d_fbp_prew_off, prew_off, "fbp preweight offsets")) ||
-        (rc = upload(&p->d_zero_row, zeros, "zero row")) ||
-        (rc = dev_alloc((void**)&p->d_imgT, sizeof(float) * (size_t)img, "transposed image")) ||
         (rc = dev_alloc((void**)&p->d_sino_ws, sizeof(float) * (size_t)sino, "sinogram workspace")) ||
         // the beam-hardening passes' reduction partials and outputs: their calls
         // allocate nothing (and can be captured into a graph)
@@ -671,7 +725,10 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
         (rc = dev_alloc((void**)&p->d_red_out, sizeof(double) * (size_t)bhc_ie_nvals(CTPRJ_MAX_E),
                         "reduction output")) ||
         (rc = p->build_geometry(p->tune.flags, *p)) || (rc = p->build_fwd_items(p->tune, *p)) ||
-        (rc = p->build_adj_items(p->tune, *p))) {
+        (rc = p->build_adj_items(p->tune, *p)) ||
+        (rc = grow(&p->d_imgT, &p->imgT_cap, p->n_sym < nslices ? img : 0, "transposed image")) ||
+        (rc = grow(&p->d_orb, &p->orb_cap, p->orb_floats, "orbit image")) ||
+        (rc = grow(&p->d_os, &p->os_cap, p->os_floats, "orbit sinogram"))) {
         delete p;
         return rc;
     }
@@ -714,6 +771,26 @@ extern "C" int ctprj_plan_layout(const ctprj_plan* p, long long* img_elems,
 
 namespace ctprj {
 
+// The symmetric slices' forward: per chunk, its orbit image, then one launch per group.
+int Plan::launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st)
+{
+    if (bhc) bhc->part_off = 0;
+    for (int c = 0; n_sym && c < chunks(); ++c) {
+        launch_orbit_image(orb_start[c + 1] - orb_start[c], d_desc, d_orb_items + orb_start[c],
+                           d_img, d_orb, st);
+        for (int g = 1; g < 4; ++g) {
+            const int n = symf[c].count[g];
+            if (!n) continue;
+            launch_forward_sym(g, tune.fwd_seg, tune.fwd_split, d_split, n, d_desc,
+                               d_symf_items + symf[c].start[g], d_views, d_rays, d_orb, d_sino,
+                               bhc, st);
+            if (bhc) bhc->part_off += n;
+        }
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : hip_fail(e, "forward launch");
+}
+
 int Plan::launch_forward(const float* d_img, float* d_sino, hipStream_t st, bool count)
 {
     if (count && n_sym) return fail(CTPRJ_EINVAL, "internal: count needs the general kernels");
@@ -721,37 +798,15 @@ int Plan::launch_forward(const float* d_img, float* d_sino, hipStream_t st, bool
     if (n_fwd_items)
         launch_forward_kernel(count, tune.fwd_block, n_fwd_items, d_desc, d_fwd_items, d_views,
                               d_rays, d_img, d_imgT, d_sino, st);
-    for (int g = 1; g < 4; ++g)
-        if (symf_count[g])
-            launch_forward_sym(g, tune.fwd_seg, tune.fwd_split, d_split, symf_count[g], d_desc,
-                               d_symf_items + symf_start[g], d_views, d_rays, d_img, d_imgT,
-                               d_sino, nullptr, st);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : hip_fail(e, "forward launch");
+    return launch_symf(d_img, d_sino, nullptr, st);
 }
 
-long long Plan::bhc_fused_parts() const
-{
-    if (n_fwd_items) return -1;
-    long long n = 0;
-    for (int g = 1; g < 4; ++g) n += symf_count[g];
-    return n;
-}
+long long Plan::bhc_fused_parts() const { return n_fwd_items ? -1 : n_symf_items; }
 
 int Plan::launch_forward_bhc(const float* d_img, float* d_w, BhcStore bhc, hipStream_t st)
 {
     if (n_fwd_items) return fail(CTPRJ_EINVAL, "internal: fused store needs symmetric slices");
-    launch_transpose(n_tr_items, d_desc, d_tr_items, d_img, d_imgT, st);
-    bhc.part_off = 0;
-    for (int g = 1; g < 4; ++g)
-        if (symf_count[g]) {
-            launch_forward_sym(g, tune.fwd_seg, tune.fwd_split, d_split, symf_count[g], d_desc,
-                               d_symf_items + symf_start[g], d_views, d_rays, d_img, d_imgT,
-                               d_w, &bhc, st);
-            bhc.part_off += symf_count[g];
-        }
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : hip_fail(e, "forward launch");
+    return launch_symf(d_img, d_w, &bhc, st);
 }
 
 int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool fbp,
@@ -762,17 +817,18 @@ int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool
     if (n_adj_items)
         launch_adjoint_kernel(tune.adj_tile, fbp, n_adj_items, d_desc, d_adj_items, d_views,
                               d_rays, d_sino, d_img, st);
-    if (n_syma_items) {
-        bool first = true;
-        for (int g = 1; g < 4; ++g)
-            if (syma_count[g]) {
-                launch_adjoint_sym(fbp, g, tune.adj_seg, (tune.flags & 16) ? 3 : 4,
-                                   (tune.flags & 32) != 0, tune.adj_split,
-                                   d_split, syma_count[g], d_desc, d_syma_items + syma_start[g],
-                                   d_views, d_rays, d_sino, d_zero_row, d_symtab, d_img,
-                                   first ? job : RedJob{}, st);
-                first = false;
-            }
+    bool first = true;
+    for (int c = 0; n_sym && c < chunks(); ++c) {
+        launch_orbit_sino(os_start[c + 1] - os_start[c], max_W, d_desc, d_os_items + os_start[c],
+                          d_symtab, d_sino, d_os, st);
+        for (int g = 1; g < 4; ++g) {
+            const int n = syma[c].count[g];
+            if (!n) continue;
+            launch_adjoint_sym(fbp, g, tune.adj_seg, tune.adj_split, d_split, n, d_desc,
+                               d_syma_items + syma[c].start[g], d_views, d_rays, d_os, d_img,
+                               first ? job : RedJob{}, st);
+            first = false;
+        }
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : hip_fail(e, "adjoint launch");
@@ -875,21 +931,24 @@ extern "C" int ctprj_plan_set_tune(ctprj_plan* p, const ctprj_tune* t)
     // the parts this change rebuilds go into N; the plan keeps its tables until all of
     // them (and the split partial-sum space) exist
     ctprj_tune nt = *t;
-    const bool geo = nt.flags != p->tune.flags;
-    const bool fwd = geo || nt.fwd_block != p->tune.fwd_block;
-    const bool adj = geo || nt.adj_tile != p->tune.adj_tile;
+    // the geometry depends on the symmetry flags (bits 0-2), the work lists on the order too
+    const bool geo = (nt.flags & 7) != (p->tune.flags & 7);
+    const bool order = geo || (nt.flags & 8) != (p->tune.flags & 8);
+    const bool fwd = order || nt.fwd_block != p->tune.fwd_block;
+    const bool adj = order || nt.adj_tile != p->tune.adj_tile;
     Tables N;
     int rc = 0;
-    if (geo) rc = p->build_geometry(nt.flags, N);
-    if (geo && !rc) {
-        // the work lists read the new slice groups
-        if (!(rc = p->build_fwd_items(nt, N))) rc = p->build_adj_items(nt, N);
-    } else if (!rc) {
+    if (geo) {
+        rc = p->build_geometry(nt.flags, N);
+    } else {
         // same geometry: build the lists from the plan's slice groups
         N.slice_sym = p->slice_sym;
-        if (fwd) rc = p->build_fwd_items(nt, N);
-        if (adj && !rc) rc = p->build_adj_items(nt, N);
+        N.slice_chunk = p->slice_chunk;
+        N.orb_start = p->orb_start;
+        N.os_start = p->os_start;
     }
+    if (fwd && !rc) rc = p->build_fwd_items(nt, N);
+    if (adj && !rc) rc = p->build_adj_items(nt, N);
     if (rc) return rc;  // N frees what it holds; the plan is unchanged
     const Tables& F = fwd ? N : *static_cast<const Tables*>(p);
     const Tables& A = adj ? N : *static_cast<const Tables*>(p);
@@ -901,19 +960,21 @@ extern "C" int ctprj_plan_set_tune(ctprj_plan* p, const ctprj_tune* t)
         nt.adj_split = nt.fwd_split = 1;
         need = 0;
     }
-    float* split = nullptr;
-    if (need > p->split_cap && (rc = dev_alloc((void**)&split, sizeof(float) * need,
-                                                "split partial sums")))
+    // workspaces only grow, and serve the old tables as well as the new
+    if (geo && ((rc = grow(&p->d_imgT, &p->imgT_cap, N.n_sym < p->nslices ? p->img_elems : 0,
+                           "transposed image")) ||
+                (rc = grow(&p->d_orb, &p->orb_cap, N.orb_floats, "orbit image")) ||
+                (rc = grow(&p->d_os, &p->os_cap, N.os_floats, "orbit sinogram"))))
         return rc;
+    if (need > p->split_cap) {
+        long long cap = (long long)p->split_cap;
+        if ((rc = grow(&p->d_split, &cap, (long long)need, "split partial sums"))) return rc;
+        p->split_cap = (size_t)cap;
+    }
     // commit: swap the rebuilt parts in (N then frees the old ones)
     if (geo) p->swap_geometry(N);
     if (fwd) p->swap_fwd(N);
     if (adj) p->swap_adj(N);
-    if (split) {
-        free_ptr(p->d_split);
-        p->d_split = split;
-        p->split_cap = need;
-    }
     p->tune = nt;
     return split_rc;
 }
@@ -926,8 +987,10 @@ size_t Plan::split_need(const ctprj_tune& t, const Tables& F, const Tables& A) c
 {
     size_t need = 0;
     for (int g = 1; g < 4; ++g) {
-        if (t.fwd_split > 1) need = std::max(need, (size_t)F.symf_count[g] * t.fwd_split);
-        if (t.adj_split > 1) need = std::max(need, (size_t)A.syma_count[g] * t.adj_split);
+        if (t.fwd_split > 1)
+            for (const Segments& c : F.symf) need = std::max(need, (size_t)c.count[g] * t.fwd_split);
+        if (t.adj_split > 1)
+            for (const Segments& c : A.syma) need = std::max(need, (size_t)c.count[g] * t.adj_split);
     }
     return need * 512;
 }
@@ -967,9 +1030,8 @@ static std::string tune_key(const ctprj_plan* p, const char* arch)
 
 // Times the kernel shapes on this plan's geometry: general forward threads per group,
 // symmetric forward waves and work-groups per ray run, general adjoint tile edge,
-// symmetric adjoint waves and work-groups per tile for each bin window width (flag bit 4)
-// and gather (LDS staging, bit 5), and (several slices) the work order of tune flag bit
-// 3; keeps the symmetry flags (bits 0-2).
+// symmetric adjoint waves and work-groups per tile, and (several slices) the work order of
+// tune flag bit 3; keeps the symmetry flags (bits 0-2).
 extern "C" int ctprj_plan_autotune(ctprj_plan* p, int reps, const char* cache_path, void* stream)
 {
     if (!p) return fail(CTPRJ_EINVAL, "plan is NULL");
@@ -1040,7 +1102,7 @@ extern "C" int ctprj_plan_autotune(ctprj_plan* p, int reps, const char* cache_pa
     // than one work-group per item only while the items are too few to fill the device
     // several times over
     auto search_split = [&](int ctprj_tune::*seg, int ctprj_tune::*split, const int* segs,
-                            int ns, bool fwd, int nitems, float* out_ms = nullptr) -> int {
+                            int ns, bool fwd, int nitems) -> int {
         float best_ms = 1e30f;
         const int splits[7] = {1, 2, 3, 4, 5, 6, 8};
         const int nsplits = nitems < 8192 ? 7 : 1;
@@ -1063,7 +1125,6 @@ extern "C" int ctprj_plan_autotune(ctprj_plan* p, int reps, const char* cache_pa
                     best.*split = k;
                 }
             }
-        if (out_ms) *out_ms = best_ms;
         return ctprj_plan_set_tune(p, &best);
     };
     const int blocks[3] = {64, 128, 256}, tiles[2] = {8, 16};
@@ -1091,26 +1152,8 @@ extern "C" int ctprj_plan_autotune(ctprj_plan* p, int reps, const char* cache_pa
                           p->n_symf_items);
     if (!rc && p->n_adj_items) rc = search(&ctprj_tune::adj_tile, tiles, 2, false);
     if (!rc && p->n_syma_items) {
-        // symmetric adjoint: bin windows 4 or 3 wide (flag bit 4) and gathers per lane
-        // from L1 or staged per wave in LDS (bit 5), each variant with its best waves and
-        // work-groups per tile (the variants differ in registers, so in the shape they
-        // want)
-        const ctprj_tune start = best;
-        ctprj_tune winner = best;
-        float win_ms = 1e30f;
-        for (int v = 0; v < 4 && !rc; ++v) {
-            best = start;
-            best.flags = (start.flags & ~48) | ((v & 1) ? 16 : 0) | ((v & 2) ? 32 : 0);
-            float ms = 1e30f;
-            rc = search_split(&ctprj_tune::adj_seg, &ctprj_tune::adj_split, asegs, 4, false,
-                              p->n_syma_items, &ms);
-            if (!rc && ms < win_ms) {
-                win_ms = ms;
-                winner = best;
-            }
-        }
-        best = winner;
-        if (!rc) rc = ctprj_plan_set_tune(p, &best);
+        rc = search_split(&ctprj_tune::adj_seg, &ctprj_tune::adj_split, asegs, 4, false,
+                          p->n_syma_items);
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

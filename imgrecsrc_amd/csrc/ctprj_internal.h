@@ -24,6 +24,10 @@ struct RedJob {
 struct FwdItem {
     int slice, view, bin0, pad;
 };
+// Orbit workspaces (image and sinogram, each) of the symmetric slices: a plan whose slices
+// need more runs them in chunks of consecutive slices that share this much (one slice
+// takes what it needs).  1 GiB floats hold 1024 slices of 512^2.
+constexpr long long kOrbitChunkFloats = 1LL << 30;
 // partial-sum space of split symmetric work items: at most 256 MiB per plan
 constexpr size_t kSplitMaxFloats = (size_t)64 << 20;
 struct AdjItem {
@@ -41,20 +45,29 @@ struct Tables {
     SliceDesc* d_desc = nullptr;
     float4* d_views = nullptr;
     Ray* d_rays = nullptr;
-    int* d_symtab = nullptr;          // view-row table of the symmetric adjoint
-    AdjItem* d_tr_items = nullptr;    // transpose tiles
+    int* d_symtab = nullptr;          // view-row table of the symmetric slices
+    AdjItem* d_tr_items = nullptr;    // transpose tiles (slices on the general kernels)
+    AdjItem* d_orb_items = nullptr;   // orbit image tiles (symmetric slices)
+    int2* d_os_items = nullptr;       // orbit sinogram rows (slice, canonical view)
     int n_tr_items = 0, n_sym = 0;
     std::vector<int> slice_sym;       // per slice: symmetry group (kGrp*), 0 = general kernels
+    std::vector<int> slice_chunk;     // per slice: chunk of the orbit workspaces
+    // first orbit image tile / orbit sinogram row of every chunk, and their ends
+    std::vector<int> orb_start, os_start;
+    long long orb_floats = 0, os_floats = 0;  // workspace of the largest chunk
     FwdItem* d_fwd_items = nullptr;   // general forward
     FwdItem* d_symf_items = nullptr;  // symmetric forward
     int n_fwd_items = 0, n_symf_items = 0;
     AdjItem* d_adj_items = nullptr;   // general adjoint
     AdjItem* d_syma_items = nullptr;  // symmetric adjoint
     int n_adj_items = 0, n_syma_items = 0;
-    // symmetric work lists are grouped by symmetry group: [start, start + count) of
-    // group g (1..3) in d_symf_items / d_syma_items
-    int symf_start[4] = {0, 0, 0, 0}, symf_count[4] = {0, 0, 0, 0};
-    int syma_start[4] = {0, 0, 0, 0}, syma_count[4] = {0, 0, 0, 0};
+    // symmetric work lists: [start, start + count) of chunk c and group g in d_symf_items /
+    // d_syma_items at [c][g], g = 1..3
+    struct Segments {
+        int start[4] = {0, 0, 0, 0}, count[4] = {0, 0, 0, 0};
+    };
+    std::vector<Segments> symf, syma;
+    int chunks() const { return (int)orb_start.size() - 1; }
 
     Tables() = default;
     Tables(const Tables&) = delete;
@@ -76,14 +89,16 @@ struct Plan : Tables {
     ctprj_tune tune{64, 16, 1, 8, 8, 1, 1};
 
     int2* d_fbp_items = nullptr;
-    float* d_zero_row = nullptr;      // max_W zeros: reads of views beyond np
     float* d_fbp_kern = nullptr;
     long long* d_fbp_kern_off = nullptr;
     float* d_fbp_prew = nullptr;
     long long* d_fbp_prew_off = nullptr;
     int n_fbp_items = 0;
 
-    float* d_imgT = nullptr;     // transposed image (forward, steep views / symmetric images)
+    float* d_imgT = nullptr;     // transposed image (general forward, steep views)
+    float* d_orb = nullptr;      // orbit image of a chunk (symmetric forward)
+    float* d_os = nullptr;       // orbit sinogram of a chunk (symmetric adjoint)
+    long long imgT_cap = 0, orb_cap = 0, os_cap = 0;  // floats held by the three
     float* d_sino_ws = nullptr;  // sinogram workspace (FBP filter output, BHC ray values)
     double* d_red = nullptr;     // reduction partials (beam-hardening)
     double* d_red_out = nullptr; // reduced sums
@@ -102,6 +117,7 @@ struct Plan : Tables {
     // work lists for tune t on the geometry of G, into G
     int build_fwd_items(const ctprj_tune& t, Tables& G) const;
     int build_adj_items(const ctprj_tune& t, Tables& G) const;
+    int launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st);
     // partial-sum floats the split symmetric launches of tune t need on tables G
     size_t split_need(const ctprj_tune& t, const Tables& fwd, const Tables& adj) const;
     int launch_forward(const float* d_img, float* d_sino, hipStream_t st, bool count);
@@ -142,15 +158,19 @@ void launch_scale(float* p, long long n, float s, hipStream_t st);
 // w; one NLL partial per item at bhc->partials[bhc->part_off + item])
 void launch_forward_sym(int grp, int seg, int nsplit, float* part, int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
-                        const Ray* rays, const float* img, const float* imgT, float* sino,
-                        const BhcStore* bhc, hipStream_t st);
+                        const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
+                        hipStream_t st);
 // The same sum as a symmetric adjoint's side job, in a launch of its own.
 void launch_wave_sum(const RedJob& job, hipStream_t st);
-void launch_adjoint_sym(bool fbp, int grp, int seg, int win, bool stage, int nsplit, float* part,
-                        int nitems, const SliceDesc* desc, const AdjItem* items,
-                        const float4* views, const Ray* rays, const float* sino,
-                        const float* zero_row, const int* symtab, float* img, const RedJob& job,
+void launch_adjoint_sym(bool fbp, int grp, int seg, int nsplit, float* part, int nitems,
+                        const SliceDesc* desc, const AdjItem* items, const float4* views,
+                        const Ray* rays, const float* os, float* img, const RedJob& job,
                         hipStream_t st);
+// The orbit image (tiles) and orbit sinogram (rows) those two read.
+void launch_orbit_image(int nitems, const SliceDesc* desc, const AdjItem* items, const float* img,
+                        float* orb, hipStream_t st);
+void launch_orbit_sino(int nitems, int max_W, const SliceDesc* desc, const int2* items,
+                       const int* tab, const float* sino, float* os, hipStream_t st);
 
 // Images held by a wavelet context (rows * cols * batch).
 long long wavelet_elems(const ctprj_wavelet* w);

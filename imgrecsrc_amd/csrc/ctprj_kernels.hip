@@ -51,12 +51,12 @@ __global__ void k_build_rays(const SliceDesc* __restrict__ slices, int nslices,
         r.dc = 0.0f;
         r.hbc = S.hbd;
     }
-    const float c = fabsf(r.cosR), s = fabsf(r.sinR);
-    const float hi_ = fmaxf(c, s), lo_ = fminf(c, s);
-    r.h = 1.0f / (hi_ * S.er);
-    r.b1 = 0.5f * (hi_ - lo_);
-    r.s = lo_;
-    r.k = lo_ > 0.0f ? 0.5f / lo_ : 0.0f;
+    const double c = fabs((double)r.cosR), s = fabs((double)r.sinR);
+    const double ramp = fmax(fmin(c, s), 0x1p-24), b1 = fmax(0.5 * (fmax(c, s) - ramp), 0x1p-25);
+    r.is = (float)(1.0 / ramp);
+    r.c2 = (float)((b1 + ramp) / ramp);
+    r.ib = (float)(0.5 / b1);
+    r.a = (float)(0.5 * ramp / (ramp + 2.0 * b1));
     rays[S.ray_off + local] = r;
 }
 
@@ -107,17 +107,20 @@ __device__ __forceinline__ float forward_ray(const SliceDesc& S, const Ray& r, f
             const float x = rowmode ? (float)u : (float)v;
             const float y = rowmode ? (float)v : (float)u;
             const float dist = ray_dist(x, y, r.cosR, r.sinR, r.dc);
-            const float hb = FAN ? r.hbc * fan_depth_scale(x, y, cT, sT, S.invd) : r.hbc;
-            const float w = strip_weight(dist, hb, r);
-            if (COUNT) part += (w != 0.0f) ? 1.0f : 0.0f;
-            else part = fmaf(w, row[u], part);
+            if (COUNT) {
+                const float qd = fmaf(fmaf(x, sT, -(y * cT)), S.invd, 1.0f);
+                part += strip_hits(dist, FAN ? r.hbc * qd : r.hbc, r) ? 1.0f : 0.0f;
+            } else {
+                const float qd = FAN ? fan_depth_scale(x, y, cT, sT, S.invd) : 1.0f;
+                part = fmaf(strip_area(dist, FAN ? r.hbc * qd : r.hbc, r), row[u], part);
+            }
         }
         if (((v + H) & 3) == 3 || v == H) {
             acc.add(part);
             part = 0.0f;
         }
     }
-    return acc.s;
+    return COUNT ? acc.s : acc.s * S.inver;
 }
 
 template <bool COUNT>
@@ -189,7 +192,7 @@ __device__ __forceinline__ float adjoint_pixel(const SliceDesc& S, int x, int y,
         } else {
             const Ray r = rays[S.ray_off + a];
             const float center = fmaf(fx, cT, fy * sT);
-            const float ext = r.b1 + r.s + r.hbc + kSupportMargin;
+            const float ext = 0.5f * (fabsf(cT) + fabsf(sT)) + r.hbc + kSupportMargin;
             blo = (int)ceilf((center - ext) * S.invDSize + (float)S.pC);
             bhi = (int)floorf((center + ext) * S.invDSize + (float)S.pC);
         }
@@ -201,7 +204,7 @@ __device__ __forceinline__ float adjoint_pixel(const SliceDesc& S, int x, int y,
             for (int b = blo; b <= bhi; ++b) {
                 const Ray r = rr[b];
                 const float dist = ray_dist(fx, fy, r.cosR, r.sinR, r.dc);
-                const float w = strip_weight(dist, r.hbc * qd, r);
+                const float w = strip_area(dist, r.hbc * qd, r);
                 part = fmaf(w, srow[b], part);
             }
             if (FBP) part *= 1.0f / (qd * qd);  // d^2/qe^2, prj/cpuPrj.c:258
@@ -210,7 +213,7 @@ __device__ __forceinline__ float adjoint_pixel(const SliceDesc& S, int x, int y,
             for (int b = blo; b <= bhi; ++b) {
                 const float dc = (float)(b - S.pC) * S.dSize;
                 const float dist = ray_dist(fx, fy, r.cosR, r.sinR, dc);
-                const float w = strip_weight(dist, r.hbc, r);
+                const float w = strip_area(dist, r.hbc, r);
                 part = fmaf(w, srow[b], part);
             }
         }
@@ -239,10 +242,11 @@ __global__ __launch_bounds__(TILE* TILE) void k_adjoint(const SliceDesc* __restr
     if (row >= S.n || col >= S.n) return;
     const int x = col - S.half, y = row - S.half;
     float val = 0.0f;
+    // even n: row 0 and column 0 stay 0
     if (x >= -S.H && x <= S.H && y >= -S.H && y <= S.H) {
         if (S.fan) val = adjoint_pixel<true, FBP>(S, x, y, views, rays, sino);
         else val = adjoint_pixel<false, FBP>(S, x, y, views, rays, sino);
-        if (FBP) val *= S.fbp_scale;
+        val *= FBP ? S.fbp_scale * S.inver : S.inver;
     }
     img[S.img_off + (long long)row * S.n + col] = val;
 }

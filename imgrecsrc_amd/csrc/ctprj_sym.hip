@@ -18,6 +18,8 @@
 // into [0, 180) and folds, the forward takes half the detector with all the images.
 // |dist| in the weight makes W(a0, b, p) == W(a0, 2pC - b, R^2 p) exactly.
 #include "ctprj_internal.h"
+#include <type_traits>
+
 #include "bhc_device.h"
 
 namespace ctprj {
@@ -56,43 +58,45 @@ __device__ __forceinline__ int map_view(const SliceDesc& S, int k, int m, int a0
     return v;
 }
 
-__device__ __forceinline__ bool mirror_view(const SliceDesc& S, int a0)
-{
-    return a0 == 0 || group_masks(S.sym).q * a0 == S.P;
-}
-
-// Candidate bins of pixel (x, y) for a view (shared with the general adjoint's rule).
+// Per canonical view, what the candidate bins of a pixel need (wave-uniform values).  With
+// the pixel's centre at (oc, qe) across and along the central ray and
+// rho = (|cos| + |sin|) / 2 half the pixel's extent in any direction, the strips that meet
+// the pixel, |dist| < b2 + hb in the weight's terms, are those of the bins at t between
+//   parallel: oc -+ (rho + hbd);   fan: (d (oc -+ rho) -+ hbd qe) / (qe +- rho),
+// hbd being half the strip's width on the detector (fan: the ray at t has
+// dist = (d oc - t qe) / sqrt(d^2 + t^2), and its footprint is at most
+// (d m + t n) / (2 sqrt(d^2 + t^2)) wide, |m|, |n| <= 2 rho), and kSupportMargin px more are
+// taken.  The sign before rho in the fan's denominator is the numerator's on the left, its
+// opposite on the right: the smaller (larger) of two ratios of linear functions of the
+// pixel, so over a square of pixels the extreme bounds are those of its corner pixels.
 template <bool FAN>
-__device__ __forceinline__ void pixel_bins(const SliceDesc& S, const Ray* rays_view, float fx,
-                                           float fy, float cT, float sT, int& blo, int& bhi)
-{
-    if (FAN) {
-        // the pixel's shadow on the virtual detector lies within t_c +- ext: a corner
-        // offset (do, dq) of the projected coordinates (|do|, |dq| <= rho) moves
-        // t = d oc/qe by d |do qe - oc dq| / (qe (qe + dq)) <= d rho (qe + |oc|) / (qe (qe - rho))
-        const float oc = fmaf(fx, cT, fy * sT);
-        const float qe = fmaf(fx, sT, fmaf(-fy, cT, S.d));
-        const float rho = 0.5f * (fabsf(cT) + fabsf(sT));
-        const float iq = fast_rcp(qe), iqr = fast_rcp(qe - rho);
-        const float tc = S.d * oc * iq;
-        const float ext = S.d * rho * (qe + fabsf(oc)) * iq * iqr;
-        const float m = ext + S.hbd + kSupportMargin * S.dSize;
-        blo = (int)ceilf((tc - m) * S.invDSize + (float)S.pC);
-        bhi = (int)floorf((tc + m) * S.invDSize + (float)S.pC);
-        if (!(qe - rho > 0.0f)) {  // the source within a pixel: every bin is a candidate
-            blo = S.blo;
-            bhi = S.bhi;
-        }
-    } else {
-        const Ray r = rays_view[0];
-        const float center = fmaf(fx, cT, fy * sT);
-        const float ext = r.b1 + r.s + r.hbc + kSupportMargin;
-        blo = (int)ceilf((center - ext) * S.invDSize + (float)S.pC);
-        bhi = (int)floorf((center + ext) * S.invDSize + (float)S.pC);
+struct BinBounds {
+    float cT, sT, rho, d, hbd, scale, left, right;
+    int blo, bhi;
+
+    // last: the last bin of the lane's pixels (below the first: none)
+    __device__ __forceinline__ BinBounds(const SliceDesc& S, float c, float s, const Ray& r, int last)
+        : cT(c), sT(s), d(S.d), hbd(S.hbd), scale(S.invDSize), blo(S.blo), bhi(last)
+    {
+        rho = 0.5f * (fabsf(c) + fabsf(s));
+        const float m = FAN ? kSupportMargin * S.dSize : rho + r.hbc + kSupportMargin;
+        left = (float)S.pC - m * S.invDSize;
+        right = (float)S.pC + m * S.invDSize;
     }
-    blo = max(blo, S.blo);
-    bhi = min(bhi, S.bhi);
-}
+    __device__ __forceinline__ void operator()(float fx, float fy, int& lo, int& hi) const
+    {
+        const float oc = fmaf(fx, cT, fy * sT);
+        float l = oc, h = oc;
+        if (FAN) {
+            const float qe = fmaf(fx, sT, fmaf(-fy, cT, d)), hq = hbd * qe;
+            const float a = fmaf(d, oc - rho, -hq), b = fmaf(d, oc + rho, hq);
+            l = a * fast_rcp(qe + copysignf(rho, a));
+            h = b * fast_rcp(qe - copysignf(rho, b));
+        }
+        lo = max((int)ceilf(fmaf(l, scale, left)), blo);
+        hi = min((int)fmaf(h, scale, right), bhi);  // towards 0: at least the last bin
+    }
+};
 
 // The sum of a RedJob by one wave: lane l adds in[l], in[l + 64], ... in order, then a
 // butterfly over the lanes; the order is fixed, so every caller gets the same value.
@@ -120,132 +124,364 @@ void launch_wave_sum(const RedJob& job, hipStream_t st)
 // while the compensation costs a quarter of a per-row update.
 constexpr int kRowBlock = 4;
 
-// Raw buffer view of one slice's array: loads take a wave-uniform byte offset (a row) in
-// an SGPR and a 32-bit per-lane byte offset (a column), so an address costs one integer
-// add per lane instead of a 64-bit pointer update.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t slice_rsrc(const float* base, int elems)
+// Raw buffer view of `bytes` bytes from a wave-uniform base: loads take a wave-uniform
+// byte offset in an SGPR and a 32-bit per-lane byte offset, and return 0 past the end.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float* base, int bytes)
 {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, elems * 4,
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, bytes,
                                              kBufferWord3);
 }
 
-__device__ __forceinline__ float ldb(__amdgpu_buffer_rsrc_t r, int voff, int soff)
-{
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-}
-
-// Four consecutive floats at a 4-byte aligned offset (one 16-byte load per lane).
-struct Quad {
-    float q[4];
-};
-
-// N (3 or 4) consecutive floats at a 4-byte aligned offset: one 12- or 16-byte load.
-template <int N>
-struct Win {
-    float q[N];
-};
-
-template <int N>
-__device__ __forceinline__ Win<N> ldbw(__amdgpu_buffer_rsrc_t r, int voff, int soff)
-{
-    Win<N> w;
-    if constexpr (N == 4) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w.q[k] = __uint_as_float(v[k]);
-    } else {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, voff, soff, 0);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) w.q[k] = __uint_as_float(v[k]);
-    }
-    return w;
-}
-
-__device__ __forceinline__ Quad ldb4(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+__device__ __forceinline__ float4 ldb128(__amdgpu_buffer_rsrc_t r, int voff, int soff)
 {
     const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-    return Quad{{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
-                 __uint_as_float(v[3])}};
+    return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
+                       __uint_as_float(v[3]));
 }
 
-// One ray of canonical view a0 against every image g p of the pixels p it meets, for
-// the elements g in MASK.  Rows mode walks image rows v = y with u = x inside; columns
-// mode (canonical views steeper than 45 degrees) walks v = x with u = y inside.  Each
-// image pixel g (x, y) is read from the image or its transpose at row +-v, column +-u,
-// whichever makes u the contiguous index.  The pixels [lo, hi] a ray meets in one row
-// are read as 4-pixel windows [s, s+3] (one 16-byte load per image instead of one load
-// per pixel and image); windows are clamped into [-H, H] so they never leave the row
-// (n >= 5), and pixels outside [lo, hi] or already taken by the previous window are
-// skipped.
-template <bool FAN, unsigned MASK, bool COLS>
-__device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, float cT, float sT,
-                                             const float* __restrict__ img,
-                                             const float* __restrict__ imgT, int vlo, int vhi,
-                                             KahanAcc* acc)
+// Orders this wave's LDS writes before its later reads (and reads before later writes).
+__device__ __forceinline__ void wave_lds_sync()
 {
-    const RowBounds rb = row_bounds(r, cT, sT, FAN ? S.invd : 0.0f, !COLS);
-    const int H = S.H, n = S.n, half = S.half;
-    const __amdgpu_buffer_rsrc_t RI = slice_rsrc(img + S.img_off, n * n);
-    const __amdgpu_buffer_rsrc_t RT = slice_rsrc(imgT + S.img_off, n * n);
-    // rows mode: g (u, v) of element e at [RI|RT](row +-v, col +-u); columns mode swaps
-    // the two arrays' roles
-    const __amdgpu_buffer_rsrc_t RA = COLS ? RT : RI;
-    const __amdgpu_buffer_rsrc_t RB = COLS ? RI : RT;
-    float part[8];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Wave minimum of lo and maximum of hi: prefix reductions inside each row of 16 lanes
+// (DPP row shifts; lanes with no source read the operation's identity, which lets the
+// compiler fold each shift into the min / max), then the four rows' last lanes.  The
+// two chains are interleaved so that each DPP read finds its operand already written.
+__device__ __forceinline__ void wave_range_i32(int lo, int hi, int& wlo, int& whi)
+{
+    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x111, 0xf, 0xf, false));
+    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x111, 0xf, 0xf, false));
+    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x112, 0xf, 0xf, false));
+    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x112, 0xf, 0xf, false));
+    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x114, 0xf, 0xf, false));
+    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x114, 0xf, 0xf, false));
+    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x118, 0xf, 0xf, false));
+    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x118, 0xf, 0xf, false));
+    const int a = __builtin_amdgcn_readlane(lo, 15), b = __builtin_amdgcn_readlane(lo, 31);
+    const int c = __builtin_amdgcn_readlane(lo, 47), d = __builtin_amdgcn_readlane(lo, 63);
+    const int e = __builtin_amdgcn_readlane(hi, 15), f = __builtin_amdgcn_readlane(hi, 31);
+    const int g = __builtin_amdgcn_readlane(hi, 47), h = __builtin_amdgcn_readlane(hi, 63);
+    wlo = min(min(a, b), min(c, d));
+    whi = max(max(e, f), max(g, h));
+}
+
+// ------------------------------------------------------------ orbit image ---
+//
+// The forward reads its pixels from the orbit image: for every pixel p of the walk, the
+// group's values img[g p] side by side, so that a ray's step to the next pixel is one
+// contiguous read for all the images instead of one read per image.  Rows are walk rows
+// v, columns u in [-H, H] (orb_pitch of them).  One row holds, for each u,
+//   D4: plane 0 = elements 0..3, plane 1 = elements 4..7 (orb_pitch float4 each),
+//   V4: elements 0, 2, 4, 6 (float4),   Z2: elements 0, 6 (float2).
+// Rows mode (v = y, u = x) comes first, then, for V4 and Z2, columns mode (v = x, u = y)
+// of the canonical views steeper than 45 degrees.  Rows v < 0 are not stored where an
+// element of the group maps v to -v and keeps u (all but Z2's rows mode): there the
+// values at -v are those at v with the slots exchanged (neg_xor), and the forward
+// exchanges its sums once, where the walk crosses v = 0.  The orbit image of a slice
+// takes 4 n^2 floats (Z2: 3 n^2).
+template <int GRP>
+struct Orbit {
+    static constexpr int N = group_masks(GRP).order;
+    static constexpr int kPlane = N >= 4 ? 4 : 2;  // floats of one pixel in one plane
+    // pixels of a row that a wave stages at once, and the 16-byte loads per lane it takes
+    static constexpr int kPixels = 128;
+    static constexpr int kLoads = kPixels * N / 256;
+    __host__ __device__ static constexpr int elem(int s)
+    {
+        return GRP == kGrpD4 ? s : GRP == kGrpV4 ? 2 * s : 6 * s;
+    }
+    __host__ __device__ static constexpr int slot(int e)
+    {
+        return GRP == kGrpD4 ? e : GRP == kGrpV4 ? e >> 1 : (e != 0);
+    }
+    // slot s at walk row -v is slot s ^ neg_xor at v; 0: the rows v < 0 are stored
+    __host__ __device__ static constexpr int neg_xor(bool cols)
+    {
+        return GRP == kGrpD4 ? 4 : GRP == kGrpV4 ? (cols ? 3 : 2) : (cols ? 1 : 0);
+    }
+};
+
+// Walk row v of the orbit image of S (floats from the slice's base).
+template <int GRP, bool COLS>
+__device__ __forceinline__ const float* orbit_row(const SliceDesc& S, const float* orb, int v)
+{
+    using O = Orbit<GRP>;
+    const int rec = O::N * S.orb_pitch;
+    const float* base = orb + S.orb_off;
+    if (COLS) base += (long long)(O::neg_xor(false) ? S.H + 1 : 2 * S.H + 1) * rec;
+    return base + (long long)(O::neg_xor(COLS) ? abs(v) : v + S.H) * rec;
+}
+
+// One 32 x 32 tile of the orbit image per work-group: item (slice, first stored row, first
+// column; pad = 1: columns mode).  Images whose u runs along image columns are read
+// straight, the others through an LDS transpose, so every read and write is coalesced.
+// Bound by its writes (16 n^2 bytes): one extra pass over a small array, 5-6 us at 1024^2.
+template <int GRP, bool COLS>
+__device__ __forceinline__ void orbit_tile(const SliceDesc& S, int r0, int u0,
+                                           const float* __restrict__ img,
+                                           float* __restrict__ orb, float (*tile)[32][33])
+{
+    using O = Orbit<GRP>;
+    constexpr int neg = O::neg_xor(COLS);
+    const int H = S.H, tx = (int)threadIdx.x & 31, ty = (int)threadIdx.x >> 5;
+    const float* src = img + S.img_off + (long long)S.half * S.n + S.half;
+    const int v0 = neg ? r0 : r0 - H;
+    // u is a row index of the source where the element's rotation (and the walk) swap axes
+    constexpr auto swapped = [](int e) constexpr { return ((e & 1) != 0) != COLS; };
 #pragma unroll
-    for (int e = 0; e < 8; ++e) part[e] = 0.0f;
-    int inblock = 0;
-    for (int v = vlo; v <= vhi; ++v) {
-        int lo, hi;
-        row_range(rb, (float)v, H, lo, hi);
-        const int op = (v + half) * n * 4;  // byte offset of row  v
-        const int om = (half - v) * n * 4;  // byte offset of row -v
-        const float fv = (float)v;
-        for (int s0 = lo; s0 <= hi; s0 += 4) {
-            const int s = min(s0, H - 3);
-            const int cp = (half + s) * 4;      // window [s, s+3]
-            const int cm = (half - s - 3) * 4;  // window [-(s+3), -s]
-            // rows: e0 ( x, y) A[v][u]   e1 (-y, x) B[-v][u]  e2 (-x,-y) A[-v][-u]
-            //       e3 ( y,-x) B[v][-u]  e4 ( x,-y) A[-v][u]  e5 ( y, x) B[v][u]
-            //       e6 (-x, y) A[v][-u]  e7 (-y,-x) B[-v][-u]          (A = img, B = imgT)
-            // cols: e0 A[v][u]  e1 B[v][-u]  e2 A[-v][-u]  e3 B[-v][u]
-            //       e4 A[v][-u] e5 B[v][u]   e6 A[-v][u]   e7 B[-v][-u]  (A = imgT, B = img)
-            Quad w8[8];
-            if (MASK & 0x01) w8[0] = ldb4(RA, cp, op);
-            if (MASK & 0x02) w8[1] = COLS ? ldb4(RB, cm, op) : ldb4(RB, cp, om);
-            if (MASK & 0x04) w8[2] = ldb4(RA, cm, om);
-            if (MASK & 0x08) w8[3] = COLS ? ldb4(RB, cp, om) : ldb4(RB, cm, op);
-            if (MASK & 0x10) w8[4] = COLS ? ldb4(RA, cm, op) : ldb4(RA, cp, om);
-            if (MASK & 0x20) w8[5] = ldb4(RB, cp, op);
-            if (MASK & 0x40) w8[6] = COLS ? ldb4(RA, cp, om) : ldb4(RA, cm, op);
-            if (MASK & 0x80) w8[7] = ldb4(RB, cm, om);
-            // which images read column +u (window index j) and which -u (index 3 - j)
-            constexpr unsigned PLUS = COLS ? 0x69u : 0x33u;
+    for (int s = 0; s < O::N; ++s) {
+        const int e = O::elem(s);
+        if (!swapped(e)) continue;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int u = s + j;
-                if (u < s0 || u > hi) continue;
-                const float fu = (float)u;
-                const float fx = COLS ? fv : fu, fy = COLS ? fu : fv;
-                const float dist = ray_dist(fx, fy, r.cosR, r.sinR, r.dc);
-                const float hb = FAN ? r.hbc * fan_depth_scale(fx, fy, cT, sT, S.invd) : r.hbc;
-                const float w = strip_weight(dist, hb, r);
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (MASK >> e & 1u)
-                        part[e] = fmaf(w, w8[e].q[(PLUS >> e & 1u) ? j : 3 - j], part[e]);
-            }
-        }
-        if (++inblock == kRowBlock || v == vhi) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (!(MASK >> e & 1u)) continue;
-                acc[e].add(part[e]);
-                part[e] = 0.0f;
-            }
-            inblock = 0;
+        for (int k = 0; k < 32; k += 8) {
+            const int v = v0 + tx, u = u0 - H + ty + k;
+            int x, y;
+            apply_px(e & 3, e >> 2, COLS ? v : u, COLS ? u : v, x, y);
+            if (v <= H && u <= H) tile[s >> (O::N == 8 ? 1 : 0)][ty + k][tx] = src[(long long)y * S.n + x];
         }
     }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 32; k += 8) {
+        const int v = v0 + ty + k, u = u0 - H + tx;
+        if (v > H || u > H) continue;
+        float q[O::N];
+#pragma unroll
+        for (int s = 0; s < O::N; ++s) {
+            const int e = O::elem(s);
+            if (swapped(e)) q[s] = tile[s >> (O::N == 8 ? 1 : 0)][tx][ty + k];
+            else {
+                int x, y;
+                apply_px(e & 3, e >> 2, COLS ? v : u, COLS ? u : v, x, y);
+                q[s] = src[(long long)y * S.n + x];
+            }
+        }
+        float* out = const_cast<float*>(orbit_row<GRP, COLS>(S, orb, v));
+        const int c = u + H;
+        if constexpr (O::N == 2) {
+            reinterpret_cast<float2*>(out)[c] = make_float2(q[0], q[1]);
+        } else {
+#pragma unroll
+            for (int p = 0; p < O::N / 4; ++p)
+                reinterpret_cast<float4*>(out)[p * S.orb_pitch + c] =
+                    make_float4(q[4 * p], q[4 * p + 1], q[4 * p + 2], q[4 * p + 3]);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_orbit_image(const SliceDesc* __restrict__ slices,
+                                                     const AdjItem* __restrict__ items,
+                                                     const float* __restrict__ img,
+                                                     float* __restrict__ orb)
+{
+    __shared__ float tile[4][32][33];
+    const AdjItem it = items[blockIdx.x];
+    const SliceDesc S = slices[it.slice];
+    // uniform over the work-group
+    if (S.sym == kGrpD4) orbit_tile<kGrpD4, false>(S, it.row0, it.col0, img, orb, tile);
+    else if (S.sym == kGrpV4 && !it.pad) orbit_tile<kGrpV4, false>(S, it.row0, it.col0, img, orb, tile);
+    else if (S.sym == kGrpV4) orbit_tile<kGrpV4, true>(S, it.row0, it.col0, img, orb, tile);
+    else if (!it.pad) orbit_tile<kGrpZ2, false>(S, it.row0, it.col0, img, orb, tile);
+    else orbit_tile<kGrpZ2, true>(S, it.row0, it.col0, img, orb, tile);
+}
+
+void launch_orbit_image(int nitems, const SliceDesc* desc, const AdjItem* items, const float* img,
+                        float* orb, hipStream_t st)
+{
+    if (nitems > 0)
+        hipLaunchKernelGGL(k_orbit_image, dim3(nitems), dim3(256), 0, st, desc, items, img, orb);
+}
+
+// ------------------------------------------------------------------ ray walk ---
+
+// One canonical ray per lane against the group's images of the pixels it meets, over the
+// walk rows [vlo, vhi].  Rows mode walks v = y with u = x inside, columns mode (canonical
+// views steeper than 45 degrees) v = x with u = y.  The wave stages the orbit-image row
+// that its 64 neighbouring rays cross in LDS (one 16-byte load per lane brings 64 16-byte
+// units; the next row is loaded while this one is summed), and every lane then reads its
+// own pixels [lo, hi] there.  Read straight from memory, a row took eight 16-byte loads
+// per lane (one per image) and the vector-memory unit, at about 16 cycles a load, bounded
+// the kernel; now three loads serve the wave's row.
+// The staged columns start at the first pixel of an end lane (the rays of a wave are
+// ordered).  Waves for which that does not hold over all of their rows, or whose rays
+// cross more than kPixels pixels of a row (coarse detectors), form the true range at each
+// row and stage it piece by piece, in increasing order.
+template <bool FAN, int GRP, bool COLS>
+__device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, float cT, float sT,
+                                             const float* __restrict__ orb, int vlo, int vhi,
+                                             KahanAcc* acc, float4* __restrict__ st)
+{
+    using O = Orbit<GRP>;
+    constexpr int N = O::N, CH = O::kPixels, neg = O::neg_xor(COLS);
+    const int lane = (int)threadIdx.x & 63, H = S.H;
+    if (vlo > vhi) return;  // uniform over the wave
+    const float fH = (float)H, qs = sT * S.invd, qc = cT * S.invd;
+    // The pixels of walk row v that the lane's ray meets are u in [lo, hi] (bounds as in
+    // row_range) between two lines in v, (ua + v ub) and (la + v lb).
+    const RowBounds rb = row_bounds(r, cT, sT, FAN ? S.invd : 0.0f, !COLS);
+    const float ua = rb.U0 * rb.iu, ub = -rb.U1 * rb.iu, la = rb.L0 * rb.il, lb = -rb.L1 * rb.il;
+    // Regular waves: at the first and the last row, and hence (all are linear in v) at every
+    // row between, each lane's lines keep their order, no lane starts more than a pixel
+    // before the end lane `edge` that starts first at both, and all end within the staged
+    // pixels.  Others form the wave's range row by row.
+    const float fa = (float)vlo, fb = (float)vhi;
+    const float ea = fmaf(fa, ub, ua), eb = fmaf(fb, ub, ua);
+    const float ga = fmaf(fa, lb, la), gb = fmaf(fb, lb, la);
+    const bool left = ga + gb <= ea + eb;  // the second line is the left one
+    const float La = left ? ga : ea, Lb = left ? gb : eb, Ra = left ? ea : ga, Rb = left ? eb : gb;
+    auto lane_f = [](float x, int l) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+    };
+    const int edge = lane_f(La, 0) + lane_f(Lb, 0) <= lane_f(La, 63) + lane_f(Lb, 63) ? 0 : 63;
+    const float sa = lane_f(La, edge), sb = lane_f(Lb, edge);
+    // (the image's width bounds the pixels, too)
+    auto within = [&](float px) { return (Ra - sa < px && Rb - sb < px) || 2.0f * fH < px; };
+    const bool regular = __all(La <= Ra && Lb <= Rb && La >= sa - 0.9f && Lb >= sb - 0.9f &&
+                               within((float)(CH - 3)));
+    const bool wide = !(regular && __all(within(61.0f)));
+    const float l0 = left ? la : ua, l1 = left ? lb : ub, r0 = left ? ua : la, r1 = left ? ub : lb;
+    auto row_setup = [&](float fv, float& lo, float& hi, int& ilo, int& c0) {
+        const float e = fmaf(fv, l1, l0), f = fmaf(fv, r1, r0);
+        if (regular) {
+            lo = fmaxf(ceilf(e), -fH);
+            hi = fminf(f, fH);
+        } else {
+            lo = fmaxf(ceilf(fminf(e, f)), -fH);
+            hi = fminf(fmaxf(e, f), fH);
+        }
+        ilo = (int)lo;
+        // one pixel of slack; a row that no lane meets takes any column, so that its load
+        // stays inside
+        c0 = min(max(__builtin_amdgcn_readlane(ilo, edge) - 1, -H), H);
+    };
+    // 16-byte unit 64 j + lane of a staged piece: pixel unit % CH of plane unit / CH; units
+    // past a narrow wave's pixels are not read (offsets beyond the row load as 0)
+    int voff[O::kLoads];
+#pragma unroll
+    for (int j = 0; j < O::kLoads; ++j) {
+        const int unit = 64 * j + lane;
+        voff[j] = N == 8 && unit >= CH ? (S.orb_pitch + unit - CH) * 16 : unit * 16;
+        if (N >= 4 && (j & 1) && !wide) voff[j] = 0x7ffffff0;
+    }
+    auto load = [&](const float* row, int c0, float4* g) {
+        const __amdgpu_buffer_rsrc_t R = row_rsrc(row, N * S.orb_pitch * 4);
+#pragma unroll
+        for (int j = 0; j < O::kLoads; ++j) g[j] = ldb128(R, voff[j], (c0 + H) * O::kPlane * 4);
+    };
+    auto stage = [&](const float4* g) {
+        wave_lds_sync();  // the previous piece's reads are done
+#pragma unroll
+        for (int j = 0; j < O::kLoads; ++j) st[64 * j + lane] = g[j];
+        wave_lds_sync();  // staged values visible to every lane
+    };
+    auto pixel = [&](int at, float* q) {
+        if constexpr (N == 2) {
+            const float2 a = reinterpret_cast<const float2*>(st)[at];
+            q[0] = a.x;
+            q[1] = a.y;
+        } else {
+#pragma unroll
+            for (int p = 0; p < N / 4; ++p) {
+                const float4 a = st[p * CH + at];
+                q[4 * p] = a.x;
+                q[4 * p + 1] = a.y;
+                q[4 * p + 2] = a.z;
+                q[4 * p + 3] = a.w;
+            }
+        }
+    };
+    float part[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) part[s] = 0.0f;
+    // the pixels [lo, hi] of walk row fv from the staged pixel of lo on
+    auto sum = [&](float fv, float lo, float hi, int at) {
+        const float rowd = COLS ? 0.0f : fmaf(fv, r.sinR, -r.dc);
+        const float rowq = FAN && !COLS ? fmaf(-fv, qc, 1.0f) : 0.0f;
+        for (float fu = lo; fu <= hi; fu += 1.0f, ++at) {
+            float q[N];
+            pixel(at, q);
+            // ray_dist and fan_depth_scale at (x, y) = (fu, fv), columns mode (fv, fu)
+            const float dist = COLS ? fmaf(fv, r.cosR, fmaf(fu, r.sinR, -r.dc))
+                                    : fmaf(fu, r.cosR, rowd);
+            const float qd = COLS ? fmaf(fv, qs, fmaf(-fu, qc, 1.0f)) : fmaf(fu, qs, rowq);
+            const float w = strip_area(dist, FAN ? r.hbc * qd : r.hbc, r);
+#pragma unroll
+            for (int s = 0; s < N; ++s) part[s] = fmaf(w, q[s], part[s]);
+        }
+    };
+    // rows v < 0 first, then v >= 0: the sums are held by the slots of the current sign
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        const int va = half ? max(vlo, 0) : vlo, vb = half ? vhi : min(vhi, -1);
+        if (va <= vb) {
+            const float* row = orbit_row<GRP, COLS>(S, orb, va);
+            const long long step = neg && !half ? -(long long)N * S.orb_pitch : N * S.orb_pitch;
+            float fv = (float)va, lo, hi;
+            int ilo, c0;
+            float4 g[O::kLoads];
+            row_setup(fv, lo, hi, ilo, c0);
+            load(row, c0, g);
+#pragma unroll 1
+            for (int v = va; v <= vb;) {
+                const int vend = min(v + kRowBlock - 1, vb);
+#pragma unroll 1
+                for (; v <= vend; ++v) {
+                    stage(g);
+                    const float pv = fv, plo = lo, phi = hi;
+                    const int pilo = ilo;
+                    const float* prow = row;
+                    int p = c0, last = c0;
+                    if (v < vb) {
+                        fv += 1.0f;
+                        row += step;
+                        row_setup(fv, lo, hi, ilo, c0);
+                        load(row, c0, g);
+                    }
+                    float first = plo;
+                    if (!regular) {
+                        const int ihi = (int)phi;  // towards 0: at least the last pixel
+                        wave_range_i32(plo <= phi ? pilo : INT_MAX, plo <= phi ? ihi : INT_MIN, p,
+                                       last);
+                        if (p > last) continue;  // no lane meets this row
+                        float4 h[O::kLoads];
+                        load(prow, p, h);
+                        stage(h);
+                        first = (float)max(pilo, p);
+                    }
+                    int at = max(pilo, p) - p;
+                    for (;;) {
+                        sum(pv, first, regular ? phi : fminf(phi, (float)(p + CH - 1)), at);
+                        p += CH;
+                        if (regular || p > last) break;  // wave-uniform
+                        float4 h[O::kLoads];
+                        load(prow, p, h);
+                        stage(h);
+                        first = (float)max(pilo, p);
+                        at = max(pilo, p) - p;
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < N; ++s) {
+                    acc[s].add(part[s]);
+                    part[s] = 0.0f;
+                }
+            }
+        }
+        if (neg && half == 0)
+#pragma unroll
+            for (int s = 0; s < N; ++s)
+                if (s < (s ^ neg)) {
+                    const KahanAcc t = acc[s];
+                    acc[s] = acc[s ^ neg];
+                    acc[s ^ neg] = t;
+                }
+    }
+#pragma unroll
+    for (int s = 0; s < N; ++s) acc[s].s *= S.inver;
 }
 
 // Kernel argument of the forward launches: empty, or (BHC) the beam-hardening ray pass
@@ -312,27 +548,27 @@ __device__ __forceinline__ double fwd_sym_store(const SliceDesc& S, const FwdIte
     }
 }
 
-// One canonical ray run over the images in MASK (the group, or its rotations on a
-// mirror view).  The image rows are cut into nsplit * SEG segments: this work-group
-// walks segments split * SEG + wave.  nsplit == 1 writes the sinogram; otherwise the
-// work-group's sums go to part[e * 64 + lane] for k_forward_sym_combine.
-template <bool FAN, unsigned MASK, bool COLS, int SEG, bool BHC>
+// One canonical ray run over the group's images.  The image rows are cut into
+// nsplit * SEG segments: this work-group walks segments split * SEG + wave.  nsplit == 1
+// writes the sinogram; otherwise the work-group's sums go to part[e * 64 + lane] for
+// k_forward_sym_combine.  Lanes past the detector's ends repeat the nearest ray and are
+// not stored; on a mirror view the rotations alone are.
+template <bool FAN, bool COLS, int SEG, int GRP, bool BHC>
 __device__ __forceinline__ void fwd_sym_run(const SliceDesc& S, const FwdItem& it, float cT,
-                                            float sT, int a0, const Ray* __restrict__ rays,
-                                            const float* __restrict__ img,
-                                            const float* __restrict__ imgT,
+                                            float sT, int a0, unsigned mask,
+                                            const Ray* __restrict__ rays,
+                                            const float* __restrict__ orb,
                                             float* __restrict__ sino, float (*red)[8][64],
                                             int split, int nsplit, float* __restrict__ part,
-                                            float (*tb)[64])
+                                            float (*tb)[64], float4* __restrict__ stage)
 {
+    using O = Orbit<GRP>;
     // the wave index is uniform over the wave: the row loop then runs on scalar registers
     const int lane = (int)threadIdx.x & 63;
     const int seg = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int b = it.bin0 + lane;
-    const int bmax = S.fold ? S.pC : S.bhi;
-    const bool active = b >= S.blo && b <= bmax;
-    KahanAcc acc[8];
-    if (active) {
+    const int b = min(max(it.bin0 + lane, S.blo), S.fold ? S.pC : S.bhi);
+    KahanAcc acc[O::N];
+    {
         Ray r;
         if (FAN) r = rays[S.ray_off + (long long)it.view * S.W + b];
         else {
@@ -341,21 +577,22 @@ __device__ __forceinline__ void fwd_sym_run(const SliceDesc& S, const FwdItem& i
         }
         const int nrow = 2 * S.H + 1, nseg = SEG * nsplit, per = (nrow + nseg - 1) / nseg;
         const int vlo = -S.H + (split * SEG + seg) * per, vhi = min(S.H, vlo + per - 1);
-        fwd_sym_rows<FAN, MASK, COLS>(S, r, cT, sT, img, imgT, vlo, vhi, acc);
+        fwd_sym_rows<FAN, GRP, COLS>(S, r, cT, sT, orb, vlo, vhi, acc,
+                                     stage + seg * O::kLoads * 64);
     }
     if (SEG > 1) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (MASK >> e & 1u) red[seg][e][lane] = acc[e].s;
+        for (int s = 0; s < O::N; ++s) red[seg][O::elem(s)][lane] = acc[s].s;
         __syncthreads();
     }
     // wave w finalises the images e = w (mod SEG): the sum of the waves' partials in wave
     // order.  BHC: the sums wait in tb[e][lane] for the kernel's one fused store loop (a
     // single inlined copy of the spectrum sums)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        if (!(MASK >> e & 1u) || (SEG > 1 && e % SEG != seg)) continue;
-        float t = acc[e].s;
+    for (int s = 0; s < O::N; ++s) {
+        const int e = O::elem(s);
+        if (!(mask >> e & 1u) || (SEG > 1 && e % SEG != seg)) continue;
+        float t = acc[s].s;
         if (SEG > 1) {
             t = red[0][e][lane];
 #pragma unroll
@@ -367,38 +604,11 @@ __device__ __forceinline__ void fwd_sym_run(const SliceDesc& S, const FwdItem& i
     }
 }
 
-template <bool FAN, int SEG, int GRP, bool BHC>
-__device__ __forceinline__ void fwd_sym_group(const SliceDesc& S, const FwdItem& it, float cT,
-                                              float sT, int a0, bool mirror,
-                                              const Ray* __restrict__ rays,
-                                              const float* __restrict__ img,
-                                              const float* __restrict__ imgT,
-                                              float* __restrict__ sino, float (*red)[8][64],
-                                              int split, int nsplit, float* __restrict__ part,
-                                              float (*tb)[64])
-{
-    // D4's canonical views lie in [0, 45] degrees and always walk rows; V4's reach 90 and
-    // Z2's 180 degrees, and the steep ones walk columns
-    constexpr GroupMasks GM = group_masks(GRP);
-    const bool cols = GRP != kGrpD4 && fabsf(cT) < fabsf(sT);
-#define CTPRJ_RUN(MASK, COLS)                                                                 \
-    fwd_sym_run<FAN, MASK, COLS, SEG, BHC>(S, it, cT, sT, a0, rays, img, imgT, sino, red, split, \
-                                           nsplit, part, tb)
-    if (GRP != kGrpD4 && cols) {
-        if (mirror) CTPRJ_RUN(GM.rot, GRP != kGrpD4);
-        else CTPRJ_RUN(GM.all, GRP != kGrpD4);
-    } else {
-        if (mirror) CTPRJ_RUN(GM.rot, false);
-        else CTPRJ_RUN(GM.all, false);
-    }
-#undef CTPRJ_RUN
-}
-
 // Work-group -> (split, item): the first nitems work-groups take split 0 of every item,
 // the next nitems split 1, and so on.
 __device__ __forceinline__ void split_item(int nitems, int& split, int& idx)
 {
-    split = (int)blockIdx.x / nitems;
+    split = __builtin_amdgcn_readfirstlane((int)blockIdx.x / nitems);
     idx = (int)blockIdx.x - split * nitems;
 }
 
@@ -412,13 +622,13 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
                                                           const FwdItem* __restrict__ items,
                                                           const float4* __restrict__ views,
                                                           const Ray* __restrict__ rays,
-                                                          const float* __restrict__ img,
-                                                          const float* __restrict__ imgT,
+                                                          const float* __restrict__ orb,
                                                           float* __restrict__ sino, int nitems,
                                                           int nsplit, float* __restrict__ part,
                                                           const FwdBhc<BHC> B)
 {
-    __shared__ float red[SEG][8][64];
+    __shared__ float red[SEG > 1 ? SEG : 1][8][64];
+    __shared__ float4 stage[SEG * Orbit<GRP>::kLoads * 64 + 1];  // + 1: read past a row's end, unused
     int split, idx;
     split_item(nitems, split, idx);
     const FwdItem it = items[idx];
@@ -430,22 +640,29 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
     const SliceDesc S = slices[it.slice];
     const float4 T = views[S.view_off + it.view];
     const int a0 = __float_as_int(T.z);
-    const bool mirror = a0 == 0 || group_masks(GRP).q * a0 == S.P;
+    constexpr GroupMasks GM = group_masks(GRP);
+    const unsigned mask = (a0 == 0 || GM.q * a0 == S.P) ? GM.rot : GM.all;
     float* mine = part ? part + (long long)blockIdx.x * 512 : nullptr;
-    // (fan, mirror, walk) are uniform over the work-group: the barrier inside is reached
-    // by all of its waves
     __shared__ float tb[BHC ? 8 : 1][64];  // BHC: each lane's final sums, by image
-    if (S.fan)
-        fwd_sym_group<true, SEG, GRP, BHC>(S, it, T.x, T.y, a0, mirror, rays, img, imgT, sino,
-                                           red, split, nsplit, mine, tb);
-    else
-        fwd_sym_group<false, SEG, GRP, BHC>(S, it, T.x, T.y, a0, mirror, rays, img, imgT, sino,
-                                            red, split, nsplit, mine, tb);
+    // D4's canonical views lie in [0, 45] degrees and always walk rows; V4's reach 90 and
+    // Z2's 180 degrees, and the steep ones walk columns.  (fan, walk) are uniform over the
+    // work-group: the barrier inside is reached by all of its waves
+    const bool cols = GRP != kGrpD4 && fabsf(T.x) < fabsf(T.y);
+#define CTPRJ_RUN(FAN, COLS)                                                                      \
+    fwd_sym_run<FAN, COLS, SEG, GRP, BHC>(S, it, T.x, T.y, a0, mask, rays, orb, sino, red, split, \
+                                          nsplit, mine, tb, stage)
+    if (GRP != kGrpD4 && cols) {
+        if (S.fan) CTPRJ_RUN(true, GRP != kGrpD4);
+        else CTPRJ_RUN(false, GRP != kGrpD4);
+    } else {
+        if (S.fan) CTPRJ_RUN(true, false);
+        else CTPRJ_RUN(false, false);
+    }
+#undef CTPRJ_RUN
     if constexpr (BHC) {
         if (!mine) {  // uniform: the fused store of this lane's images, then the NLL partial
             const int lane = (int)threadIdx.x & 63;
             const int seg = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-            const unsigned mask = mirror ? group_masks(GRP).rot : group_masks(GRP).all;
             double f = 0.0;
             // each lane reads back only its own entries: no barrier
 #pragma unroll 1
@@ -494,433 +711,235 @@ __global__ __launch_bounds__(512) void k_forward_sym_combine(const SliceDesc* __
 }
 
 // ------------------------------------------------------------------ adjoint ---
-
-// Orbit gather for one canonical view and one group element g' = (k2, m2): the weight
-// W(a0, b, g'^-1 q0) is shared by the orbit pixels h q0 for h in HMASK, which read view
-// h g' (a0, b).  On a mirror view rotations g' pair with rotation h and reflections
-// with reflection h, so that h g' is always a rotation: every entry then takes the
-// forward's key (a0, b, R^-k q) and the two directions evaluate the same float weight.
-// `tab` holds the view-row entries of (a0, g') for the eight h (wave-uniform).  The
-// bins [blo, bhi] of the pixel are read as 4-bin windows (one 16-byte load per image),
-// clamped into [0, W - 4] so they stay inside the row, reflected rows at 2pC - b.
-template <bool FAN, bool FBP, unsigned HMASK, int WIN>
-__device__ __forceinline__ void adj_sym_elem(const SliceDesc& S, const Ray* __restrict__ rview,
-                                             __amdgpu_buffer_rsrc_t RS, __amdgpu_buffer_rsrc_t RZ,
-                                             const int* __restrict__ tab, float cT, float sT,
-                                             int k2, int m2, int x0, int y0, float* vpart)
-{
-    // p = g'^-1 q0; (R^k M)^-1 = R^k M, (R^k)^-1 = R^-k
-    int px, py;
-    if (m2) apply_px(k2, 1, x0, y0, px, py);
-    else apply_px(4 - k2, 0, x0, y0, px, py);
-    const float fx = (float)px, fy = (float)py;
-    int blo, bhi;
-    pixel_bins<FAN>(S, rview, fx, fy, cT, sT, blo, bhi);
-    if (blo > bhi) return;
-    __amdgpu_buffer_rsrc_t rs[8];
-    int soff[8];
-    bool flip[8];
-#pragma unroll
-    for (int h = 0; h < 8; ++h) {
-        if (!(HMASK >> h & 1u)) continue;
-        const int t = tab[h];
-        const bool none = (t & kRowNone) != 0;
-        rs[h] = none ? RZ : RS;
-        soff[h] = none ? 0 : (t & ~(kRowFlip | kRowNone));
-        flip[h] = (t & kRowFlip) != 0;
-    }
-    const float qd = FAN ? fan_depth_scale(fx, fy, cT, sT, S.invd) : 1.0f;
-    float part[8];
-#pragma unroll
-    for (int h = 0; h < 8; ++h) part[h] = 0.0f;
-    const int two_pc = 2 * S.pC, smax = S.W - WIN;
-    for (int s0 = blo; s0 <= bhi; s0 += WIN) {
-        const int s = min(s0, smax);
-        // windows [s, s+WIN-1] and the reflected [2pC-s-WIN+1, 2pC-s]
-        const int ob = s * 4, of = (two_pc - s - (WIN - 1)) * 4;
-        Win<WIN> q[8];
-#pragma unroll
-        for (int h = 0; h < 8; ++h)
-            if (HMASK >> h & 1u) q[h] = ldbw<WIN>(rs[h], flip[h] ? of : ob, soff[h]);
-#pragma unroll
-        for (int j = 0; j < WIN; ++j) {
-            const int b = s + j;
-            if (b < s0 || b > bhi) continue;
-            Ray r;
-            if (FAN) r = rview[b];
-            else {
-                r = rview[0];
-                r.dc = (float)(b - S.pC) * S.dSize;
-            }
-            const float dist = ray_dist(fx, fy, r.cosR, r.sinR, r.dc);
-            const float w = strip_weight(dist, FAN ? r.hbc * qd : r.hbc, r);
-#pragma unroll
-            for (int h = 0; h < 8; ++h)
-                if (HMASK >> h & 1u)
-                    part[h] = fmaf(w, flip[h] ? q[h].q[WIN - 1 - j] : q[h].q[j], part[h]);
-        }
-    }
-    // FBP fan weight d^2/qe^2 (prj/cpuPrj.c:258); qe of g'^-1 q0 at a0 is the depth of
-    // every orbit pixel at its own view
-    const float fw = (FBP && FAN) ? 1.0f / (qd * qd) : 1.0f;
-#pragma unroll
-    for (int h = 0; h < 8; ++h)
-        if (HMASK >> h & 1u) vpart[h] += (FBP && FAN) ? part[h] * fw : part[h];
-}
-
-// One fan-beam ray record through a buffer view of the slice's ray table (byte offsets:
-// voff the bin, soff the view row).
-__device__ __forceinline__ Ray ldray(__amdgpu_buffer_rsrc_t r, int voff, int soff)
-{
-    const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-    const auto b = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16, soff, 0);
-    Ray x;
-    x.cosR = __uint_as_float(a[0]);
-    x.sinR = __uint_as_float(a[1]);
-    x.dc = __uint_as_float(a[2]);
-    x.hbc = __uint_as_float(a[3]);
-    x.h = __uint_as_float(b[0]);
-    x.b1 = __uint_as_float(b[1]);
-    x.s = __uint_as_float(b[2]);
-    x.k = __uint_as_float(b[3]);
-    return x;
-}
-
-// The same gather for a canonical view off the mirror lines and a compile-time element
-// g' = E2: the reflection of every view row is fixed (elem_flip), so windows and bins are
-// indexed without selects.  Sums go straight into the view's partials; views beyond np
-// read the zero row (a wave-uniform choice of buffer), which adds exact zeros.  Fan beam:
-// the rays of a window's first three bins are loaded together before the image windows
-// (a pixel meets at most three bins when the detector pitch is at least the pixel's;
-// the fourth is loaded where needed), RR being the slice's ray table and rrow the
-// view's row.
-template <bool FAN, bool FBP, unsigned HMASK, int E2, bool FOLD, int WIN>
-__device__ __forceinline__ void adj_sym_elem_ct(const SliceDesc& S, const Ray* __restrict__ rview,
-                                                __amdgpu_buffer_rsrc_t RS, __amdgpu_buffer_rsrc_t RZ,
-                                                __amdgpu_buffer_rsrc_t RR, int rrow,
-                                                const int* __restrict__ tab, float cT, float sT,
-                                                int x0, int y0, float* vpart)
-{
-    constexpr int K2 = E2 & 3, M2 = E2 >> 2;
-    int px, py;
-    if (M2) apply_px(K2, 1, x0, y0, px, py);
-    else apply_px(4 - K2, 0, x0, y0, px, py);
-    const float fx = (float)px, fy = (float)py;
-    int blo, bhi;
-    pixel_bins<FAN>(S, rview, fx, fy, cT, sT, blo, bhi);
-    if (blo > bhi) return;
-    // rows of views beyond np read the zero row (wave-uniform resource selects)
-    __amdgpu_buffer_rsrc_t rs[8];
-    int soff[8];
-#pragma unroll
-    for (int h = 0; h < 8; ++h) {
-        if (!(HMASK >> h & 1u)) continue;
-        const int t = tab[h];
-        const bool none = (t & kRowNone) != 0;
-        rs[h] = none ? RZ : RS;
-        soff[h] = none ? 0 : (t & ~(kRowFlip | kRowNone));
-    }
-    const float qd = FAN ? fan_depth_scale(fx, fy, cT, sT, S.invd) : 1.0f;
-    // FBP fan weight d^2/qe^2 (prj/cpuPrj.c:258), folded into each weight
-    const float fw = (FBP && FAN) ? 1.0f / (qd * qd) : 1.0f;
-    const int two_pc = 2 * S.pC, smax = S.W - WIN;
-    for (int s0 = blo; s0 <= bhi; s0 += WIN) {
-        const int s = min(s0, smax);
-        // windows [s, s+WIN-1] and the reflected [2pC-s-WIN+1, 2pC-s]
-        const int ob = s * 4, of = (two_pc - s - (WIN - 1)) * 4;
-        Ray rq[3];
-        if (FAN) {
-#pragma unroll
-            for (int j = 0; j < 3; ++j) rq[j] = ldray(RR, (s + j) * (int)sizeof(Ray), rrow);
-        }
-        Win<WIN> q[8];
-#pragma unroll
-        for (int h = 0; h < 8; ++h)
-            if (HMASK >> h & 1u) q[h] = ldbw<WIN>(rs[h], elem_flip(h, E2, FOLD) ? of : ob, soff[h]);
-#pragma unroll
-        for (int j = 0; j < WIN; ++j) {
-            const int b = s + j;
-            Ray r;
-            if (FAN) r = j < 3 ? rq[j] : ldray(RR, b * (int)sizeof(Ray), rrow);
-            else {
-                r = rview[0];
-                r.dc = (float)(b - S.pC) * S.dSize;
-            }
-            const float dist = ray_dist(fx, fy, r.cosR, r.sinR, r.dc);
-            float w = strip_weight(dist, FAN ? r.hbc * qd : r.hbc, r);
-            if (FBP && FAN) w *= fw;
-            // bins of the window outside [s0, bhi] (taken by the previous window, or past
-            // the pixel's candidates) add an exact zero
-            w = (b >= s0 && b <= bhi) ? w : 0.0f;
-#pragma unroll
-            for (int h = 0; h < 8; ++h)
-                if (HMASK >> h & 1u)
-                    vpart[h] = fmaf(w, q[h].q[elem_flip(h, E2, FOLD) ? WIN - 1 - j : j], vpart[h]);
-        }
-    }
-}
-
-// ------------------------------------------------- LDS-staged adjoint gather ---
 //
-// The direct gather above has every lane load its own 3- or 4-bin windows of the eight
-// sinogram rows and (fan beam) three 32-byte ray records per window, so neighbouring
-// lanes fetch the same bins again through the vector-memory pipeline, the kernel's
-// busiest unit.  The staged gather lets the wave fetch each (canonical view, element g')
-// once: the bins [L0, L0 + kStageBins) that any of its 64 orbit pixels can read (the
-// wave minimum of the pixels' first candidate bins, up to the maximum of their last
-// candidate plus the window width), one load per sinogram row and one for the ray
-// records, into a wave-private LDS area; the pixels then read their windows from LDS.
-// Every pixel still forms the same weights from the same ray records and sums its bins
-// in the same order, so the image is bit-identical.  A wave whose range exceeds
-// kStageBins bins (fine detector pitch) stages it in chunks of kStageBins bins.
+// The adjoint reads its bins from the orbit sinogram: for every canonical view a0 and bin
+// b, the values of the group's rays g (a0, b) side by side (element e in slot e; a half-turn
+// scan's folded views at their reflected bin; 0 for views beyond np, bins that carry no
+// ray, and, on a mirror view, the reflections).  Orbit pixel h q0 under group element g'
+// reads ray h g' (a0, b), so for a fixed g' the eight pixels of an orbit read the same
+// entry with its slots permuted by the product h g', known at compile time.  One row
+// holds, for each bin, D4: plane 0 = elements 0..3, plane 1 = elements 4..7 (os_pitch
+// float4 each), V4: elements 0, 2, 4, 6 (float4), Z2: elements 0, 6 (float2).
+
+// Element product h g' = (k1, m1) (k2, m2), R^k M^m each.
+__host__ __device__ constexpr int elem_mul(int h, int e2)
+{
+    const int k1 = h & 3, m1 = h >> 2, k2 = e2 & 3, m2 = e2 >> 2;
+    return ((k1 + (m1 ? -k2 : k2)) & 3) + 4 * (m1 ^ m2);
+}
+
+// Rows of the orbit sinogram: item (slice, canonical view), 256 bins per work-group.
+// tab: 8 entries per canonical view, the sinogram row of element e (byte offset | kRowFlip,
+// or kRowNone).  The values are stored divided by the effectiveRate.
+template <int GRP>
+__device__ __forceinline__ void orbit_sino_bin(const SliceDesc& S, int i, int b,
+                                               const int* __restrict__ tab,
+                                               const float* __restrict__ sino,
+                                               float* __restrict__ os)
+{
+    using O = Orbit<GRP>;
+    const int* t = tab + S.tab_off + (long long)i * 8;
+    const float* in = sino + S.sino_off;
+    const bool ray = b >= S.blo && b <= S.bhi;
+    float q[O::N];
+#pragma unroll
+    for (int s = 0; s < O::N; ++s) {
+        const int r = t[O::elem(s)];
+        q[s] = 0.0f;
+        if (ray && !(r & kRowNone))
+            q[s] = S.inver * in[((r & ~(kRowFlip | kRowNone)) >> 2) + ((r & kRowFlip) ? 2 * S.pC - b : b)];
+    }
+    float* out = os + S.os_off + (long long)i * (O::N * S.os_pitch);
+    if constexpr (O::N == 2) {
+        reinterpret_cast<float2*>(out)[b] = make_float2(q[0], q[1]);
+    } else {
+#pragma unroll
+        for (int p = 0; p < O::N / 4; ++p)
+            reinterpret_cast<float4*>(out)[p * S.os_pitch + b] =
+                make_float4(q[4 * p], q[4 * p + 1], q[4 * p + 2], q[4 * p + 3]);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_orbit_sino(const SliceDesc* __restrict__ slices,
+                                                    const int2* __restrict__ items,
+                                                    const int* __restrict__ tab,
+                                                    const float* __restrict__ sino,
+                                                    float* __restrict__ os)
+{
+    const int2 it = items[blockIdx.x];
+    const SliceDesc S = slices[it.x];
+    const int b = (int)(blockIdx.y * 256 + threadIdx.x);
+    if (b >= S.W) return;
+    if (S.sym == kGrpD4) orbit_sino_bin<kGrpD4>(S, it.y, b, tab, sino, os);
+    else if (S.sym == kGrpV4) orbit_sino_bin<kGrpV4>(S, it.y, b, tab, sino, os);
+    else orbit_sino_bin<kGrpZ2>(S, it.y, b, tab, sino, os);
+}
+
+void launch_orbit_sino(int nitems, int max_W, const SliceDesc* desc, const int2* items,
+                       const int* tab, const float* sino, float* os, hipStream_t st)
+{
+    if (nitems > 0)
+        hipLaunchKernelGGL(k_orbit_sino, dim3(nitems, (max_W + 255) / 256), dim3(256), 0, st, desc,
+                           items, tab, sino, os);
+}
+
+// Bins a wave stages at once per (canonical view, element): every pixel of an 8 x 8 tile
+// reads bins within about 11 pixels' shadow of each other.
 constexpr int kStageBins = 32;
 
+// One wave's LDS area, addressed by one offset 16 k for bin k: its orbit values at val[k]
+// (and val[kStageBins + k], D4's plane 1), and (fan beam) its ray record at ray[k] and
+// ray[kStageBins + k].
 struct AdjStage {
-    float4 ray[2 * kStageBins];  // fan beam: bin k's record at ray[2k], ray[2k+1]
-    // bin k's value in orbit image h's row at val[k][h]; the 48-byte stride spreads a
-    // staging store's lanes (bins 4 q + j of rows h) over the LDS banks
-    float val[kStageBins][12];
+    float4 val[64];
+    float4 ray[64];
 };
 
-// Byte offset past the end of every slice's sinogram buffer (whose size is below 2^31
-// bytes): a 16-byte raw buffer load there is out of range in every dword and reads 0.
-constexpr int kStageNoRow = 0x7ffffff0;
-
-// Wave minimum of lo and maximum of hi: prefix reductions inside each row of 16 lanes
-// (DPP row shifts; lanes with no source read the operation's identity, which lets the
-// compiler fold each shift into the min / max), then the four rows' last lanes.  The
-// two chains are interleaved so that each DPP read finds its operand already written.
-__device__ __forceinline__ void wave_range_i32(int lo, int hi, int& wlo, int& whi)
-{
-    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x111, 0xf, 0xf, false));
-    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x111, 0xf, 0xf, false));
-    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x112, 0xf, 0xf, false));
-    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x112, 0xf, 0xf, false));
-    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x114, 0xf, 0xf, false));
-    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x114, 0xf, 0xf, false));
-    lo = min(lo, __builtin_amdgcn_update_dpp(INT_MAX, lo, 0x118, 0xf, 0xf, false));
-    hi = max(hi, __builtin_amdgcn_update_dpp(INT_MIN, hi, 0x118, 0xf, 0xf, false));
-    const int a = __builtin_amdgcn_readlane(lo, 15), b = __builtin_amdgcn_readlane(lo, 31);
-    const int c = __builtin_amdgcn_readlane(lo, 47), d = __builtin_amdgcn_readlane(lo, 63);
-    const int e = __builtin_amdgcn_readlane(hi, 15), f = __builtin_amdgcn_readlane(hi, 31);
-    const int g = __builtin_amdgcn_readlane(hi, 47), h = __builtin_amdgcn_readlane(hi, 63);
-    wlo = min(min(a, b), min(c, d));
-    whi = max(max(e, f), max(g, h));
-}
-
-// Orders this wave's LDS writes before its later reads (and reads before later writes).
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// The gather of adj_sym_elem_ct through the wave's LDS area.  Every lane of the wave
-// takes part (the staging loads are the wave's); lanes with valid == false or an empty
-// candidate range add nothing.
-// One chunk of adj_sym_elem_lds: bins [L0, L0 + kStageBins) staged by the wave, then this
-// lane's candidates blo..bhi inside the chunk summed.  Every lane of the wave takes part.
-template <bool FAN, bool FBP, unsigned HMASK>
-__device__ __forceinline__ void adj_sym_chunk(const SliceDesc& S, const Ray* __restrict__ rview,
-                                              __amdgpu_buffer_rsrc_t RS, __amdgpu_buffer_rsrc_t RR,
-                                              int rrow, int e2, int tl, float cT, float sT,
-                                              float fx, float fy, int blo, int bhi, int L0,
-                                              float* vpart, AdjStage* __restrict__ st)
-{
-    const int lane = (int)threadIdx.x & 63;
-    // lane 8 ql + hl fetches bins L0 + 4 ql .. L0 + 4 ql + 3 of orbit image hl's row with
-    // one 16-byte load, so one wave load brings the eight rows' kStageBins bins.  Reflected
-    // rows read the reversed block at 2pC - b; its offsets may fall outside the row (into
-    // a neighbouring row, or below the array, which reads 0) only for bins beyond the
-    // detector or the pixels' candidates, whose weights are exact zeros.  Rows of views
-    // beyond np, and images outside HMASK, give 0.
-    const int hl = lane & 7, ql = lane >> 3;
-    wave_lds_sync();  // the previous element's reads are done
-    // lane hl's row entry tab[hl] = entry 8 e2 + hl of the view, which lane 8 e2 + hl
-    // holds in tl (images outside the group have kRowNone entries)
-    const int t = __builtin_amdgcn_ds_bpermute((8 * e2 + hl) << 2, tl);
-    // the row's reflection from its entry (equal to elem_flip, checked when the table is
-    // built): a per-view value keeps the store addresses below from being hoisted out of
-    // the view loop as eight per-element sets
-    const bool fl = (t & kRowFlip) != 0;
-    const int b0 = L0 + 4 * ql;
-    // a row without an entry reads past the buffer's end, which gives zeros (no branch)
-    const int voff = (t & kRowNone) ? kStageNoRow
-                                    : (t & ~(kRowFlip | kRowNone)) + 4 * (fl ? 2 * S.pC - b0 - 3 : b0);
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(RS, voff, 0, 0);
-    const float x0 = __uint_as_float(v[0]), x1 = __uint_as_float(v[1]);
-    const float x2 = __uint_as_float(v[2]), x3 = __uint_as_float(v[3]);
-    float4 rv;
-    if (FAN) {  // ray records of bins L0 .. L0 + kStageBins - 1: 16 bytes per lane
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(RR, L0 * (int)sizeof(Ray) + lane * 16,
-                                                             rrow, 0);
-        rv = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
-                         __uint_as_float(v[3]));
-    }
-    // xj is bin b0 + j, or b0 + 3 - j of a reflected row: reversed in registers, so that
-    // the stores keep per-lane addresses
-    st->val[4 * ql + 0][hl] = fl ? x3 : x0;
-    st->val[4 * ql + 1][hl] = fl ? x2 : x1;
-    st->val[4 * ql + 2][hl] = fl ? x1 : x2;
-    st->val[4 * ql + 3][hl] = fl ? x0 : x3;
-    if (FAN) st->ray[lane] = rv;
-    wave_lds_sync();  // staged values visible to every lane
-    if (blo > bhi) return;  // no candidate of this lane in the chunk
-    const float qd = FAN ? fan_depth_scale(fx, fy, cT, sT, S.invd) : 1.0f;
-    // FBP fan weight d^2/qe^2 (prj/cpuPrj.c:258), folded into each weight
-    const float fw = (FBP && FAN) ? 1.0f / (qd * qd) : 1.0f;
-    // exactly the pixel's candidate bins, in increasing order: the per-lane gathers add
-    // the same products plus exact zeros (bins of a window past bhi), which change no sum
-    // (a partial sum that starts at +0 never becomes -0)
-    for (int b = blo; b <= bhi; ++b) {
-        const int k = b - L0;
-        Ray r;
-        if (FAN) {
-            const float4 a = st->ray[2 * k], c = st->ray[2 * k + 1];
-            r.cosR = a.x;
-            r.sinR = a.y;
-            r.dc = a.z;
-            r.hbc = a.w;
-            r.h = c.x;
-            r.b1 = c.y;
-            r.s = c.z;
-            r.k = c.w;
-        } else {
-            r = rview[0];
-            r.dc = (float)(b - S.pC) * S.dSize;
-        }
-        const float dist = ray_dist(fx, fy, r.cosR, r.sinR, r.dc);
-        float w = strip_weight(dist, FAN ? r.hbc * qd : r.hbc, r);
-        if (FBP && FAN) w *= fw;
-        const float4 lo = *reinterpret_cast<const float4*>(&st->val[k][0]);
-        const float4 hi = *reinterpret_cast<const float4*>(&st->val[k][4]);
-        const float q[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-#pragma unroll
-        for (int h = 0; h < 8; ++h)
-            if (HMASK >> h & 1u) vpart[h] = fmaf(w, q[h], vpart[h]);
-    }
-}
-
-// The gather of adj_sym_elem_ct through the wave's LDS area, for element g' = e2 (a
-// canonical view off the mirror lines) and the orbit images in HMASK.  Every lane of the
-// wave takes part; lanes with valid == false or no candidate add nothing.  A range wider
-// than kStageBins bins (fine detector pitch) is staged and summed in chunks of kStageBins
-// bins, in increasing order, so the sums are bit-identical to the per-lane gathers'.
-template <bool FAN, bool FBP, unsigned HMASK>
-__device__ __forceinline__ void adj_sym_elem_lds(const SliceDesc& S, const Ray* __restrict__ rview,
-                                                 __amdgpu_buffer_rsrc_t RS,
-                                                 __amdgpu_buffer_rsrc_t RR, int rrow, int e2,
-                                                 int tl, float cT, float sT, int x0, int y0,
-                                                 bool valid, float* vpart,
-                                                 AdjStage* __restrict__ st)
-{
-    const int k2 = e2 & 3, m2 = e2 >> 2;
-    int px, py;
-    if (m2) apply_px(k2, 1, x0, y0, px, py);
-    else apply_px(4 - k2, 0, x0, y0, px, py);
-    const float fx = (float)px, fy = (float)py;
-    int blo, bhi;
-    pixel_bins<FAN>(S, rview, fx, fy, cT, sT, blo, bhi);
-    if (!valid || blo > bhi) {
-        blo = INT_MAX;
-        bhi = INT_MIN;
-    }
-    int L0, Lmax;
-    wave_range_i32(blo, bhi, L0, Lmax);
-    // wave-uniform; one chunk unless the range is wider than kStageBins bins
-    for (int c0 = L0; c0 <= Lmax; c0 += kStageBins)
-        adj_sym_chunk<FAN, FBP, HMASK>(S, rview, RS, RR, rrow, e2, tl, cT, sT, fx, fy,
-                                       max(blo, c0), min(bhi, c0 + kStageBins - 1), c0, vpart,
-                                       st);
-}
-
-// All elements of a canonical view off the mirror lines, unrolled at compile time.
-// With STAGE the wave stages each element's bins in LDS (every lane takes part),
-// otherwise the valid lanes gather directly.
-template <bool FAN, bool FBP, int GRP, bool FOLD, int WIN, bool STAGE>
-__device__ __forceinline__ void adj_sym_view_ct(const SliceDesc& S, const Ray* __restrict__ rview,
-                                                __amdgpu_buffer_rsrc_t RS, __amdgpu_buffer_rsrc_t RZ,
-                                                __amdgpu_buffer_rsrc_t RR, int rrow,
-                                                const int* __restrict__ tv, float cT, float sT,
-                                                int x0, int y0, bool valid, float* vpart,
-                                                AdjStage* __restrict__ st)
-{
-    constexpr GroupMasks G = group_masks(GRP);
-    constexpr unsigned GSET = FOLD ? G.fold : G.all;
-    // the view's 64 row entries, entry l in lane l (the staged gathers pick theirs with a
-    // lane permute)
-    const int tl = STAGE ? tv[threadIdx.x & 63] : 0;
-#define CTPRJ_E(E2)                                                                             \
-    if constexpr ((GSET >> E2) & 1u) {                                                           \
-        if (STAGE)                                                                               \
-            adj_sym_elem_lds<FAN, FBP, G.all>(S, rview, RS, RR, rrow, E2, tl, cT, sT, x0, y0,     \
-                                              valid, vpart, st);                                 \
-        else if (valid)                                                                          \
-            adj_sym_elem_ct<FAN, FBP, G.all, E2, FOLD, WIN>(S, rview, RS, RZ, RR, rrow,          \
-                                                            tv + 8 * E2, cT, sT, x0, y0, vpart); \
-    }
-    CTPRJ_E(0) CTPRJ_E(1) CTPRJ_E(2) CTPRJ_E(3) CTPRJ_E(4) CTPRJ_E(5) CTPRJ_E(6) CTPRJ_E(7)
-#undef CTPRJ_E
-}
-
-// Canonical views i = i0, i0 + step, ... for the orbit of (x0, y0) under group GRP.
-// Every lane of the wave runs the view loop (the staged gather needs them all); lanes
-// with valid == false add nothing.
-template <bool FAN, bool FBP, int GRP, int WIN, bool STAGE>
+// Canonical views i = i0, i0 + step, ... for the orbit of (x0, y0) under group GRP: for
+// each view and each element g' the wave stages the bins that its 64 orbit pixels can
+// read (one load per lane for the values, one for the fan-beam ray records; the next
+// element's are loaded while this one's are summed), and every lane sums its own candidate
+// bins from LDS, in increasing order: the weight W(a0, b, g'^-1 q0) is formed once and
+// serves every pixel of the orbit.  On a mirror view the reflected rays' zeros leave
+// rotations g' paired with rotation pixels and reflections with reflected ones, so every
+// entry has the forward's key.  A folded scan takes the half set of elements that maps the
+// canonical range into [0, 180).  The staged range starts at the smallest first bin of the
+// tile's corner pixels (the extremes, see BinBounds); should a lane's bins lie outside,
+// the wave takes the true range, piece by piece where it is wider than kStageBins.
+// Bound by VALU issue (4 cycles a wave instruction): what is not a weight or an update is
+// kept to the candidate bounds (about 25 instructions per element) and the loop's two.
+template <bool FAN, bool FBP, int GRP, bool FOLD>
 __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* __restrict__ views,
                                               const Ray* __restrict__ rays,
-                                              const float* __restrict__ sino,
-                                              const float* __restrict__ zero_row,
-                                              const int* __restrict__ symtab, int x0, int y0,
+                                              const float* __restrict__ os, int x0, int y0,
                                               bool valid, int i0, int step, KahanAcc* acc,
                                               AdjStage* __restrict__ st)
 {
+    using O = Orbit<GRP>;
+    constexpr int N = O::N, CH = kStageBins;
     constexpr GroupMasks G = group_masks(GRP);
-    constexpr unsigned REF = G.all & ~G.rot;
-    const __amdgpu_buffer_rsrc_t RS = slice_rsrc(sino + S.sino_off, S.np * S.W);
-    const __amdgpu_buffer_rsrc_t RZ = slice_rsrc(zero_row, S.W);
-    // fan: the slice's ray table (ncanon rows of W records, below 2 GiB)
-    const __amdgpu_buffer_rsrc_t RR = slice_rsrc(
-        reinterpret_cast<const float*>(rays + S.ray_off),
-        FAN ? S.ncanon * S.W * (int)(sizeof(Ray) / sizeof(float)) : 0);
+    constexpr unsigned GSET = FOLD ? G.fold : G.all;
+    const int lane = (int)threadIdx.x & 63;
+    const float gx = (float)x0, gy = (float)y0;
+    // lane's part of a staged piece, bytes from the first bin's: values, ray records
+    const int voff = N == 8 && lane >= CH ? (S.os_pitch + lane - CH) * 16 : lane * O::kPlane * 4;
+    const int roff = (lane & (CH - 1)) * (int)sizeof(Ray) + (lane >= CH ? 16 : 0);
+    const int rec = N * S.os_pitch, last_bin = valid ? S.bhi : INT_MIN;
     for (int i = i0; i < S.ncanon; i += step) {
         const float4 T = views[S.view_off + i];
-        const int a0 = __float_as_int(T.z);
-        const Ray* rview = FAN ? rays + S.ray_off + (long long)i * S.W : rays + S.ray_off + i;
-        const int* tv = symtab + S.tab_off + (long long)i * 64;
-        const int rrow = FAN ? i * S.W * (int)sizeof(Ray) : 0;
-        float vpart[8];  // this view's sums; compensated once per view
+        const float* osrow = os + S.os_off + (long long)i * rec;
+        const __amdgpu_buffer_rsrc_t RV = row_rsrc(osrow, rec * 4);
+        const Ray* rview = rays + S.ray_off + (FAN ? (long long)i * S.W : i);
+        const __amdgpu_buffer_rsrc_t RR = row_rsrc(reinterpret_cast<const float*>(rview),
+                                                   FAN ? S.W * (int)sizeof(Ray) : 0);
+        const Ray r0 = rview[0];  // parallel beam: the view's ray constants
+        const BinBounds<FAN> bounds(S, T.x, T.y, r0, last_bin);
+        float vpart[N];  // this view's sums; compensated once per view
 #pragma unroll
-        for (int h = 0; h < 8; ++h) vpart[h] = 0.0f;
-        if (a0 == 0 || G.q * a0 == S.P) {
-            // rotations g' -> rotation orbit pixels, reflections g' -> reflected ones
-            const unsigned grot = S.fold ? G.mfold_rot : G.rot;
-            const unsigned gref = S.fold ? G.mfold_ref : REF;
-            if (valid) {
-#pragma unroll 1
-                for (int e = 0; e < 8; ++e)
-                    if (grot >> e & 1u)
-                        adj_sym_elem<FAN, FBP, G.rot, WIN>(S, rview, RS, RZ, tv + 8 * e, T.x, T.y,
-                                                           e & 3, e >> 2, x0, y0, vpart);
-#pragma unroll 1
-                for (int e = 0; e < 8; ++e)
-                    if (gref >> e & 1u)
-                        adj_sym_elem<FAN, FBP, REF, WIN>(S, rview, RS, RZ, tv + 8 * e, T.x, T.y,
-                                                         e & 3, e >> 2, x0, y0, vpart);
+        for (int s = 0; s < N; ++s) vpart[s] = 0.0f;
+        // the pixel g'^-1 q0: (R^k M)^-1 = R^k M, (R^k)^-1 = R^-k
+        auto pixel = [&](int e2, float& fx, float& fy) {
+            const float y = (e2 >> 2) ? -gy : gy;
+            switch ((e2 >> 2) ? (e2 & 3) : (-e2 & 3)) {
+                case 0: fx = gx; fy = y; break;
+                case 1: fx = -y; fy = gx; break;
+                case 2: fx = -gx; fy = -y; break;
+                default: fx = y; fy = -gx; break;
             }
-        } else if (GRP != kGrpZ2 && S.fold) {
-            // a half-turn parallel scan takes the half set that maps the canonical range
-            // into [0, 180) and reads the rest folded
-            adj_sym_view_ct<FAN, FBP, GRP, GRP != kGrpZ2, WIN, STAGE>(
-                S, rview, RS, RZ, RR, rrow, tv, T.x, T.y, x0, y0, valid, vpart, st);
-        } else {
-            adj_sym_view_ct<FAN, FBP, GRP, false, WIN, STAGE>(S, rview, RS, RZ, RR, rrow, tv, T.x,
-                                                              T.y, x0, y0, valid, vpart, st);
-        }
+        };
+        // the lane's candidate bins under element e2, and the wave's first
+        auto range = [&](int e2, int& blo, int& bhi, int& c0) {
+            float fx, fy;
+            pixel(e2, fx, fy);
+            bounds(fx, fy, blo, bhi);
+            c0 = min(min(__builtin_amdgcn_readlane(blo, 0), __builtin_amdgcn_readlane(blo, 7)),
+                     min(__builtin_amdgcn_readlane(blo, 56), __builtin_amdgcn_readlane(blo, 63)));
+            // (no candidates: any bin, so that the load stays inside)
+            c0 = __builtin_amdgcn_readfirstlane(min(c0, S.bhi));
+        };
+        auto load = [&](int c0, float4& val, float4& ray) {
+            if constexpr (N == 2) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(RV, voff, c0 * 8, 0);
+                val.x = __uint_as_float(v[0]);
+                val.y = __uint_as_float(v[1]);
+            } else {
+                val = ldb128(RV, voff, c0 * 16);
+            }
+            if (FAN) ray = ldb128(RR, roff, c0 * (int)sizeof(Ray));
+        };
+        auto stage = [&](const float4& val, const float4& ray) {
+            wave_lds_sync();  // the previous piece's reads are done
+            if constexpr (N == 2) *reinterpret_cast<float2*>(&st->val[lane]) = make_float2(val.x, val.y);
+            else st->val[lane] = val;
+            if (FAN) st->ray[lane] = ray;
+            wave_lds_sync();  // staged values visible to every lane
+        };
+        // bins blo..bhi, staged from c0 on
+        auto sum = [&](auto e2c, int blo, int bhi, int c0) {
+            constexpr int e2 = decltype(e2c)::value;
+            if (blo > bhi) return;
+            float fx, fy;
+            pixel(e2, fx, fy);
+            const float qd = FAN ? fan_depth_scale(fx, fy, T.x, T.y, S.invd) : 1.0f;
+            // FBP fan weight d^2/qe^2 (prj/cpuPrj.c:258), folded into each weight
+            const float fw = (FBP && FAN) ? 1.0f / (qd * qd) : 1.0f;
+            const float4* at = st->val + (blo - c0);
+            const float4* const end = st->val + (bhi - c0);
+            float fb = (float)(blo - S.pC);  // parallel beam
+            do {
+                Ray r = r0;
+                if (FAN) {
+                    const float4 a = at[64], c = at[64 + CH];
+                    r = Ray{a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+                } else {
+                    r.dc = fb * S.dSize;
+                    fb += 1.0f;
+                }
+                const float4 va = at[0], vb = at[N == 8 ? CH : 0];
+                const float q[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
+                const float dist = ray_dist(fx, fy, r.cosR, r.sinR, r.dc);
+                float w = strip_area(dist, FAN ? r.hbc * qd : r.hbc, r);
+                if (FBP && FAN) w *= fw;
 #pragma unroll
-        for (int h = 0; h < 8; ++h)
-            if (G.all >> h & 1u) acc[h].add(vpart[h]);
+                for (int s = 0; s < N; ++s)
+                    vpart[s] = fmaf(w, q[O::slot(elem_mul(O::elem(s), e2))], vpart[s]);
+            } while (++at <= end);
+        };
+        int blo, bhi, c0;
+        float4 val{}, ray{};
+        range(0, blo, bhi, c0);  // element 0 is in every set
+        load(c0, val, ray);
+        // element E2, the first piece of the next element of the set on its way meanwhile
+#define CTPRJ_E(E2)                                                                          \
+    if constexpr ((GSET >> E2) & 1u) {                                                       \
+        constexpr unsigned rest = GSET & ~((2u << E2) - 1u);                                 \
+        constexpr int NX = rest ? __builtin_ctz(rest) : 0;                                   \
+        const int l = blo, h = bhi;                                                          \
+        int p = c0, last = c0;                                                               \
+        stage(val, ray);                                                                     \
+        if (rest) {                                                                          \
+            range(NX, blo, bhi, c0);                                                         \
+            load(c0, val, ray);                                                              \
+        }                                                                                    \
+        if (__any(l <= h && (l < p || h >= p + CH))) {                                       \
+            wave_range_i32(l <= h ? l : INT_MAX, l <= h ? h : INT_MIN, p, last);             \
+            float4 v2{}, r2{};                                                               \
+            load(p, v2, r2);                                                                 \
+            stage(v2, r2);                                                                   \
+        }                                                                                    \
+        for (;;) {                                                                           \
+            sum(std::integral_constant<int, E2>{}, max(l, p), min(h, p + CH - 1), p);        \
+            p += CH;                                                                         \
+            if (p > last) break;                                                             \
+            float4 v2{}, r2{};                                                               \
+            load(p, v2, r2);                                                                 \
+            stage(v2, r2);                                                                   \
+        }                                                                                    \
+    }
+        CTPRJ_E(0) CTPRJ_E(1) CTPRJ_E(2) CTPRJ_E(3) CTPRJ_E(4) CTPRJ_E(5) CTPRJ_E(6) CTPRJ_E(7)
+#undef CTPRJ_E
+#pragma unroll
+        for (int s = 0; s < N; ++s) acc[s].add(vpart[s]);
     }
 }
 
@@ -971,38 +990,32 @@ __device__ __forceinline__ void adj_sym_store(const SliceDesc& S, int x0, int y0
 // The canonical views are cut into nsplit * SEG strided sets: wave w of this work-group
 // takes i = split * SEG + w + j * nsplit * SEG.  nsplit == 1 writes the image; otherwise
 // the work-group's sums go to part[h * 64 + lane] for k_adjoint_sym_combine.
-template <bool FBP, int SEG, int GRP, int WIN, bool STAGE>
+template <bool FAN, bool FBP, int SEG, int GRP>
 __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& it,
                                              const float4* __restrict__ views,
                                              const Ray* __restrict__ rays,
-                                             const float* __restrict__ sino,
-                                             const float* __restrict__ zero_row,
-                                             const int* __restrict__ symtab,
+                                             const float* __restrict__ os,
                                              float* __restrict__ img, float (*red)[8][64],
                                              int split, int nsplit, float* __restrict__ part,
                                              AdjStage* __restrict__ stage)
 {
-    constexpr GroupMasks G = group_masks(GRP);
+    using O = Orbit<GRP>;
     // the wave index is uniform over the wave: the view loop then runs on scalar registers
     const int lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int x0, y0;
     const bool valid = adj_sym_base<GRP>(S, it, lane, x0, y0);
-    KahanAcc acc[8];
-    if (STAGE || valid) {
-        const int i0 = split * SEG + wave, step = SEG * nsplit;
-        AdjStage* st = STAGE ? stage + wave : nullptr;
-        if (S.fan)
-            adj_sym_pixel<true, FBP, GRP, WIN, STAGE>(S, views, rays, sino, zero_row, symtab, x0,
-                                                      y0, valid, i0, step, acc, st);
-        else
-            adj_sym_pixel<false, FBP, GRP, WIN, STAGE>(S, views, rays, sino, zero_row, symtab, x0,
-                                                       y0, valid, i0, step, acc, st);
-    }
+    KahanAcc acc[O::N];
+    const int i0 = split * SEG + wave, step = SEG * nsplit;
+    if (!FAN && GRP != kGrpZ2 && S.fold)
+        adj_sym_pixel<FAN, FBP, GRP, !FAN && GRP != kGrpZ2>(S, views, rays, os, x0, y0, valid, i0,
+                                                            step, acc, stage + wave);
+    else
+        adj_sym_pixel<FAN, FBP, GRP, false>(S, views, rays, os, x0, y0, valid, i0, step, acc,
+                                            stage + wave);
     if (SEG > 1) {
 #pragma unroll
-        for (int h = 0; h < 8; ++h)
-            if (G.all >> h & 1u) red[wave][h][lane] = acc[h].s;
+        for (int s = 0; s < O::N; ++s) red[wave][O::elem(s)][lane] = acc[s].s;
         __syncthreads();
     }
     if (!part && it.pad) sym_zero_border(S, img);
@@ -1010,9 +1023,10 @@ __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& 
     // wave w finalises the elements h = w (mod SEG): the sum of the waves' partials in
     // wave order
 #pragma unroll
-    for (int h = 0; h < 8; ++h) {
-        if (!(G.all >> h & 1u) || (SEG > 1 && h % SEG != wave)) continue;
-        float t = acc[h].s;
+    for (int s = 0; s < O::N; ++s) {
+        const int h = O::elem(s);
+        if (SEG > 1 && h % SEG != wave) continue;
+        float t = acc[s].s;
         if (SEG > 1) {
             t = red[0][h][lane];
 #pragma unroll
@@ -1026,36 +1040,32 @@ __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& 
 // One launch per symmetry group; SEG waves split the canonical views (wave w takes
 // i = w, w + SEG, ...) and then share the final sums; with nsplit > 1, nsplit
 // work-groups share the views of a tile and leave their sums in part (512 floats per
-// work-group) for k_adjoint_sym_combine.  STAGE: the gathers off the mirror views go
-// through each wave's LDS area (adj_sym_elem_lds).  The staged 4-bin-window variants ask
-// for at least five waves per SIMD (96 VGPRs; D4 would take 99, four waves); the same
-// request spills on the staged 3-bin D4 variants, which keep the compiler's own schedule
-// (the window width matters there only on the mirror views' per-lane gathers).
-template <bool FBP, int SEG, int GRP, int WIN, bool STAGE>
-__global__ __launch_bounds__(64 * SEG)
-__attribute__((amdgpu_waves_per_eu((STAGE && WIN == 4) ? 5 : 1))) void k_adjoint_sym(const SliceDesc* __restrict__ slices,
+// work-group) for k_adjoint_sym_combine.
+template <bool FBP, int SEG, int GRP>
+__global__ __launch_bounds__(64 * SEG) void k_adjoint_sym(const SliceDesc* __restrict__ slices,
                                                           const AdjItem* __restrict__ items,
                                                           const float4* __restrict__ views,
                                                           const Ray* __restrict__ rays,
-                                                          const float* __restrict__ sino,
-                                                          const float* __restrict__ zero_row,
-                                                          const int* __restrict__ symtab,
+                                                          const float* __restrict__ os,
                                                           float* __restrict__ img, int nitems,
                                                           int nsplit, float* __restrict__ part,
                                                           const RedJob job)
 {
     __shared__ float red[SEG][8][64];
-    __shared__ AdjStage stage[STAGE ? SEG : 1];
+    __shared__ AdjStage stage[SEG];
     if (job.out && blockIdx.x == 0 && threadIdx.x < 64) wave_sum_job(job);  // on the side
     int split, idx;
     split_item(nitems, split, idx);
     const AdjItem it = items[idx];
     if (it.slice < 0) return;  // uniform over the work-group
     const SliceDesc S = slices[it.slice];
-    adj_sym_tile<FBP, SEG, GRP, WIN, STAGE>(S, it, views, rays, sino, zero_row, symtab, img, red,
-                                            split, nsplit,
-                                            part ? part + (long long)blockIdx.x * 512 : nullptr,
-                                            stage);
+    float* mine = part ? part + (long long)blockIdx.x * 512 : nullptr;
+    if (S.fan)
+        adj_sym_tile<true, FBP, SEG, GRP>(S, it, views, rays, os, img, red, split, nsplit, mine,
+                                          stage);
+    else
+        adj_sym_tile<false, FBP, SEG, GRP>(S, it, views, rays, os, img, red, split, nsplit, mine,
+                                           stage);
 }
 
 // The nsplit partial sums of each orbit image of a tile, added in split order and
@@ -1088,14 +1098,14 @@ __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __
 template <int GRP, bool BHC>
 static void launch_forward_sym_g(int seg, int nsplit, float* part, int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
-                                 const Ray* rays, const float* img, const float* imgT, float* sino,
+                                 const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
 {
     float* pp = nsplit > 1 ? part : nullptr;
     const dim3 grid((unsigned)nitems * (unsigned)nsplit);
 #define CTPRJ_LAUNCH(SEG)                                                                       \
     hipLaunchKernelGGL((k_forward_sym<SEG, GRP, BHC>), grid, dim3(64 * SEG), 0, st, desc, items, \
-                       views, rays, img, imgT, sino, nitems, nsplit, pp, B)
+                       views, rays, orb, sino, nitems, nsplit, pp, B)
     switch (seg) {
         case 1: CTPRJ_LAUNCH(1); break;
         case 2: CTPRJ_LAUNCH(2); break;
@@ -1112,62 +1122,52 @@ static void launch_forward_sym_g(int seg, int nsplit, float* part, int nitems,
 template <bool BHC>
 static void launch_forward_sym_b(int grp, int seg, int nsplit, float* part, int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
-                                 const Ray* rays, const float* img, const float* imgT, float* sino,
+                                 const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
 {
     if (grp == kGrpD4)
         launch_forward_sym_g<kGrpD4, BHC>(seg, nsplit, part, nitems, desc, items, views, rays,
-                                          img, imgT, sino, B, st);
+                                          orb, sino, B, st);
     else if (grp == kGrpV4)
         launch_forward_sym_g<kGrpV4, BHC>(seg, nsplit, part, nitems, desc, items, views, rays,
-                                          img, imgT, sino, B, st);
+                                          orb, sino, B, st);
     else
         launch_forward_sym_g<kGrpZ2, BHC>(seg, nsplit, part, nitems, desc, items, views, rays,
-                                          img, imgT, sino, B, st);
+                                          orb, sino, B, st);
 }
 
 void launch_forward_sym(int grp, int seg, int nsplit, float* part, int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
-                        const Ray* rays, const float* img, const float* imgT, float* sino,
-                        const BhcStore* bhc, hipStream_t st)
+                        const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
+                        hipStream_t st)
 {
     if (bhc) {
         FwdBhc<true> B;
         static_cast<BhcStore&>(B) = *bhc;
-        launch_forward_sym_b<true>(grp, seg, nsplit, part, nitems, desc, items, views, rays, img,
-                                   imgT, sino, B, st);
+        launch_forward_sym_b<true>(grp, seg, nsplit, part, nitems, desc, items, views, rays, orb,
+                                   sino, B, st);
     } else {
-        launch_forward_sym_b<false>(grp, seg, nsplit, part, nitems, desc, items, views, rays, img,
-                                    imgT, sino, FwdBhc<false>{}, st);
+        launch_forward_sym_b<false>(grp, seg, nsplit, part, nitems, desc, items, views, rays, orb,
+                                    sino, FwdBhc<false>{}, st);
     }
 }
 
-template <bool FBP, int GRP, int WIN>
-static void launch_adjoint_sym_t(int seg, bool stage, int nsplit, float* part, int nitems,
+template <bool FBP, int GRP>
+static void launch_adjoint_sym_t(int seg, int nsplit, float* part, int nitems,
                                  const SliceDesc* desc, const AdjItem* items, const float4* views,
-                                 const Ray* rays, const float* sino, const float* zero_row,
-                                 const int* symtab, float* img, const RedJob& job, hipStream_t st)
+                                 const Ray* rays, const float* os, float* img, const RedJob& job,
+                                 hipStream_t st)
 {
     float* pp = nsplit > 1 ? part : nullptr;
     const dim3 grid((unsigned)nitems * (unsigned)nsplit);
-#define CTPRJ_LAUNCH(SEG, STAGE)                                                                 \
-    hipLaunchKernelGGL((k_adjoint_sym<FBP, SEG, GRP, WIN, STAGE>), grid, dim3(64 * SEG), 0, st,  \
-                       desc, items, views, rays, sino, zero_row, symtab, img, nitems, nsplit, pp, \
-                       job)
-    if (stage) {
-        switch (seg) {
-            case 1: CTPRJ_LAUNCH(1, true); break;
-            case 2: CTPRJ_LAUNCH(2, true); break;
-            case 4: CTPRJ_LAUNCH(4, true); break;
-            default: CTPRJ_LAUNCH(8, true); break;
-        }
-    } else {
-        switch (seg) {
-            case 1: CTPRJ_LAUNCH(1, false); break;
-            case 2: CTPRJ_LAUNCH(2, false); break;
-            case 4: CTPRJ_LAUNCH(4, false); break;
-            default: CTPRJ_LAUNCH(8, false); break;
-        }
+#define CTPRJ_LAUNCH(SEG)                                                                      \
+    hipLaunchKernelGGL((k_adjoint_sym<FBP, SEG, GRP>), grid, dim3(64 * SEG), 0, st, desc, items, \
+                       views, rays, os, img, nitems, nsplit, pp, job)
+    switch (seg) {
+        case 1: CTPRJ_LAUNCH(1); break;
+        case 2: CTPRJ_LAUNCH(2); break;
+        case 4: CTPRJ_LAUNCH(4); break;
+        default: CTPRJ_LAUNCH(8); break;
     }
 #undef CTPRJ_LAUNCH
     if (pp)
@@ -1175,42 +1175,34 @@ static void launch_adjoint_sym_t(int seg, bool stage, int nsplit, float* part, i
                            st, desc, items, nitems, nsplit, pp, img);
 }
 
-template <bool FBP, int WIN>
-static void launch_adjoint_sym_f(int grp, int seg, bool stage, int nsplit, float* part, int nitems,
+template <bool FBP>
+static void launch_adjoint_sym_f(int grp, int seg, int nsplit, float* part, int nitems,
                                  const SliceDesc* desc, const AdjItem* items, const float4* views,
-                                 const Ray* rays, const float* sino, const float* zero_row,
-                                 const int* symtab, float* img, const RedJob& job, hipStream_t st)
+                                 const Ray* rays, const float* os, float* img, const RedJob& job,
+                                 hipStream_t st)
 {
     if (grp == kGrpD4)
-        launch_adjoint_sym_t<FBP, kGrpD4, WIN>(seg, stage, nsplit, part, nitems, desc, items,
-                                               views, rays, sino, zero_row, symtab, img, job, st);
+        launch_adjoint_sym_t<FBP, kGrpD4>(seg, nsplit, part, nitems, desc, items, views, rays, os,
+                                          img, job, st);
     else if (grp == kGrpV4)
-        launch_adjoint_sym_t<FBP, kGrpV4, WIN>(seg, stage, nsplit, part, nitems, desc, items,
-                                               views, rays, sino, zero_row, symtab, img, job, st);
+        launch_adjoint_sym_t<FBP, kGrpV4>(seg, nsplit, part, nitems, desc, items, views, rays, os,
+                                          img, job, st);
     else
-        launch_adjoint_sym_t<FBP, kGrpZ2, WIN>(seg, stage, nsplit, part, nitems, desc, items,
-                                               views, rays, sino, zero_row, symtab, img, job, st);
+        launch_adjoint_sym_t<FBP, kGrpZ2>(seg, nsplit, part, nitems, desc, items, views, rays, os,
+                                          img, job, st);
 }
 
-void launch_adjoint_sym(bool fbp, int grp, int seg, int win, bool stage, int nsplit, float* part,
-                        int nitems, const SliceDesc* desc, const AdjItem* items,
-                        const float4* views, const Ray* rays, const float* sino,
-                        const float* zero_row, const int* symtab, float* img, const RedJob& job,
+void launch_adjoint_sym(bool fbp, int grp, int seg, int nsplit, float* part, int nitems,
+                        const SliceDesc* desc, const AdjItem* items, const float4* views,
+                        const Ray* rays, const float* os, float* img, const RedJob& job,
                         hipStream_t st)
 {
-    if (fbp && win == 3)
-        launch_adjoint_sym_f<true, 3>(grp, seg, stage, nsplit, part, nitems, desc, items, views,
-                                      rays, sino, zero_row, symtab, img, job, st);
-    else if (fbp)
-        launch_adjoint_sym_f<true, 4>(grp, seg, stage, nsplit, part, nitems, desc, items, views,
-                                      rays, sino, zero_row, symtab, img, job, st);
-    else if (win == 3)
-        launch_adjoint_sym_f<false, 3>(grp, seg, stage, nsplit, part, nitems, desc, items, views,
-                                       rays, sino, zero_row, symtab, img, job, st);
+    if (fbp)
+        launch_adjoint_sym_f<true>(grp, seg, nsplit, part, nitems, desc, items, views, rays, os,
+                                   img, job, st);
     else
-        launch_adjoint_sym_f<false, 4>(grp, seg, stage, nsplit, part, nitems, desc, items, views,
-                                       rays, sino, zero_row, symtab, img, job, st);
+        launch_adjoint_sym_f<false>(grp, seg, nsplit, part, nitems, desc, items, views, rays, os,
+                                    img, job, st);
 }
-
 
 }  // namespace ctprj
