@@ -703,6 +703,7 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
             prew.push_back((float)w);
         }
         max_W = std::max(max_W, W);
+        p->max_n = std::max(p->max_n, g.n);
     }
     p->img_elems = img;
     p->sino_elems = sino;
@@ -728,7 +729,9 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
         (rc = p->build_adj_items(p->tune, *p)) ||
         (rc = grow(&p->d_imgT, &p->imgT_cap, p->n_sym < nslices ? img : 0, "transposed image")) ||
         (rc = grow(&p->d_orb, &p->orb_cap, p->orb_floats, "orbit image")) ||
-        (rc = grow(&p->d_os, &p->os_cap, p->os_floats, "orbit sinogram"))) {
+        (rc = grow(&p->d_os, &p->os_cap, p->os_floats, "orbit sinogram")) ||
+        (rc = grow(&p->d_split, &p->split_cap, (long long)p->split_need(p->tune, *p, *p),
+                   "split partial sums"))) {
         delete p;
         return rc;
     }
@@ -771,6 +774,28 @@ extern "C" int ctprj_plan_layout(const ctprj_plan* p, long long* img_elems,
 
 namespace ctprj {
 
+// A new plan's shape, 8 waves in one work-group per item, stands for the plan's own choice:
+// as it is where every image is at most kSmallEdge wide, else 4 waves and as many
+// work-groups per item as give about kFillItems of them (two at least in the forward, whose
+// items differ in cost), within the partial sums' space.
+// Measured (us, 8 x 1 against the choice): forward 64^2 14.8 / 16.4, 256^2 parallel 31.4 /
+// 22.3, 512^2 fan 108 / 78, 769^2 fan of odd views 343 / 319, 1024^2 fan 207 / 183, 16
+// ragged slices 1265 / 1230, 32 x 512^2 3505 / 3352; adjoint 15.6 / 17.4, 19.4 / 15.3,
+// 67 / 49, 306 / 304, 176 / 159, 1027 / 1023, 2028 / 1993.  The line: at 64^2 the second
+// launch that adds the partial sums costs more than the split gains, at 160^2 (25.6 / 17.6)
+// less; small slices keep one shape so that a batch gives each of them the bits of a
+// one-slice plan.
+constexpr int kSmallEdge = 224, kFillItems = 9000;
+
+Plan::Shape Plan::sym_shape(const ctprj_tune& t, bool fwd, int items) const
+{
+    const Shape set = fwd ? Shape{t.fwd_seg, t.fwd_split} : Shape{t.adj_seg, t.adj_split};
+    if (set.seg != 8 || set.split != 1 || max_n <= kSmallEdge || items < 1) return set;
+    int split = std::min(std::max((kFillItems + items - 1) / items, fwd ? 2 : 1), 8);
+    while (split > 1 && (size_t)items * split * 512 > kSplitMaxFloats) --split;
+    return Shape{4, split};
+}
+
 // The symmetric slices' forward: per chunk, its orbit image, then one launch per group.
 int Plan::launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st)
 {
@@ -781,7 +806,8 @@ int Plan::launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStrea
         for (int g = 1; g < 4; ++g) {
             const int n = symf[c].count[g];
             if (!n) continue;
-            launch_forward_sym(g, tune.fwd_seg, tune.fwd_split, d_split, n, d_desc,
+            const Shape sh = sym_shape(tune, true, n);
+            launch_forward_sym(g, sh.seg, sh.split, d_split, n, d_desc,
                                d_symf_items + symf[c].start[g], d_views, d_rays, d_orb, d_sino,
                                bhc, st);
             if (bhc) bhc->part_off += n;
@@ -824,7 +850,8 @@ int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool
         for (int g = 1; g < 4; ++g) {
             const int n = syma[c].count[g];
             if (!n) continue;
-            launch_adjoint_sym(fbp, g, tune.adj_seg, tune.adj_split, d_split, n, d_desc,
+            const Shape sh = sym_shape(tune, false, n);
+            launch_adjoint_sym(fbp, g, sh.seg, sh.split, d_split, n, d_desc,
                                d_syma_items + syma[c].start[g], d_views, d_rays, d_os, d_img,
                                first ? job : RedJob{}, st);
             first = false;
@@ -958,7 +985,7 @@ extern "C" int ctprj_plan_set_tune(ctprj_plan* p, const ctprj_tune* t)
         split_rc = fail(CTPRJ_EINVAL, "split work items need %zu MiB of partial sums (at most %zu)",
                         need * sizeof(float) >> 20, kSplitMaxFloats * sizeof(float) >> 20);
         nt.adj_split = nt.fwd_split = 1;
-        need = 0;
+        need = p->split_need(nt, F, A);
     }
     // workspaces only grow, and serve the old tables as well as the new
     if (geo && ((rc = grow(&p->d_imgT, &p->imgT_cap, N.n_sym < p->nslices ? p->img_elems : 0,
@@ -966,11 +993,7 @@ extern "C" int ctprj_plan_set_tune(ctprj_plan* p, const ctprj_tune* t)
                 (rc = grow(&p->d_orb, &p->orb_cap, N.orb_floats, "orbit image")) ||
                 (rc = grow(&p->d_os, &p->os_cap, N.os_floats, "orbit sinogram"))))
         return rc;
-    if (need > p->split_cap) {
-        long long cap = (long long)p->split_cap;
-        if ((rc = grow(&p->d_split, &cap, (long long)need, "split partial sums"))) return rc;
-        p->split_cap = (size_t)cap;
-    }
+    if ((rc = grow(&p->d_split, &p->split_cap, (long long)need, "split partial sums"))) return rc;
     // commit: swap the rebuilt parts in (N then frees the old ones)
     if (geo) p->swap_geometry(N);
     if (fwd) p->swap_fwd(N);
@@ -986,11 +1009,13 @@ namespace ctprj {
 size_t Plan::split_need(const ctprj_tune& t, const Tables& F, const Tables& A) const
 {
     size_t need = 0;
+    auto add = [&](bool fwd, int items) {
+        const Shape sh = sym_shape(t, fwd, items);
+        if (sh.split > 1) need = std::max(need, (size_t)items * sh.split);
+    };
     for (int g = 1; g < 4; ++g) {
-        if (t.fwd_split > 1)
-            for (const Segments& c : F.symf) need = std::max(need, (size_t)c.count[g] * t.fwd_split);
-        if (t.adj_split > 1)
-            for (const Segments& c : A.syma) need = std::max(need, (size_t)c.count[g] * t.adj_split);
+        for (const Segments& c : F.symf) add(true, c.count[g]);
+        for (const Segments& c : A.syma) add(false, c.count[g]);
     }
     return need * 512;
 }

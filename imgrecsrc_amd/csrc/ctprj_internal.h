@@ -85,7 +85,7 @@ struct Plan : Tables {
     std::vector<ctprj_geom> geoms;
     std::vector<long long> img_offsets, sino_offsets;
     long long img_elems = 0, sino_elems = 0;
-    int max_W = 0;
+    int max_W = 0, max_n = 0;
     ctprj_tune tune{64, 16, 1, 8, 8, 1, 1};
 
     int2* d_fbp_items = nullptr;
@@ -109,7 +109,7 @@ struct Plan : Tables {
     float* d_ie_phi = nullptr;   // I-epsilon step: basis matrix of its projection
     size_t ie_phi_cap = 0;       // bytes held by d_ie_phi
     float* d_split = nullptr;    // partial sums of split symmetric work items
-    size_t split_cap = 0;        // floats held by d_split
+    long long split_cap = 0;     // floats held by d_split
 
     ~Plan();
     // geometry tables for tune flags `flags` into G
@@ -118,6 +118,11 @@ struct Plan : Tables {
     int build_fwd_items(const ctprj_tune& t, Tables& G) const;
     int build_adj_items(const ctprj_tune& t, Tables& G) const;
     int launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st);
+    // waves per item and work-groups per item of a symmetric launch of `items` items
+    struct Shape {
+        int seg, split;
+    };
+    Shape sym_shape(const ctprj_tune& t, bool fwd, int items) const;
     // partial-sum floats the split symmetric launches of tune t need on tables G
     size_t split_need(const ctprj_tune& t, const Tables& fwd, const Tables& adj) const;
     int launch_forward(const float* d_img, float* d_sino, hipStream_t st, bool count);

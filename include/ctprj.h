@@ -127,7 +127,9 @@ typedef struct ctprj_tune {
                         above 1 their partial sums are added in a fixed order by a second
                         launch (more work-groups for small slices) */
     int fwd_split;   /* symmetric forward: work-groups per 64 canonical rays splitting the
-                        image rows, 1-8, the same way */
+                        image rows, 1-8, the same way.  In either direction 8 waves (seg)
+                        with one work-group (split), a new plan's values, leave the shape to
+                        the plan, which takes it from its sizes */
 } ctprj_tune;
 int ctprj_plan_get_tune(const ctprj_plan* plan, ctprj_tune* tune);
 /* Out-of-range fields are refused (CTPRJ_EINVAL) and change nothing.  Splits whose
