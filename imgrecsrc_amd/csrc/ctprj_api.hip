@@ -710,7 +710,7 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
     p->max_W = max_W;
     std::vector<int2> fbpi;
     for (int s = 0; s < nslices; ++s)
-        for (int a = 0; a < geoms[s].np; ++a) fbpi.push_back(make_int2(s, a));
+        for (int a = 0; a < geoms[s].np; a += kFbpItemViews) fbpi.push_back(make_int2(s, a));
     p->n_fbp_items = (int)fbpi.size();
     p->red_cap = bhc_red_doubles(sino);
     if ((rc = upload(&p->d_fbp_items, fbpi, "fbp work list")) ||
@@ -863,9 +863,9 @@ int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool
 
 int Plan::launch_fbp(const float* d_sino, float* d_img, hipStream_t st)
 {
-    const size_t shmem = sizeof(float) * 3 * (size_t)max_W;
-    if (shmem > 160 * 1024) return fail(CTPRJ_EINVAL, "FBP: prjWidth %d too large", max_W);
-    launch_fbp_filter(n_fbp_items, shmem, d_desc, d_fbp_items, d_fbp_kern, d_fbp_kern_off,
+    if (sizeof(float) * 3 * (size_t)max_W > 160 * 1024)
+        return fail(CTPRJ_EINVAL, "FBP: prjWidth %d too large", max_W);
+    launch_fbp_filter(n_fbp_items, max_W, d_desc, d_fbp_items, d_fbp_kern, d_fbp_kern_off,
                       d_fbp_prew, d_fbp_prew_off, d_sino, d_sino_ws, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "fbp filter launch");

@@ -152,7 +152,9 @@ void launch_forward_kernel(bool count, int block, int nitems, const SliceDesc* d
 void launch_adjoint_kernel(int tile, bool fbp, int nitems, const SliceDesc* desc,
                            const AdjItem* items, const float4* views, const Ray* rays,
                            const float* sino, float* img, hipStream_t st);
-void launch_fbp_filter(int nitems, size_t shmem, const SliceDesc* desc, const int2* items,
+// items: (slice, first of up to kFbpItemViews views)
+constexpr int kFbpItemViews = 4;
+void launch_fbp_filter(int nitems, int max_W, const SliceDesc* desc, const int2* items,
                        const float* kern, const long long* kern_off, const float* prew,
                        const long long* prew_off, const float* sino, float* out,
                        hipStream_t st);

@@ -254,43 +254,97 @@ __global__ __launch_bounds__(TILE* TILE) void k_adjoint(const SliceDesc* __restr
 // --------------------------------------------------------------------------- FBP ---
 
 // Fan cosine pre-weight (prj/cpuPrj.c:737-751) and Hann-windowed ramp filter
-// (prj/utils.h:94-151) of one view per work-group.  The FFT filter of the reference is
-// a circular convolution over 2W samples of the zero-padded view with
-// g = 0.5 h + 0.25 h(.-1) + 0.25 h(.+1), h the periodic Ram-Lak kernel; g is tabulated
-// on the host (2W floats per slice at kern_off).  out[i] = sum_j v[j] g[(i-j) mod 2W].
-__global__ __launch_bounds__(256) void k_fbp_filter(const SliceDesc* __restrict__ slices,
-                                                    const int2* __restrict__ items,
-                                                    const float* __restrict__ kern,
-                                                    const long long* __restrict__ kern_off,
-                                                    const float* __restrict__ preweight,
-                                                    const long long* __restrict__ prew_off,
-                                                    const float* __restrict__ sino,
-                                                    float* __restrict__ out)
+// (prj/utils.h:94-151).  The FFT filter of the reference is a circular convolution over 2W
+// samples of the zero-padded view with g = 0.5 h + 0.25 h(.-1) + 0.25 h(.+1), h the periodic
+// Ram-Lak kernel; g is tabulated on the host (2W floats per slice at kern_off).
+// out[i] = sum_j v[j] g[(i-j) mod 2W]: a product with a Toeplitz matrix.
+//
+// A work-group forms 256 outputs of four views; its eight waves split the taps j of each
+// chunk, and a lane keeps 4 outputs x 4 views: per 8 taps it reads 12 values of g (three
+// 16-byte reads, each serving up to 16 products) and 8 x 4 samples (broadcast) for 128 FMAs.
+// One view per work-group with an LDS read of g and of v per product was bound by those
+// reads: 360 views of 729 bins 73 us, now 18.  Products are summed in runs of kFbpRun taps
+// and the runs, and then the eight waves, with compensation.
+constexpr int kFbpViews = kFbpItemViews, kFbpOuts = 256, kFbpWaves = 8, kFbpRun = 64;
+constexpr int kFbpChunk = 1024;  // taps staged at once: a multiple of 8 taps per wave
+
+__global__ __launch_bounds__(64 * kFbpWaves) void k_fbp_filter(
+    const SliceDesc* __restrict__ slices, const int2* __restrict__ items,
+    const float* __restrict__ kern, const long long* __restrict__ kern_off,
+    const float* __restrict__ preweight, const long long* __restrict__ prew_off,
+    const float* __restrict__ sino, float* __restrict__ out)
 {
-    extern __shared__ float sh[];  // W weighted samples + 2W kernel taps
+    __shared__ float4 v[kFbpChunk];                   // v[tap]: the four views' samples
+    __shared__ __attribute__((aligned(16))) float g[kFbpChunk + kFbpOuts];
+    __shared__ float red[kFbpWaves][kFbpViews][kFbpOuts];
     const int2 it = items[blockIdx.x];
     const SliceDesc S = slices[it.x];
-    const int W = S.W, L = 2 * W;
-    float* v = sh;
-    float* g = sh + W;
+    const int W = S.W, L = 2 * W, i0 = (int)blockIdx.y * kFbpOuts;
+    if (i0 >= W) return;  // uniform over the work-group
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
     const float* src = sino + S.sino_off + (long long)it.y * W;
     const float* pw = preweight + prew_off[it.x];
     const float* kk = kern + kern_off[it.x];
-    for (int j = threadIdx.x; j < W; j += blockDim.x) v[j] = src[j] * (S.fan ? pw[j] : 1.0f);
-    for (int j = threadIdx.x; j < L; j += blockDim.x) g[j] = kk[j];
-    __syncthreads();
-    float* dst = out + S.sino_off + (long long)it.y * W;
-    for (int i = threadIdx.x; i < W; i += blockDim.x) {
-        KahanAcc acc;
-        float part = 0.0f;
-        for (int j = 0; j < W; ++j) {
-            int k = i - j;
-            k += (k < 0) ? L : 0;
-            part = fmaf(v[j], g[k], part);
-            if ((j & 63) == 63) { acc.add(part); part = 0.0f; }
+    const int nview = min(kFbpViews, S.np - it.y);
+    KahanAcc acc[kFbpViews][4];
+    for (int j0 = 0; j0 < W; j0 += kFbpChunk) {
+        // taps of this chunk, a multiple of 8 per wave; samples past W are 0
+        const int taps = min(kFbpChunk, (W - j0 + 8 * kFbpWaves - 1) / (8 * kFbpWaves) * (8 * kFbpWaves));
+        __syncthreads();  // the previous chunk's reads are done
+        for (int j = t; j < taps; j += 64 * kFbpWaves) {
+            float q[kFbpViews];
+            const bool in = j0 + j < W;
+            const float w = in && S.fan ? pw[j0 + j] : 1.0f;
+#pragma unroll
+            for (int a = 0; a < kFbpViews; ++a)
+                q[a] = in && a < nview ? src[(long long)a * W + j0 + j] * w : 0.0f;
+            v[j] = make_float4(q[0], q[1], q[2], q[3]);
         }
-        acc.add(part);
-        dst[i] = acc.s;
+        // g[x] is the kernel at i - j = x + i0 - j0 - taps (0 where no output needs it)
+        for (int x = t; x < taps + kFbpOuts; x += 64 * kFbpWaves) {
+            const int k = x + i0 - j0 - taps;
+            g[x] = k > -W && k < W ? kk[k < 0 ? k + L : k] : 0.0f;
+        }
+        __syncthreads();
+        const int per = taps / kFbpWaves, ja = wave * per, jb = ja + per;
+        for (int jr = ja; jr < jb; jr += kFbpRun) {
+            float part[kFbpViews][4] = {};
+            for (int j = jr; j < min(jb, jr + kFbpRun); j += 8) {
+                // outputs i0 + 4 lane + r, taps j0 + j + s: kernel value r - s + 8 of the window
+                const float4* w4 = reinterpret_cast<const float4*>(g + 4 * lane - j + taps - 8);
+                const float4 wa = w4[0], wb = w4[1], wc = w4[2];
+                const float w[12] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y,
+                                     wb.z, wb.w, wc.x, wc.y, wc.z, wc.w};
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    const float4 q = v[j + s];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        part[0][r] = fmaf(q.x, w[r - s + 8], part[0][r]);
+                        part[1][r] = fmaf(q.y, w[r - s + 8], part[1][r]);
+                        part[2][r] = fmaf(q.z, w[r - s + 8], part[2][r]);
+                        part[3][r] = fmaf(q.w, w[r - s + 8], part[3][r]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < kFbpViews; ++a)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[a][r].add(part[a][r]);
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < kFbpViews; ++a)
+        *reinterpret_cast<float4*>(&red[wave][a][4 * lane]) =
+            make_float4(acc[a][0].s, acc[a][1].s, acc[a][2].s, acc[a][3].s);
+    __syncthreads();
+    for (int x = t; x < kFbpViews * kFbpOuts; x += 64 * kFbpWaves) {
+        const int a = x / kFbpOuts, i = x % kFbpOuts;
+        if (a >= nview || i0 + i >= W) continue;
+        KahanAcc sum;
+#pragma unroll
+        for (int w = 0; w < kFbpWaves; ++w) sum.add(red[w][a][i]);
+        out[S.sino_off + (long long)(it.y + a) * W + i0 + i] = sum.s;
     }
 }
 
@@ -355,12 +409,13 @@ void launch_adjoint_kernel(int tile, bool fbp, int nitems, const SliceDesc* desc
     }
 }
 
-void launch_fbp_filter(int nitems, size_t shmem, const SliceDesc* desc, const int2* items,
+void launch_fbp_filter(int nitems, int max_W, const SliceDesc* desc, const int2* items,
                        const float* kern, const long long* kern_off, const float* prew,
                        const long long* prew_off, const float* sino, float* out, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_fbp_filter, dim3(nitems), dim3(256), shmem, st, desc, items, kern,
-                       kern_off, prew, prew_off, sino, out);
+    hipLaunchKernelGGL(k_fbp_filter, dim3(nitems, (max_W + kFbpOuts - 1) / kFbpOuts),
+                       dim3(64 * kFbpWaves), 0, st, desc, items, kern, kern_off, prew, prew_off,
+                       sino, out);
 }
 
 void launch_scale(float* p, long long n, float s, hipStream_t st)
