@@ -2,16 +2,20 @@
 // D >= 0 by the fast gradient projection on the dual (utils/denoise_bound_mod.m, as
 // utils/TV.m:56-80 calls it), isotropic or l1 TV (utils/tlv.m), and the TV value.
 //
-// One iteration is two launches over the pixels: the primal step (C = X - lambda
+// One iteration is one launch over the pixels: the primal step (C = X - lambda
 // Lforward(R), D = max(C, 0), with the FP64 partial sums of ||D - Dold||^2, ||D||^2,
-// ||C - D||^2 and ||C||^2) and the dual step (P = proj(R + Ltrans(D)/(8 lambda)), then
-// the momentum R = P + (tk - 1)(P - Pold)/tkp1).  The dual fields P1 (vertical
-// differences, rows 0..m-2) and P2 (horizontal, columns 0..n-2) are stored padded to
-// m x n.  A one-work-group launch per iteration adds the four sums for the stopping test
-// and the momentum restart and keeps the loop state on the device; the host reads it once
-// per four iterations.  All arithmetic is FP64 in the reference's order; images are FP32.
+// ||C - D||^2 and ||C||^2) at a pixel and its lower and right neighbours, and the pixel's
+// dual step (P = proj(R + Ltrans(D)/(8 lambda)), then the momentum
+// R = P + (tk - 1)(P - Pold)/tkp1, into the other of two R buffers).  Every work-group first
+// adds the previous iteration's partial sums for itself, in one fixed order, and so knows
+// the stopping test's and the momentum restart's outcome without a launch in between.  The
+// dual fields P1 (vertical differences, rows 0..m-2) and P2 (horizontal, columns 0..n-2)
+// are stored padded to m x n.  The host reads the state once per eight iterations, from
+// host memory that a one-work-group launch writes.  All arithmetic is FP64 in the
+// reference's order; images are FP32.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <new>
 #include <vector>
@@ -21,31 +25,45 @@
 namespace ctprj {
 
 constexpr int kTvBlock = 256;
+// Work-groups of an iteration, at most: every one of them reads all the partial sums (32 B
+// each), which 1024 keep at 32 MB a launch from L2; larger images give a group several runs
+// of kTvBlock pixels.  24 iterations at 512^2, 800^2 and 2048^2: 392, 600 and 2357 us with
+// 1024, 401, 728 and 3489 with 512, 452, 1051 and 5868 with 256.
+constexpr long long kTvGroups = 1024;
 
-__device__ __forceinline__ void tv_block_sum4(const double v[4], double* part)
+// Sum of four values over the work-group, the same in every thread: each wave's lanes by
+// a butterfly, then the waves in order.
+__device__ __forceinline__ void tv_group_sum4(double v[4])
 {
-    __shared__ double sh[4][kTvBlock];
-    const int t = threadIdx.x;
+    __shared__ double sh[kTvBlock / 64][4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) sh[k][t] = v[k];
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] += __shfl_xor(v[k], off, 64);
+    const int wave = (int)threadIdx.x >> 6;
+    __syncthreads();  // an earlier call's reads are done
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sh[wave][k] = v[k];
     __syncthreads();
-    for (int off = kTvBlock / 2; off > 0; off >>= 1) {
-        if (t < off) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) sh[k][t] += sh[k][t + off];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
+    for (int k = 0; k < 4; ++k) {
+        v[k] = sh[0][k];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) part[4 * (long long)blockIdx.x + k] = sh[k][0];
+        for (int w = 1; w < kTvBlock / 64; ++w) v[k] += sh[w][k];
     }
 }
 
-// primal step (utils/denoise_bound_mod.m:118-119 with utils/Lforward.m)
-// FGP loop state on the device (utils/denoise_bound_mod.m:95-150): the iteration's
-// kernels read tk from here and k_tv_ctrl updates it, so the host looks at the state once
-// per chunk of iterations; kernels queued after the stop return at once.
+__device__ __forceinline__ void tv_block_sum4(double v[4], double* part)
+{
+    tv_group_sum4(v);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) part[4 * (long long)blockIdx.x + k] = v[k];
+}
+
+// FGP loop state (utils/denoise_bound_mod.m:95-150) before an iteration; launches queued
+// after the stop do nothing.
 struct TvCtl {
     double t;     // tk of the next iteration (the last tkp1, or 1 after a restart)
     double fval;  // objective of the last iteration
@@ -55,126 +73,151 @@ struct TvCtl {
 // tkp1 from tk (utils/denoise_bound_mod.m:117), the same expression wherever it is formed
 __device__ __forceinline__ double tv_next_t(double tk) { return (1.0 + sqrt(1.0 + 4.0 * tk * tk)) / 2.0; }
 
-__global__ __launch_bounds__(kTvBlock) void k_tv_primal(const double* __restrict__ X,
-                                                        double* __restrict__ D,
-                                                        const double* __restrict__ R1,
-                                                        const double* __restrict__ R2, int m,
-                                                        int n, long long total, double lam,
-                                                        double* __restrict__ part,
-                                                        const TvCtl* __restrict__ c)
-{
-    if (c->done) return;  // uniform
-    const long long t = (long long)blockIdx.x * kTvBlock + threadIdx.x;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    if (t < total) {
-        const int j = (int)(t % n);
-        const int i = (int)((t / n) % m);
-        const double x = (i == 0) ? R1[t] : (i == m - 1 ? -R1[t - n] : R1[t] - R1[t - n]);
-        const double y = (j == 0) ? R2[t] : (j == n - 1 ? -R2[t - 1] : R2[t] - R2[t - 1]);
-        const double c = __dsub_rn(X[t], __dmul_rn(lam, x + y));
-        const double d = fmax(c, 0.0);
-        const double e = d - D[t], f = c - d;
-        D[t] = d;
-        v[0] = e * e;
-        v[1] = d * d;
-        v[2] = f * f;
-        v[3] = c * c;
-    }
-    tv_block_sum4(v, part);
-}
-
-// dual step (utils/denoise_bound_mod.m:120-144 with utils/Ltrans.m)
-__global__ __launch_bounds__(kTvBlock) void k_tv_dual(const double* __restrict__ D,
-                                                      double* __restrict__ P1,
-                                                      double* __restrict__ P2,
-                                                      double* __restrict__ R1,
-                                                      double* __restrict__ R2, int m, int n,
-                                                      long long total, double lam, int iso,
-                                                      const TvCtl* __restrict__ c)
-{
-    if (c->done) return;  // uniform
-    const double tk = c->t, tkp1 = tv_next_t(tk);
-    const long long t = (long long)blockIdx.x * kTvBlock + threadIdx.x;
-    if (t >= total) return;
-    const int j = (int)(t % n);
-    const int i = (int)((t / n) % m);
-    const bool has1 = i < m - 1, has2 = j < n - 1;
-    const double d = D[t];
-    const double l8 = 8.0 * lam;
-    double p1 = has1 ? R1[t] + (d - D[t + n]) / l8 : 0.0;
-    double p2 = has2 ? R2[t] + (d - D[t + 1]) / l8 : 0.0;
-    if (iso) {
-        const double a = sqrt(fmax(__dadd_rn(__dmul_rn(p1, p1), __dmul_rn(p2, p2)), 1.0));
-        p1 = p1 / a;
-        p2 = p2 / a;
-    } else {
-        p1 = fmax(fmin(p1, 1.0), -1.0);
-        p2 = fmax(fmin(p2, 1.0), -1.0);
-    }
-    if (has1) {
-        const double o = P1[t];
-        P1[t] = p1;
-        R1[t] = p1 + (tk - 1.0) * (p1 - o) / tkp1;
-    }
-    if (has2) {
-        const double o = P2[t];
-        P2[t] = p2;
-        R2[t] = p2 + (tk - 1.0) * (p2 - o) / tkp1;
-    }
-}
-
-// D = P = R = 0 and the loop state: tk = 1, no iteration yet (utils/denoise_bound_mod.m:60-86)
-__global__ void k_tv_start(double* __restrict__ D, double* __restrict__ P1, double* __restrict__ P2,
-                           double* __restrict__ R1, double* __restrict__ R2, long long total,
-                           int maxIter, TvCtl* __restrict__ c)
-{
-    const long long t = (long long)blockIdx.x * kTvBlock + threadIdx.x;
-    if (t < total) D[t] = P1[t] = P2[t] = R1[t] = R2[t] = 0.0;
-    if (t == 0) {
-        c->t = 1.0;
-        c->fval = INFINITY;
-        c->i = 0;
-        c->count = 0;
-        c->done = maxIter <= 0;
-    }
-}
-
 // End of an iteration (utils/denoise_bound_mod.m:146-150): re = ||D - Dold|| / ||D||
 // counts towards the stop below epsilon, fval = -||C - D||^2 + ||C||^2, a rising fval
 // restarts the momentum (tkp1 = 1); stop after maxIter iterations or 5 in a row below
-// epsilon.  The per-group partials are summed in a fixed order.
-__global__ __launch_bounds__(kTvBlock) void k_tv_ctrl(const double* __restrict__ part,
-                                                      long long nblk, double epsilon,
-                                                      int maxIter, TvCtl* __restrict__ c)
+// epsilon.  The per-group partials are summed in a fixed order; every thread of the
+// work-group gets the state.
+__device__ __forceinline__ TvCtl tv_advance(TvCtl c, const double* __restrict__ part,
+                                            long long nblk, double epsilon, int maxIter)
 {
-    if (c->done) return;
-    __shared__ double sh[4][kTvBlock];
-    const int t = threadIdx.x;
+    if (c.done) return c;  // uniform
     double a[4] = {0.0, 0.0, 0.0, 0.0};
-    for (long long b = t; b < nblk; b += kTvBlock)
+    for (long long b = threadIdx.x; b < nblk; b += kTvBlock)
 #pragma unroll
         for (int k = 0; k < 4; ++k) a[k] += part[4 * b + k];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) sh[k][t] = a[k];
-    __syncthreads();
-    for (int off = kTvBlock / 2; off > 0; off >>= 1) {
-        if (t < off) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) sh[k][t] += sh[k][t + off];
+    tv_group_sum4(a);
+    const double re = sqrt(a[0]) / sqrt(a[1]);
+    const double fval = -a[2] + a[3];
+    const double tkp1 = tv_next_t(c.t);
+    c.count = (re < epsilon) ? c.count + 1 : 0;
+    c.t = (fval > c.fval) ? 1.0 : tkp1;
+    c.fval = fval;
+    c.i += 1;
+    c.done = c.i >= maxIter || c.count >= 5;
+    return c;
+}
+
+// What an iteration reads at pixel t = (i, j) of its image: X and R at the pixel, its lower
+// and right neighbours and what their differences take (zero outside the image), D and P.
+struct TvPix {
+    int i, j;
+    double x, xd, xr;              // X at t, t + n, t + 1
+    double r1, r1u, r1d, r1r, r1q;  // R1 at t, t - n, t + n, t + 1, t + 1 - n
+    double r2, r2l, r2r, r2d, r2q;  // R2 at t, t - 1, t + 1, t + n, t + n - 1
+    double d, p1, p2;
+};
+
+__device__ __forceinline__ TvPix tv_load(const double* __restrict__ X, const double* D,
+                                         const double* P1, const double* P2,
+                                         const double* __restrict__ R1,
+                                         const double* __restrict__ R2, long long t, int m, int n)
+{
+    TvPix q;
+    const unsigned row = (unsigned)t / (unsigned)n;  // fewer than 2^31 pixels
+    q.j = (int)((unsigned)t - row * (unsigned)n);
+    q.i = (int)(row % (unsigned)m);
+    const bool up = q.i > 0, left = q.j > 0, down = q.i < m - 1, right = q.j < n - 1;
+    q.x = X[t];
+    q.xd = down ? X[t + n] : 0.0;
+    q.xr = right ? X[t + 1] : 0.0;
+    q.r1 = R1[t];
+    q.r1u = up ? R1[t - n] : 0.0;
+    q.r1d = down ? R1[t + n] : 0.0;
+    q.r1r = right ? R1[t + 1] : 0.0;
+    q.r1q = right && up ? R1[t + 1 - n] : 0.0;
+    q.r2 = R2[t];
+    q.r2l = left ? R2[t - 1] : 0.0;
+    q.r2r = right ? R2[t + 1] : 0.0;
+    q.r2d = down ? R2[t + n] : 0.0;
+    q.r2q = down && left ? R2[t + n - 1] : 0.0;
+    q.d = D[t];
+    q.p1 = P1[t];
+    q.p2 = P2[t];
+    return q;
+}
+
+// C = X - lambda Lforward(R) (utils/Lforward.m) from X and R1, R2 at the pixel and at the
+// upper and left ones; R1 is zero on the last row and R2 on the last column.
+__device__ __forceinline__ double tv_primal(double x, double r1, double r1u, double r2, double r2l,
+                                            double lam)
+{
+    return __dsub_rn(x, __dmul_rn(lam, (r1 - r1u) + (r2 - r2l)));
+}
+
+// Iteration c0's state says (utils/denoise_bound_mod.m:118-144 with utils/Lforward.m and
+// utils/Ltrans.m).  first: that state is complete; otherwise it is the previous
+// iteration's, whose partial sums are in part0.  Group 0 keeps the new state in c1.
+// Bound by the chain state -> partial sums -> pixels -> partial sums at small images, by the
+// 88 B a pixel moves at large ones; so a group's first pixels are requested before the sums
+// are added: 24 iterations with their launches take 358 us at 512^2 and 2.04 ms at 2048^2, 398
+// and 2.36 ms without that, and 586 and 2.65 ms as primal, dual and control launches.
+__global__ __launch_bounds__(kTvBlock) void k_tv_iter(
+    const double* __restrict__ X, double* __restrict__ D, double* __restrict__ P1,
+    double* __restrict__ P2, const double* __restrict__ R1, const double* __restrict__ R2,
+    double* __restrict__ N1, double* __restrict__ N2, int m, int n, long long total,
+    long long chunk, double lam, int iso, double epsilon, int maxIter, int first,
+    const double* __restrict__ part0, double* __restrict__ part1, const TvCtl* __restrict__ c0,
+    TvCtl* __restrict__ c1)
+{
+    const long long end = min(total, (blockIdx.x + 1) * chunk);
+    long long t = blockIdx.x * chunk + threadIdx.x;
+    TvPix q = {};
+    if (t < end) q = tv_load(X, D, P1, P2, R1, R2, t, m, n);
+    TvCtl c = *c0;
+    if (!first) c = tv_advance(c, part0, gridDim.x, epsilon, maxIter);
+    if (c1 != c0 && blockIdx.x == 0 && threadIdx.x == 0) *c1 = c;
+    if (c.done) return;  // uniform
+    const double tk = c.t, tkp1 = tv_next_t(tk), l8 = 8.0 * lam;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    while (t < end) {
+        const bool has1 = q.i < m - 1, has2 = q.j < n - 1;
+        const double cc = tv_primal(q.x, q.r1, q.r1u, q.r2, q.r2l, lam);
+        const double d = fmax(cc, 0.0);
+        const double e = d - q.d, f = cc - d;
+        D[t] = d;
+        v[0] += e * e;
+        v[1] += d * d;
+        v[2] += f * f;
+        v[3] += cc * cc;
+        double p1 = 0.0, p2 = 0.0;
+        if (has1)
+            p1 = q.r1 + (d - fmax(tv_primal(q.xd, q.r1d, q.r1, q.r2d, q.r2q, lam), 0.0)) / l8;
+        if (has2)
+            p2 = q.r2 + (d - fmax(tv_primal(q.xr, q.r1r, q.r1q, q.r2r, q.r2, lam), 0.0)) / l8;
+        if (iso) {
+            // (inside the unit ball the divisor is 1)
+            const double s = fmax(__dadd_rn(__dmul_rn(p1, p1), __dmul_rn(p2, p2)), 1.0);
+            if (s > 1.0) {
+                const double a = sqrt(s);
+                p1 = p1 / a;
+                p2 = p2 / a;
+            }
+        } else {
+            p1 = fmax(fmin(p1, 1.0), -1.0);
+            p2 = fmax(fmin(p2, 1.0), -1.0);
         }
-        __syncthreads();
+        // (zero on the last row and on the last column)
+        P1[t] = p1;
+        N1[t] = p1 + (tk - 1.0) * (p1 - q.p1) / tkp1;
+        P2[t] = p2;
+        N2[t] = p2 + (tk - 1.0) * (p2 - q.p2) / tkp1;
+        t += kTvBlock;
+        if (t < end) q = tv_load(X, D, P1, P2, R1, R2, t, m, n);
     }
-    if (t != 0) return;
-    const double re = sqrt(sh[0][0]) / sqrt(sh[1][0]);
-    const int count = (re < epsilon) ? c->count + 1 : 0;
-    const double fval = -sh[2][0] + sh[3][0];
-    const double tkp1 = tv_next_t(c->t);
-    const int i = c->i + 1;
-    c->t = (fval > c->fval) ? 1.0 : tkp1;
-    c->fval = fval;
-    c->count = count;
-    c->i = i;
-    c->done = i >= maxIter || count >= 5;
+    tv_block_sum4(v, part1);
+}
+
+// The state after an iteration, into c1 and host memory.
+__global__ __launch_bounds__(kTvBlock) void k_tv_state(const double* __restrict__ part,
+                                                       long long nblk, double epsilon,
+                                                       int maxIter, const TvCtl* __restrict__ c0,
+                                                       TvCtl* __restrict__ c1, TvCtl* host)
+{
+    const TvCtl c = tv_advance(*c0, part, nblk, epsilon, maxIter);
+    if (threadIdx.x != 0) return;
+    *c1 = c;
+    *host = c;
 }
 
 // Support mask (utils/maskFunc.m): pixels where mask is 0 are zero; NULL keeps all.
@@ -202,11 +245,19 @@ __global__ __launch_bounds__(kTvBlock) void k_tv_value(const float* __restrict__
     tv_block_sum4(v, part);
 }
 
-__global__ void k_tv_in(const float* __restrict__ in, double* __restrict__ out, long long n,
-                        const float* __restrict__ mask)
+// The input image and D = 0, P = proj(Ltrans(0)) = 0, R = P, and the loop state: tk = 1, no
+// iteration yet (utils/denoise_bound_mod.m:60-86)
+__global__ void k_tv_in(const float* __restrict__ in, double* __restrict__ X,
+                        double* __restrict__ D, double* __restrict__ P1, double* __restrict__ P2,
+                        double* __restrict__ R1, double* __restrict__ R2, long long n,
+                        const float* __restrict__ mask, TvCtl* __restrict__ c)
 {
     const long long i = (long long)blockIdx.x * kTvBlock + threadIdx.x;
-    if (i < n) out[i] = tv_masked(mask, i, (double)in[i]);
+    if (i < n) {
+        X[i] = tv_masked(mask, i, (double)in[i]);
+        D[i] = P1[i] = P2[i] = R1[i] = R2[i] = 0.0;
+    }
+    if (i == 0) *c = TvCtl{1.0, INFINITY, 0, 0, 0, 0};
 }
 
 __global__ void k_tv_out(const double* __restrict__ in, float* __restrict__ out, long long n,
@@ -223,16 +274,20 @@ using namespace ctprj;
 struct ctprj_tv {
     int rows = 0, cols = 0, batch = 0, iso = 1;
     long long n = 0, blocks = 0;
-    double *d_X = nullptr, *d_D = nullptr, *d_P1 = nullptr, *d_P2 = nullptr, *d_R1 = nullptr,
-           *d_R2 = nullptr, *d_part = nullptr;
-    TvCtl* d_ctl = nullptr;   // the FGP loop's state
+    double *d_X = nullptr, *d_D = nullptr, *d_P1 = nullptr, *d_P2 = nullptr, *d_part = nullptr;
+    double *d_R1[2] = {nullptr, nullptr}, *d_R2[2] = {nullptr, nullptr};  // by parity of the iteration
+    double* d_sums = nullptr;  // partial sums of an iteration, by its parity
+    TvCtl* d_ctl = nullptr;    // the FGP loop's state, by the iteration's parity
+    TvCtl* h_ctl = nullptr;    // ... as the host reads it (pinned)
     float* d_mask = nullptr;  // support (NULL: every pixel)
     std::vector<double> part;
     ~ctprj_tv()
     {
-        for (void* p : {(void*)d_X, (void*)d_D, (void*)d_P1, (void*)d_P2, (void*)d_R1, (void*)d_R2,
-                        (void*)d_part, (void*)d_ctl, (void*)d_mask})
+        for (void* p : {(void*)d_X, (void*)d_D, (void*)d_P1, (void*)d_P2, (void*)d_R1[0],
+                        (void*)d_R1[1], (void*)d_R2[0], (void*)d_R2[1], (void*)d_part,
+                        (void*)d_sums, (void*)d_ctl, (void*)d_mask})
             if (p) (void)hipFree(p);
+        if (h_ctl) (void)hipHostFree(h_ctl);
     }
 };
 
@@ -256,10 +311,13 @@ extern "C" int ctprj_tv_create(int rows, int cols, int batch, int iso, ctprj_tv*
     w->blocks = (n + kTvBlock - 1) / kTvBlock;
     w->part.assign((size_t)4 * w->blocks, 0.0);
     hipError_t e = hipSuccess;
-    for (double** p : {&w->d_X, &w->d_D, &w->d_P1, &w->d_P2, &w->d_R1, &w->d_R2})
+    for (double** p : {&w->d_X, &w->d_D, &w->d_P1, &w->d_P2, &w->d_R1[0], &w->d_R1[1], &w->d_R2[0],
+                       &w->d_R2[1]})
         if (e == hipSuccess) e = hipMalloc((void**)p, sizeof(double) * (size_t)n);
     if (e == hipSuccess) e = hipMalloc((void**)&w->d_part, sizeof(double) * 4 * (size_t)w->blocks);
-    if (e == hipSuccess) e = hipMalloc((void**)&w->d_ctl, sizeof(TvCtl));
+    if (e == hipSuccess) e = hipMalloc((void**)&w->d_sums, sizeof(double) * 8 * kTvGroups);
+    if (e == hipSuccess) e = hipMalloc((void**)&w->d_ctl, 2 * sizeof(TvCtl));
+    if (e == hipSuccess) e = hipHostMalloc((void**)&w->h_ctl, sizeof(TvCtl), hipHostMallocDefault);
     if (e != hipSuccess) {
         delete w;
         return fail(CTPRJ_ENOMEM, "tv workspace: %s", hipGetErrorString(e));
@@ -326,36 +384,38 @@ extern "C" int ctprj_tv_denoise(ctprj_tv* w, const float* d_x, double lambda, do
     hipStream_t st = (hipStream_t)stream;
     const long long n = w->n;
     const unsigned g = (unsigned)w->blocks;
-    hipLaunchKernelGGL(k_tv_in, dim3(g), dim3(kTvBlock), 0, st, d_x, w->d_X, n, w->d_mask);
-    // D = 0, P = proj(Ltrans(0)) = 0, R = P   (utils/denoise_bound_mod.m:60-86)
+    // a group's pixels: a multiple of kTvBlock, kTvGroups groups at most
+    const long long chunk = (w->blocks + kTvGroups - 1) / kTvGroups * kTvBlock;
+    const unsigned groups = (unsigned)((n + chunk - 1) / chunk);
     TvCtl* C = w->d_ctl;
-    hipLaunchKernelGGL(k_tv_start, dim3(g), dim3(kTvBlock), 0, st, w->d_D, w->d_P1, w->d_P2,
-                       w->d_R1, w->d_R2, n, maxIter, C);
-    // iterations in chunks of kTvChunk, the host reading the state after each chunk
-    constexpr int kTvChunk = 4;
-    TvCtl h{};
-    // the stop comes after at most maxIter iterations
-    const long long max_chunks = (long long)maxIter / kTvChunk + 2;
-    for (long long chunk = 0;; ++chunk) {
-        if (chunk == max_chunks)
-            return fail(CTPRJ_EHIP, "tv_denoise: the loop state did not stop");
-        for (int k = 0; k < kTvChunk; ++k) {
-            hipLaunchKernelGGL(k_tv_primal, dim3(g), dim3(kTvBlock), 0, st, w->d_X, w->d_D,
-                               w->d_R1, w->d_R2, w->rows, w->cols, n, lambda, w->d_part, C);
-            hipLaunchKernelGGL(k_tv_dual, dim3(g), dim3(kTvBlock), 0, st, w->d_D, w->d_P1,
-                               w->d_P2, w->d_R1, w->d_R2, w->rows, w->cols, n, lambda, w->iso, C);
-            hipLaunchKernelGGL(k_tv_ctrl, dim3(1), dim3(kTvBlock), 0, st, w->d_part, w->blocks,
-                               epsilon, maxIter, C);
+    hipLaunchKernelGGL(k_tv_in, dim3(g), dim3(kTvBlock), 0, st, d_x, w->d_X, w->d_D, w->d_P1,
+                       w->d_P2, w->d_R1[0], w->d_R2[0], n, w->d_mask, C);
+    // iterations in batches of kTvBatch, the host reading the state after each
+    constexpr int kTvBatch = 8;
+    int it = 0;
+    bool done = maxIter <= 0;
+    while (!done) {
+        const int stop = it + std::min(kTvBatch, maxIter - it);
+        for (const int begin = it; it < stop; ++it) {
+            const int a = it & 1, first = it == begin;
+            hipLaunchKernelGGL(k_tv_iter, dim3(groups), dim3(kTvBlock), 0, st, w->d_X, w->d_D,
+                               w->d_P1, w->d_P2, w->d_R1[a], w->d_R2[a], w->d_R1[1 - a],
+                               w->d_R2[1 - a], w->rows, w->cols, n, chunk, lambda, w->iso,
+                               epsilon, maxIter, first, w->d_sums + 4 * kTvGroups * (1 - a),
+                               w->d_sums + 4 * kTvGroups * a, first ? C + a : C + 1 - a, C + a);
         }
+        const int a = (it - 1) & 1;
+        hipLaunchKernelGGL(k_tv_state, dim3(1), dim3(kTvBlock), 0, st,
+                           w->d_sums + 4 * kTvGroups * a, (long long)groups, epsilon, maxIter,
+                           C + a, C + 1 - a, w->h_ctl);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "tv iteration launch");
-        e = hipMemcpyAsync(&h, C, sizeof(h), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) return hip_fail(e, "tv state");
-        if (h.done) break;
+        if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(e, "tv state");
+        done = w->h_ctl->done != 0;
+        if (!done && it >= maxIter) return fail(CTPRJ_EHIP, "tv_denoise: the loop state did not stop");
     }
     hipLaunchKernelGGL(k_tv_out, dim3(g), dim3(kTvBlock), 0, st, w->d_D, d_out, n, w->d_mask);
-    if (iterations) *iterations = h.i;
+    if (iterations) *iterations = maxIter <= 0 ? 0 : w->h_ctl->i;
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : hip_fail(e, "tv output");
 }

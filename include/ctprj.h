@@ -328,7 +328,7 @@ int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, double u, double
  * Total-variation proximal step (opt.proximal = 'tvl1' / 'tviso',
  * bhc/beamhardenSpline.m:215-224 -> utils/TV.m:56-80 -> utils/denoise_bound_mod.m): a
  * context holds `batch` images of rows x cols (rows, cols >= 2) and the TV type
- * (iso != 0: isotropic, else l1).  FP64 state (six image-sized buffers), FP32 images.
+ * (iso != 0: isotropic, else l1).  FP64 state (eight image-sized buffers), FP32 images.
  * ------------------------------------------------------------------------------ */
 typedef struct ctprj_tv ctprj_tv;
 int ctprj_tv_create(int rows, int cols, int batch, int iso, ctprj_tv** out);
@@ -343,7 +343,7 @@ int ctprj_tv_value(ctprj_tv* w, const float* d_x, double* tv, void* stream);
  * maxIter iterations or when ||D - Dold|| / ||D|| < epsilon five times in a row; the
  * dual starts at zero (TV.denoise does not forward its init).  Norms and the stopping
  * test run over all images of the context together.  *iterations gets the count.
- * The loop state stays on the device; the host reads it once per four iterations. */
+ * The loop state stays on the device; the host reads it once per eight iterations. */
 int ctprj_tv_denoise(ctprj_tv* w, const float* d_a, double lambda, double epsilon,
                      int maxIter, float* d_out, int* iterations, void* stream);
 
