@@ -12,7 +12,7 @@
 // all coarser levels there.  The taps are kernel arguments.  All arithmetic is FP64 in
 // the reference's summation order; images enter and leave as FP32.  The ADMM loop keeps
 // its state (rho, counters, the stop flag) on the device and is read by the host once
-// per chunk of iterations.
+// per chunk of iterations; with two taps one launch does a whole iteration.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -654,6 +654,416 @@ __global__ void k_admm_final(const double* __restrict__ a, const double* __restr
                      scale);
 }
 
+// ---- the two-tap ADMM (taps of length 2: Haar's) --------------------------------------
+// Without overlap between taps the L levels of a transform are 2^L x 2^L blocks that know
+// nothing of each other, so an iteration of the ADMM is one launch: a work-group takes a
+// tile of S x S pixels (S = 32 for up to 5 levels, 64 for 6), reads its coefficients,
+// forms Psi(s + nu), alpha, Psit(alpha) and the shrink, and writes the coefficients back.
+// A thread owns a 2 x 2 quad of the finest level and at most one quad of a coarser level;
+// the approximations pass through LDS, one barrier per level.  Every work-group first adds
+// the previous iteration's partial sums, in one order, and knows the loop state from them.
+// Sums and products within the transforms are those of the level kernels, in their order.
+// Bound by latency (64 work-groups at 512^2 and 6 levels, 12.5 us an iteration where its 14 MB
+// would take 3): 13 iterations there take 206 us, as 11 launches each 836.
+
+struct HaarTaps {
+    double lo0, lo1, hi0, hi1, e0, e1, o0, o1;
+};
+
+constexpr int kHaarMaxLevels = 6;
+constexpr int kHaarGroups = 1024;  // work-groups of an iteration, at most: each reads all the sums
+
+constexpr __host__ __device__ int haar_tile(int L) { return L > 5 ? 64 : 32; }
+
+// Offset of level l's approximations within the tile's (side S >> (l + 1) each)
+template <int S>
+constexpr __host__ __device__ int haar_off(int l)
+{
+    int o = 0;
+    for (int m = 0; m < l; ++m) o += (S >> (m + 1)) * (S >> (m + 1));
+    return o;
+}
+
+// A quad of coefficients: the approximation (only at the last level), and the details of
+// (low row, high column), (high, low), (high, high).
+struct HaarQuad {
+    int lev, r, c;  // level and place in the tile
+    bool on, ll;    // inside the image; the last level
+    unsigned g[4];
+    double s[4], nu[4];
+};
+
+// the quad's indices in image `img` for the tile at (r0, c0)
+template <int S>
+__device__ __forceinline__ void haar_place(HaarQuad& q, int img, int r0, int c0, int rows, int cols,
+                                           int L)
+{
+    const int l1 = q.lev + 1, P = (r0 >> l1) + q.r, Q = (c0 >> l1) + q.c, M = rows >> l1,
+              H = cols >> l1;
+    q.on = q.lev < L && P < M && Q < H;
+    q.ll = q.lev == L - 1;
+    const unsigned b = (unsigned)img * (unsigned)rows * (unsigned)cols;
+    q.g[0] = b + (unsigned)P * cols + Q;
+    q.g[1] = q.g[0] + H;
+    q.g[2] = q.g[0] + (unsigned)M * cols;
+    q.g[3] = q.g[2] + H;
+}
+
+__device__ __forceinline__ void haar_read(HaarQuad& q, const double* s, const double* nu)
+{
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const bool have = q.on && (k > 0 || q.ll);
+        q.s[k] = have ? s[q.g[k]] : 0.0;
+        q.nu[k] = have ? nu[q.g[k]] : 0.0;
+    }
+}
+
+// Pixels (0,0) (0,1) (1,0) (1,1) of a quad from its coefficients: columns, then rows.
+__device__ __forceinline__ void haar_synth(const HaarTaps& T, const double v[4], double x[4])
+{
+    auto pair = [](double lo, double a, double hi, double b) {
+        return __dadd_rn(__dadd_rn(0.0, __dmul_rn(lo, a)), __dmul_rn(hi, b));
+    };
+    const double el = pair(v[0], T.e0, v[2], T.e1), ol = pair(v[0], T.o0, v[2], T.o1);
+    const double eh = pair(v[1], T.e0, v[3], T.e1), oh = pair(v[1], T.o0, v[3], T.o1);
+    x[0] = pair(el, T.e0, eh, T.e1);
+    x[1] = pair(el, T.o0, eh, T.o1);
+    x[2] = pair(ol, T.e0, oh, T.e1);
+    x[3] = pair(ol, T.o0, oh, T.o1);
+}
+
+// ... and back: rows, then columns.
+__device__ __forceinline__ void haar_analyse(const HaarTaps& T, const double x[4], double v[4])
+{
+    auto pair = [](double a, double ta, double b, double tb) {
+        return __dadd_rn(__dadd_rn(0.0, __dmul_rn(a, ta)), __dmul_rn(b, tb));
+    };
+    const double l0 = pair(x[0], T.lo0, x[1], T.lo1), h0 = pair(x[0], T.hi0, x[1], T.hi1);
+    const double l1 = pair(x[2], T.lo0, x[3], T.lo1), h1 = pair(x[2], T.hi0, x[3], T.hi1);
+    v[0] = pair(l0, T.lo0, l1, T.lo1);
+    v[1] = pair(h0, T.lo0, h1, T.lo1);
+    v[2] = pair(l0, T.hi0, l1, T.hi1);
+    v[3] = pair(h0, T.hi0, h1, T.hi1);
+}
+
+// Sums of two values over a work-group of NT threads, the same in every thread.
+template <int NT>
+__device__ __forceinline__ void haar_sum2(double& a, double& b)
+{
+    __shared__ double sh[NT / 64][2];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off, 64);
+        b += __shfl_xor(b, off, 64);
+    }
+    __syncthreads();  // an earlier call's reads are done
+    if ((threadIdx.x & 63) == 0) {
+        sh[threadIdx.x >> 6][0] = a;
+        sh[threadIdx.x >> 6][1] = b;
+    }
+    __syncthreads();
+    a = sh[0][0];
+    b = sh[0][1];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) {
+        a += sh[w][0];
+        b += sh[w][1];
+    }
+}
+
+template <int NT>
+__device__ __forceinline__ void haar_total2(const double* __restrict__ part, int nparts, double& a,
+                                            double& b)
+{
+    a = b = 0.0;
+    for (int i = threadIdx.x; i < nparts; i += NT) {
+        a += part[2 * i];
+        b += part[2 * i + 1];
+    }
+    haar_sum2<NT>(a, b);
+}
+
+// The loop state after the iteration whose partial sums are ds2 and rs2 (npg/admm.m:35-50),
+// as k_admm_ctrl forms it.
+__device__ __forceinline__ AdmmCtl haar_advance(AdmmCtl c, double ds2, double rs2)
+{
+    c.itr += 1;
+    c.cnt += 1;
+    c.f = 1.0;
+    const double difS = sqrt(ds2), residual = sqrt(rs2);
+    c.done = c.itr > c.maxItr || (difS <= c.relTol && residual <= c.relTol);
+    if (!c.done && c.cnt > 20) {
+        if (difS > 10 * residual) {
+            c.rho = c.rho / 2;
+            c.f = 2.0;
+            c.cnt = 0;
+        } else if (difS < residual / 10) {
+            c.rho = c.rho * 2;
+            c.f = 0.5;
+            c.cnt = 0;
+        }
+    }
+    return c;
+}
+
+// The input with its support, kept in FP32 (a copy: the caller may reuse its own before the
+// output is written), and the partial sums of its squares.
+__global__ __launch_bounds__(kWvBlock) void k_haar_in(const float* __restrict__ in,
+                                                      float* __restrict__ a, long long n,
+                                                      const float* __restrict__ mask,
+                                                      double* __restrict__ part)
+{
+    double q = 0.0, z = 0.0;
+    for (long long i = (long long)blockIdx.x * kWvBlock + threadIdx.x; i < n;
+         i += (long long)gridDim.x * kWvBlock) {
+        const double v = masked(mask, i, (double)in[i]);
+        a[i] = (float)v;
+        q += v * v;
+    }
+    haar_sum2<kWvBlock>(q, z);
+    if (threadIdx.x == 0) {
+        part[2 * blockIdx.x] = q;
+        part[2 * blockIdx.x + 1] = 0.0;
+    }
+}
+
+enum HaarMode { kHaarFirst, kHaarFresh, kHaarNext, kHaarFinal };
+
+struct HaarArgs {
+    HaarTaps T;
+    const float *a, *init, *mask, *cmask;
+    double *s, *nu;
+    float* out;
+    int rows, cols, batch, L;
+    double u, relTol;
+    int maxItr, nparts;
+    const double* part0;
+    double* part1;
+    const AdmmCtl* c0;
+    AdmmCtl* c1;
+};
+
+// MODE kHaarFirst: the state from the input's sums, s = preS = Psit(init / scale), nu = 0,
+// then the first iteration; kHaarFresh: an iteration from the complete state c0; kHaarNext:
+// one whose predecessor's sums are in part0, the state kept in c1; kHaarFinal: the output
+// (npg/admm.m:52).
+template <int S, int MODE>
+__global__ __launch_bounds__(S* S / 4) void k_haar_admm(HaarArgs A)
+{
+    constexpr int NT = S * S / 4;
+    __shared__ __attribute__((aligned(16))) double LL[haar_off<S>(kHaarMaxLevels)];
+    const int t = threadIdx.x;
+    const int tr = (A.rows + S - 1) / S, tc = (A.cols + S - 1) / S, tiles = tr * tc * A.batch;
+    HaarQuad q0, q1;
+    q0.lev = 0;
+    q0.r = t / (S / 2);
+    q0.c = t % (S / 2);
+    q1.lev = kHaarMaxLevels;  // none
+    q1.r = q1.c = 0;
+#pragma unroll
+    for (int l = 1; l < kHaarMaxLevels && (S >> (l + 1)) > 0; ++l) {
+        const int side = S >> (l + 1), i = t - (haar_off<S>(l) - haar_off<S>(1));
+        if (i >= 0 && i < side * side) {
+            q1.lev = l;
+            q1.r = i / side;
+            q1.c = i % side;
+        }
+    }
+    const int side1 = S >> (q1.lev + 1);
+    int own = 0, from = 0;  // the coarser quad's own approximation and the finer level's
+#pragma unroll
+    for (int l = 1; l < kHaarMaxLevels; ++l)
+        if (q1.lev == l) {
+            own = haar_off<S>(l) + q1.r * side1 + q1.c;
+            from = haar_off<S>(l - 1) + 2 * q1.r * (2 * side1) + 2 * q1.c;
+        }
+    double2* fine0 = (double2*)(LL + from);
+    double2* fine1 = (double2*)(LL + from + 2 * side1);
+    const int own0 = q0.r * (S / 2) + q0.c;
+
+    auto synth = [&](double x[4]) {  // Psi(s + nu) at the thread's pixels
+        double v[4];
+        for (int l = A.L - 1; l > 0; --l) {
+            if (q1.lev == l) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = q1.s[k] + q1.nu[k];
+                if (!q1.ll) v[0] = LL[own];
+                haar_synth(A.T, v, x);
+                *fine0 = make_double2(x[0], x[1]);
+                *fine1 = make_double2(x[2], x[3]);
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = q0.s[k] + q0.nu[k];
+        if (!q0.ll) v[0] = LL[own0];
+        haar_synth(A.T, v, x);
+    };
+    // Psit of the thread's pixels: its quads' coefficients, zero off their support
+    auto analyse = [&](const double x[4], double p0[4], double p1[4]) {
+        haar_analyse(A.T, x, p0);
+        if (!q0.ll) LL[own0] = p0[0];
+        for (int l = 1; l < A.L; ++l) {
+            __syncthreads();
+            if (q1.lev == l) {
+                const double2 a = *fine0, b = *fine1;
+                const double y[4] = {a.x, a.y, b.x, b.y};
+                haar_analyse(A.T, y, p1);
+                if (!q1.ll) LL[own] = p1[0];
+            }
+        }
+    };
+
+    double ds = 0.0, rs = 0.0;
+    AdmmCtl c;
+    bool have = false;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int img = tile / (tr * tc), ij = tile - img * (tr * tc), ti = ij / tc,
+                  r0 = ti * S, c0 = (ij - ti * tc) * S;
+        haar_place<S>(q0, img, r0, c0, A.rows, A.cols, A.L);
+        haar_place<S>(q1, img, r0, c0, A.rows, A.cols, A.L);
+        // the quad's pixels
+        const bool px = q0.on;
+        const unsigned i0 = (unsigned)img * (unsigned)A.rows * (unsigned)A.cols +
+                            (unsigned)(r0 + 2 * q0.r) * A.cols + (unsigned)(c0 + 2 * q0.c);
+        const unsigned at[4] = {i0, i0 + 1, i0 + A.cols, i0 + A.cols + 1};
+        double a[4];
+        bool in[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            a[k] = px ? (double)A.a[at[k]] : 0.0;
+            in[k] = px && (!A.mask || A.mask[at[k]] != 0.0f);
+        }
+        double x[4] = {0.0, 0.0, 0.0, 0.0};
+        if (MODE == kHaarFirst) {
+            if (A.init) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[k] = in[k] ? (double)A.init[at[k]] : 0.0;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[k] = in[k] ? a[k] : 0.0;
+            }
+        } else {
+            haar_read(q0, A.s, A.nu);
+            haar_read(q1, A.s, A.nu);
+        }
+        // which coefficients are on their support
+        bool m0[4], m1[4];
+        if (MODE != kHaarFinal) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                m0[k] = q0.on && (k > 0 || q0.ll) && (!A.cmask || A.cmask[q0.g[k]] != 0.0f);
+                m1[k] = q1.on && (k > 0 || q1.ll) && (!A.cmask || A.cmask[q1.g[k]] != 0.0f);
+            }
+        }
+        if (!have) {  // the state, once the first tile's loads are on their way
+            have = true;
+            if (MODE == kHaarFirst) {  // npg/admm.m:17-18
+                double sq, z;
+                haar_total2<NT>(A.part0, A.nparts, sq, z);
+                c.scale = sqrt(sq);
+                c.inv = 1.0 / c.scale;
+                c.u = A.u / c.scale;
+                c.rho = c.f = 1.0;
+                c.itr = c.cnt = c.pad = 0;
+                c.zero = c.done = c.scale == 0.0;
+                c.relTol = A.relTol;
+                c.maxItr = A.maxItr;
+            } else {
+                c = *A.c0;
+                if (MODE == kHaarNext && !c.done) {
+                    double ds2, rs2;
+                    haar_total2<NT>(A.part0, A.nparts, ds2, rs2);
+                    c = haar_advance(c, ds2, rs2);
+                }
+            }
+            if ((MODE == kHaarFirst || MODE == kHaarNext) && blockIdx.x == 0 && t == 0) *A.c1 = c;
+            if (MODE != kHaarFinal && c.done) return;  // uniform
+        }
+        if (MODE == kHaarFinal && c.zero) {
+            if (px)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) A.out[at[k]] = 0.0f;
+            continue;  // uniform
+        }
+        double p0[4] = {0.0, 0.0, 0.0, 0.0}, p1[4] = {0.0, 0.0, 0.0, 0.0};
+        if (MODE == kHaarFirst) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = in[k] ? x[k] * c.inv : 0.0;
+            analyse(x, p0, p1);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                q0.s[k] = m0[k] ? p0[k] : 0.0;
+                q1.s[k] = m1[k] ? p1[k] : 0.0;
+                q0.nu[k] = q1.nu[k] = 0.0;
+            }
+            // the synthesis writes what the analysis read: same thread, no barrier needed
+        } else if (c.f != 1.0) {  // a rho change (npg/admm.m:43-49)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                q0.nu[k] *= c.f;
+                q1.nu[k] *= c.f;
+            }
+        }
+        synth(x);
+        const double rho = c.rho;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            x[k] = fmax(__dadd_rn(a[k] * c.inv, __dmul_rn(rho, in[k] ? x[k] : 0.0)) / (1.0 + rho),
+                        0.0);
+        if (MODE == kHaarFinal) {
+            if (px)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) A.out[at[k]] = (float)(x[k] * c.scale);
+            continue;
+        }
+        analyse(x, p0, p1);
+        // shrink (npg/admm.m:27-33), s before it being preS
+        const double th = fabs(c.u / rho);
+        auto shrink = [&](const HaarQuad& q, const bool m[4], const double p4[4]) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (!(q.on && (k > 0 || q.ll))) continue;
+                const double p = m[k] ? p4[k] : 0.0;
+                const double y = p - q.nu[k];
+                const double si = y > th ? y - th : (y < -th ? y + th : 0.0);
+                A.s[q.g[k]] = si;
+                A.nu[q.g[k]] = q.nu[k] + si - p;
+                const double d = si - q.s[k], r = si - p;
+                ds += d * d;
+                rs += r * r;
+            }
+        };
+        shrink(q0, m0, p0);
+        shrink(q1, m1, p1);
+    }
+    if (MODE != kHaarFinal) {
+        haar_sum2<NT>(ds, rs);
+        if (t == 0) {
+            A.part1[2 * blockIdx.x] = ds;
+            A.part1[2 * blockIdx.x + 1] = rs;
+        }
+    }
+}
+
+// The state after an iteration, into c1 and host memory; the sums in k_haar_admm's order.
+template <int NT>
+__global__ __launch_bounds__(NT) void k_haar_state(const double* __restrict__ part, int nparts,
+                                                   const AdmmCtl* __restrict__ c0,
+                                                   AdmmCtl* __restrict__ c1, AdmmCtl* host)
+{
+    AdmmCtl c = *c0;
+    if (!c.done) {
+        double ds2, rs2;
+        haar_total2<NT>(part, nparts, ds2, rs2);
+        c = haar_advance(c, ds2, rs2);
+    }
+    if (threadIdx.x != 0) return;
+    *c1 = c;
+    *host = c;
+}
+
 }  // namespace ctprj
 
 using namespace ctprj;
@@ -665,7 +1075,9 @@ struct ctprj_wavelet {
     double *d_x = nullptr, *d_y = nullptr;                  // transform ping-pong
     double *d_a = nullptr, *d_s = nullptr, *d_nu = nullptr, *d_pre = nullptr, *d_pa = nullptr;
     double* d_part = nullptr;
-    AdmmCtl* d_ctl = nullptr;  // the prox loop's state
+    AdmmCtl* d_ctl = nullptr;  // the prox loop's state (two-tap: two, by the iteration's parity)
+    double* d_sums = nullptr;  // two-tap prox: an iteration's partial sums, by its parity
+    AdmmCtl* h_ctl = nullptr;  // ... and the state as the host reads it (pinned)
     float* d_mask = nullptr;   // image support (NULL: every pixel)
     hipStream_t cap_stream = nullptr;        // where the ADMM chunk is captured
     hipGraphExec_t chunk_exec = nullptr;     // the captured chunk (rebuilt with new masks)
@@ -678,8 +1090,9 @@ struct ctprj_wavelet {
         if (cap_stream) (void)hipStreamDestroy(cap_stream);
         for (void* p : {(void*)d_x, (void*)d_y, (void*)d_a, (void*)d_s, (void*)d_nu,
                         (void*)d_pre, (void*)d_pa, (void*)d_part, (void*)d_ctl, (void*)d_mask,
-                        (void*)d_cmask})
+                        (void*)d_cmask, (void*)d_sums})
             if (p) (void)hipFree(p);
+        if (h_ctl) (void)hipHostFree(h_ctl);
     }
 };
 
@@ -867,7 +1280,10 @@ extern "C" int ctprj_wavelet_create(int rows, int cols, int batch, const double*
     for (double** p : {&w->d_x, &w->d_y, &w->d_a, &w->d_s, &w->d_nu, &w->d_pre, &w->d_pa})
         if (e == hipSuccess) e = hipMalloc((void**)p, sizeof(double) * (size_t)n);
     if (e == hipSuccess) e = hipMalloc((void**)&w->d_part, sizeof(double) * 2 * (size_t)w->blocks);
-    if (e == hipSuccess) e = hipMalloc((void**)&w->d_ctl, sizeof(AdmmCtl));
+    if (e == hipSuccess) e = hipMalloc((void**)&w->d_ctl, 2 * sizeof(AdmmCtl));
+    if (e == hipSuccess) e = hipMalloc((void**)&w->d_sums, sizeof(double) * 4 * kHaarGroups);
+    if (e == hipSuccess)
+        e = hipHostMalloc((void**)&w->h_ctl, sizeof(AdmmCtl), hipHostMallocDefault);
     if (e != hipSuccess) {
         delete w;
         return fail(CTPRJ_ENOMEM, "wavelet workspace: %s", hipGetErrorString(e));
@@ -1014,6 +1430,76 @@ int admm_graph(ctprj_wavelet* w)
     return e == hipSuccess ? 0 : hip_fail(e, "admm graph");
 }
 
+// The two-tap prox: batches of kHaarBatch iterations, one launch each, the host reading the
+// state after each batch.
+template <int S>
+int haar_admm(ctprj_wavelet* w, const float* d_a, double u, double relTol, int maxItr,
+              const float* d_init, float* d_out, int* iterations, hipStream_t st)
+{
+    constexpr int NT = S * S / 4, kHaarBatch = 8;
+    const long long tiles = (long long)((w->rows + S - 1) / S) * ((w->cols + S - 1) / S) * w->batch;
+    const int groups = (int)std::min<long long>(tiles, kHaarGroups);
+    const int in_groups = (int)std::min<long long>(w->blocks, kHaarGroups);
+    double* sums[2] = {w->d_sums, w->d_sums + 2 * kHaarGroups};
+    AdmmCtl* C = w->d_ctl;
+    HaarArgs A{};
+    const WvTaps& T = w->T;
+    A.T = HaarTaps{T.lo[0], T.lo[1], T.hi[0], T.hi[1], T.e0[0], T.e1[0], T.o0[0], T.o1[0]};
+    float* a = reinterpret_cast<float*>(w->d_a);
+    A.a = a;
+    A.init = d_init;
+    A.mask = w->d_mask;
+    A.cmask = w->d_cmask;
+    A.s = w->d_s;
+    A.nu = w->d_nu;
+    A.out = d_out;
+    A.rows = w->rows;
+    A.cols = w->cols;
+    A.batch = w->batch;
+    A.L = w->L;
+    A.u = u;
+    A.relTol = relTol;
+    A.maxItr = maxItr;
+    const dim3 G((unsigned)groups), B(NT);
+    hipLaunchKernelGGL(k_haar_in, dim3((unsigned)in_groups), dim3(kWvBlock), 0, st, d_a, a, w->n,
+                       w->d_mask, sums[1]);
+    // at most maxItr + 1 iterations
+    const long long most = (long long)maxItr + 1;
+    long long it = 0;
+    for (bool done = false; !done;) {
+        const long long stop = it + std::min<long long>(kHaarBatch, most - it);
+        for (const long long begin = it; it < stop; ++it) {
+            const int p = (int)(it & 1);
+            // iteration `it` reads the state C[p] where the batch begins, else its
+            // predecessor's C[1 - p] and sums, and leaves its own state in C[p]
+            A.part0 = sums[1 - p];
+            A.part1 = sums[p];
+            A.nparts = it == 0 ? in_groups : groups;
+            A.c0 = it == begin ? C + p : C + 1 - p;
+            A.c1 = C + p;
+            if (it == 0)
+                hipLaunchKernelGGL((k_haar_admm<S, kHaarFirst>), G, B, 0, st, A);
+            else if (it == begin)
+                hipLaunchKernelGGL((k_haar_admm<S, kHaarFresh>), G, B, 0, st, A);
+            else
+                hipLaunchKernelGGL((k_haar_admm<S, kHaarNext>), G, B, 0, st, A);
+        }
+        const int p = (int)((it - 1) & 1);
+        hipLaunchKernelGGL((k_haar_state<NT>), dim3(1), B, 0, st, sums[p], groups, C + p, C + 1 - p,
+                           w->h_ctl);
+        int rc = last("admm iteration launch");
+        if (rc) return rc;
+        hipError_t e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return hip_fail(e, "admm state");
+        done = w->h_ctl->done != 0;
+        if (!done && it >= most) return fail(CTPRJ_EHIP, "admm: the loop state did not stop");
+    }
+    A.c0 = C + (it & 1);
+    hipLaunchKernelGGL((k_haar_admm<S, kHaarFinal>), G, B, 0, st, A);
+    if (iterations) *iterations = w->h_ctl->itr;
+    return last("admm output");
+}
+
 }  // namespace
 
 extern "C" int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, double u,
@@ -1027,6 +1513,13 @@ extern "C" int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, doubl
     const long long n = w->n;
     const unsigned g = grid1(n);
     relTol = std::min(1e-3, relTol);  // npg/admm.m:14
+    // taps of length 2 on up to 6 levels: an iteration is one launch (13 iterations of 6 levels
+    // at 512^2: 206 us, 836 by the levels' own launches below; at 96^2 72 and 147 for a call
+    // that stops early)
+    if (w->T.lh == 2 && w->L <= kHaarMaxLevels)
+        return haar_tile(w->L) == 64
+                   ? haar_admm<64>(w, d_a, u, relTol, maxItr, d_init, d_out, iterations, st)
+                   : haar_admm<32>(w, d_a, u, relTol, maxItr, d_init, d_out, iterations, st);
     AdmmCtl* C = w->d_ctl;
     const int* stop = &C->done;
     // scale = ||a||, a /= scale, u /= scale  (npg/admm.m:17-18)
