@@ -569,9 +569,17 @@ static std::vector<Item> group_segments(const std::vector<Item> (&by)[4], const 
     return out;
 }
 
+// Four neighbouring canonical views of a slice on the same walk and bins (fewer at the end
+// of a walk: the others are padding): the items of one work-group of k_forward_views.
+struct FwdQuad {
+    int slice;
+    FwdItem it[4];
+};
+
 int Plan::build_fwd_items(const ctprj_tune& t, Tables& G) const
 {
-    std::vector<FwdItem> items, by[4];
+    std::vector<FwdItem> items;
+    std::vector<FwdQuad> by[4];
     const int B = t.fwd_block;
     for (int s = 0; s < nslices; ++s) {
         const ctprj_geom& g = geoms[s];
@@ -581,9 +589,17 @@ int Plan::build_fwd_items(const ctprj_tune& t, Tables& G) const
             bool fold = false;
             choose_group(g, t.flags, &fold, &canon);
             const int bmax = fold ? pC : bhi;
-            for (int i = 0; i < (int)canon.size(); ++i)
-                for (int b0 = 0; b0 <= bmax; b0 += 64)
-                    by[G.slice_sym[s]].push_back(FwdItem{s, i, b0, 0});
+            // the views steeper than 45 degrees walk columns (none under D4)
+            auto cols = [&](int i) { return 8LL * canon[i] > g.prjFull && 8LL * canon[i] < 3LL * g.prjFull; };
+            for (int i = 0, m; i < (int)canon.size(); i += m) {
+                m = 1;
+                while (m < 4 && i + m < (int)canon.size() && cols(i + m) == cols(i)) ++m;
+                for (int b0 = 0; b0 <= bmax; b0 += 64) {
+                    FwdQuad q{s, {}};
+                    for (int k = 0; k < 4; ++k) q.it[k] = FwdItem{k < m ? s : -1, i + k, b0, cols(i)};
+                    by[G.slice_sym[s]].push_back(q);
+                }
+            }
         } else {
             for (int a = 0; a < g.np; ++a)
                 for (int b0 = 0; b0 < g.prjWidth; b0 += B) items.push_back(FwdItem{s, a, b0, 0});
@@ -591,7 +607,17 @@ int Plan::build_fwd_items(const ctprj_tune& t, Tables& G) const
     }
     const bool spread = !(t.flags & 8);
     items = batch_order(items, geoms, spread, true);
-    std::vector<FwdItem> sym = group_segments(by, G, geoms, spread, true, &G.symf);
+    std::vector<FwdItem> sym;
+    for (const FwdQuad& q : group_segments(by, G, geoms, spread, true, &G.symf))
+        for (FwdItem it : q.it) {
+            if (q.slice < 0) it.slice = -1;
+            sym.push_back(it);
+        }
+    for (Tables::Segments& c : G.symf)
+        for (int g = 1; g < 4; ++g) {
+            c.start[g] *= 4;
+            c.count[g] *= 4;
+        }
     G.n_fwd_items = (int)items.size();
     G.n_symf_items = (int)sym.size();
     int rc = upload(&G.d_fwd_items, items, "forward work list");
@@ -776,24 +802,40 @@ namespace ctprj {
 
 // A new plan's shape, 8 waves in one work-group per item, stands for the plan's own choice:
 // as it is where every image is at most kSmallEdge wide, else 4 waves and as many
-// work-groups per item as give about kFillItems of them (two at least in the forward, whose
-// items differ in cost), within the partial sums' space.
+// work-groups as give about kFill of them, within the partial sums' space.
 // Measured (us, 8 x 1 against the choice): forward 64^2 14.8 / 16.4, 256^2 parallel 31.4 /
-// 22.3, 512^2 fan 108 / 78, 769^2 fan of odd views 343 / 319, 1024^2 fan 207 / 183, 16
-// ragged slices 1265 / 1230, 32 x 512^2 3505 / 3352; adjoint 15.6 / 17.4, 19.4 / 15.3,
-// 67 / 49, 306 / 304, 176 / 159, 1027 / 1023, 2028 / 1993.  The line: at 64^2 the second
-// launch that adds the partial sums costs more than the split gains, at 160^2 (25.6 / 17.6)
-// less; small slices keep one shape so that a batch gives each of them the bits of a
-// one-slice plan.
-constexpr int kSmallEdge = 224, kFillItems = 9000;
+// 22.3, 512^2 fan 108 / 75; adjoint 15.6 / 17.4, 19.4 / 15.3, 67 / 49, 769^2 fan of odd views
+// 306 / 304, 1024^2 fan 176 / 159, 16 ragged slices 1027 / 1023, 32 x 512^2 2028 / 1993.  The
+// line: at 64^2 the second launch that adds the partial sums costs more than the split
+// gains, at 160^2 (25.6 / 17.6) less; small slices keep one shape so that a batch gives each
+// of them the bits of a one-slice plan.
+// Four waves of the forward share the staged rows of four neighbouring views (`views`) from
+// kViewRows rows of such work-groups on, else they cut one view's rows into four: with few
+// work-groups the shorter walks count for more.  Rows of one view against rows of four (us):
+// 256^2 parallel (9.3e3 rows) 21.7 / 28.2, 384^2 fan (42e3) 48.7 / 57.8, 512^2 fan (71e3)
+// 73.8 / 75.4, 8 x 256^2 (74e3) 75.6 / 75.7, 640^2 fan (115e3) 100 / 94, 512^2 parallel
+// (142e3) 122 / 112, 1024^2 fan (210e3) 179 / 151, 512^2 fan of odd views (222e3) 114 / 96,
+// 769^2 (748e3) 352 / 251, 32 x 512^2 3350 / 2340.
+// kFillQuads: split 2, 4, 8, 16 of 1024^2 334, 196, 176, 158, of 512^2 173, 108, 84, 74,
+// of 769^2 302, 276, 251, 255, of 8 x 512^2 646, 607, 613, 639; 32 x 512^2 1, 2, 3: 2343,
+// 2285, 2265, less than the second launch costs where the store evaluates the spectrum.
+constexpr int kSmallEdge = 224, kFillItems = 9000, kFillQuads = 8000;
+constexpr long long kViewRows = 80000;
 
 Plan::Shape Plan::sym_shape(const ctprj_tune& t, bool fwd, int items) const
 {
-    const Shape set = fwd ? Shape{t.fwd_seg, t.fwd_split} : Shape{t.adj_seg, t.adj_split};
-    if (set.seg != 8 || set.split != 1 || max_n <= kSmallEdge || items < 1) return set;
-    int split = std::min(std::max((kFillItems + items - 1) / items, fwd ? 2 : 1), 8);
-    while (split > 1 && (size_t)items * split * 512 > kSplitMaxFloats) --split;
-    return Shape{4, split};
+    Shape sh = fwd ? Shape{t.fwd_seg, t.fwd_split, false} : Shape{t.adj_seg, t.adj_split, false};
+    const bool own = sh.seg == 8 && sh.split == 1 && max_n > kSmallEdge && items > 0;
+    if (own) sh.seg = 4;
+    sh.views = fwd && sh.seg == 4 && (long long)(items / 4) * max_n >= kViewRows;
+    if (own) {
+        const int groups = sh.views ? items / 4 : items;
+        const int want = ((sh.views ? kFillQuads : kFillItems) + groups - 1) / groups;
+        // (the forward's items differ in cost: two work-groups each at least)
+        sh.split = std::min(std::max(want, fwd && !sh.views ? 2 : 1), sh.views ? 16 : 8);
+        while (sh.split > 1 && (size_t)items * sh.split * 512 > kSplitMaxFloats) --sh.split;
+    }
+    return sh;
 }
 
 // The symmetric slices' forward: per chunk, its orbit image, then one launch per group.
@@ -807,7 +849,7 @@ int Plan::launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStrea
             const int n = symf[c].count[g];
             if (!n) continue;
             const Shape sh = sym_shape(tune, true, n);
-            launch_forward_sym(g, sh.seg, sh.split, d_split, n, d_desc,
+            launch_forward_sym(g, sh.seg, sh.views, sh.split, d_split, n, d_desc,
                                d_symf_items + symf[c].start[g], d_views, d_rays, d_orb, d_sino,
                                bhc, st);
             if (bhc) bhc->part_off += n;

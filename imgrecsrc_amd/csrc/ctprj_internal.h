@@ -118,9 +118,11 @@ struct Plan : Tables {
     int build_fwd_items(const ctprj_tune& t, Tables& G) const;
     int build_adj_items(const ctprj_tune& t, Tables& G) const;
     int launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st);
-    // waves per item and work-groups per item of a symmetric launch of `items` items
+    // waves and work-groups per item of a symmetric launch of `items` items; views: the four
+    // waves of a forward work-group take four items instead of one item's rows
     struct Shape {
         int seg, split;
+        bool views;
     };
     Shape sym_shape(const ctprj_tune& t, bool fwd, int items) const;
     // partial-sum floats the split symmetric launches of tune t need on tables G
@@ -163,7 +165,7 @@ void launch_scale(float* p, long long n, float s, hipStream_t st);
 // per item leave partial sums in part (nitems * nsplit * 512 floats), added by a second
 // launch.  bhc != NULL: the beam-hardening alpha pass fused into the store (sino receives
 // w; one NLL partial per item at bhc->partials[bhc->part_off + item])
-void launch_forward_sym(int grp, int seg, int nsplit, float* part, int nitems,
+void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, float* part, int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
                         const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
                         hipStream_t st);

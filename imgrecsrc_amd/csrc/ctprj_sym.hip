@@ -484,6 +484,201 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
     for (int s = 0; s < N; ++s) acc[s].s *= S.inver;
 }
 
+// The walk of four canonical views at once: the work-group's four waves take the same 64
+// bins of neighbouring views, whose rays cross nearly the same pixels of a row.  kRows rows
+// of the orbit image, kUnits 16-byte units of each plane, are staged for all four in one of
+// two buffers (each wave brings one plane of one row, kChunks loads of 64 units as far as
+// the rays need them), the next rows' loads being on their way while these are summed: one
+// barrier per kRows rows.
+// Staging per wave, the vector memory unit (three 16-byte loads a row under D4, about 16
+// cycles each), LDS (three writes and the reads) and VALU were each busy two thirds of the
+// time; a row now takes one load and one write a wave, and VALU issue bounds the walk.
+// Forward of 32 x 512^2 parallel 3350 -> 2340 us, 769^2 fan of odd views 352 -> 251, 1024^2
+// fan 175 -> 158, 16 ragged slices 1230 -> 985.  Five waves per SIMD under D4 (96 VGPRs, 5
+// spilled outside the pixel loop) against four: 8 x 512^2 607 us against 667.
+template <int GRP>
+struct ViewStage {
+    using O = Orbit<GRP>;
+    static constexpr int kPlanes = O::N == 8 ? 2 : 1;
+    static constexpr int kRows = 4 / kPlanes;
+    static constexpr int kChunks = O::N == 2 ? 2 : 3;
+    static constexpr int kUnits = 64 * kChunks;           // of one plane of a row
+    static constexpr int kUnitPixels = O::N == 2 ? 2 : 1;
+    static constexpr int kPixels = kUnits * kUnitPixels;
+    static constexpr int kBuffer = kRows * kPlanes * kUnits;
+    // the rows that fwd_sym_rows stages for each wave fit, too
+    static constexpr int kStage = 2 * kBuffer > 4 * O::kLoads * 64 ? 2 * kBuffer : 4 * O::kLoads * 64;
+};
+
+__device__ __forceinline__ float wave_min(float x)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x = fminf(x, __shfl_xor(x, off, 64));
+    return x;
+}
+
+// As fwd_sym_rows, for the four waves of a work-group (every one calls it with the same
+// rows, and with the same slice, bins and walk).  A wave without a view (!active) helps to
+// stage and sums nothing.
+// What the staged columns must hold: the lanes' lines in v are straight, so their smallest
+// start lies above its chord over [vlo, vhi] and their largest end below its own, and both
+// chords are known from the two end rows.  Work-groups whose lanes' lines change order or
+// leave more than kPixels between the chords walk each wave by itself.
+template <bool FAN, int GRP, bool COLS>
+__device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, float cT, float sT,
+                                              const float* __restrict__ orb, int vlo, int vhi,
+                                              bool active, int wave, KahanAcc* acc,
+                                              float4* __restrict__ st, float (*ends)[4])
+{
+    using O = Orbit<GRP>;
+    using V = ViewStage<GRP>;
+    constexpr int N = O::N, R = V::kRows, neg = O::neg_xor(COLS);
+    const int lane = (int)threadIdx.x & 63, H = S.H;
+    if (vlo > vhi) return;  // uniform over the work-group
+    const float fH = (float)H, qs = sT * S.invd, qc = cT * S.invd;
+    const RowBounds rb = row_bounds(r, cT, sT, FAN ? S.invd : 0.0f, !COLS);
+    const float ua = rb.U0 * rb.iu, ub = -rb.U1 * rb.iu, la = rb.L0 * rb.il, lb = -rb.L1 * rb.il;
+    const float fa = (float)vlo, fb = (float)vhi;
+    const float ea = fmaf(fa, ub, ua), eb = fmaf(fb, ub, ua);
+    const float ga = fmaf(fa, lb, la), gb = fmaf(fb, lb, la);
+    const bool left = ga + gb <= ea + eb;  // the second line is the left one
+    float lo_a = left ? ga : ea, lo_b = left ? gb : eb, hi_a = left ? ea : ga, hi_b = left ? eb : gb;
+    const bool ordered = __all(lo_a <= hi_a && lo_b <= hi_b);
+    lo_a = wave_min(lo_a);
+    lo_b = wave_min(lo_b);
+    hi_a = -wave_min(-hi_a);
+    hi_b = -wave_min(-hi_b);
+    if (lane == 0) {
+        ends[wave][0] = lo_a;
+        ends[wave][1] = lo_b;
+        ends[wave][2] = ordered ? hi_a : INFINITY;
+        ends[wave][3] = hi_b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        lo_a = fminf(lo_a, ends[w][0]);
+        lo_b = fminf(lo_b, ends[w][1]);
+        hi_a = fmaxf(hi_a, ends[w][2]);
+        hi_b = fmaxf(hi_b, ends[w][3]);
+    }
+    // first staged column of the rows v..v + R - 1: c + (v - vlo) slope, less a pixel of slack
+    const float slope = vhi > vlo ? (lo_b - lo_a) / (float)(vhi - vlo) : 0.0f;
+    const float c = lo_a - 1.0f + fminf(0.0f, slope * (float)(R - 1));
+    const float span = fmaxf(hi_a - lo_a, hi_b - lo_b) + fabsf(slope) * (float)(R - 1) + 3.0f;
+    // (the image's width bounds the pixels, too); unordered lanes have left span = inf
+    const float px = fminf(span, 2.0f * fH + 2.0f);
+    const bool fits = span < INFINITY && px < (float)(V::kPixels - 1);
+    if (!__builtin_amdgcn_readfirstlane((int)fits)) {
+        fwd_sym_rows<FAN, GRP, COLS>(S, r, cT, sT, orb, vlo, vhi, acc, st + wave * O::kLoads * 64);
+        return;
+    }
+    const int chunks = __builtin_amdgcn_readfirstlane((int)px + 1 + 64 * V::kUnitPixels) /
+                       (64 * V::kUnitPixels);
+    const float none = 1e30f;  // beyond any pixel
+    const float l0 = !active ? none : (left ? la : ua), l1 = !active ? 0.0f : (left ? lb : ub);
+    const float r0 = !active ? -none : (left ? ua : la), r1 = !active ? 0.0f : (left ? ub : lb);
+    const int my_row = wave / V::kPlanes, my_plane = wave % V::kPlanes;
+    float4* const mine = st + wave * V::kUnits + lane;
+    auto column = [&](int v) {
+        const int k = (int)floorf(fmaf((float)(v - vlo), slope, c));
+        return __builtin_amdgcn_readfirstlane(min(max(k, -H), H));
+    };
+    auto load = [&](int v, int vb, int c0, float4* g) {
+        const __amdgpu_buffer_rsrc_t B =
+            row_rsrc(orbit_row<GRP, COLS>(S, orb, min(v + my_row, vb)), N * S.orb_pitch * 4);
+#pragma unroll
+        for (int k = 0; k < V::kChunks; ++k)
+            if (k < chunks)
+                g[k] = ldb128(B, (my_plane * S.orb_pitch + 64 * k + lane) * 16, (c0 + H) * O::kPlane * 4);
+    };
+    auto store = [&](int buf, const float4* g) {
+#pragma unroll
+        for (int k = 0; k < V::kChunks; ++k)
+            if (k < chunks) mine[buf * V::kBuffer + 64 * k] = g[k];
+    };
+    float part[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) part[s] = 0.0f;
+    auto flush = [&]() {
+#pragma unroll
+        for (int s = 0; s < N; ++s) {
+            acc[s].add(part[s]);
+            part[s] = 0.0f;
+        }
+    };
+    int buf = 0;
+    // rows v < 0 first, then v >= 0: the sums are held by the slots of the current sign
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        const int va = half ? max(vlo, 0) : vlo, vb = half ? vhi : min(vhi, -1);
+        if (va <= vb) {
+            float4 g[V::kChunks] = {};
+            int c0 = column(va);
+            load(va, vb, c0, g);
+            store(buf, g);
+            __syncthreads();
+#pragma unroll 1
+            for (int v = va; v <= vb; v += R) {
+                const int now = c0, last = min(v + R - 1, vb);
+                const bool more = v + R <= vb;
+                if (more) {
+                    c0 = column(v + R);
+                    load(v + R, vb, c0, g);
+                }
+                const float4* row = st + buf * V::kBuffer;
+#pragma unroll 1
+                for (int y = v; y <= last; ++y, row += V::kPlanes * V::kUnits) {
+                    const float fv = (float)y;
+                    const float lo = fmaxf(ceilf(fmaf(fv, l1, l0)), -fH);
+                    const float hi = fminf(fmaf(fv, r1, r0), fH);
+                    const float rowd = COLS ? 0.0f : fmaf(fv, r.sinR, -r.dc);
+                    const float rowq = FAN && !COLS ? fmaf(-fv, qc, 1.0f) : 0.0f;
+                    int at = (int)lo - now;
+                    for (float fu = lo; fu <= hi; fu += 1.0f, ++at) {
+                        float q[N];
+                        if constexpr (N == 2) {
+                            const float2 a = reinterpret_cast<const float2*>(row)[at];
+                            q[0] = a.x;
+                            q[1] = a.y;
+                        } else {
+#pragma unroll
+                            for (int p = 0; p < V::kPlanes; ++p) {
+                                const float4 a = row[p * V::kUnits + at];
+                                q[4 * p] = a.x;
+                                q[4 * p + 1] = a.y;
+                                q[4 * p + 2] = a.z;
+                                q[4 * p + 3] = a.w;
+                            }
+                        }
+                        // ray_dist and fan_depth_scale at (x, y) = (fu, fv), columns mode (fv, fu)
+                        const float dist = COLS ? fmaf(fv, r.cosR, fmaf(fu, r.sinR, -r.dc))
+                                                : fmaf(fu, r.cosR, rowd);
+                        const float qd = COLS ? fmaf(fv, qs, fmaf(-fu, qc, 1.0f)) : fmaf(fu, qs, rowq);
+                        const float w = strip_area(dist, FAN ? r.hbc * qd : r.hbc, r);
+#pragma unroll
+                        for (int s = 0; s < N; ++s) part[s] = fmaf(w, q[s], part[s]);
+                    }
+                    if (((y - va) & (kRowBlock - 1)) == kRowBlock - 1 || y == vb) flush();
+                }
+                if (more) store(buf ^ 1, g);
+                __syncthreads();
+                buf ^= 1;
+            }
+        }
+        if (neg && half == 0)
+#pragma unroll
+            for (int s = 0; s < N; ++s)
+                if (s < (s ^ neg)) {
+                    const KahanAcc t = acc[s];
+                    acc[s] = acc[s ^ neg];
+                    acc[s ^ neg] = t;
+                }
+    }
+#pragma unroll
+    for (int s = 0; s < N; ++s) acc[s].s *= S.inver;
+}
+
 // Kernel argument of the forward launches: empty, or (BHC) the beam-hardening ray pass
 // fused into the final store (ctprj_bhc_grad_alpha): every sinogram entry is stored
 // once, as w of bhc_ray at Ts times its ray sum, and its FP64 NLL term goes into the
@@ -671,6 +866,95 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
             const double tot = group_sum(f);
             if (threadIdx.x == 0) B.partials[B.part_off + blockIdx.x] = tot;
         }
+    }
+}
+
+// Four neighbouring canonical views (four consecutive items: one slice, one walk, the same
+// bins; the first is there unless all are padding), one wave each: see fwd_view_rows.  With
+// nsplit > 1, nsplit work-groups share the rows and leave their sums in part, as in
+// k_forward_sym.
+template <int GRP, bool BHC>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(GRP == kGrpD4 ? 5 : GRP == kGrpV4 ? 6 : 8)))
+void k_forward_views(const SliceDesc* __restrict__ slices,
+                                                       const FwdItem* __restrict__ items,
+                                                       const float4* __restrict__ views,
+                                                       const Ray* __restrict__ rays,
+                                                       const float* __restrict__ orb,
+                                                       float* __restrict__ sino, int nitems,
+                                                       int nsplit, float* __restrict__ part,
+                                                       const FwdBhc<BHC> B)
+{
+    using O = Orbit<GRP>;
+    __shared__ float4 stage[ViewStage<GRP>::kStage + 1];  // + 1: read past a row's end, unused
+    __shared__ float ends[4][4];
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int split, quad;
+    split_item(nitems / 4, split, quad);
+    const FwdItem lead = items[4 * quad];
+    if (lead.slice < 0) {  // uniform over the work-group: padding items
+        if constexpr (BHC)
+            if (!part && threadIdx.x < 4) B.partials[B.part_off + 4 * quad + threadIdx.x] = 0.0;
+        return;
+    }
+    FwdItem it = items[4 * quad + wave];
+    const bool active = it.slice >= 0;
+    if (!active) it = lead;
+    const SliceDesc S = slices[lead.slice];
+    const float4 T = views[S.view_off + it.view];
+    const int a0 = __float_as_int(T.z);
+    constexpr GroupMasks GM = group_masks(GRP);
+    const unsigned mask = !active ? 0u : (a0 == 0 || GM.q * a0 == S.P) ? GM.rot : GM.all;
+    const int b = min(max(it.bin0 + lane, S.blo), S.fold ? S.pC : S.bhi);
+    KahanAcc acc[O::N];
+    {
+        Ray r;
+        if (S.fan) r = rays[S.ray_off + (long long)it.view * S.W + b];
+        else {
+            r = rays[S.ray_off + it.view];
+            r.dc = (float)(b - S.pC) * S.dSize;
+        }
+        const int nrow = 2 * S.H + 1, per = (nrow + nsplit - 1) / nsplit;
+        const int vlo = -S.H + split * per, vhi = min(S.H, vlo + per - 1);
+        const bool cols = GRP != kGrpD4 && lead.pad;  // the walk, uniform over the work-group
+#define CTPRJ_RUN(FAN, COLS)                                                                     \
+    fwd_view_rows<FAN, GRP, COLS>(S, r, T.x, T.y, orb, vlo, vhi, active, wave, acc, stage, ends)
+        if (GRP != kGrpD4 && cols) {
+            if (S.fan) CTPRJ_RUN(true, GRP != kGrpD4);
+            else CTPRJ_RUN(false, GRP != kGrpD4);
+        } else {
+            if (S.fan) CTPRJ_RUN(true, false);
+            else CTPRJ_RUN(false, false);
+        }
+#undef CTPRJ_RUN
+    }
+    if (part) {
+        float* mine = part + ((long long)split * nitems + 4 * quad + wave) * 512;
+#pragma unroll
+        for (int s = 0; s < O::N; ++s)
+            if (mask >> O::elem(s) & 1u) mine[O::elem(s) * 64 + lane] = acc[s].s;
+        return;
+    }
+    if constexpr (!BHC) {
+#pragma unroll
+        for (int s = 0; s < O::N; ++s)
+            if (mask >> O::elem(s) & 1u)
+                fwd_sym_store<false>(S, it, a0, O::elem(s), lane, acc[s].s, sino, B);
+    } else {
+        // each lane's sums wait in LDS for one fused store loop (a single inlined copy of the
+        // spectrum sums); each lane reads back only its own entries
+        float(*tb)[64] = reinterpret_cast<float(*)[64]>(stage) + 8 * wave;
+        __syncthreads();  // every wave's rows are read
+#pragma unroll
+        for (int s = 0; s < O::N; ++s) tb[O::elem(s)][lane] = acc[s].s;
+        double f = 0.0;
+#pragma unroll 1
+        for (int e = 0; e < 8; ++e)
+            if (mask >> e & 1u) f += fwd_sym_store<true>(S, it, a0, e, lane, tb[e][lane], sino, B);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) f += __shfl_xor(f, off, 64);
+        if (lane == 0) B.partials[B.part_off + 4 * quad + wave] = f;
     }
 }
 
@@ -1096,7 +1380,7 @@ __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __
 // ----------------------------------------------------------------- launchers ---
 
 template <int GRP, bool BHC>
-static void launch_forward_sym_g(int seg, int nsplit, float* part, int nitems,
+static void launch_forward_sym_g(int seg, bool four_views, int nsplit, float* part, int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
                                  const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
@@ -1106,7 +1390,11 @@ static void launch_forward_sym_g(int seg, int nsplit, float* part, int nitems,
 #define CTPRJ_LAUNCH(SEG)                                                                       \
     hipLaunchKernelGGL((k_forward_sym<SEG, GRP, BHC>), grid, dim3(64 * SEG), 0, st, desc, items, \
                        views, rays, orb, sino, nitems, nsplit, pp, B)
-    switch (seg) {
+    if (seg == 4 && four_views)
+        hipLaunchKernelGGL((k_forward_views<GRP, BHC>),
+                           dim3((unsigned)(nitems / 4) * (unsigned)nsplit), dim3(256), 0, st, desc,
+                           items, views, rays, orb, sino, nitems, nsplit, pp, B);
+    else switch (seg) {
         case 1: CTPRJ_LAUNCH(1); break;
         case 2: CTPRJ_LAUNCH(2); break;
         case 4: CTPRJ_LAUNCH(4); break;
@@ -1120,23 +1408,23 @@ static void launch_forward_sym_g(int seg, int nsplit, float* part, int nitems,
 }
 
 template <bool BHC>
-static void launch_forward_sym_b(int grp, int seg, int nsplit, float* part, int nitems,
+static void launch_forward_sym_b(int grp, int seg, bool four_views, int nsplit, float* part, int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
                                  const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
 {
     if (grp == kGrpD4)
-        launch_forward_sym_g<kGrpD4, BHC>(seg, nsplit, part, nitems, desc, items, views, rays,
+        launch_forward_sym_g<kGrpD4, BHC>(seg, four_views, nsplit, part, nitems, desc, items, views, rays,
                                           orb, sino, B, st);
     else if (grp == kGrpV4)
-        launch_forward_sym_g<kGrpV4, BHC>(seg, nsplit, part, nitems, desc, items, views, rays,
+        launch_forward_sym_g<kGrpV4, BHC>(seg, four_views, nsplit, part, nitems, desc, items, views, rays,
                                           orb, sino, B, st);
     else
-        launch_forward_sym_g<kGrpZ2, BHC>(seg, nsplit, part, nitems, desc, items, views, rays,
+        launch_forward_sym_g<kGrpZ2, BHC>(seg, four_views, nsplit, part, nitems, desc, items, views, rays,
                                           orb, sino, B, st);
 }
 
-void launch_forward_sym(int grp, int seg, int nsplit, float* part, int nitems,
+void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, float* part, int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
                         const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
                         hipStream_t st)
@@ -1144,10 +1432,10 @@ void launch_forward_sym(int grp, int seg, int nsplit, float* part, int nitems,
     if (bhc) {
         FwdBhc<true> B;
         static_cast<BhcStore&>(B) = *bhc;
-        launch_forward_sym_b<true>(grp, seg, nsplit, part, nitems, desc, items, views, rays, orb,
+        launch_forward_sym_b<true>(grp, seg, four_views, nsplit, part, nitems, desc, items, views, rays, orb,
                                    sino, B, st);
     } else {
-        launch_forward_sym_b<false>(grp, seg, nsplit, part, nitems, desc, items, views, rays, orb,
+        launch_forward_sym_b<false>(grp, seg, four_views, nsplit, part, nitems, desc, items, views, rays, orb,
                                     sino, FwdBhc<false>{}, st);
     }
 }
