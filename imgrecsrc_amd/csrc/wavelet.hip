@@ -664,7 +664,7 @@ __global__ void k_admm_final(const double* __restrict__ a, const double* __restr
 // the previous iteration's partial sums, in one order, and knows the loop state from them.
 // Sums and products within the transforms are those of the level kernels, in their order.
 // Bound by latency (64 work-groups at 512^2 and 6 levels, 12.5 us an iteration where its 14 MB
-// would take 3): 13 iterations there take 206 us, as 11 launches each 836.
+// would take 3): 13 iterations there take 192 us, as 11 launches each 836.
 
 struct HaarTaps {
     double lo0, lo1, hi0, hi1, e0, e1, o0, o1;
@@ -1077,7 +1077,8 @@ struct ctprj_wavelet {
     double* d_part = nullptr;
     AdmmCtl* d_ctl = nullptr;  // the prox loop's state (two-tap: two, by the iteration's parity)
     double* d_sums = nullptr;  // two-tap prox: an iteration's partial sums, by its parity
-    AdmmCtl* h_ctl = nullptr;  // ... and the state as the host reads it (pinned)
+    AdmmCtl* h_ctl = nullptr;  // ... and the state as the host reads it (pinned), by the batch's parity
+    hipEvent_t ev[2] = {nullptr, nullptr};  // ... the batch's state is written
     float* d_mask = nullptr;   // image support (NULL: every pixel)
     hipStream_t cap_stream = nullptr;        // where the ADMM chunk is captured
     hipGraphExec_t chunk_exec = nullptr;     // the captured chunk (rebuilt with new masks)
@@ -1093,6 +1094,8 @@ struct ctprj_wavelet {
                         (void*)d_cmask, (void*)d_sums})
             if (p) (void)hipFree(p);
         if (h_ctl) (void)hipHostFree(h_ctl);
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
     }
 };
 
@@ -1283,7 +1286,9 @@ extern "C" int ctprj_wavelet_create(int rows, int cols, int batch, const double*
     if (e == hipSuccess) e = hipMalloc((void**)&w->d_ctl, 2 * sizeof(AdmmCtl));
     if (e == hipSuccess) e = hipMalloc((void**)&w->d_sums, sizeof(double) * 4 * kHaarGroups);
     if (e == hipSuccess)
-        e = hipHostMalloc((void**)&w->h_ctl, sizeof(AdmmCtl), hipHostMallocDefault);
+        e = hipHostMalloc((void**)&w->h_ctl, 2 * sizeof(AdmmCtl), hipHostMallocDefault);
+    for (hipEvent_t& v : w->ev)
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
     if (e != hipSuccess) {
         delete w;
         return fail(CTPRJ_ENOMEM, "wavelet workspace: %s", hipGetErrorString(e));
@@ -1430,8 +1435,10 @@ int admm_graph(ctprj_wavelet* w)
     return e == hipSuccess ? 0 : hip_fail(e, "admm graph");
 }
 
-// The two-tap prox: batches of kHaarBatch iterations, one launch each, the host reading the
-// state after each batch.
+// The two-tap prox: batches of kHaarBatch iterations, one launch each.  The host waits for a
+// batch's state only when the next batch (or the output) is queued: with a wait between them
+// the GPU stood still for about 30 us a batch, more than the launches of a batch past the stop
+// take (8 x 2.5 us).  13 iterations of 6 levels at 512^2: 206 -> 192 us.
 template <int S>
 int haar_admm(ctprj_wavelet* w, const float* d_a, double u, double relTol, int maxItr,
               const float* d_init, float* d_out, int* iterations, hipStream_t st)
@@ -1466,7 +1473,8 @@ int haar_admm(ctprj_wavelet* w, const float* d_a, double u, double relTol, int m
     // at most maxItr + 1 iterations
     const long long most = (long long)maxItr + 1;
     long long it = 0;
-    for (bool done = false; !done;) {
+    int batches = 0;
+    auto queue = [&]() -> int {
         const long long stop = it + std::min<long long>(kHaarBatch, most - it);
         for (const long long begin = it; it < stop; ++it) {
             const int p = (int)(it & 1);
@@ -1484,20 +1492,35 @@ int haar_admm(ctprj_wavelet* w, const float* d_a, double u, double relTol, int m
             else
                 hipLaunchKernelGGL((k_haar_admm<S, kHaarNext>), G, B, 0, st, A);
         }
-        const int p = (int)((it - 1) & 1);
+        const int p = (int)((it - 1) & 1), slot = batches++ & 1;
         hipLaunchKernelGGL((k_haar_state<NT>), dim3(1), B, 0, st, sums[p], groups, C + p, C + 1 - p,
-                           w->h_ctl);
-        int rc = last("admm iteration launch");
-        if (rc) return rc;
-        hipError_t e = hipStreamSynchronize(st);
+                           w->h_ctl + slot);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipEventRecord(w->ev[slot], st);
+        return e == hipSuccess ? 0 : hip_fail(e, "admm iteration launch");
+    };
+    auto output = [&]() -> int {  // after the last queued batch
+        A.c0 = C + (it & 1);
+        hipLaunchKernelGGL((k_haar_admm<S, kHaarFinal>), G, B, 0, st, A);
+        return last("admm output");
+    };
+    int rc = queue();
+    if (rc) return rc;
+    for (bool done = false, out = false; !done;) {
+        const AdmmCtl* h = w->h_ctl + ((batches - 1) & 1);
+        const hipEvent_t ev = w->ev[(batches - 1) & 1];
+        out = it >= most;
+        if ((rc = out ? output() : queue())) return rc;
+        const hipError_t e = hipEventSynchronize(ev);
         if (e != hipSuccess) return hip_fail(e, "admm state");
-        done = w->h_ctl->done != 0;
-        if (!done && it >= most) return fail(CTPRJ_EHIP, "admm: the loop state did not stop");
+        done = h->done != 0;
+        if (!done && out) return fail(CTPRJ_EHIP, "admm: the loop state did not stop");
+        if (done) {
+            if (iterations) *iterations = h->itr;
+            if (!out) return output();
+        }
     }
-    A.c0 = C + (it & 1);
-    hipLaunchKernelGGL((k_haar_admm<S, kHaarFinal>), G, B, 0, st, A);
-    if (iterations) *iterations = w->h_ctl->itr;
-    return last("admm output");
+    return 0;
 }
 
 }  // namespace
@@ -1510,11 +1533,15 @@ extern "C" int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, doubl
     if (!std::isfinite(u) || !std::isfinite(relTol) || maxItr < 0)
         return fail(CTPRJ_EINVAL, "prox_wavelet_admm: bad u, tolerance or maxItr");
     hipStream_t st = (hipStream_t)stream;
+    hipStreamCaptureStatus cap;
+    hipError_t ce = hipStreamIsCapturing(st, &cap);
+    if (ce == hipSuccess && cap != hipStreamCaptureStatusNone) ce = hipErrorStreamCaptureUnsupported;
+    if (ce != hipSuccess) return hip_fail(ce, "prox_wavelet_admm");  // the host reads the state
     const long long n = w->n;
     const unsigned g = grid1(n);
     relTol = std::min(1e-3, relTol);  // npg/admm.m:14
     // taps of length 2 on up to 6 levels: an iteration is one launch (13 iterations of 6 levels
-    // at 512^2: 206 us, 836 by the levels' own launches below; at 96^2 72 and 147 for a call
+    // at 512^2: 192 us, 836 by the levels' own launches below; at 96^2 72 and 147 for a call
     // that stops early)
     if (w->T.lh == 2 && w->L <= kHaarMaxLevels)
         return haar_tile(w->L) == 64
