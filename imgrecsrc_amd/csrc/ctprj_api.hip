@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -170,6 +171,7 @@ void Tables::swap_geometry(Tables& o)
     slice_chunk.swap(o.slice_chunk);
     orb_start.swap(o.orb_start);
     os_start.swap(o.os_start);
+    loads.swap(o.loads);
 }
 
 void Tables::swap_fwd(Tables& o)
@@ -391,6 +393,9 @@ static int host_map_view(int P, bool fold, int k, int m, int a0, bool* flip)
     return v;
 }
 
+// Forward items that are few: each gets a compute unit of its own.
+constexpr long long kFewItems = 256;
+
 int Plan::build_geometry(int flags, Tables& G) const
 {
     std::vector<SliceDesc> desc(nslices);
@@ -406,6 +411,7 @@ int Plan::build_geometry(int flags, Tables& G) const
     G.os_start.assign(1, 0);
     G.orb_floats = G.os_floats = 0;
     G.n_sym = 0;
+    G.loads.assign(1, Tables::Loads{});
     for (int s = 0; s < nslices; ++s) {
         const ctprj_geom& g = geoms[s];
         SliceDesc& D = desc[s];
@@ -464,6 +470,7 @@ int Plan::build_geometry(int flags, Tables& G) const
                 orb_used = os_used = 0;  // a new chunk
                 G.orb_start.push_back((int)orbi.size());
                 G.os_start.push_back((int)osi.size());
+                G.loads.push_back(Tables::Loads{});
             }
             D.orb_off = orb_used;
             D.os_off = os_used;
@@ -484,6 +491,21 @@ int Plan::build_geometry(int flags, Tables& G) const
                 std::memcpy(&tag, &a0, sizeof(tag));
                 views.push_back(make_float4(c, si, tag, 0.0f));
             }
+            // a small plan's own shapes (see sym_shape)
+            const long long fitems = (long long)D.ncanon * ((fold ? D.pC : D.bhi) / 64 + 1);
+            const int elems = fold ? M.order / 2 : M.order;
+            const int steps = (D.ncanon + 7) / 8 * elems;  // of one of eight waves
+            D.fcap = fitems <= kFewItems ? 2 : 1;
+            D.acap = steps <= 16 ? 1 : std::min((steps + 7) / 8, 8);
+            const long long nt = (D.H + 8) / 8, nty = grp == kGrpZ2 ? (2 * D.H + 8) / 8 : nt;
+            Tables::Loads& L = G.loads.back();
+            L.fmin[grp] = std::min(L.fmin[grp], D.fcap);
+            L.fmax[grp] = std::max(L.fmax[grp], D.fcap);
+            L.amax[grp] = std::max(L.amax[grp], D.acap);
+            L.fitems[grp] += fitems;
+            L.asteps += (grp == kGrpD4 ? nt * (nt + 1) / 2 : nt * nty) * D.ncanon * elems;
+            // (byte offsets into a sinogram that is read directly are 32-bit)
+            if ((double)g.np * g.prjWidth * 4.0 >= 2147483648.0) L.asteps = LLONG_MAX / 2;
             G.slice_sym[s] = grp;
             G.slice_chunk[s] = (int)G.orb_start.size() - 1;
             ++G.n_sym;
@@ -756,7 +778,7 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
         (rc = grow(&p->d_imgT, &p->imgT_cap, p->n_sym < nslices ? img : 0, "transposed image")) ||
         (rc = grow(&p->d_orb, &p->orb_cap, p->orb_floats, "orbit image")) ||
         (rc = grow(&p->d_os, &p->os_cap, p->os_floats, "orbit sinogram")) ||
-        (rc = grow(&p->d_split, &p->split_cap, (long long)p->split_need(p->tune, *p, *p),
+        (rc = grow(&p->d_split, &p->split_cap, (long long)p->split_need(p->tune, *p, *p, *p),
                    "split partial sums"))) {
         delete p;
         return rc;
@@ -800,15 +822,23 @@ extern "C" int ctprj_plan_layout(const ctprj_plan* p, long long* img_elems,
 
 namespace ctprj {
 
-// A new plan's shape, 8 waves in one work-group per item, stands for the plan's own choice:
-// as it is where every image is at most kSmallEdge wide, else 4 waves and as many
-// work-groups as give about kFill of them, within the partial sums' space.
-// Measured (us, 8 x 1 against the choice): forward 64^2 14.8 / 16.4, 256^2 parallel 31.4 /
-// 22.3, 512^2 fan 108 / 75; adjoint 15.6 / 17.4, 19.4 / 15.3, 67 / 49, 769^2 fan of odd views
-// 306 / 304, 1024^2 fan 176 / 159, 16 ragged slices 1027 / 1023, 32 x 512^2 2028 / 1993.  The
-// line: at 64^2 the second launch that adds the partial sums costs more than the split
-// gains, at 160^2 (25.6 / 17.6) less; small slices keep one shape so that a batch gives each
-// of them the bits of a one-slice plan.
+// A new plan's shape, 8 waves in one work-group per item, stands for the plan's own choice.
+// Where an image is more than kSmallEdge wide: 4 waves and as many work-groups as give about
+// kFill of them, within the partial sums' space.
+// Measured (us, 8 x 1 against the choice): forward 256^2 parallel 31.4 / 22.3, 512^2 fan 108 /
+// 75; adjoint 19.4 / 15.3, 67 / 49, 769^2 fan of odd views 306 / 304, 1024^2 fan 176 / 159, 16
+// ragged slices 1027 / 1023, 32 x 512^2 2028 / 1993.
+// Up to kSmallEdge the shape is each slice's own (fcap, acap), so that a batch gives it the
+// bits of a one-slice plan:
+//   adjoint: 8 waves; a wave's steps (bins of one view under one element, about 0.5 us each in
+//   a chain) above 16 are cut to about 8 by work-groups; the second launch that adds them
+//   costs about 2 us.  8 x 1 against the choice: 60^2 half turn 22.8 / 12.2, 93^2 fan 31.3 /
+//   12.0, 128^2 parallel 16.0 / 12.1, 224^2 fan of 600 views 45.7 / 22.2; kept: 48^2 9.4, 64^2
+//   11.6 (11.3 as 8 x 2).
+//   forward: 16 walks where a slice has few items, else 8: one work-group of 16 waves if the
+//   launch's items are few, two of 8 in a batch.  8 waves / 16: 64^2 fan 12.8 / 11.8, 93^2 fan
+//   16.1 / 14.4, 128^2 parallel 19.0 / 16.0, 160^2 fan 21.8 / 18.5; with more than 256 items
+//   93^2 parallel 19.6 / 21.0, 128^2 of odd views 15.9 / 18.0, 224^2 fan 34.8 / 36.6.
 // Four waves of the forward share the staged rows of four neighbouring views (`views`) from
 // kViewRows rows of such work-groups on, else they cut one view's rows into four: with few
 // work-groups the shorter walks count for more.  Rows of one view against rows of four (us):
@@ -822,10 +852,20 @@ namespace ctprj {
 constexpr int kSmallEdge = 224, kFillItems = 9000, kFillQuads = 8000;
 constexpr long long kViewRows = 80000;
 
-Plan::Shape Plan::sym_shape(const ctprj_tune& t, bool fwd, int items) const
+Plan::Shape Plan::sym_shape(const ctprj_tune& t, bool fwd, int items, const Tables& G, int c,
+                            int g) const
 {
-    Shape sh = fwd ? Shape{t.fwd_seg, t.fwd_split, false} : Shape{t.adj_seg, t.adj_split, false};
-    const bool own = sh.seg == 8 && sh.split == 1 && max_n > kSmallEdge && items > 0;
+    Shape sh = fwd ? Shape{t.fwd_seg, t.fwd_split, false, false}
+                   : Shape{t.adj_seg, t.adj_split, false, false};
+    const bool own = sh.seg == 8 && sh.split == 1 && items > 0;
+    if (own && max_n <= kSmallEdge) {
+        const Loads& L = G.loads[c];
+        if (fwd && L.fmin[g] == 2 && L.fitems[g] <= kFewItems) return Shape{16, 1, false, false};
+        sh.split = fwd ? L.fmax[g] : L.amax[g];
+        sh.capped = true;
+        while (sh.split > 1 && (size_t)items * sh.split * 512 > kSplitMaxFloats) --sh.split;
+        return sh;
+    }
     if (own) sh.seg = 4;
     sh.views = fwd && sh.seg == 4 && (long long)(items / 4) * max_n >= kViewRows;
     if (own) {
@@ -848,8 +888,8 @@ int Plan::launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStrea
         for (int g = 1; g < 4; ++g) {
             const int n = symf[c].count[g];
             if (!n) continue;
-            const Shape sh = sym_shape(tune, true, n);
-            launch_forward_sym(g, sh.seg, sh.views, sh.split, d_split, n, d_desc,
+            const Shape sh = sym_shape(tune, true, n, *this, c, g);
+            launch_forward_sym(g, sh.seg, sh.views, sh.split, sh.capped, d_split, n, d_desc,
                                d_symf_items + symf[c].start[g], d_views, d_rays, d_orb, d_sino,
                                bhc, st);
             if (bhc) bhc->part_off += n;
@@ -877,6 +917,14 @@ int Plan::launch_forward_bhc(const float* d_img, float* d_w, BhcStore bhc, hipSt
     return launch_symf(d_img, d_w, &bhc, st);
 }
 
+// Up to kDirectSteps steps of the adjoint it reads the sinogram itself: the launch that makes
+// the orbit sinogram (3 to 4 us with its gap) then costs more than the four loads of a value
+// do.  Adjoint with / without that launch, us, at steps: 48^2 parallel 0.3e3 12.1 / 9.7, 64^2
+// fan 0.8e3 14.3 / 11.4, 160^2 fan 20e3 33.0 / 31.4, 256^2 parallel 25e3 14.7 / 12.2, 224^2 fan
+// 64e3 23.3 / 20.9, 320^2 fan 77e3 26.0 / 24.6, 256^2 of odd views 185e3 34.7 / 34.2, 200^2 of
+// odd views 188e3 55.9 / 56.8, 512^2 fan 194e3 46.2 / 47.1, 512^2 of odd views 741e3 112 / 115.
+constexpr long long kDirectSteps = 100000;
+
 int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool fbp,
                          const RedJob& job)
 {
@@ -887,14 +935,17 @@ int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool
                               d_rays, d_sino, d_img, st);
     bool first = true;
     for (int c = 0; n_sym && c < chunks(); ++c) {
-        launch_orbit_sino(os_start[c + 1] - os_start[c], max_W, d_desc, d_os_items + os_start[c],
-                          d_symtab, d_sino, d_os, st);
+        const bool direct = loads[c].asteps <= kDirectSteps;
+        if (!direct)
+            launch_orbit_sino(os_start[c + 1] - os_start[c], max_W, d_desc,
+                              d_os_items + os_start[c], d_symtab, d_sino, d_os, st);
         for (int g = 1; g < 4; ++g) {
             const int n = syma[c].count[g];
             if (!n) continue;
-            const Shape sh = sym_shape(tune, false, n);
-            launch_adjoint_sym(fbp, g, sh.seg, sh.split, d_split, n, d_desc,
-                               d_syma_items + syma[c].start[g], d_views, d_rays, d_os, d_img,
+            const Shape sh = sym_shape(tune, false, n, *this, c, g);
+            launch_adjoint_sym(fbp, g, sh.seg, sh.split, sh.capped, d_split, n, d_desc,
+                               d_syma_items + syma[c].start[g], d_views, d_rays,
+                               direct ? d_sino : d_os, direct ? d_symtab : nullptr, d_img,
                                first ? job : RedJob{}, st);
             first = false;
         }
@@ -1019,15 +1070,16 @@ extern "C" int ctprj_plan_set_tune(ctprj_plan* p, const ctprj_tune* t)
     if (fwd && !rc) rc = p->build_fwd_items(nt, N);
     if (adj && !rc) rc = p->build_adj_items(nt, N);
     if (rc) return rc;  // N frees what it holds; the plan is unchanged
+    const Tables& L = geo ? N : *static_cast<const Tables*>(p);
     const Tables& F = fwd ? N : *static_cast<const Tables*>(p);
     const Tables& A = adj ? N : *static_cast<const Tables*>(p);
     int split_rc = 0;
-    size_t need = p->split_need(nt, F, A);
+    size_t need = p->split_need(nt, L, F, A);
     if (need > kSplitMaxFloats) {
         split_rc = fail(CTPRJ_EINVAL, "split work items need %zu MiB of partial sums (at most %zu)",
                         need * sizeof(float) >> 20, kSplitMaxFloats * sizeof(float) >> 20);
         nt.adj_split = nt.fwd_split = 1;
-        need = p->split_need(nt, F, A);
+        need = p->split_need(nt, L, F, A);
     }
     // workspaces only grow, and serve the old tables as well as the new
     if (geo && ((rc = grow(&p->d_imgT, &p->imgT_cap, N.n_sym < p->nslices ? p->img_elems : 0,
@@ -1048,16 +1100,16 @@ namespace ctprj {
 
 // Partial-sum space of the split symmetric launches: per group launch nitems * nsplit
 // work-groups of 512 floats; the launches of one call run in stream order and share it.
-size_t Plan::split_need(const ctprj_tune& t, const Tables& F, const Tables& A) const
+size_t Plan::split_need(const ctprj_tune& t, const Tables& G, const Tables& F, const Tables& A) const
 {
     size_t need = 0;
-    auto add = [&](bool fwd, int items) {
-        const Shape sh = sym_shape(t, fwd, items);
+    auto add = [&](bool fwd, int items, int c, int g) {
+        const Shape sh = sym_shape(t, fwd, items, G, c, g);
         if (sh.split > 1) need = std::max(need, (size_t)items * sh.split);
     };
     for (int g = 1; g < 4; ++g) {
-        for (const Segments& c : F.symf) add(true, c.count[g]);
-        for (const Segments& c : A.syma) add(false, c.count[g]);
+        for (int c = 0; c < (int)F.symf.size(); ++c) add(true, F.symf[c].count[g], c, g);
+        for (int c = 0; c < (int)A.syma.size(); ++c) add(false, A.syma[c].count[g], c, g);
     }
     return need * 512;
 }
@@ -1134,23 +1186,23 @@ extern "C" int ctprj_plan_autotune(ctprj_plan* p, int reps, const char* cache_pa
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
     ctprj_tune best = p->tune;
-    // average time of `reps` launches of one direction after one untimed launch
+    // time of `reps` launches of one direction, one after the other as a solver makes them,
+    // after one untimed launch
     auto time_dir = [&](bool fwd, float* out) -> int {
-        float ms = 0;
         for (int r = -1; r < reps; ++r) {
-            (void)hipEventRecord(e0, st);
+            if (r == 0) (void)hipEventRecord(e0, st);
             const int rc2 = fwd ? p->launch_forward(d_img, d_sino, st, false)
                                 : p->launch_adjoint(d_sino, d_img, st, false);
             if (rc2) return rc2;
-            (void)hipEventRecord(e1, st);
-            (void)hipEventSynchronize(e1);
-            float m = 0;
-            (void)hipEventElapsedTime(&m, e0, e1);
-            if (r >= 0) ms += m;
         }
-        *out = ms;
+        (void)hipEventRecord(e1, st);
+        (void)hipEventSynchronize(e1);
+        (void)hipEventElapsedTime(out, e0, e1);
         return 0;
     };
+    // a few ms of launches first, so that the early candidates meet the clocks of the late ones
+    float warm = 0, ms0 = 0;
+    for (int k = 0; k < 64 && warm < 4.0f && !rc; ++k, warm += ms0) rc = time_dir(true, &ms0);
     // one knob at a time, the others held at the best found so far
     auto search = [&](int ctprj_tune::*knob, const int* vals, int nv, bool fwd) -> int {
         float best_ms = 1e30f;

@@ -69,6 +69,8 @@ struct SliceDesc {
     // (offsets into the workspaces of the slice's chunk, elements per row of one plane)
     long long tab_off, orb_off, os_off;
     int orb_pitch, os_pitch;
+    // work-groups per forward / adjoint item in a small plan's own launch shape
+    int fcap, acap;
 };
 
 // Per-ray footprint constants.  Parallel beam: one entry per view (dc unused, the bin

@@ -67,6 +67,14 @@ struct Tables {
         int start[4] = {0, 0, 0, 0}, count[4] = {0, 0, 0, 0};
     };
     std::vector<Segments> symf, syma;
+    // what a plan's own launch shapes go by, of chunk c and group g: the slices' least and
+    // largest fcap, largest acap and forward items; (whole chunk) the adjoint's steps, a step
+    // being a tile's bins of one canonical view under one element
+    struct Loads {
+        int fmin[4] = {8, 8, 8, 8}, fmax[4] = {1, 1, 1, 1}, amax[4] = {1, 1, 1, 1};
+        long long fitems[4] = {0, 0, 0, 0}, asteps = 0;
+    };
+    std::vector<Loads> loads;
     int chunks() const { return (int)orb_start.size() - 1; }
 
     Tables() = default;
@@ -118,15 +126,17 @@ struct Plan : Tables {
     int build_fwd_items(const ctprj_tune& t, Tables& G) const;
     int build_adj_items(const ctprj_tune& t, Tables& G) const;
     int launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st);
-    // waves and work-groups per item of a symmetric launch of `items` items; views: the four
-    // waves of a forward work-group take four items instead of one item's rows
+    // waves and work-groups per item of a symmetric launch of `items` items of chunk c and
+    // group g; views: the four waves of a forward work-group take four items instead of one
+    // item's rows; capped: a slice's items take its fcap / acap work-groups at most
     struct Shape {
         int seg, split;
-        bool views;
+        bool views, capped;
     };
-    Shape sym_shape(const ctprj_tune& t, bool fwd, int items) const;
-    // partial-sum floats the split symmetric launches of tune t need on tables G
-    size_t split_need(const ctprj_tune& t, const Tables& fwd, const Tables& adj) const;
+    Shape sym_shape(const ctprj_tune& t, bool fwd, int items, const Tables& G, int c, int g) const;
+    // partial-sum floats the split symmetric launches of tune t need on geometry G and these
+    // work lists
+    size_t split_need(const ctprj_tune& t, const Tables& G, const Tables& fwd, const Tables& adj) const;
     int launch_forward(const float* d_img, float* d_sino, hipStream_t st, bool count);
     // Number of NLL partials of launch_forward_bhc (the symmetric forward items), or -1
     // when the plan has slices on the general kernels (no fused store there).
@@ -162,19 +172,22 @@ void launch_fbp_filter(int nitems, int max_W, const SliceDesc* desc, const int2*
                        hipStream_t st);
 void launch_scale(float* p, long long n, float s, hipStream_t st);
 // symmetric kernels (ctprj_sym.hip), one launch per symmetry group; nsplit > 1 work-groups
-// per item leave partial sums in part (nitems * nsplit * 512 floats), added by a second
+// per item (capped: at most the slice's fcap / acap) leave partial sums in part (nitems * nsplit * 512 floats), added by a second
 // launch.  bhc != NULL: the beam-hardening alpha pass fused into the store (sino receives
 // w; one NLL partial per item at bhc->partials[bhc->part_off + item])
-void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, float* part, int nitems,
+void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, bool capped, float* part,
+                        int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
                         const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
                         hipStream_t st);
 // The same sum as a symmetric adjoint's side job, in a launch of its own.
 void launch_wave_sum(const RedJob& job, hipStream_t st);
-void launch_adjoint_sym(bool fbp, int grp, int seg, int nsplit, float* part, int nitems,
+// direct: the view-row table, os being the sinogram itself; NULL: os is the orbit sinogram
+void launch_adjoint_sym(bool fbp, int grp, int seg, int nsplit, bool capped, float* part,
+                        int nitems,
                         const SliceDesc* desc, const AdjItem* items, const float4* views,
-                        const Ray* rays, const float* os, float* img, const RedJob& job,
-                        hipStream_t st);
+                        const Ray* rays, const float* os, const int* direct, float* img,
+                        const RedJob& job, hipStream_t st);
 // The orbit image (tiles) and orbit sinogram (rows) those two read.
 void launch_orbit_image(int nitems, const SliceDesc* desc, const AdjItem* items, const float* img,
                         float* orb, hipStream_t st);

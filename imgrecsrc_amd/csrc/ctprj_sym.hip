@@ -791,7 +791,13 @@ __device__ __forceinline__ void fwd_sym_run(const SliceDesc& S, const FwdItem& i
         if (SEG > 1) {
             t = red[0][e][lane];
 #pragma unroll
-            for (int q = 1; q < SEG; ++q) t += red[q][e][lane];
+            for (int q = 1; q < (SEG > 8 ? 8 : SEG); ++q) t += red[q][e][lane];
+        }
+        if (SEG > 8) {  // as two work-groups of eight waves add them
+            float u = red[SEG > 8 ? 8 : 0][e][lane];
+#pragma unroll
+            for (int q = 9; q < SEG; ++q) u += red[q][e][lane];
+            t += u;
         }
         if (part) part[e * 64 + lane] = t;
         else if (BHC) tb[e][lane] = t;
@@ -807,6 +813,7 @@ __device__ __forceinline__ void split_item(int nitems, int& split, int& idx)
     idx = (int)blockIdx.x - split * nitems;
 }
 
+// capped: a slice's items take its fcap (acap) of the nsplit work-groups, the others end.
 // One work item: (slice, canonical view index, first bin of 64) of a slice under group
 // GRP (one launch per group keeps each variant's registers to its own images).  SEG
 // waves share the 64 rays, each walking 1/SEG of the work-group's image rows, and then
@@ -819,7 +826,8 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
                                                           const Ray* __restrict__ rays,
                                                           const float* __restrict__ orb,
                                                           float* __restrict__ sino, int nitems,
-                                                          int nsplit, float* __restrict__ part,
+                                                          int nsplit, bool capped,
+                                                          float* __restrict__ part,
                                                           const FwdBhc<BHC> B)
 {
     __shared__ float red[SEG > 1 ? SEG : 1][8][64];
@@ -833,6 +841,8 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
         return;
     }
     const SliceDesc S = slices[it.slice];
+    if (capped) nsplit = min(nsplit, S.fcap);
+    if (split >= nsplit) return;  // uniform over the work-group
     const float4 T = views[S.view_off + it.view];
     const int a0 = __float_as_int(T.z);
     constexpr GroupMasks GM = group_masks(GRP);
@@ -961,7 +971,7 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
 // The nsplit partial sums of each canonical ray and image of an item, added in split
 // order and written like the one-work-group path (512 threads: image e = thread / 64 of
 // ray lane = thread % 64).
-template <int GRP, bool BHC>
+template <int GRP, bool BHC, bool CAPPED>
 __global__ __launch_bounds__(512) void k_forward_sym_combine(const SliceDesc* __restrict__ slices,
                                                              const FwdItem* __restrict__ items,
                                                              const float4* __restrict__ views,
@@ -977,6 +987,7 @@ __global__ __launch_bounds__(512) void k_forward_sym_combine(const SliceDesc* __
         return;
     }
     const SliceDesc S = slices[it.slice];
+    if (CAPPED) nsplit = min(nsplit, S.fcap);
     const int a0 = __float_as_int(views[S.view_off + it.view].z);
     constexpr GroupMasks GM = group_masks(GRP);
     const unsigned mask = (a0 == 0 || GM.q * a0 == S.P) ? GM.rot : GM.all;
@@ -1092,10 +1103,14 @@ struct AdjStage {
 // the wave takes the true range, piece by piece where it is wider than kStageBins.
 // Bound by VALU issue (4 cycles a wave instruction): what is not a weight or an update is
 // kept to the candidate bounds (about 25 instructions per element) and the loop's two.
-template <bool FAN, bool FBP, int GRP, bool FOLD>
+// DIRECT: os is the sinogram itself and tab the view-row table; a staged value is then
+// gathered from the rows of its slots' elements, one 4-byte load each, instead of read from
+// the orbit sinogram with one 16-byte load.
+template <bool FAN, bool FBP, int GRP, bool FOLD, bool DIRECT>
 __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* __restrict__ views,
                                               const Ray* __restrict__ rays,
-                                              const float* __restrict__ os, int x0, int y0,
+                                              const float* __restrict__ os,
+                                              const int* __restrict__ tab, int x0, int y0,
                                               bool valid, int i0, int step, KahanAcc* acc,
                                               AdjStage* __restrict__ st)
 {
@@ -1111,8 +1126,22 @@ __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* 
     const int rec = N * S.os_pitch, last_bin = valid ? S.bhi : INT_MIN;
     for (int i = i0; i < S.ncanon; i += step) {
         const float4 T = views[S.view_off + i];
-        const float* osrow = os + S.os_off + (long long)i * rec;
-        const __amdgpu_buffer_rsrc_t RV = row_rsrc(osrow, rec * 4);
+        const float* osrow = DIRECT ? os + S.sino_off : os + S.os_off + (long long)i * rec;
+        const __amdgpu_buffer_rsrc_t RV = row_rsrc(osrow, DIRECT ? S.np * S.W * 4 : rec * 4);
+        // DIRECT: the lane's slots read bin c0 + lane (reflected rows: 2 pC less it) of their rows
+        // at byte at0 + dir * c0; rows without an entry lie past the end and read as 0
+        int at0[O::kPlane], dir[O::kPlane];
+        if constexpr (DIRECT) {
+            const int* t = tab + S.tab_off + (long long)i * 8 + (N == 8 && lane >= CH ? 4 : 0);
+            const int k = N == 8 ? lane & (CH - 1) : lane;
+#pragma unroll
+            for (int q = 0; q < O::kPlane; ++q) {
+                const int r = t[N == 8 ? q : O::elem(q)];
+                const bool none = r & kRowNone, flip = r & kRowFlip;
+                at0[q] = none ? 0x7ffffff0 : (r & ~(kRowFlip | kRowNone)) + 4 * (flip ? 2 * S.pC - k : k);
+                dir[q] = none ? 0 : flip ? -4 : 4;
+            }
+        }
         const Ray* rview = rays + S.ray_off + (FAN ? (long long)i * S.W : i);
         const __amdgpu_buffer_rsrc_t RR = row_rsrc(reinterpret_cast<const float*>(rview),
                                                    FAN ? S.W * (int)sizeof(Ray) : 0);
@@ -1142,7 +1171,13 @@ __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* 
             c0 = __builtin_amdgcn_readfirstlane(min(c0, S.bhi));
         };
         auto load = [&](int c0, float4& val, float4& ray) {
-            if constexpr (N == 2) {
+            if constexpr (DIRECT) {
+                float* v = &val.x;
+#pragma unroll
+                for (int q = 0; q < O::kPlane; ++q)
+                    v[q] = __uint_as_float(
+                        __builtin_amdgcn_raw_buffer_load_b32(RV, at0[q] + dir[q] * c0, 0, 0));
+            } else if constexpr (N == 2) {
                 const auto v = __builtin_amdgcn_raw_buffer_load_b64(RV, voff, c0 * 8, 0);
                 val.x = __uint_as_float(v[0]);
                 val.y = __uint_as_float(v[1]);
@@ -1151,7 +1186,15 @@ __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* 
             }
             if (FAN) ray = ldb128(RR, roff, c0 * (int)sizeof(Ray));
         };
-        auto stage = [&](const float4& val, const float4& ray) {
+        auto stage = [&](float4 val, const float4& ray) {
+            if constexpr (DIRECT) {  // (the orbit sinogram holds the values divided by the rate)
+                val.x *= S.inver;
+                val.y *= S.inver;
+                if constexpr (N > 2) {
+                    val.z *= S.inver;
+                    val.w *= S.inver;
+                }
+            }
             wave_lds_sync();  // the previous piece's reads are done
             if constexpr (N == 2) *reinterpret_cast<float2*>(&st->val[lane]) = make_float2(val.x, val.y);
             else st->val[lane] = val;
@@ -1274,11 +1317,12 @@ __device__ __forceinline__ void adj_sym_store(const SliceDesc& S, int x0, int y0
 // The canonical views are cut into nsplit * SEG strided sets: wave w of this work-group
 // takes i = split * SEG + w + j * nsplit * SEG.  nsplit == 1 writes the image; otherwise
 // the work-group's sums go to part[h * 64 + lane] for k_adjoint_sym_combine.
-template <bool FAN, bool FBP, int SEG, int GRP>
+template <bool FAN, bool FBP, int SEG, int GRP, bool DIRECT>
 __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& it,
                                              const float4* __restrict__ views,
                                              const Ray* __restrict__ rays,
                                              const float* __restrict__ os,
+                                             const int* __restrict__ tab,
                                              float* __restrict__ img, float (*red)[8][64],
                                              int split, int nsplit, float* __restrict__ part,
                                              AdjStage* __restrict__ stage)
@@ -1292,11 +1336,11 @@ __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& 
     KahanAcc acc[O::N];
     const int i0 = split * SEG + wave, step = SEG * nsplit;
     if (!FAN && GRP != kGrpZ2 && S.fold)
-        adj_sym_pixel<FAN, FBP, GRP, !FAN && GRP != kGrpZ2>(S, views, rays, os, x0, y0, valid, i0,
-                                                            step, acc, stage + wave);
+        adj_sym_pixel<FAN, FBP, GRP, !FAN && GRP != kGrpZ2, DIRECT>(
+            S, views, rays, os, tab, x0, y0, valid, i0, step, acc, stage + wave);
     else
-        adj_sym_pixel<FAN, FBP, GRP, false>(S, views, rays, os, x0, y0, valid, i0, step, acc,
-                                            stage + wave);
+        adj_sym_pixel<FAN, FBP, GRP, false, DIRECT>(S, views, rays, os, tab, x0, y0, valid, i0, step,
+                                                    acc, stage + wave);
     if (SEG > 1) {
 #pragma unroll
         for (int s = 0; s < O::N; ++s) red[wave][O::elem(s)][lane] = acc[s].s;
@@ -1325,14 +1369,16 @@ __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& 
 // i = w, w + SEG, ...) and then share the final sums; with nsplit > 1, nsplit
 // work-groups share the views of a tile and leave their sums in part (512 floats per
 // work-group) for k_adjoint_sym_combine.
-template <bool FBP, int SEG, int GRP>
+template <bool FBP, int SEG, int GRP, bool DIRECT>
 __global__ __launch_bounds__(64 * SEG) void k_adjoint_sym(const SliceDesc* __restrict__ slices,
                                                           const AdjItem* __restrict__ items,
                                                           const float4* __restrict__ views,
                                                           const Ray* __restrict__ rays,
                                                           const float* __restrict__ os,
+                                                          const int* __restrict__ tab,
                                                           float* __restrict__ img, int nitems,
-                                                          int nsplit, float* __restrict__ part,
+                                                          int nsplit, bool capped,
+                                                          float* __restrict__ part,
                                                           const RedJob job)
 {
     __shared__ float red[SEG][8][64];
@@ -1343,19 +1389,21 @@ __global__ __launch_bounds__(64 * SEG) void k_adjoint_sym(const SliceDesc* __res
     const AdjItem it = items[idx];
     if (it.slice < 0) return;  // uniform over the work-group
     const SliceDesc S = slices[it.slice];
+    if (capped) nsplit = min(nsplit, S.acap);
+    if (split >= nsplit) return;  // uniform over the work-group
     float* mine = part ? part + (long long)blockIdx.x * 512 : nullptr;
     if (S.fan)
-        adj_sym_tile<true, FBP, SEG, GRP>(S, it, views, rays, os, img, red, split, nsplit, mine,
-                                          stage);
+        adj_sym_tile<true, FBP, SEG, GRP, DIRECT>(S, it, views, rays, os, tab, img, red, split,
+                                                  nsplit, mine, stage);
     else
-        adj_sym_tile<false, FBP, SEG, GRP>(S, it, views, rays, os, img, red, split, nsplit, mine,
-                                           stage);
+        adj_sym_tile<false, FBP, SEG, GRP, DIRECT>(S, it, views, rays, os, tab, img, red, split,
+                                                   nsplit, mine, stage);
 }
 
 // The nsplit partial sums of each orbit image of a tile, added in split order and
 // written like the one-work-group path (512 threads: orbit image h = thread / 64 of base
 // pixel lane = thread % 64).
-template <bool FBP, int GRP>
+template <bool FBP, int GRP, bool CAPPED>
 __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __restrict__ slices,
                                                              const AdjItem* __restrict__ items,
                                                              int nitems, int nsplit,
@@ -1365,6 +1413,7 @@ __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __
     const AdjItem it = items[blockIdx.x];
     if (it.slice < 0) return;
     const SliceDesc S = slices[it.slice];
+    if (CAPPED) nsplit = min(nsplit, S.acap);
     constexpr GroupMasks G = group_masks(GRP);
     if (it.pad) sym_zero_border(S, img);
     const int h = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
@@ -1380,7 +1429,8 @@ __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __
 // ----------------------------------------------------------------- launchers ---
 
 template <int GRP, bool BHC>
-static void launch_forward_sym_g(int seg, bool four_views, int nsplit, float* part, int nitems,
+static void launch_forward_sym_g(int seg, bool four_views, int nsplit, bool capped, float* part,
+                                 int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
                                  const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
@@ -1389,7 +1439,7 @@ static void launch_forward_sym_g(int seg, bool four_views, int nsplit, float* pa
     const dim3 grid((unsigned)nitems * (unsigned)nsplit);
 #define CTPRJ_LAUNCH(SEG)                                                                       \
     hipLaunchKernelGGL((k_forward_sym<SEG, GRP, BHC>), grid, dim3(64 * SEG), 0, st, desc, items, \
-                       views, rays, orb, sino, nitems, nsplit, pp, B)
+                       views, rays, orb, sino, nitems, nsplit, capped, pp, B)
     if (seg == 4 && four_views)
         hipLaunchKernelGGL((k_forward_views<GRP, BHC>),
                            dim3((unsigned)(nitems / 4) * (unsigned)nsplit), dim3(256), 0, st, desc,
@@ -1402,29 +1452,32 @@ static void launch_forward_sym_g(int seg, bool four_views, int nsplit, float* pa
         default: CTPRJ_LAUNCH(16); break;
     }
 #undef CTPRJ_LAUNCH
-    if (pp)
-        hipLaunchKernelGGL((k_forward_sym_combine<GRP, BHC>), dim3((unsigned)nitems), dim3(512), 0,
-                           st, desc, items, views, nitems, nsplit, pp, sino, B);
+    if (!pp) return;
+    auto* combine = capped ? k_forward_sym_combine<GRP, BHC, true> : k_forward_sym_combine<GRP, BHC, false>;
+    hipLaunchKernelGGL(combine, dim3((unsigned)nitems), dim3(512), 0, st, desc, items, views, nitems,
+                       nsplit, pp, sino, B);
 }
 
 template <bool BHC>
-static void launch_forward_sym_b(int grp, int seg, bool four_views, int nsplit, float* part, int nitems,
+static void launch_forward_sym_b(int grp, int seg, bool four_views, int nsplit, bool capped,
+                                 float* part, int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
                                  const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
 {
     if (grp == kGrpD4)
-        launch_forward_sym_g<kGrpD4, BHC>(seg, four_views, nsplit, part, nitems, desc, items, views, rays,
-                                          orb, sino, B, st);
+        launch_forward_sym_g<kGrpD4, BHC>(seg, four_views, nsplit, capped, part, nitems, desc, items,
+                                          views, rays, orb, sino, B, st);
     else if (grp == kGrpV4)
-        launch_forward_sym_g<kGrpV4, BHC>(seg, four_views, nsplit, part, nitems, desc, items, views, rays,
-                                          orb, sino, B, st);
+        launch_forward_sym_g<kGrpV4, BHC>(seg, four_views, nsplit, capped, part, nitems, desc, items,
+                                          views, rays, orb, sino, B, st);
     else
-        launch_forward_sym_g<kGrpZ2, BHC>(seg, four_views, nsplit, part, nitems, desc, items, views, rays,
-                                          orb, sino, B, st);
+        launch_forward_sym_g<kGrpZ2, BHC>(seg, four_views, nsplit, capped, part, nitems, desc, items,
+                                          views, rays, orb, sino, B, st);
 }
 
-void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, float* part, int nitems,
+void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, bool capped, float* part,
+                        int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
                         const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
                         hipStream_t st)
@@ -1432,25 +1485,27 @@ void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, float* pa
     if (bhc) {
         FwdBhc<true> B;
         static_cast<BhcStore&>(B) = *bhc;
-        launch_forward_sym_b<true>(grp, seg, four_views, nsplit, part, nitems, desc, items, views, rays, orb,
-                                   sino, B, st);
+        launch_forward_sym_b<true>(grp, seg, four_views, nsplit, capped, part, nitems, desc, items,
+                                   views, rays, orb, sino, B, st);
     } else {
-        launch_forward_sym_b<false>(grp, seg, four_views, nsplit, part, nitems, desc, items, views, rays, orb,
-                                    sino, FwdBhc<false>{}, st);
+        launch_forward_sym_b<false>(grp, seg, four_views, nsplit, capped, part, nitems, desc, items,
+                                    views, rays, orb, sino, FwdBhc<false>{}, st);
     }
 }
 
 template <bool FBP, int GRP>
-static void launch_adjoint_sym_t(int seg, int nsplit, float* part, int nitems,
+static void launch_adjoint_sym_t(int seg, int nsplit, bool capped, float* part, int nitems,
                                  const SliceDesc* desc, const AdjItem* items, const float4* views,
-                                 const Ray* rays, const float* os, float* img, const RedJob& job,
-                                 hipStream_t st)
+                                 const Ray* rays, const float* os, const int* direct, float* img,
+                                 const RedJob& job, hipStream_t st)
 {
     float* pp = nsplit > 1 ? part : nullptr;
     const dim3 grid((unsigned)nitems * (unsigned)nsplit);
 #define CTPRJ_LAUNCH(SEG)                                                                      \
-    hipLaunchKernelGGL((k_adjoint_sym<FBP, SEG, GRP>), grid, dim3(64 * SEG), 0, st, desc, items, \
-                       views, rays, os, img, nitems, nsplit, pp, job)
+    hipLaunchKernelGGL((direct ? k_adjoint_sym<FBP, SEG, GRP, true>                            \
+                               : k_adjoint_sym<FBP, SEG, GRP, false>),                         \
+                       grid, dim3(64 * SEG), 0, st, desc, items, views, rays, os, direct, img, \
+                       nitems, nsplit, capped, pp, job)
     switch (seg) {
         case 1: CTPRJ_LAUNCH(1); break;
         case 2: CTPRJ_LAUNCH(2); break;
@@ -1458,39 +1513,41 @@ static void launch_adjoint_sym_t(int seg, int nsplit, float* part, int nitems,
         default: CTPRJ_LAUNCH(8); break;
     }
 #undef CTPRJ_LAUNCH
-    if (pp)
-        hipLaunchKernelGGL((k_adjoint_sym_combine<FBP, GRP>), dim3((unsigned)nitems), dim3(512), 0,
-                           st, desc, items, nitems, nsplit, pp, img);
+    if (!pp) return;
+    auto* combine = capped ? k_adjoint_sym_combine<FBP, GRP, true> : k_adjoint_sym_combine<FBP, GRP, false>;
+    hipLaunchKernelGGL(combine, dim3((unsigned)nitems), dim3(512), 0, st, desc, items, nitems, nsplit,
+                       pp, img);
 }
 
 template <bool FBP>
-static void launch_adjoint_sym_f(int grp, int seg, int nsplit, float* part, int nitems,
+static void launch_adjoint_sym_f(int grp, int seg, int nsplit, bool capped, float* part, int nitems,
                                  const SliceDesc* desc, const AdjItem* items, const float4* views,
-                                 const Ray* rays, const float* os, float* img, const RedJob& job,
-                                 hipStream_t st)
+                                 const Ray* rays, const float* os, const int* direct, float* img,
+                                 const RedJob& job, hipStream_t st)
 {
     if (grp == kGrpD4)
-        launch_adjoint_sym_t<FBP, kGrpD4>(seg, nsplit, part, nitems, desc, items, views, rays, os,
-                                          img, job, st);
+        launch_adjoint_sym_t<FBP, kGrpD4>(seg, nsplit, capped, part, nitems, desc, items, views, rays, os,
+                                          direct, img, job, st);
     else if (grp == kGrpV4)
-        launch_adjoint_sym_t<FBP, kGrpV4>(seg, nsplit, part, nitems, desc, items, views, rays, os,
-                                          img, job, st);
+        launch_adjoint_sym_t<FBP, kGrpV4>(seg, nsplit, capped, part, nitems, desc, items, views, rays, os,
+                                          direct, img, job, st);
     else
-        launch_adjoint_sym_t<FBP, kGrpZ2>(seg, nsplit, part, nitems, desc, items, views, rays, os,
-                                          img, job, st);
+        launch_adjoint_sym_t<FBP, kGrpZ2>(seg, nsplit, capped, part, nitems, desc, items, views, rays, os,
+                                          direct, img, job, st);
 }
 
-void launch_adjoint_sym(bool fbp, int grp, int seg, int nsplit, float* part, int nitems,
+void launch_adjoint_sym(bool fbp, int grp, int seg, int nsplit, bool capped, float* part,
+                        int nitems,
                         const SliceDesc* desc, const AdjItem* items, const float4* views,
-                        const Ray* rays, const float* os, float* img, const RedJob& job,
-                        hipStream_t st)
+                        const Ray* rays, const float* os, const int* direct, float* img,
+                        const RedJob& job, hipStream_t st)
 {
     if (fbp)
-        launch_adjoint_sym_f<true>(grp, seg, nsplit, part, nitems, desc, items, views, rays, os,
-                                   img, job, st);
+        launch_adjoint_sym_f<true>(grp, seg, nsplit, capped, part, nitems, desc, items, views, rays, os,
+                                   direct, img, job, st);
     else
-        launch_adjoint_sym_f<false>(grp, seg, nsplit, part, nitems, desc, items, views, rays, os,
-                                    img, job, st);
+        launch_adjoint_sym_f<false>(grp, seg, nsplit, capped, part, nitems, desc, items, views, rays, os,
+                                    direct, img, job, st);
 }
 
 }  // namespace ctprj
