@@ -634,17 +634,19 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
                     const float hi = fminf(fmaf(fv, r1, r0), fH);
                     const float rowd = COLS ? 0.0f : fmaf(fv, r.sinR, -r.dc);
                     const float rowq = FAN && !COLS ? fmaf(-fv, qc, 1.0f) : 0.0f;
-                    int at = (int)lo - now;
-                    for (float fu = lo; fu <= hi; fu += 1.0f, ++at) {
+                    // (the byte offset of the pixel is kept, not its index: one add a pixel less)
+                    int at = ((int)lo - now) * (O::kPlane * 4) + (int)((const char*)row - (const char*)st);
+                    for (float fu = lo; fu <= hi; fu += 1.0f, at += O::kPlane * 4) {
+                        const char* px = (const char*)st + at;
                         float q[N];
                         if constexpr (N == 2) {
-                            const float2 a = reinterpret_cast<const float2*>(row)[at];
+                            const float2 a = *reinterpret_cast<const float2*>(px);
                             q[0] = a.x;
                             q[1] = a.y;
                         } else {
 #pragma unroll
                             for (int p = 0; p < V::kPlanes; ++p) {
-                                const float4 a = row[p * V::kUnits + at];
+                                const float4 a = reinterpret_cast<const float4*>(px)[p * V::kUnits];
                                 q[4 * p] = a.x;
                                 q[4 * p + 1] = a.y;
                                 q[4 * p + 2] = a.z;
@@ -1100,13 +1102,17 @@ struct AdjStage {
 // entry has the forward's key.  A folded scan takes the half set of elements that maps the
 // canonical range into [0, 180).  The staged range starts at the smallest first bin of the
 // tile's corner pixels (the extremes, see BinBounds); should a lane's bins lie outside,
-// the wave takes the true range, piece by piece where it is wider than kStageBins.
+// the wave takes the true range, piece by piece where it is wider than kStageBins.  COMPACT
+// (see adj_compact): they cannot, and the check, the pieces and their bounds are left out,
+// about 7 of 130 instructions an element: adjoint of 8 x 512^2 parallel 473 -> 440 us.
+// The fan beam keeps them: without, 512^2 took 47.3 us against 46.1 and 512^2 of odd views 118
+// against 112.
 // Bound by VALU issue (4 cycles a wave instruction): what is not a weight or an update is
 // kept to the candidate bounds (about 25 instructions per element) and the loop's two.
 // DIRECT: os is the sinogram itself and tab the view-row table; a staged value is then
 // gathered from the rows of its slots' elements, one 4-byte load each, instead of read from
 // the orbit sinogram with one 16-byte load.
-template <bool FAN, bool FBP, int GRP, bool FOLD, bool DIRECT>
+template <bool FAN, bool FBP, int GRP, bool FOLD, bool DIRECT, bool COMPACT>
 __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* __restrict__ views,
                                               const Ray* __restrict__ rays,
                                               const float* __restrict__ os,
@@ -1248,19 +1254,23 @@ __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* 
             range(NX, blo, bhi, c0);                                                         \
             load(c0, val, ray);                                                              \
         }                                                                                    \
-        if (__any(l <= h && (l < p || h >= p + CH))) {                                       \
-            wave_range_i32(l <= h ? l : INT_MAX, l <= h ? h : INT_MIN, p, last);             \
-            float4 v2{}, r2{};                                                               \
-            load(p, v2, r2);                                                                 \
-            stage(v2, r2);                                                                   \
-        }                                                                                    \
-        for (;;) {                                                                           \
-            sum(std::integral_constant<int, E2>{}, max(l, p), min(h, p + CH - 1), p);        \
-            p += CH;                                                                         \
-            if (p > last) break;                                                             \
-            float4 v2{}, r2{};                                                               \
-            load(p, v2, r2);                                                                 \
-            stage(v2, r2);                                                                   \
+        if constexpr (COMPACT) {                                                             \
+            sum(std::integral_constant<int, E2>{}, l, h, p);                                 \
+        } else {                                                                             \
+            if (__any(l <= h && (l < p || h >= p + CH))) {                                   \
+                wave_range_i32(l <= h ? l : INT_MAX, l <= h ? h : INT_MIN, p, last);         \
+                float4 v2{}, r2{};                                                           \
+                load(p, v2, r2);                                                             \
+                stage(v2, r2);                                                               \
+            }                                                                                \
+            for (;;) {                                                                       \
+                sum(std::integral_constant<int, E2>{}, max(l, p), min(h, p + CH - 1), p);    \
+                p += CH;                                                                     \
+                if (p > last) break;                                                         \
+                float4 v2{}, r2{};                                                           \
+                load(p, v2, r2);                                                             \
+                stage(v2, r2);                                                               \
+            }                                                                                \
         }                                                                                    \
     }
         CTPRJ_E(0) CTPRJ_E(1) CTPRJ_E(2) CTPRJ_E(3) CTPRJ_E(4) CTPRJ_E(5) CTPRJ_E(6) CTPRJ_E(7)
@@ -1317,6 +1327,17 @@ __device__ __forceinline__ void adj_sym_store(const SliceDesc& S, int x0, int y0
 // The canonical views are cut into nsplit * SEG strided sets: wave w of this work-group
 // takes i = split * SEG + w + j * nsplit * SEG.  nsplit == 1 writes the image; otherwise
 // the work-group's sums go to part[h * 64 + lane] for k_adjoint_sym_combine.
+// Parallel beam: whether the bins that the pixels of any tile can read lie within one staged
+// piece from its corners' first bin on, at any view.  The first bin is a sum of rounded
+// monotone terms of the pixel, so no pixel's lies before the corners'; the pixels are 7 sqrt(2)
+// < 9.91 apart, a pixel's footprint is sqrt(2) wide at most, and the strip and the margins
+// come to it; two bins are rounding at both ends.
+__device__ __forceinline__ bool adj_compact(const SliceDesc& S)
+{
+    return (9.91f + 1.42f + 2.0f * (S.hbd + kSupportMargin)) * 1.001f * S.invDSize + 2.0f <
+           (float)kStageBins;
+}
+
 template <bool FAN, bool FBP, int SEG, int GRP, bool DIRECT>
 __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& it,
                                              const float4* __restrict__ views,
@@ -1335,12 +1356,18 @@ __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& 
     const bool valid = adj_sym_base<GRP>(S, it, lane, x0, y0);
     KahanAcc acc[O::N];
     const int i0 = split * SEG + wave, step = SEG * nsplit;
-    if (!FAN && GRP != kGrpZ2 && S.fold)
-        adj_sym_pixel<FAN, FBP, GRP, !FAN && GRP != kGrpZ2, DIRECT>(
-            S, views, rays, os, tab, x0, y0, valid, i0, step, acc, stage + wave);
-    else
-        adj_sym_pixel<FAN, FBP, GRP, false, DIRECT>(S, views, rays, os, tab, x0, y0, valid, i0, step,
-                                                    acc, stage + wave);
+    constexpr bool kPar = !FAN, kFold = kPar && GRP != kGrpZ2;
+#define CTPRJ_RUN(FOLD, COMPACT)                                                               \
+    adj_sym_pixel<FAN, FBP, GRP, FOLD, DIRECT, COMPACT>(S, views, rays, os, tab, x0, y0, valid, \
+                                                        i0, step, acc, stage + wave)
+    if (kPar && adj_compact(S)) {  // uniform over the launch's work-groups of the slice
+        if (kFold && S.fold) CTPRJ_RUN(kFold, kPar);
+        else CTPRJ_RUN(false, kPar);
+    } else {
+        if (kFold && S.fold) CTPRJ_RUN(kFold, false);
+        else CTPRJ_RUN(false, false);
+    }
+#undef CTPRJ_RUN
     if (SEG > 1) {
 #pragma unroll
         for (int s = 0; s < O::N; ++s) red[wave][O::elem(s)][lane] = acc[s].s;
