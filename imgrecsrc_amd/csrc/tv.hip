@@ -62,6 +62,50 @@ __device__ __forceinline__ void tv_block_sum4(double v[4], double* part)
         for (int k = 0; k < 4; ++k) part[4 * (long long)blockIdx.x + k] = v[k];
 }
 
+// The work-group's sums of four values as an iteration keeps them: sum k of group b at
+// part[k nblk + b].  A wave's lanes halve the values they hold with the first two exchanges
+// (lane l ends with value l / 16, summed over lanes of equal l % 16 first), 14 shuffled words
+// where a butterfly of all four takes 48: LDS, which carries the shuffles, is a good part of a
+// small iteration's time.
+__device__ __forceinline__ void tv_store_sum4(const double v[4], double* part, long long nblk)
+{
+    __shared__ double sh[kTvBlock / 64][4];
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const bool hi = lane & 32, up = lane & 16;
+    const double a0 = hi ? v[2] : v[0], a1 = hi ? v[3] : v[1];
+    const double b0 = hi ? v[0] : v[2], b1 = hi ? v[1] : v[3];
+    const double c0 = a0 + __shfl_xor(b0, 32, 64), c1 = a1 + __shfl_xor(b1, 32, 64);
+    double s = (up ? c1 : c0) + __shfl_xor(up ? c0 : c1, 16, 64);
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((lane & 15) == 0) sh[wave][lane >> 4] = s;
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        double t = sh[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kTvBlock / 64; ++w) t += sh[w][threadIdx.x];
+        part[threadIdx.x * nblk + blockIdx.x] = t;
+    }
+}
+
+// Those sums over all groups, the same in every thread: wave k adds value k.
+__device__ __forceinline__ void tv_total4(const double* __restrict__ part, long long nblk, double a[4])
+{
+    static_assert(kTvBlock == 256, "a wave per value");
+    __shared__ double sh[4];
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const double* p = part + wave * nblk;
+    double s = 0.0;
+#pragma unroll 4
+    for (int b = lane; b < (int)nblk; b += 64) s += p[b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) sh[wave] = s;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) a[k] = sh[k];
+}
+
 // FGP loop state (utils/denoise_bound_mod.m:95-150) before an iteration; launches queued
 // after the stop do nothing.
 struct TvCtl {
@@ -82,11 +126,8 @@ __device__ __forceinline__ TvCtl tv_advance(TvCtl c, const double* __restrict__ 
                                             long long nblk, double epsilon, int maxIter)
 {
     if (c.done) return c;  // uniform
-    double a[4] = {0.0, 0.0, 0.0, 0.0};
-    for (long long b = threadIdx.x; b < nblk; b += kTvBlock)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] += part[4 * b + k];
-    tv_group_sum4(a);
+    double a[4];
+    tv_total4(part, nblk, a);
     const double re = sqrt(a[0]) / sqrt(a[1]);
     const double fval = -a[2] + a[3];
     const double tkp1 = tv_next_t(c.t);
@@ -205,7 +246,7 @@ __global__ __launch_bounds__(kTvBlock) void k_tv_iter(
         t += kTvBlock;
         if (t < end) q = tv_load(X, D, P1, P2, R1, R2, t, m, n);
     }
-    tv_block_sum4(v, part1);
+    tv_store_sum4(v, part1, gridDim.x);
 }
 
 // The state after an iteration, into c1 and host memory.
