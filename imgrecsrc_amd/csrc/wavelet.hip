@@ -663,8 +663,8 @@ __global__ void k_admm_final(const double* __restrict__ a, const double* __restr
 // the approximations pass through LDS, one barrier per level.  Every work-group first adds
 // the previous iteration's partial sums, in one order, and knows the loop state from them.
 // Sums and products within the transforms are those of the level kernels, in their order.
-// Bound by latency (64 work-groups at 512^2 and 6 levels, 12.5 us an iteration where its 14 MB
-// would take 3): 13 iterations there take 192 us, as 11 launches each 836.
+// Bound by latency (64 work-groups at 512^2 and 6 levels, 10.5 us an iteration where its 14 MB
+// would take 3): 13 iterations there take 166 us, as 11 launches each 836.
 
 struct HaarTaps {
     double lo0, lo1, hi0, hi1, e0, e1, o0, o1;
@@ -747,22 +747,21 @@ __device__ __forceinline__ void haar_analyse(const HaarTaps& T, const double x[4
     v[3] = pair(h0, T.hi0, h1, T.hi1);
 }
 
-// Sums of two values over a work-group of NT threads, the same in every thread.
+// Sums of two values over a work-group of NT threads, in thread 0: the lower half of a wave's
+// lanes goes on with the first value, the upper with the second (12 shuffled words, not 24); with haar_total2, 13 iterations at 512^2
+// 192 -> 166 us.
 template <int NT>
 __device__ __forceinline__ void haar_sum2(double& a, double& b)
 {
     __shared__ double sh[NT / 64][2];
+    const int lane = (int)threadIdx.x & 63;
+    const bool hi = lane & 32;
+    double s = (hi ? b : a) + __shfl_xor(hi ? a : b, 32, 64);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off, 64);
-        b += __shfl_xor(b, off, 64);
-    }
-    __syncthreads();  // an earlier call's reads are done
-    if ((threadIdx.x & 63) == 0) {
-        sh[threadIdx.x >> 6][0] = a;
-        sh[threadIdx.x >> 6][1] = b;
-    }
+    for (int off = 16; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((lane & 31) == 0) sh[threadIdx.x >> 6][lane >> 5] = s;
     __syncthreads();
+    if (threadIdx.x != 0) return;
     a = sh[0][0];
     b = sh[0][1];
 #pragma unroll
@@ -772,16 +771,25 @@ __device__ __forceinline__ void haar_sum2(double& a, double& b)
     }
 }
 
+// The two sums over all groups' partial sums, the same in every thread: the first wave adds
+// one of them, the second the other.
 template <int NT>
 __device__ __forceinline__ void haar_total2(const double* __restrict__ part, int nparts, double& a,
                                             double& b)
 {
-    a = b = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += NT) {
-        a += part[2 * i];
-        b += part[2 * i + 1];
+    __shared__ double sh[2];
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    if (wave < 2) {
+        double s = 0.0;
+#pragma unroll 4
+        for (int i = lane; i < nparts; i += 64) s += part[2 * i + wave];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (lane == 0) sh[wave] = s;
     }
-    haar_sum2<NT>(a, b);
+    __syncthreads();
+    a = sh[0];
+    b = sh[1];
 }
 
 // The loop state after the iteration whose partial sums are ds2 and rs2 (npg/admm.m:35-50),
@@ -1541,7 +1549,7 @@ extern "C" int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, doubl
     const unsigned g = grid1(n);
     relTol = std::min(1e-3, relTol);  // npg/admm.m:14
     // taps of length 2 on up to 6 levels: an iteration is one launch (13 iterations of 6 levels
-    // at 512^2: 192 us, 836 by the levels' own launches below; at 96^2 72 and 147 for a call
+    // at 512^2: 166 us, 836 by the levels' own launches below; at 96^2 72 and 147 for a call
     // that stops early)
     if (w->T.lh == 2 && w->L <= kHaarMaxLevels)
         return haar_tile(w->L) == 64
