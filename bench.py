@@ -673,25 +673,30 @@ def main():
     t_fwd = timed(lambda: P.forward(img, out=sino), reps, stream)
     t_adj = timed(lambda: P.adjoint(sino, out=back), reps, stream)
     sfx = "_sym" if P.modes()[0] != 0 else ""
-    # the forward call also runs the 32x32 transpose of the image (a few microseconds)
+    # each call also runs the pass that lays out its orbit array (a few microseconds)
     dom_name, dom_ms = (f"k_adjoint{sfx}", t_adj) if t_adj >= t_fwd else (f"k_forward{sfx}", t_fwd)
-    launches = (["k_adjoint_sym"] + (["k_adjoint_sym_combine"] if tune["adj_split"] > 1 else [])
+    # 8 waves with one work-group stand for the plan's own shape: four views a work-group
+    # and split items at this size
+    own = (tune["fwd_seg"], tune["fwd_split"]) == (8, 1)
+    adj_parts = tune["adj_split"] > 1 or tune["adj_seg"] == 8
+    launches = (["k_orbit_sino", "k_adjoint_sym"] + (["k_adjoint_sym_combine"] if adj_parts else [])
                 if dom_name.startswith("k_adjoint") else
-                ["k_transpose", "k_forward_sym"] + (["k_forward_sym_combine"]
-                                                    if tune["fwd_split"] > 1 else []))
+                ["k_orbit_image",
+                 "k_forward_views" if own or tune["fwd_seg"] == 4 else "k_forward_sym"] +
+                (["k_forward_sym_combine"] if own or tune["fwd_split"] > 1 else []))
     tag = f"{'adjoint' if dom_name.startswith('k_adjoint') else 'forward'}_{args.workload}"
     roofline = roofline_entry(tag, dom_name, dom_ms, launches, nnz, tune,
                               t_fwd if dom_name.startswith("k_adjoint") else t_adj)
 
     # the pair replayed as one HIP graph next to the same pair launched eagerly: what
-    # the call's launches (transpose, forward, its combine, adjoint, its combine) cost
+    # the call's launches (orbit pass, forward, its combine, the same of the adjoint) cost
     step()
     torch.cuda.synchronize()
     back_eager = back.clone()
     t_pair = timed(step, reps, stream)
     t_pair_graph, _, pair_graph = graph_timed(step, reps, stream)
     pair_replay = {"eager_ms": round(t_pair, 4), "graph_ms": round(t_pair_graph, 4),
-                   "launches_per_pair": (2 + (tune["fwd_split"] > 1)) + (1 + (tune["adj_split"] > 1)),
+                   "launches_per_pair": 4 + (own or tune["fwd_split"] > 1) + adj_parts,
                    "replay_equals_eager": bool(torch.equal(back, back_eager))}
     del pair_graph
     log(f"pair eager {t_pair:.4f} ms, graph replay {t_pair_graph:.4f} ms")

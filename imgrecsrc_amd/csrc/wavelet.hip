@@ -748,8 +748,8 @@ __device__ __forceinline__ void haar_analyse(const HaarTaps& T, const double x[4
 }
 
 // Sums of two values over a work-group of NT threads, in thread 0: the lower half of a wave's
-// lanes goes on with the first value, the upper with the second (12 shuffled words, not 24); with haar_total2, 13 iterations at 512^2
-// 192 -> 166 us.
+// lanes goes on with the first value, the upper with the second (12 shuffled words, not 24);
+// with haar_total2, 13 iterations at 512^2 192 -> 166 us.
 template <int NT>
 __device__ __forceinline__ void haar_sum2(double& a, double& b)
 {
