@@ -1576,7 +1576,7 @@ extern "C" int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, doubl
     // iterations in chunks of kAdmmChunk (one graph launch), the host reading the state
     // after each chunk
     if ((rc = admm_graph(w))) return rc;
-    AdmmCtl h{};
+    AdmmCtl& h = *w->h_ctl;  // pinned: a pageable copy waits for staging, 9 us a chunk
     // the stop comes after at most maxItr + 1 iterations
     const long long max_chunks = ((long long)maxItr + 1) / kAdmmChunk + 2;
     for (long long chunk = 0;; ++chunk) {
