@@ -1024,6 +1024,9 @@ __global__ __launch_bounds__(S* S / 4) void k_haar_admm(HaarArgs A)
             if (px)
 #pragma unroll
                 for (int k = 0; k < 4; ++k) A.out[at[k]] = (float)(x[k] * c.scale);
+            // the approximations are read before the next tile's synthesis writes them (the
+            // other modes analyse in between; more levels have a barrier before the finest)
+            __syncthreads();
             continue;
         }
         analyse(x, p0, p1);
