@@ -393,8 +393,18 @@ static int host_map_view(int P, bool fold, int k, int m, int a0, bool* flip)
     return v;
 }
 
-// Forward items that are few: each gets a compute unit of its own.
-constexpr long long kFewItems = 256;
+constexpr long long kViewRows = 40000;  // rows of four-view work-groups: see fwd_shape
+
+// Whether canonical view i of a slice walks columns (steeper than 45 degrees; none under D4),
+// and how many views from i on share a four-view work-group.
+static bool walks_columns(int a0, int P) { return 8LL * a0 > P && 8LL * a0 < 3LL * P; }
+static int quad_views(const std::vector<int>& canon, int i, int P)
+{
+    int m = 1;
+    while (m < 4 && i + m < (int)canon.size() && walks_columns(canon[i + m], P) == walks_columns(canon[i], P))
+        ++m;
+    return m;
+}
 
 int Plan::build_geometry(int flags, Tables& G) const
 {
@@ -491,19 +501,28 @@ int Plan::build_geometry(int flags, Tables& G) const
                 std::memcpy(&tag, &a0, sizeof(tag));
                 views.push_back(make_float4(c, si, tag, 0.0f));
             }
-            // a small plan's own shapes (see sym_shape)
-            const long long fitems = (long long)D.ncanon * ((fold ? D.pC : D.bhi) / 64 + 1);
+            // the slice's own cut of rows and views (see above fwd_shape), and what its launches
+            // go by
+            const long long nt = (D.H + 8) / 8, nty = grp == kGrpZ2 ? (2 * D.H + 8) / 8 : nt;
+            const long long tiles = grp == kGrpD4 ? nt * (nt + 1) / 2 : nt * nty;
+            const long long bins = (fold ? D.pC : D.bhi) / 64 + 1;
+            long long quads = 0;
+            for (int i = 0; i < D.ncanon; i += quad_views(canon, i, D.P)) quads += bins;
+            const long long fitems = D.ncanon * bins, rows = quads * (2 * D.H + 1);
             const int elems = fold ? M.order / 2 : M.order;
             const int steps = (D.ncanon + 7) / 8 * elems;  // of one of eight waves
-            D.fcap = fitems <= kFewItems ? 2 : 1;
-            D.acap = steps <= 16 ? 1 : std::min((steps + 7) / 8, 8);
-            const long long nt = (D.H + 8) / 8, nty = grp == kGrpZ2 ? (2 * D.H + 8) / 8 : nt;
+            const bool longer = rows < kViewRows && g.n * std::max(1.0f, g.dSize) >= 350.0f;
+            D.fgroups = g.n <= 48 ? 2 : g.n > 224 && (fitems <= 150 || longer) ? 8 : 4;
+            const long long fill = tiles < 40 ? 16 : tiles <= 160 ? 8 : tiles <= 320 ? 4 : std::min(8LL, (9000 + tiles - 1) / tiles);
+            D.agroups = steps <= 16 ? 2 : (int)std::min((steps + 7) / 8 * 2LL, fill);
             Tables::Loads& L = G.loads.back();
-            L.fmin[grp] = std::min(L.fmin[grp], D.fcap);
-            L.fmax[grp] = std::max(L.fmax[grp], D.fcap);
-            L.amax[grp] = std::max(L.amax[grp], D.acap);
+            L.fmin[grp] = std::min(L.fmin[grp], D.fgroups);
+            L.fmax[grp] = std::max(L.fmax[grp], D.fgroups);
+            L.amin[grp] = std::min(L.amin[grp], D.agroups);
+            L.amax[grp] = std::max(L.amax[grp], D.agroups);
             L.fitems[grp] += fitems;
-            L.asteps += (grp == kGrpD4 ? nt * (nt + 1) / 2 : nt * nty) * D.ncanon * elems;
+            L.frows[grp] += rows;
+            L.asteps += tiles * D.ncanon * elems;
             // (byte offsets into a sinogram that is read directly are 32-bit)
             if ((double)g.np * g.prjWidth * 4.0 >= 2147483648.0) L.asteps = LLONG_MAX / 2;
             G.slice_sym[s] = grp;
@@ -611,14 +630,12 @@ int Plan::build_fwd_items(const ctprj_tune& t, Tables& G) const
             bool fold = false;
             choose_group(g, t.flags, &fold, &canon);
             const int bmax = fold ? pC : bhi;
-            // the views steeper than 45 degrees walk columns (none under D4)
-            auto cols = [&](int i) { return 8LL * canon[i] > g.prjFull && 8LL * canon[i] < 3LL * g.prjFull; };
             for (int i = 0, m; i < (int)canon.size(); i += m) {
-                m = 1;
-                while (m < 4 && i + m < (int)canon.size() && cols(i + m) == cols(i)) ++m;
+                m = quad_views(canon, i, g.prjFull);
+                const int cols = walks_columns(canon[i], g.prjFull);
                 for (int b0 = 0; b0 <= bmax; b0 += 64) {
                     FwdQuad q{s, {}};
-                    for (int k = 0; k < 4; ++k) q.it[k] = FwdItem{k < m ? s : -1, i + k, b0, cols(i)};
+                    for (int k = 0; k < 4; ++k) q.it[k] = FwdItem{k < m ? s : -1, i + k, b0, cols};
                     by[G.slice_sym[s]].push_back(q);
                 }
             }
@@ -751,7 +768,6 @@ static int plan_new(const ctprj_geom* geoms, int nslices, int flags, Plan** out)
             prew.push_back((float)w);
         }
         max_W = std::max(max_W, W);
-        p->max_n = std::max(p->max_n, g.n);
     }
     p->img_elems = img;
     p->sino_elems = sino;
@@ -823,58 +839,87 @@ extern "C" int ctprj_plan_layout(const ctprj_plan* p, long long* img_elems,
 namespace ctprj {
 
 // A new plan's shape, 8 waves in one work-group per item, stands for the plan's own choice.
-// Where an image is more than kSmallEdge wide: 4 waves and as many work-groups as give about
-// kFill of them, within the partial sums' space.
-// Measured (us, 8 x 1 against the choice): forward 256^2 parallel 31.4 / 22.3, 512^2 fan 108 /
-// 75; adjoint 19.4 / 15.3, 67 / 49, 769^2 fan of odd views 306 / 304, 1024^2 fan 176 / 159, 16
-// ragged slices 1027 / 1023, 32 x 512^2 2028 / 1993.
-// Up to kSmallEdge the shape is each slice's own (fcap, acap), so that a batch gives it the
-// bits of a one-slice plan:
-//   adjoint: 8 waves; a wave's steps (bins of one view under one element, about 0.5 us each in
-//   a chain) above 16 are cut to about 8 by work-groups; the second launch that adds them
-//   costs about 2 us.  8 x 1 against the choice: 60^2 half turn 22.8 / 12.2, 93^2 fan 31.3 /
-//   12.0, 128^2 parallel 16.0 / 12.1, 224^2 fan of 600 views 45.7 / 22.2; kept: 48^2 9.4, 64^2
-//   11.6 (11.3 as 8 x 2).
-//   forward: 16 walks where a slice has few items, else 8: one work-group of 16 waves if the
-//   launch's items are few, two of 8 in a batch.  8 waves / 16: 64^2 fan 12.8 / 11.8, 93^2 fan
-//   16.1 / 14.4, 128^2 parallel 19.0 / 16.0, 160^2 fan 21.8 / 18.5; with more than 256 items
-//   93^2 parallel 19.6 / 21.0, 128^2 of odd views 15.9 / 18.0, 224^2 fan 34.8 / 36.6.
-// Four waves of the forward share the staged rows of four neighbouring views (`views`) from
-// kViewRows rows of such work-groups on, else they cut one view's rows into four: with few
-// work-groups the shorter walks count for more.  Rows of one view against rows of four (us):
-// 256^2 parallel (9.3e3 rows) 21.7 / 28.2, 384^2 fan (42e3) 48.7 / 57.8, 512^2 fan (71e3)
-// 73.8 / 75.4, 8 x 256^2 (74e3) 75.6 / 75.7, 640^2 fan (115e3) 100 / 94, 512^2 parallel
-// (142e3) 122 / 112, 1024^2 fan (210e3) 179 / 151, 512^2 fan of odd views (222e3) 114 / 96,
-// 769^2 (748e3) 352 / 251, 32 x 512^2 3350 / 2340.
-// kFillQuads: split 2, 4, 8, 16 of 1024^2 334, 196, 176, 158, of 512^2 173, 108, 84, 74,
-// of 769^2 302, 276, 251, 255, of 8 x 512^2 646, 607, 613, 639; 32 x 512^2 1, 2, 3: 2343,
-// 2285, 2265, less than the second launch costs where the store evaluates the spectrum.
-constexpr int kSmallEdge = 224, kFillItems = 9000, kFillQuads = 8000;
-constexpr long long kViewRows = 80000;
+//
+// The sums are the slice's own.  Every symmetric slice's rows (views) are cut into `fgroups`
+// (`agroups`) groups of four segments (strided sets), numbers that follow from this slice
+// alone: a wave sums a segment, four segments make a group, in order, and the groups make the
+// ray (pixel), in order.  What a launch chooses, by everything in it, is only which waves and
+// work-groups do that, so a slice has the same bits alone, in any batch and in either work
+// order.
+//
+// agroups.  Sets of a slice's canonical views, as many groups as fill the device in one round
+// (about 1280 work-groups of four waves fit), or, where four already exceed it, up to 8 for a
+// shorter last round.  Adjoint, us, by groups: 512^2 fan 4: 50.7, 8: 48.1; 300^2 4: 18.4, 6:
+// 20.4; 16 x 300^2 152, 160, 8: 165; 224^2 fan 8: 16.1, 16: 18.1; 93^2 of 536 views 8: 14.1,
+// 16: 11.3.  Slices of 16 steps of one of eight waves and fewer (a step being about 0.5 us)
+// take two groups, which are one work-group of eight waves: 64^2 fan 11.4 us, without the
+// second launch's 2 us.
+//
+// fgroups.  4 for most: 256^2 parallel 2, 3, 4, 6, 8 groups 32.2, 26.1, 24.2, 22.2, 21.2 us
+// alone, but 64 of them 392, 382, 387, 410, 437; so 8 only above 224^2 where the items are few
+// (a slice that does not fill the device) or their walks long, in rows or in pixels of a row:
+// 512^2 parallel of 180 views and pitch 1.6 81 with four, 54 with eight.  Up to 48^2 two: 100 x
+// 48^2 48 us with four, 40 with two, one alone the same.
+constexpr long long kFewItems = 256;    // forward items that get a compute unit each
 
-Plan::Shape Plan::sym_shape(const ctprj_tune& t, bool fwd, int items, const Tables& G, int c,
-                            int g) const
+// Forward launches, by the rows of four-view work-groups in them (us):
+//   many (kViewRows): k_forward_views; 512^2 fan (71e3) 71.5, as four waves on one view's rows
+//   80; 512^2 parallel (142e3) 69.5 / 78; 16 x 192^2 (174e3) 140 / 158; 4 x 224^2 fan (54e3)
+//   69 / 70; 8 x 256^2 (74e3) 79 / 83; 16 x 93^2 of 536 views (100e3) 104 / 119; 100 x 64^2
+//   fan (63e3) 63 / 65; below: 256^2 (9.3e3) 25 / 21, 16 x 64^2 (24e3) 29 / 27.
+//     A work-group takes every group (level -1) where work-groups and rows per work-group say
+//     that the partial sums cost more than a longer last round: 200 x 128^2 (4800 work-groups)
+//     440, as groups 486; 100 x 128^2 odd 352 / 400; 8 x 512^2 odd (4416) 740 / 690; 32 x
+//     512^2 (8864) 2400 / 2350, less than the second launch with the spectrum costs.  It takes
+//     one segment (level 0) where they are few and long: 1024^2 fan (276) 183, as groups 246;
+//     769^2 odd (972) 247 / 267; 2 x 1024^2 (552) 326 / 385; 16 x 224^2 fan (960) 217 / 189.
+//     Between, a group, or two, four, ... of them while 8000 work-groups are left: 64 x 256^2
+//     two 427, one 442.
+//   fewer: four waves on one view's rows, one work-group per group; or the groups together in
+//   one work-group of 8 (two groups) or 16 waves, without a second launch, where those are at
+//   most kFewItems: 64^2 fan 11.7 / 13.5, 128^2 15.9 / 15.7.
+Plan::Shape Plan::fwd_shape(const ctprj_tune& t, int items, const Tables& G, int c, int g) const
 {
-    Shape sh = fwd ? Shape{t.fwd_seg, t.fwd_split, false, false}
-                   : Shape{t.adj_seg, t.adj_split, false, false};
-    const bool own = sh.seg == 8 && sh.split == 1 && items > 0;
-    if (own && max_n <= kSmallEdge) {
-        const Loads& L = G.loads[c];
-        if (fwd && L.fmin[g] == 2 && L.fitems[g] <= kFewItems) return Shape{16, 1, false, false};
-        sh.split = fwd ? L.fmax[g] : L.amax[g];
-        sh.capped = true;
-        while (sh.split > 1 && (size_t)items * sh.split * 512 > kSplitMaxFloats) --sh.split;
-        return sh;
+    const Loads& L = G.loads[c];
+    Shape sh{t.fwd_seg, t.fwd_split, false, 0, t.fwd_seg == 8 && t.fwd_split == 1, items, 0};
+    const long long quads = items / 4, most = L.fmax[g];
+    sh.views = L.frows[g] >= kViewRows && (sh.capped || sh.seg == 4);
+    if (!sh.capped) {
+        sh.level = 1;
+    } else if (sh.views) {
+        const long long rows = L.frows[g] / quads;  // of a work-group, padding included
+        sh.seg = 4;
+        sh.level = quads >= std::max(2500LL, 15 * rows) ? -1 : 10 * most * quads < 52 * rows ? 0 : 1;
+        while (sh.level > 0 && 2 * sh.level <= most && quads * most >= 16000LL * sh.level) sh.level *= 2;
+        sh.split = sh.level < 0 ? 1 : sh.level == 0 ? 4 * (int)most : (int)most;
+    } else if (L.fmin[g] == most && (most == 2 || (most == 4 && L.fitems[g] <= kFewItems))) {
+        sh.seg = 4 * (int)most;
+    } else {
+        sh.seg = 4;
+        sh.split = (int)most;
     }
-    if (own) sh.seg = 4;
-    sh.views = fwd && sh.seg == 4 && (long long)(items / 4) * max_n >= kViewRows;
-    if (own) {
-        const int groups = sh.views ? items / 4 : items;
-        const int want = ((sh.views ? kFillQuads : kFillItems) + groups - 1) / groups;
-        // (the forward's items differ in cost: two work-groups each at least)
-        sh.split = std::min(std::max(want, fwd && !sh.views ? 2 : 1), sh.views ? 16 : 8);
-        while (sh.split > 1 && (size_t)items * sh.split * 512 > kSplitMaxFloats) --sh.split;
+    const long long per = 512LL * (sh.split > 1 ? sh.split : sh.views && sh.level < 0 && most > 1);
+    const long long all = (long long)kSplitMaxFloats;
+    if (sh.capped && per * items > all) {  // pieces of equal size
+        const long long n = (items + all / per / 32 * 32 - 1) / (all / per / 32 * 32);
+        sh.piece = (int)((items + 32 * n - 1) / (32 * n) * 32);
     }
+    sh.part = (size_t)(per * sh.piece);
+    return sh;
+}
+
+// Adjoint launches: one work-group per group while there are few items, then one per tile,
+// which goes through the groups: 64 x 192^2 (4992 items) 186 / 168 us, 8 x 512^2 fan (4488) 309 /
+// 314, 100 x 160^2 (7800) 235 / 217, 200 x 128^2 (7200) 296 / 259.
+Plan::Shape Plan::adj_shape(const ctprj_tune& t, int items, const Tables& G, int c, int g) const
+{
+    const Loads& L = G.loads[c];
+    Shape sh{t.adj_seg, t.adj_split, false, 0, t.adj_seg == 8 && t.adj_split == 1, items, 0};
+    if (sh.capped && !(L.amin[g] == 2 && L.amax[g] == 2 && items < 2000)) {
+        sh.seg = 4;
+        sh.split = items >= 4600 ? 1 : L.amax[g];
+    }
+    sh.part = sh.split > 1 ? (size_t)items * sh.split * 512 : 0;
     return sh;
 }
 
@@ -888,11 +933,14 @@ int Plan::launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStrea
         for (int g = 1; g < 4; ++g) {
             const int n = symf[c].count[g];
             if (!n) continue;
-            const Shape sh = sym_shape(tune, true, n, *this, c, g);
-            launch_forward_sym(g, sh.seg, sh.views, sh.split, sh.capped, d_split, n, d_desc,
-                               d_symf_items + symf[c].start[g], d_views, d_rays, d_orb, d_sino,
-                               bhc, st);
-            if (bhc) bhc->part_off += n;
+            const Shape sh = fwd_shape(tune, n, *this, c, g);
+            for (int i = 0; i < n; i += sh.piece) {
+                const int m = std::min(sh.piece, n - i);
+                launch_forward_sym(g, sh.seg, sh.views, sh.level, sh.split, sh.capped, d_split, m, d_desc,
+                                   d_symf_items + symf[c].start[g] + i, d_views, d_rays, d_orb,
+                                   d_sino, bhc, st);
+                if (bhc) bhc->part_off += m;
+            }
         }
     }
     hipError_t e = hipGetLastError();
@@ -942,7 +990,7 @@ int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool
         for (int g = 1; g < 4; ++g) {
             const int n = syma[c].count[g];
             if (!n) continue;
-            const Shape sh = sym_shape(tune, false, n, *this, c, g);
+            const Shape sh = adj_shape(tune, n, *this, c, g);
             launch_adjoint_sym(fbp, g, sh.seg, sh.split, sh.capped, d_split, n, d_desc,
                                d_syma_items + syma[c].start[g], d_views, d_rays,
                                direct ? d_sino : d_os, direct ? d_symtab : nullptr, d_img,
@@ -1103,15 +1151,13 @@ namespace ctprj {
 size_t Plan::split_need(const ctprj_tune& t, const Tables& G, const Tables& F, const Tables& A) const
 {
     size_t need = 0;
-    auto add = [&](bool fwd, int items, int c, int g) {
-        const Shape sh = sym_shape(t, fwd, items, G, c, g);
-        if (sh.split > 1) need = std::max(need, (size_t)items * sh.split);
-    };
     for (int g = 1; g < 4; ++g) {
-        for (int c = 0; c < (int)F.symf.size(); ++c) add(true, F.symf[c].count[g], c, g);
-        for (int c = 0; c < (int)A.syma.size(); ++c) add(false, A.syma[c].count[g], c, g);
+        for (int c = 0; c < (int)F.symf.size(); ++c)
+            if (F.symf[c].count[g]) need = std::max(need, fwd_shape(t, F.symf[c].count[g], G, c, g).part);
+        for (int c = 0; c < (int)A.syma.size(); ++c)
+            if (A.syma[c].count[g]) need = std::max(need, adj_shape(t, A.syma[c].count[g], G, c, g).part);
     }
-    return need * 512;
+    return need;
 }
 
 }  // namespace ctprj

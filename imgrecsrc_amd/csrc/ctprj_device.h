@@ -69,8 +69,9 @@ struct SliceDesc {
     // (offsets into the workspaces of the slice's chunk, elements per row of one plane)
     long long tab_off, orb_off, os_off;
     int orb_pitch, os_pitch;
-    // work-groups per forward / adjoint item in a small plan's own launch shape
-    int fcap, acap;
+    // groups of four into which a plan of its own shape cuts a forward item's rows and a tile's
+    // views: by this slice alone, so that its sums are the same whatever else the plan holds
+    int fgroups, agroups;
 };
 
 // Per-ray footprint constants.  Parallel beam: one entry per view (dc unused, the bin

@@ -67,12 +67,13 @@ struct Tables {
         int start[4] = {0, 0, 0, 0}, count[4] = {0, 0, 0, 0};
     };
     std::vector<Segments> symf, syma;
-    // what a plan's own launch shapes go by, of chunk c and group g: the slices' least and
-    // largest fcap, largest acap and forward items; (whole chunk) the adjoint's steps, a step
-    // being a tile's bins of one canonical view under one element
+    // what a launch of chunk c and group g goes by: the slices' least and largest
+    // fgroups and agroups, forward items and rows of four-view work-groups; (whole chunk) the adjoint's steps, a
+    // step being a tile's bins of one canonical view under one element
     struct Loads {
-        int fmin[4] = {8, 8, 8, 8}, fmax[4] = {1, 1, 1, 1}, amax[4] = {1, 1, 1, 1};
-        long long fitems[4] = {0, 0, 0, 0}, asteps = 0;
+        int fmin[4] = {16, 16, 16, 16}, fmax[4] = {1, 1, 1, 1};
+        int amin[4] = {16, 16, 16, 16}, amax[4] = {1, 1, 1, 1};
+        long long fitems[4] = {0, 0, 0, 0}, frows[4] = {0, 0, 0, 0}, asteps = 0;
     };
     std::vector<Loads> loads;
     int chunks() const { return (int)orb_start.size() - 1; }
@@ -93,7 +94,7 @@ struct Plan : Tables {
     std::vector<ctprj_geom> geoms;
     std::vector<long long> img_offsets, sino_offsets;
     long long img_elems = 0, sino_elems = 0;
-    int max_W = 0, max_n = 0;
+    int max_W = 0;
     ctprj_tune tune{64, 16, 1, 8, 8, 1, 1};
 
     int2* d_fbp_items = nullptr;
@@ -128,12 +129,18 @@ struct Plan : Tables {
     int launch_symf(const float* d_img, float* d_sino, BhcStore* bhc, hipStream_t st);
     // waves and work-groups per item of a symmetric launch of `items` items of chunk c and
     // group g; views: the four waves of a forward work-group take four items instead of one
-    // item's rows; capped: a slice's items take its fcap / acap work-groups at most
+    // item's rows, at a level (see k_forward_views); capped: a slice's items are cut into its own
+    // fgroups / agroups; piece: items of one launch, at most
     struct Shape {
         int seg, split;
-        bool views, capped;
+        bool views;
+        int level;
+        bool capped;
+        int piece;
+        size_t part;  // floats of partial sums
     };
-    Shape sym_shape(const ctprj_tune& t, bool fwd, int items, const Tables& G, int c, int g) const;
+    Shape fwd_shape(const ctprj_tune& t, int items, const Tables& G, int c, int g) const;
+    Shape adj_shape(const ctprj_tune& t, int items, const Tables& G, int c, int g) const;
     // partial-sum floats the split symmetric launches of tune t need on geometry G and these
     // work lists
     size_t split_need(const ctprj_tune& t, const Tables& G, const Tables& fwd, const Tables& adj) const;
@@ -172,10 +179,12 @@ void launch_fbp_filter(int nitems, int max_W, const SliceDesc* desc, const int2*
                        hipStream_t st);
 void launch_scale(float* p, long long n, float s, hipStream_t st);
 // symmetric kernels (ctprj_sym.hip), one launch per symmetry group; nsplit > 1 work-groups
-// per item (capped: at most the slice's fcap / acap) leave partial sums in part (nitems * nsplit * 512 floats), added by a second
-// launch.  bhc != NULL: the beam-hardening alpha pass fused into the store (sino receives
+// per item (capped: the slice's fgroups / agroups, at most) leave partial sums in part
+// (nitems * nsplit * 512 floats), added by a second launch; views4, level: k_forward_views and
+// what a work-group of it takes (level -1: nsplit = 1, and part holds nitems * 512 floats
+// where a slice has several groups).  bhc != NULL: the beam-hardening alpha pass fused into the store (sino receives
 // w; one NLL partial per item at bhc->partials[bhc->part_off + item])
-void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, bool capped, float* part,
+void launch_forward_sym(int grp, int seg, bool views4, int level, int nsplit, bool capped, float* part,
                         int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
                         const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,

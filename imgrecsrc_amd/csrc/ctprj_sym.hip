@@ -480,8 +480,6 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
                     acc[s ^ neg] = t;
                 }
     }
-#pragma unroll
-    for (int s = 0; s < N; ++s) acc[s].s *= S.inver;
 }
 
 // The walk of four canonical views at once: the work-group's four waves take the same 64
@@ -494,8 +492,9 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
 // cycles each), LDS (three writes and the reads) and VALU were each busy two thirds of the
 // time; a row now takes one load and one write a wave, and VALU issue bounds the walk.
 // Forward of 32 x 512^2 parallel 3350 -> 2340 us, 769^2 fan of odd views 352 -> 251, 1024^2
-// fan 175 -> 158, 16 ragged slices 1230 -> 985.  Five waves per SIMD under D4 (96 VGPRs, 5
-// spilled outside the pixel loop) against four: 8 x 512^2 607 us against 667.
+// fan 175 -> 158, 16 ragged slices 1230 -> 985.  Five waves per SIMD under D4 (96 VGPRs, 4
+// spilled outside the pixel loop) against four: 8 x 512^2 607 us against 667; 1024^2 fan 183
+// against 203, which is why the sums' LDS is kept below the sixth granule step (kLdsSums).
 template <int GRP>
 struct ViewStage {
     using O = Orbit<GRP>;
@@ -508,6 +507,10 @@ struct ViewStage {
     static constexpr int kBuffer = kRows * kPlanes * kUnits;
     // the rows that fwd_sym_rows stages for each wave fit, too
     static constexpr int kStage = 2 * kBuffer > 4 * O::kLoads * 64 ? 2 * kBuffer : 4 * O::kLoads * 64;
+    // the first so many of a wave's sums over segments wait in LDS: under D4, whose registers
+    // are all taken, seven, which with the stage leave room for five work-groups a compute
+    // unit (25 of 128 granules of 1280 B each; eight take 26)
+    static constexpr int kLdsSums = O::N == 8 ? 7 : 0;
 };
 
 __device__ __forceinline__ float wave_min(float x)
@@ -519,16 +522,18 @@ __device__ __forceinline__ float wave_min(float x)
 
 // As fwd_sym_rows, for the four waves of a work-group (every one calls it with the same
 // rows, and with the same slice, bins and walk).  A wave without a view (!active) helps to
-// stage and sums nothing.
+// stage and sums nothing.  The rows are vlo..vhi in segments of `per` rows: after each,
+// done(acc, flip, neg) takes the sums that fwd_sym_rows gives for that segment alone, with
+// flip still in the slots of the rows v < 0 (s ^ neg for s), and clears them.
 // What the staged columns must hold: the lanes' lines in v are straight, so their smallest
 // start lies above its chord over [vlo, vhi] and their largest end below its own, and both
 // chords are known from the two end rows.  Work-groups whose lanes' lines change order or
 // leave more than kPixels between the chords walk each wave by itself.
-template <bool FAN, int GRP, bool COLS>
+template <bool FAN, int GRP, bool COLS, class Done>
 __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, float cT, float sT,
                                               const float* __restrict__ orb, int vlo, int vhi,
-                                              bool active, int wave, KahanAcc* acc,
-                                              float4* __restrict__ st, float (*ends)[4])
+                                              int per, bool active, int wave,
+                                              float4* __restrict__ st, float (*ends)[4], Done done)
 {
     using O = Orbit<GRP>;
     using V = ViewStage<GRP>;
@@ -562,6 +567,8 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
         hi_a = fmaxf(hi_a, ends[w][2]);
         hi_b = fmaxf(hi_b, ends[w][3]);
     }
+    __syncthreads();  // read: `ends` may share its place with the sums
+    KahanAcc acc[N];
     // first staged column of the rows v..v + R - 1: c + (v - vlo) slope, less a pixel of slack
     const float slope = vhi > vlo ? (lo_b - lo_a) / (float)(vhi - vlo) : 0.0f;
     const float c = lo_a - 1.0f + fminf(0.0f, slope * (float)(R - 1));
@@ -570,7 +577,11 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
     const float px = fminf(span, 2.0f * fH + 2.0f);
     const bool fits = span < INFINITY && px < (float)(V::kPixels - 1);
     if (!__builtin_amdgcn_readfirstlane((int)fits)) {
-        fwd_sym_rows<FAN, GRP, COLS>(S, r, cT, sT, orb, vlo, vhi, acc, st + wave * O::kLoads * 64);
+        for (int v = vlo; v <= vhi; v += per) {
+            fwd_sym_rows<FAN, GRP, COLS>(S, r, cT, sT, orb, v, min(v + per - 1, vhi), acc,
+                                         st + wave * O::kLoads * 64);
+            done(acc, false, std::integral_constant<int, neg>{});
+        }
         return;
     }
     const int chunks = __builtin_amdgcn_readfirstlane((int)px + 1 + 64 * V::kUnitPixels) /
@@ -607,12 +618,13 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
             part[s] = 0.0f;
         }
     };
-    int buf = 0;
+    int buf = 0, seg_end = min(vlo + per - 1, vhi);
     // rows v < 0 first, then v >= 0: the sums are held by the slots of the current sign
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
         const int va = half ? max(vlo, 0) : vlo, vb = half ? vhi : min(vhi, -1);
         if (va <= vb) {
+            int block = va + kRowBlock - 1;  // the block's last row
             float4 g[V::kChunks] = {};
             int c0 = column(va);
             load(va, vb, c0, g);
@@ -661,7 +673,14 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
 #pragma unroll
                         for (int s = 0; s < N; ++s) part[s] = fmaf(w, q[s], part[s]);
                     }
-                    if (((y - va) & (kRowBlock - 1)) == kRowBlock - 1 || y == vb) flush();
+                    if (y == min(min(block, seg_end), vb)) {
+                        flush();
+                        block = y + kRowBlock;
+                        if (y == seg_end) {
+                            done(acc, neg && !half, std::integral_constant<int, neg>{});
+                            seg_end = min(seg_end + per, vhi);
+                        }
+                    }
                 }
                 if (more) store(buf ^ 1, g);
                 __syncthreads();
@@ -677,8 +696,6 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
                     acc[s ^ neg] = t;
                 }
     }
-#pragma unroll
-    for (int s = 0; s < N; ++s) acc[s].s *= S.inver;
 }
 
 // Kernel argument of the forward launches: empty, or (BHC) the beam-hardening ray pass
@@ -779,26 +796,27 @@ __device__ __forceinline__ void fwd_sym_run(const SliceDesc& S, const FwdItem& i
     }
     if (SEG > 1) {
 #pragma unroll
-        for (int s = 0; s < O::N; ++s) red[seg][O::elem(s)][lane] = acc[s].s;
+        for (int s = 0; s < O::N; ++s) red[seg][O::elem(s)][lane] = acc[s].s * S.inver;
         __syncthreads();
     }
     // wave w finalises the images e = w (mod SEG): the sum of the waves' partials in wave
-    // order.  BHC: the sums wait in tb[e][lane] for the kernel's one fused store loop (a
-    // single inlined copy of the spectrum sums)
+    // order, more than four as groups of four.  BHC: the sums wait in tb[e][lane] for the
+    // kernel's one fused store loop (a single inlined copy of the spectrum sums)
 #pragma unroll
     for (int s = 0; s < O::N; ++s) {
         const int e = O::elem(s);
         if (!(mask >> e & 1u) || (SEG > 1 && e % SEG != seg)) continue;
-        float t = acc[s].s;
+        float t = acc[s].s * S.inver;
         if (SEG > 1) {
             t = red[0][e][lane];
 #pragma unroll
-            for (int q = 1; q < (SEG > 8 ? 8 : SEG); ++q) t += red[q][e][lane];
+            for (int q = 1; q < (SEG > 4 ? 4 : SEG); ++q) t += red[q][e][lane];
         }
-        if (SEG > 8) {  // as two work-groups of eight waves add them
-            float u = red[SEG > 8 ? 8 : 0][e][lane];
 #pragma unroll
-            for (int q = 9; q < SEG; ++q) u += red[q][e][lane];
+        for (int k = 4; k < SEG; k += 4) {  // as work-groups of four waves are added
+            float u = red[k][e][lane];
+#pragma unroll
+            for (int q = k + 1; q < k + 4; ++q) u += red[q][e][lane];
             t += u;
         }
         if (part) part[e * 64 + lane] = t;
@@ -815,12 +833,13 @@ __device__ __forceinline__ void split_item(int nitems, int& split, int& idx)
     idx = (int)blockIdx.x - split * nitems;
 }
 
-// capped: a slice's items take its fcap (acap) of the nsplit work-groups, the others end.
 // One work item: (slice, canonical view index, first bin of 64) of a slice under group
 // GRP (one launch per group keeps each variant's registers to its own images).  SEG
 // waves share the 64 rays, each walking 1/SEG of the work-group's image rows, and then
 // share the final sums; with nsplit > 1, nsplit work-groups share the rows of an item
 // and leave their sums in part (512 floats per work-group) for k_forward_sym_combine.
+// capped: a slice's items take its own number (fgroups) of the nsplit work-groups, the others
+// end.
 template <int SEG, int GRP, bool BHC>
 __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __restrict__ slices,
                                                           const FwdItem* __restrict__ items,
@@ -843,7 +862,7 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
         return;
     }
     const SliceDesc S = slices[it.slice];
-    if (capped) nsplit = min(nsplit, S.fcap);
+    if (capped) nsplit = min(nsplit, S.fgroups);
     if (split >= nsplit) return;  // uniform over the work-group
     const float4 T = views[S.view_off + it.view];
     const int a0 = __float_as_int(T.z);
@@ -882,9 +901,15 @@ __global__ __launch_bounds__(64 * SEG) void k_forward_sym(const SliceDesc* __res
 }
 
 // Four neighbouring canonical views (four consecutive items: one slice, one walk, the same
-// bins; the first is there unless all are padding), one wave each: see fwd_view_rows.  With
-// nsplit > 1, nsplit work-groups share the rows and leave their sums in part, as in
-// k_forward_sym.
+// bins; the first is there unless all are padding), one wave each: see fwd_view_rows.  The
+// rows are cut into the 4 x groups segments of k_forward_sym with four waves (groups = 0: the
+// slice's own fgroups) and a wave adds them as that kernel and its second launch do, so both
+// give the same bits; the level says what a work-group takes:
+//   0  one segment (nsplit = 4 x groups);  m >= 1  m groups of four segments (nsplit = groups /
+//   m, upwards): unless there is one group only, every segment's or group's sums go to part for
+//   k_forward_sym_combine;
+//   -1  all of them: where there is more than one group, the groups' sum waits in the item's
+//   place of part, read and written once a group.
 template <int GRP, bool BHC>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(GRP == kGrpD4 ? 5 : GRP == kGrpV4 ? 6 : 8)))
@@ -894,12 +919,18 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
                                                        const Ray* __restrict__ rays,
                                                        const float* __restrict__ orb,
                                                        float* __restrict__ sino, int nitems,
-                                                       int nsplit, float* __restrict__ part,
+                                                       int nsplit, int level, int groups,
+                                                       bool parts, float* __restrict__ part,
                                                        const FwdBhc<BHC> B)
 {
     using O = Orbit<GRP>;
-    __shared__ float4 stage[ViewStage<GRP>::kStage + 1];  // + 1: read past a row's end, unused
-    __shared__ float ends[4][4];
+    using V = ViewStage<GRP>;
+    constexpr int N = O::N;
+    // the staged rows, then the waves' sums by slot (or, + 1, what is read past a row's end);
+    // the sums' place holds the walks' ends first
+    constexpr int kSums = V::kLdsSums ? 4 * V::kLdsSums * 64 / 4 : 4;
+    __shared__ float4 stage[V::kStage + kSums];
+    float(*const ends)[4] = reinterpret_cast<float(*)[4]>(stage + V::kStage);
     const int lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int split, quad;
@@ -907,19 +938,40 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
     const FwdItem lead = items[4 * quad];
     if (lead.slice < 0) {  // uniform over the work-group: padding items
         if constexpr (BHC)
-            if (!part && threadIdx.x < 4) B.partials[B.part_off + 4 * quad + threadIdx.x] = 0.0;
+            if (!parts && threadIdx.x < 4) B.partials[B.part_off + 4 * quad + threadIdx.x] = 0.0;
         return;
     }
     FwdItem it = items[4 * quad + wave];
     const bool active = it.slice >= 0;
     if (!active) it = lead;
     const SliceDesc S = slices[lead.slice];
+    if (groups == 0) groups = S.fgroups;
+    const int nseg = level < 0 ? 4 * groups : level == 0 ? 1 : 4 * level, seg0 = split * nseg;
+    if (seg0 >= 4 * groups) return;  // uniform over the work-group
     const float4 T = views[S.view_off + it.view];
     const int a0 = __float_as_int(T.z);
     constexpr GroupMasks GM = group_masks(GRP);
     const unsigned mask = !active ? 0u : (a0 == 0 || GM.q * a0 == S.P) ? GM.rot : GM.all;
     const int b = min(max(it.bin0 + lane, S.blo), S.fold ? S.pC : S.bhi);
-    KahanAcc acc[O::N];
+    // this wave's sums by slot, and, level 2 of several groups, the place of their total
+    float reg[N];
+    // (the places are formed anew where they are used: no register holds them over the walk)
+    auto here = [&]() {
+        int l = (int)threadIdx.x;
+        asm("" : "+v"(l));
+        return l & 63;
+    };
+    auto lds = [&](int s) -> float& {
+        return reinterpret_cast<float*>(stage + V::kStage)[(wave * V::kLdsSums + s) * 64 + here()];
+    };
+    auto get = [&](int s) -> float { return s < V::kLdsSums ? lds(s) : reg[s]; };
+    auto set = [&](int s, float t) { if (s < V::kLdsSums) lds(s) = t; else reg[s] = t; };
+    // the sums of segment or group g of the item in part, or (g = 0) their total
+    auto slot = [&](int g, int s) -> float& {
+        return part[((long long)g * nitems + 4 * quad + wave) * 512 + O::elem(s) * 64 + here()];
+    };
+    const bool total = level < 0 && groups > 1;
+    int next = level == 0 ? split : level * split;  // part's next segment or group
     {
         Ray r;
         if (S.fan) r = rays[S.ray_off + (long long)it.view * S.W + b];
@@ -927,11 +979,47 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
             r = rays[S.ray_off + it.view];
             r.dc = (float)(b - S.pC) * S.dSize;
         }
-        const int nrow = 2 * S.H + 1, per = (nrow + nsplit - 1) / nsplit;
-        const int vlo = -S.H + split * per, vhi = min(S.H, vlo + per - 1);
+        const int nrow = 2 * S.H + 1;
+        const int per = __builtin_amdgcn_readfirstlane((nrow + 4 * groups - 1) / (4 * groups));
+        const int vlo = -S.H + seg0 * per, vhi = min(S.H, vlo + nseg * per - 1);
         const bool cols = GRP != kGrpD4 && lead.pad;  // the walk, uniform over the work-group
-#define CTPRJ_RUN(FAN, COLS)                                                                     \
-    fwd_view_rows<FAN, GRP, COLS>(S, r, T.x, T.y, orb, vlo, vhi, active, wave, acc, stage, ends)
+        int segs = 0;  // finished
+        bool clear = true;
+        auto done = [&](KahanAcc* acc, bool flip, auto neg) {
+            // (flip: the slots of the rows v < 0)
+            float in[N];
+#pragma unroll
+            for (int s = 0; s < N; ++s) {
+                in[s] = acc[s].s * S.inver;
+                acc[s] = KahanAcc{};
+            }
+#pragma unroll
+            for (int s = 0; s < N; ++s) {
+                const float v = flip ? in[s ^ decltype(neg)::value] : in[s];
+                set(s, clear ? v : get(s) + v);
+            }
+            ++segs;
+            clear = false;
+            if (level == 0 || segs % 4 == 0 || vlo + segs * per > vhi) {  // (the last one)
+                if (parts) {
+#pragma unroll
+                    for (int s = 0; s < N; ++s) slot(next, s) = get(s);
+                    ++next;
+                    clear = true;
+                } else if (total) {
+#pragma unroll
+                    for (int s = 0; s < N; ++s) {
+                        const float t = get(s);
+                        float& u = slot(0, s);
+                        u = segs <= 4 ? t : u + t;
+                    }
+                    clear = true;
+                }
+            }
+        };
+#define CTPRJ_RUN(FAN, COLS)                                                                    \
+    fwd_view_rows<FAN, GRP, COLS>(S, r, T.x, T.y, orb, vlo, vhi, per, active, wave, stage, ends, \
+                                  done)
         if (GRP != kGrpD4 && cols) {
             if (S.fan) CTPRJ_RUN(true, GRP != kGrpD4);
             else CTPRJ_RUN(false, GRP != kGrpD4);
@@ -941,25 +1029,28 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
         }
 #undef CTPRJ_RUN
     }
-    if (part) {
-        float* mine = part + ((long long)split * nitems + 4 * quad + wave) * 512;
+    if (parts) {  // segments or groups past the last row
+        const int end = level == 0 ? split + 1 : min(level * (split + 1), groups);
+        for (; next < end; ++next)
 #pragma unroll
-        for (int s = 0; s < O::N; ++s)
-            if (mask >> O::elem(s) & 1u) mine[O::elem(s) * 64 + lane] = acc[s].s;
+            for (int s = 0; s < N; ++s) slot(next, s) = 0.0f;
         return;
     }
+    if (total)
+#pragma unroll
+        for (int s = 0; s < N; ++s) set(s, slot(0, s));
     if constexpr (!BHC) {
 #pragma unroll
         for (int s = 0; s < O::N; ++s)
             if (mask >> O::elem(s) & 1u)
-                fwd_sym_store<false>(S, it, a0, O::elem(s), lane, acc[s].s, sino, B);
+                fwd_sym_store<false>(S, it, a0, O::elem(s), lane, get(s), sino, B);
     } else {
         // each lane's sums wait in LDS for one fused store loop (a single inlined copy of the
         // spectrum sums); each lane reads back only its own entries
         float(*tb)[64] = reinterpret_cast<float(*)[64]>(stage) + 8 * wave;
         __syncthreads();  // every wave's rows are read
 #pragma unroll
-        for (int s = 0; s < O::N; ++s) tb[O::elem(s)][lane] = acc[s].s;
+        for (int s = 0; s < O::N; ++s) tb[O::elem(s)][lane] = get(s);
         double f = 0.0;
 #pragma unroll 1
         for (int e = 0; e < 8; ++e)
@@ -971,13 +1062,13 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
 }
 
 // The nsplit partial sums of each canonical ray and image of an item, added in split
-// order and written like the one-work-group path (512 threads: image e = thread / 64 of
-// ray lane = thread % 64).
+// order (fine: by groups of four) and written like the one-work-group path (512 threads:
+// image e = thread / 64 of ray lane = thread % 64).
 template <int GRP, bool BHC, bool CAPPED>
 __global__ __launch_bounds__(512) void k_forward_sym_combine(const SliceDesc* __restrict__ slices,
                                                              const FwdItem* __restrict__ items,
                                                              const float4* __restrict__ views,
-                                                             int nitems, int nsplit,
+                                                             int nitems, int nsplit, bool fine,
                                                              const float* __restrict__ part,
                                                              float* __restrict__ sino,
                                                              const FwdBhc<BHC> B)
@@ -989,7 +1080,7 @@ __global__ __launch_bounds__(512) void k_forward_sym_combine(const SliceDesc* __
         return;
     }
     const SliceDesc S = slices[it.slice];
-    if (CAPPED) nsplit = min(nsplit, S.fcap);
+    if (CAPPED) nsplit = min(nsplit, fine ? 4 * S.fgroups : S.fgroups);
     const int a0 = __float_as_int(views[S.view_off + it.view].z);
     constexpr GroupMasks GM = group_masks(GRP);
     const unsigned mask = (a0 == 0 || GM.q * a0 == S.P) ? GM.rot : GM.all;
@@ -997,8 +1088,17 @@ __global__ __launch_bounds__(512) void k_forward_sym_combine(const SliceDesc* __
     double f = 0.0;
     if (mask >> e & 1u) {
         const float* p = part + (long long)blockIdx.x * 512 + threadIdx.x;
-        float t = p[0];
-        for (int k = 1; k < nsplit; ++k) t += p[(long long)k * nitems * 512];
+        const long long step = nitems * 512LL;
+        float t = 0.0f;
+        if (fine) {
+            for (int k = 0; k < nsplit; k += 4, p += 4 * step) {
+                const float u = ((p[0] + p[step]) + p[2 * step]) + p[3 * step];
+                t = k ? t + u : u;
+            }
+        } else {
+            t = p[0];
+            for (int k = 1; k < nsplit; ++k) t += p[k * step];
+        }
         f = fwd_sym_store<BHC>(S, it, a0, e, lane, t, sino, B);
     }
     if constexpr (BHC) {  // the work-group's NLL partial (every thread takes part)
@@ -1116,15 +1216,14 @@ template <bool FAN, bool FBP, int GRP, bool FOLD, bool DIRECT, bool COMPACT>
 __device__ __forceinline__ void adj_sym_pixel(const SliceDesc& S, const float4* __restrict__ views,
                                               const Ray* __restrict__ rays,
                                               const float* __restrict__ os,
-                                              const int* __restrict__ tab, int x0, int y0,
-                                              bool valid, int i0, int step, KahanAcc* acc,
-                                              AdjStage* __restrict__ st)
+                                              const int* __restrict__ tab, int lane, int x0,
+                                              int y0, bool valid, int i0, int step,
+                                              KahanAcc* acc, AdjStage* __restrict__ st)
 {
     using O = Orbit<GRP>;
     constexpr int N = O::N, CH = kStageBins;
     constexpr GroupMasks G = group_masks(GRP);
     constexpr unsigned GSET = FOLD ? G.fold : G.all;
-    const int lane = (int)threadIdx.x & 63;
     const float gx = (float)x0, gy = (float)y0;
     // lane's part of a staged piece, bytes from the first bin's: values, ray records
     const int voff = N == 8 && lane >= CH ? (S.os_pitch + lane - CH) * 16 : lane * O::kPlane * 4;
@@ -1324,9 +1423,6 @@ __device__ __forceinline__ void adj_sym_store(const SliceDesc& S, int x0, int y0
     img[S.img_off + (long long)(oy + S.half) * S.n + ox + S.half] = FBP ? t * S.fbp_scale : t;
 }
 
-// The canonical views are cut into nsplit * SEG strided sets: wave w of this work-group
-// takes i = split * SEG + w + j * nsplit * SEG.  nsplit == 1 writes the image; otherwise
-// the work-group's sums go to part[h * 64 + lane] for k_adjoint_sym_combine.
 // Parallel beam: whether the bins that the pixels of any tile can read lie within one staged
 // piece from its corners' first bin on, at any view.  The first bin is a sum of rounded
 // monotone terms of the pixel, so no pixel's lies before the corners'; the pixels are 7 sqrt(2)
@@ -1338,64 +1434,87 @@ __device__ __forceinline__ bool adj_compact(const SliceDesc& S)
            (float)kStageBins;
 }
 
+// The canonical views are cut into groups * SEG strided sets: set g * SEG + w, wave w's in
+// group g, holds i = g * SEG + w + j * groups * SEG.  A work-group takes the groups first..last
+// (more than one: SEG = 4 only), the waves' sums of a group being added in wave order (eight
+// waves: as two groups of four) and the groups in theirs, here or, with part, one group's
+// sums to part[h * 64 + lane], in k_adjoint_sym_combine: who adds changes no bit.
 template <bool FAN, bool FBP, int SEG, int GRP, bool DIRECT>
 __device__ __forceinline__ void adj_sym_tile(const SliceDesc& S, const AdjItem& it,
                                              const float4* __restrict__ views,
                                              const Ray* __restrict__ rays,
                                              const float* __restrict__ os,
                                              const int* __restrict__ tab,
-                                             float* __restrict__ img, float (*red)[8][64],
-                                             int split, int nsplit, float* __restrict__ part,
-                                             AdjStage* __restrict__ stage)
+                                             float* __restrict__ img,
+                                             float (*red)[SEG][Orbit<GRP>::N][64],
+                                             float (*tot)[64], int groups, int first, int last,
+                                             float* __restrict__ part, AdjStage* __restrict__ stage)
 {
     using O = Orbit<GRP>;
     // the wave index is uniform over the wave: the view loop then runs on scalar registers
-    const int lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    int x0, y0;
-    const bool valid = adj_sym_base<GRP>(S, it, lane, x0, y0);
-    KahanAcc acc[O::N];
-    const int i0 = split * SEG + wave, step = SEG * nsplit;
     constexpr bool kPar = !FAN, kFold = kPar && GRP != kGrpZ2;
 #define CTPRJ_RUN(FOLD, COMPACT)                                                               \
-    adj_sym_pixel<FAN, FBP, GRP, FOLD, DIRECT, COMPACT>(S, views, rays, os, tab, x0, y0, valid, \
-                                                        i0, step, acc, stage + wave)
-    if (kPar && adj_compact(S)) {  // uniform over the launch's work-groups of the slice
-        if (kFold && S.fold) CTPRJ_RUN(kFold, kPar);
-        else CTPRJ_RUN(false, kPar);
-    } else {
-        if (kFold && S.fold) CTPRJ_RUN(kFold, false);
-        else CTPRJ_RUN(false, false);
+    adj_sym_pixel<FAN, FBP, GRP, FOLD, DIRECT, COMPACT>(S, views, rays, os, tab, lane, x0, y0, \
+                                                        valid, i0, step, acc, stage + wave)
+    const int step = SEG * groups;
+    if (!part && it.pad) sym_zero_border(S, img);
+    if (SEG != 4) last = first;
+#pragma unroll 1
+    for (int g = first; g <= last; ++g) {
+        // (formed anew for every group: kept from one to the next, what the walk derives from
+        // the lane and its pixel takes 20 registers, a wave per SIMD)
+        int lane = (int)threadIdx.x & 63, x0, y0;
+        if (SEG == 4) asm("" : "+v"(lane));
+        const bool valid = adj_sym_base<GRP>(S, it, lane, x0, y0);
+        KahanAcc acc[O::N];
+        const int i0 = g * SEG + wave;
+        if (kPar && adj_compact(S)) {  // uniform over the launch's work-groups of the slice
+            if (kFold && S.fold) CTPRJ_RUN(kFold, kPar);
+            else CTPRJ_RUN(false, kPar);
+        } else {
+            if (kFold && S.fold) CTPRJ_RUN(kFold, false);
+            else CTPRJ_RUN(false, false);
+        }
+        // (two buffers: a wave that is a group ahead does not disturb the sums below)
+        auto* const r = red[SEG == 4 ? (g - first) & 1 : 0];
+        if (SEG > 1) {
+#pragma unroll
+            for (int s = 0; s < O::N; ++s) r[wave][s][lane] = acc[s].s;
+            __syncthreads();
+        }
+        // wave w finalises the elements h = w (mod SEG)
+#pragma unroll
+        for (int s = 0; s < O::N; ++s) {
+            const int h = O::elem(s);
+            if (SEG > 1 && h % SEG != wave) continue;
+            float t = acc[s].s;
+            if (SEG > 1) {
+                t = r[0][s][lane];
+#pragma unroll
+                for (int q = 1; q < (SEG > 4 ? 4 : SEG); ++q) t += r[q][s][lane];
+            }
+            if (SEG > 4) {
+                float u = r[SEG > 4 ? 4 : 0][s][lane];
+#pragma unroll
+                for (int q = 5; q < SEG; ++q) u += r[q][s][lane];
+                t += u;
+            }
+            if (SEG == 4 && g > first) t = tot[s][lane] + t;
+            if (SEG == 4 && g < last) tot[s][lane] = t;  // (its own lanes read it)
+            else if (!valid) continue;
+            else if (part) part[h * 64 + lane] = t;
+            else adj_sym_store<FBP, GRP>(S, x0, y0, h, t, img);
+        }
     }
 #undef CTPRJ_RUN
-    if (SEG > 1) {
-#pragma unroll
-        for (int s = 0; s < O::N; ++s) red[wave][O::elem(s)][lane] = acc[s].s;
-        __syncthreads();
-    }
-    if (!part && it.pad) sym_zero_border(S, img);
-    if (!valid) return;
-    // wave w finalises the elements h = w (mod SEG): the sum of the waves' partials in
-    // wave order
-#pragma unroll
-    for (int s = 0; s < O::N; ++s) {
-        const int h = O::elem(s);
-        if (SEG > 1 && h % SEG != wave) continue;
-        float t = acc[s].s;
-        if (SEG > 1) {
-            t = red[0][h][lane];
-#pragma unroll
-            for (int q = 1; q < SEG; ++q) t += red[q][h][lane];
-        }
-        if (part) part[h * 64 + lane] = t;
-        else adj_sym_store<FBP, GRP>(S, x0, y0, h, t, img);
-    }
 }
 
-// One launch per symmetry group; SEG waves split the canonical views (wave w takes
-// i = w, w + SEG, ...) and then share the final sums; with nsplit > 1, nsplit
-// work-groups share the views of a tile and leave their sums in part (512 floats per
-// work-group) for k_adjoint_sym_combine.
+// One launch per symmetry group; SEG waves split the canonical views and then share the final
+// sums; with nsplit > 1, nsplit work-groups share the views of a tile, one group of sets each,
+// and leave their sums in part (512 floats per work-group) for k_adjoint_sym_combine.  capped:
+// a slice's views are cut into its own number of groups of four (agroups); one work-group
+// takes them all (SEG = 4, or the two of SEG = 8) or up to nsplit do, the others end.
 template <bool FBP, int SEG, int GRP, bool DIRECT>
 __global__ __launch_bounds__(64 * SEG) void k_adjoint_sym(const SliceDesc* __restrict__ slices,
                                                           const AdjItem* __restrict__ items,
@@ -1408,7 +1527,8 @@ __global__ __launch_bounds__(64 * SEG) void k_adjoint_sym(const SliceDesc* __res
                                                           float* __restrict__ part,
                                                           const RedJob job)
 {
-    __shared__ float red[SEG][8][64];
+    __shared__ float red[SEG == 4 ? 2 : 1][SEG][Orbit<GRP>::N][64];
+    __shared__ float tot[SEG == 4 ? Orbit<GRP>::N : 1][64];
     __shared__ AdjStage stage[SEG];
     if (job.out && blockIdx.x == 0 && threadIdx.x < 64) wave_sum_job(job);  // on the side
     int split, idx;
@@ -1416,15 +1536,16 @@ __global__ __launch_bounds__(64 * SEG) void k_adjoint_sym(const SliceDesc* __res
     const AdjItem it = items[idx];
     if (it.slice < 0) return;  // uniform over the work-group
     const SliceDesc S = slices[it.slice];
-    if (capped) nsplit = min(nsplit, S.acap);
-    if (split >= nsplit) return;  // uniform over the work-group
+    const int groups = capped && SEG == 4 ? S.agroups : nsplit;
+    if (split >= groups) return;  // uniform over the work-group
+    const int last = nsplit > 1 ? split : groups - 1;
     float* mine = part ? part + (long long)blockIdx.x * 512 : nullptr;
     if (S.fan)
-        adj_sym_tile<true, FBP, SEG, GRP, DIRECT>(S, it, views, rays, os, tab, img, red, split,
-                                                  nsplit, mine, stage);
+        adj_sym_tile<true, FBP, SEG, GRP, DIRECT>(S, it, views, rays, os, tab, img, red, tot, groups,
+                                                  split, last, mine, stage);
     else
-        adj_sym_tile<false, FBP, SEG, GRP, DIRECT>(S, it, views, rays, os, tab, img, red, split,
-                                                   nsplit, mine, stage);
+        adj_sym_tile<false, FBP, SEG, GRP, DIRECT>(S, it, views, rays, os, tab, img, red, tot, groups,
+                                                   split, last, mine, stage);
 }
 
 // The nsplit partial sums of each orbit image of a tile, added in split order and
@@ -1440,7 +1561,7 @@ __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __
     const AdjItem it = items[blockIdx.x];
     if (it.slice < 0) return;
     const SliceDesc S = slices[it.slice];
-    if (CAPPED) nsplit = min(nsplit, S.acap);
+    if (CAPPED) nsplit = min(nsplit, S.agroups);
     constexpr GroupMasks G = group_masks(GRP);
     if (it.pad) sym_zero_border(S, img);
     const int h = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
@@ -1456,21 +1577,25 @@ __global__ __launch_bounds__(512) void k_adjoint_sym_combine(const SliceDesc* __
 // ----------------------------------------------------------------- launchers ---
 
 template <int GRP, bool BHC>
-static void launch_forward_sym_g(int seg, bool four_views, int nsplit, bool capped, float* part,
+static void launch_forward_sym_g(int seg, bool views4, int level, int nsplit,
+                                 bool capped, float* part,
                                  int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
                                  const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
 {
     float* pp = nsplit > 1 ? part : nullptr;
+    // work-groups per item of k_forward_views
+    const int nwg = level < 0 ? 1 : level == 0 ? nsplit : (nsplit + level - 1) / level;
     const dim3 grid((unsigned)nitems * (unsigned)nsplit);
 #define CTPRJ_LAUNCH(SEG)                                                                       \
     hipLaunchKernelGGL((k_forward_sym<SEG, GRP, BHC>), grid, dim3(64 * SEG), 0, st, desc, items, \
                        views, rays, orb, sino, nitems, nsplit, capped, pp, B)
-    if (seg == 4 && four_views)
+    if (views4)
         hipLaunchKernelGGL((k_forward_views<GRP, BHC>),
-                           dim3((unsigned)(nitems / 4) * (unsigned)nsplit), dim3(256), 0, st, desc,
-                           items, views, rays, orb, sino, nitems, nsplit, pp, B);
+                           dim3((unsigned)(nitems / 4) * (unsigned)nwg), dim3(256), 0, st, desc,
+                           items, views, rays, orb, sino, nitems, nwg, level, capped ? 0 : nsplit,
+                           pp != nullptr, part, B);
     else switch (seg) {
         case 1: CTPRJ_LAUNCH(1); break;
         case 2: CTPRJ_LAUNCH(2); break;
@@ -1482,28 +1607,30 @@ static void launch_forward_sym_g(int seg, bool four_views, int nsplit, bool capp
     if (!pp) return;
     auto* combine = capped ? k_forward_sym_combine<GRP, BHC, true> : k_forward_sym_combine<GRP, BHC, false>;
     hipLaunchKernelGGL(combine, dim3((unsigned)nitems), dim3(512), 0, st, desc, items, views, nitems,
-                       nsplit, pp, sino, B);
+                       nsplit, views4 && level == 0, pp, sino, B);
 }
 
 template <bool BHC>
-static void launch_forward_sym_b(int grp, int seg, bool four_views, int nsplit, bool capped,
+static void launch_forward_sym_b(int grp, int seg, bool views4, int level, int nsplit,
+                                 bool capped,
                                  float* part, int nitems,
                                  const SliceDesc* desc, const FwdItem* items, const float4* views,
                                  const Ray* rays, const float* orb, float* sino,
                                  const FwdBhc<BHC>& B, hipStream_t st)
 {
     if (grp == kGrpD4)
-        launch_forward_sym_g<kGrpD4, BHC>(seg, four_views, nsplit, capped, part, nitems, desc, items,
+        launch_forward_sym_g<kGrpD4, BHC>(seg, views4, level, nsplit, capped, part, nitems, desc, items,
                                           views, rays, orb, sino, B, st);
     else if (grp == kGrpV4)
-        launch_forward_sym_g<kGrpV4, BHC>(seg, four_views, nsplit, capped, part, nitems, desc, items,
+        launch_forward_sym_g<kGrpV4, BHC>(seg, views4, level, nsplit, capped, part, nitems, desc, items,
                                           views, rays, orb, sino, B, st);
     else
-        launch_forward_sym_g<kGrpZ2, BHC>(seg, four_views, nsplit, capped, part, nitems, desc, items,
+        launch_forward_sym_g<kGrpZ2, BHC>(seg, views4, level, nsplit, capped, part, nitems, desc, items,
                                           views, rays, orb, sino, B, st);
 }
 
-void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, bool capped, float* part,
+void launch_forward_sym(int grp, int seg, bool views4, int level, int nsplit,
+                                 bool capped, float* part,
                         int nitems,
                         const SliceDesc* desc, const FwdItem* items, const float4* views,
                         const Ray* rays, const float* orb, float* sino, const BhcStore* bhc,
@@ -1512,10 +1639,10 @@ void launch_forward_sym(int grp, int seg, bool four_views, int nsplit, bool capp
     if (bhc) {
         FwdBhc<true> B;
         static_cast<BhcStore&>(B) = *bhc;
-        launch_forward_sym_b<true>(grp, seg, four_views, nsplit, capped, part, nitems, desc, items,
+        launch_forward_sym_b<true>(grp, seg, views4, level, nsplit, capped, part, nitems, desc, items,
                                    views, rays, orb, sino, B, st);
     } else {
-        launch_forward_sym_b<false>(grp, seg, four_views, nsplit, capped, part, nitems, desc, items,
+        launch_forward_sym_b<false>(grp, seg, views4, level, nsplit, capped, part, nitems, desc, items,
                                     views, rays, orb, sino, FwdBhc<false>{}, st);
     }
 }

@@ -129,7 +129,8 @@ typedef struct ctprj_tune {
     int fwd_split;   /* symmetric forward: work-groups per 64 canonical rays splitting the
                         image rows, 1-8, the same way.  In either direction 8 waves (seg)
                         with one work-group (split), a new plan's values, leave the shape to
-                        the plan, which takes it from its sizes */
+                        the plan, which takes it from its sizes.  Under any one tune a slice's
+                        results are bit for bit the same alone and among other slices */
 } ctprj_tune;
 int ctprj_plan_get_tune(const ctprj_plan* plan, ctprj_tune* tune);
 /* Out-of-range fields are refused (CTPRJ_EINVAL) and change nothing.  Splits whose
