@@ -308,8 +308,15 @@ void launch_orbit_image(int nitems, const SliceDesc* desc, const AdjItem* items,
 // the kernel; now three loads serve the wave's row.
 // The staged columns start at the first pixel of an end lane (the rays of a wave are
 // ordered).  Waves for which that does not hold over all of their rows, or whose rays
-// cross more than kPixels pixels of a row (coarse detectors), form the true range at each
-// row and stage it piece by piece, in increasing order.
+// cross more than kPixels pixels of a row (coarse detectors), go another way:
+//   V4, Z2  each lane reads its own pixels straight from the orbit image, one load a pixel:
+//       hardly a pixel is shared between lanes, and a row staged in pieces leaves the lanes
+//       of the other pieces idle.  Forward, us, staged piece by piece with every load waited
+//       for / so: 1024^2 fan of 181 views, pitch 4: 342 / 181, pitch 7: 595 / 286; 512^2, pitch
+//       2.5: 90 / 59; 1024^2 parallel of 181, pitch 2: 160 / 113.
+//   D4  two loads a pixel, 64 lines each, would bound the walk (512^2 fan of 720 views, pitch 4:
+//       205); the wave forms its true range of pixels and stages it piece by piece, the next
+//       piece or row being on its way: 138 / 125 there, 1024^2 fan of 180 views, pitch 3: 208 / 190.
 template <bool FAN, int GRP, bool COLS>
 __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, float cT, float sT,
                                              const float* __restrict__ orb, int vlo, int vhi,
@@ -327,7 +334,7 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
     // Regular waves: at the first and the last row, and hence (all are linear in v) at every
     // row between, each lane's lines keep their order, no lane starts more than a pixel
     // before the end lane `edge` that starts first at both, and all end within the staged
-    // pixels.  Others form the wave's range row by row.
+    // pixels.
     const float fa = (float)vlo, fb = (float)vhi;
     const float ea = fmaf(fa, ub, ua), eb = fmaf(fb, ub, ua);
     const float ga = fmaf(fa, lb, la), gb = fmaf(fb, lb, la);
@@ -342,9 +349,10 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
     auto within = [&](float px) { return (Ra - sa < px && Rb - sb < px) || 2.0f * fH < px; };
     const bool regular = __all(La <= Ra && Lb <= Rb && La >= sa - 0.9f && Lb >= sb - 0.9f &&
                                within((float)(CH - 3)));
-    const bool wide = !(regular && __all(within(61.0f)));
+    const bool wide = !__all(within(61.0f));
     const float l0 = left ? la : ua, l1 = left ? lb : ub, r0 = left ? ua : la, r1 = left ? ub : lb;
-    auto row_setup = [&](float fv, float& lo, float& hi, int& ilo, int& c0) {
+    // the lane's pixels of row fv
+    auto row_range = [&](float fv, float& lo, float& hi) {
         const float e = fmaf(fv, l1, l0), f = fmaf(fv, r1, r0);
         if (regular) {
             lo = fmaxf(ceilf(e), -fH);
@@ -353,12 +361,25 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
             lo = fmaxf(ceilf(fminf(e, f)), -fH);
             hi = fminf(fmaxf(e, f), fH);
         }
-        ilo = (int)lo;
-        // one pixel of slack; a row that no lane meets takes any column, so that its load
-        // stays inside
-        c0 = min(max(__builtin_amdgcn_readlane(ilo, edge) - 1, -H), H);
     };
-    // 16-byte unit 64 j + lane of a staged piece: pixel unit % CH of plane unit / CH; units
+    float part[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) part[s] = 0.0f;
+    // the weight at pixel fu of a row of rowd, rowq (of fv in columns mode)
+    auto weight = [&](float fu, float fv, float rowd, float rowq) {
+        // ray_dist and fan_depth_scale at (x, y) = (fu, fv), columns mode (fv, fu)
+        const float dist = COLS ? fmaf(fv, r.cosR, fmaf(fu, r.sinR, -r.dc)) : fmaf(fu, r.cosR, rowd);
+        const float qd = COLS ? fmaf(fv, qs, fmaf(-fu, qc, 1.0f)) : fmaf(fu, qs, rowq);
+        return strip_area(dist, FAN ? r.hbc * qd : r.hbc, r);
+    };
+    auto flush = [&]() {
+#pragma unroll
+        for (int s = 0; s < N; ++s) {
+            acc[s].add(part[s]);
+            part[s] = 0.0f;
+        }
+    };
+    // 16-byte unit 64 j + lane of a staged row: pixel unit % CH of plane unit / CH; units
     // past a narrow wave's pixels are not read (offsets beyond the row load as 0)
     int voff[O::kLoads];
 #pragma unroll
@@ -367,108 +388,143 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
         voff[j] = N == 8 && unit >= CH ? (S.orb_pitch + unit - CH) * 16 : unit * 16;
         if (N >= 4 && (j & 1) && !wide) voff[j] = 0x7ffffff0;
     }
-    auto load = [&](const float* row, int c0, float4* g) {
-        const __amdgpu_buffer_rsrc_t R = row_rsrc(row, N * S.orb_pitch * 4);
-#pragma unroll
-        for (int j = 0; j < O::kLoads; ++j) g[j] = ldb128(R, voff[j], (c0 + H) * O::kPlane * 4);
-    };
-    auto stage = [&](const float4* g) {
-        wave_lds_sync();  // the previous piece's reads are done
-#pragma unroll
-        for (int j = 0; j < O::kLoads; ++j) st[64 * j + lane] = g[j];
-        wave_lds_sync();  // staged values visible to every lane
-    };
-    auto pixel = [&](int at, float* q) {
-        if constexpr (N == 2) {
-            const float2 a = reinterpret_cast<const float2*>(st)[at];
-            q[0] = a.x;
-            q[1] = a.y;
-        } else {
-#pragma unroll
-            for (int p = 0; p < N / 4; ++p) {
-                const float4 a = st[p * CH + at];
-                q[4 * p] = a.x;
-                q[4 * p + 1] = a.y;
-                q[4 * p + 2] = a.z;
-                q[4 * p + 3] = a.w;
-            }
-        }
-    };
-    float part[N];
-#pragma unroll
-    for (int s = 0; s < N; ++s) part[s] = 0.0f;
-    // the pixels [lo, hi] of walk row fv from the staged pixel of lo on
-    auto sum = [&](float fv, float lo, float hi, int at) {
-        const float rowd = COLS ? 0.0f : fmaf(fv, r.sinR, -r.dc);
-        const float rowq = FAN && !COLS ? fmaf(-fv, qc, 1.0f) : 0.0f;
-        for (float fu = lo; fu <= hi; fu += 1.0f, ++at) {
-            float q[N];
-            pixel(at, q);
-            // ray_dist and fan_depth_scale at (x, y) = (fu, fv), columns mode (fv, fu)
-            const float dist = COLS ? fmaf(fv, r.cosR, fmaf(fu, r.sinR, -r.dc))
-                                    : fmaf(fu, r.cosR, rowd);
-            const float qd = COLS ? fmaf(fv, qs, fmaf(-fu, qc, 1.0f)) : fmaf(fu, qs, rowq);
-            const float w = strip_area(dist, FAN ? r.hbc * qd : r.hbc, r);
-#pragma unroll
-            for (int s = 0; s < N; ++s) part[s] = fmaf(w, q[s], part[s]);
-        }
-    };
     // rows v < 0 first, then v >= 0: the sums are held by the slots of the current sign
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
         const int va = half ? max(vlo, 0) : vlo, vb = half ? vhi : min(vhi, -1);
-        if (va <= vb) {
-            const float* row = orbit_row<GRP, COLS>(S, orb, va);
-            const long long step = neg && !half ? -(long long)N * S.orb_pitch : N * S.orb_pitch;
-            float fv = (float)va, lo, hi;
-            int ilo, c0;
+        const float* row = va <= vb ? orbit_row<GRP, COLS>(S, orb, va) : nullptr;
+        const long long step = neg && !half ? -(long long)N * S.orb_pitch : N * S.orb_pitch;
+        float fv = (float)va, lo, hi;
+        if (va <= vb && (regular || N == 8)) {
+            // the first staged column of row fv, and (D4's irregular waves) the wave's last pixel
+            int c0, last = INT_MIN;
+            auto column = [&]() {
+                if (N < 8 || regular) {
+                    // one pixel of slack; a row that no lane meets takes any column, so that
+                    // its load stays inside
+                    c0 = min(max(__builtin_amdgcn_readlane((int)lo, edge) - 1, -H), H);
+                } else {
+                    const bool any = lo <= hi;
+                    wave_range_i32(any ? (int)lo : INT_MAX, any ? (int)hi : INT_MIN, c0, last);
+                    c0 = min(c0, H);
+                }
+            };
+            auto load = [&](int c0, float4* g) {
+                const __amdgpu_buffer_rsrc_t R = row_rsrc(row, N * S.orb_pitch * 4);
+#pragma unroll
+                for (int j = 0; j < O::kLoads; ++j) g[j] = ldb128(R, voff[j], (c0 + H) * O::kPlane * 4);
+            };
             float4 g[O::kLoads];
-            row_setup(fv, lo, hi, ilo, c0);
-            load(row, c0, g);
+            row_range(fv, lo, hi);
+            column();
+            load(c0, g);
+#pragma unroll 1
+            for (int v = va; v <= vb;) {
+                const int vend = min(v + kRowBlock - 1, vb);
+#pragma unroll 1
+                for (; v <= vend;) {
+                    wave_lds_sync();  // the previous row's reads are done
+#pragma unroll
+                    for (int j = 0; j < O::kLoads; ++j) st[64 * j + lane] = g[j];
+                    wave_lds_sync();  // staged values visible to every lane
+                    const float pv = fv;
+                    float plo = lo, phi = hi;
+                    int at = (int)fminf(lo, fH) - c0;
+                    bool more = false;  // (wave-uniform) pixels of this row past the staged ones
+                    if (N == 8 && !regular) {
+                        phi = fminf(hi, (float)(c0 + CH - 1));
+                        more = c0 + CH <= last;
+                    }
+                    if (more) {
+                        c0 += CH;
+                        lo = fmaxf(lo, (float)c0);
+                        load(c0, g);
+                    } else {
+                        if (v < vb) {
+                            fv += 1.0f;
+                            row += step;
+                            row_range(fv, lo, hi);
+                            column();
+                            load(c0, g);
+                        }
+                        ++v;
+                    }
+                    const float rowd = COLS ? 0.0f : fmaf(pv, r.sinR, -r.dc);
+                    const float rowq = FAN && !COLS ? fmaf(-pv, qc, 1.0f) : 0.0f;
+                    for (float fu = plo; fu <= phi; fu += 1.0f, ++at) {
+                        float q[N];
+                        if constexpr (N == 2) {
+                            const float2 a = reinterpret_cast<const float2*>(st)[at];
+                            q[0] = a.x;
+                            q[1] = a.y;
+                        } else {
+#pragma unroll
+                            for (int p = 0; p < N / 4; ++p) {
+                                const float4 a = st[p * CH + at];
+                                q[4 * p] = a.x;
+                                q[4 * p + 1] = a.y;
+                                q[4 * p + 2] = a.z;
+                                q[4 * p + 3] = a.w;
+                            }
+                        }
+                        const float w = weight(fu, pv, rowd, rowq);
+#pragma unroll
+                        for (int s = 0; s < N; ++s) part[s] = fmaf(w, q[s], part[s]);
+                    }
+                }
+                flush();
+            }
+        } else if (N < 8 && va <= vb) {
+            // straight from memory, a pixel (and, at its end, the next row's first) ahead
+            auto load = [&](int at, float* q) {  // past the row's end: 0, or the next plane's
+                const __amdgpu_buffer_rsrc_t R = row_rsrc(row, N * S.orb_pitch * 4);
+                if constexpr (N == 2) {
+                    const auto a = __builtin_amdgcn_raw_buffer_load_b64(R, at, 0, 0);
+                    q[0] = __uint_as_float(a[0]);
+                    q[1] = __uint_as_float(a[1]);
+                } else {
+#pragma unroll
+                    for (int p = 0; p < N / 4; ++p) {
+                        const float4 a = ldb128(R, at, p * S.orb_pitch * 16);
+                        q[4 * p] = a.x;
+                        q[4 * p + 1] = a.y;
+                        q[4 * p + 2] = a.z;
+                        q[4 * p + 3] = a.w;
+                    }
+                }
+            };
+            float q[N];
+            auto begin = [&](int& at) {
+                row_range(fv, lo, hi);
+                at = (int)(fminf(lo, fH) + fH) * (O::kPlane * 4);
+                load(at, q);
+            };
+            int at;
+            begin(at);
 #pragma unroll 1
             for (int v = va; v <= vb;) {
                 const int vend = min(v + kRowBlock - 1, vb);
 #pragma unroll 1
                 for (; v <= vend; ++v) {
-                    stage(g);
-                    const float pv = fv, plo = lo, phi = hi;
-                    const int pilo = ilo;
-                    const float* prow = row;
-                    int p = c0, last = c0;
+                    const float rowd = COLS ? 0.0f : fmaf(fv, r.sinR, -r.dc);
+                    const float rowq = FAN && !COLS ? fmaf(-fv, qc, 1.0f) : 0.0f;
+                    for (float fu = lo; fu <= hi; fu += 1.0f) {
+                        float next[N];
+                        at += O::kPlane * 4;
+                        load(at, next);
+                        const float w = weight(fu, fv, rowd, rowq);
+#pragma unroll
+                        for (int s = 0; s < N; ++s) part[s] = fmaf(w, q[s], part[s]);
+#pragma unroll
+                        for (int s = 0; s < N; ++s) q[s] = next[s];
+                    }
                     if (v < vb) {
                         fv += 1.0f;
                         row += step;
-                        row_setup(fv, lo, hi, ilo, c0);
-                        load(row, c0, g);
-                    }
-                    float first = plo;
-                    if (!regular) {
-                        const int ihi = (int)phi;  // towards 0: at least the last pixel
-                        wave_range_i32(plo <= phi ? pilo : INT_MAX, plo <= phi ? ihi : INT_MIN, p,
-                                       last);
-                        if (p > last) continue;  // no lane meets this row
-                        float4 h[O::kLoads];
-                        load(prow, p, h);
-                        stage(h);
-                        first = (float)max(pilo, p);
-                    }
-                    int at = max(pilo, p) - p;
-                    for (;;) {
-                        sum(pv, first, regular ? phi : fminf(phi, (float)(p + CH - 1)), at);
-                        p += CH;
-                        if (regular || p > last) break;  // wave-uniform
-                        float4 h[O::kLoads];
-                        load(prow, p, h);
-                        stage(h);
-                        first = (float)max(pilo, p);
-                        at = max(pilo, p) - p;
+                        begin(at);
                     }
                 }
-#pragma unroll
-                for (int s = 0; s < N; ++s) {
-                    acc[s].add(part[s]);
-                    part[s] = 0.0f;
-                }
+                flush();
             }
         }
         if (neg && half == 0)
