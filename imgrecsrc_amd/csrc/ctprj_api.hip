@@ -393,7 +393,7 @@ static int host_map_view(int P, bool fold, int k, int m, int a0, bool* flip)
     return v;
 }
 
-constexpr long long kViewRows = 40000;  // rows of four-view work-groups: see fwd_shape
+constexpr long long kViewRows = 50000;  // rows of four-view work-groups: see fwd_shape
 
 // Whether canonical view i of a slice walks columns (steeper than 45 degrees; none under D4),
 // and how many views from i on share a four-view work-group.
@@ -511,7 +511,7 @@ int Plan::build_geometry(int flags, Tables& G) const
             const long long fitems = D.ncanon * bins, rows = quads * (2 * D.H + 1);
             const int elems = fold ? M.order / 2 : M.order;
             const int steps = (D.ncanon + 7) / 8 * elems;  // of one of eight waves
-            const bool longer = rows < kViewRows && g.n * std::max(1.0f, g.dSize) >= 350.0f;
+            const bool longer = rows < 40000 && g.n * std::max(1.0f, g.dSize) >= 350.0f;
             D.fgroups = g.n <= 48 ? 2 : g.n > 224 && (fitems <= 150 || longer) ? 8 : 4;
             const long long fill = tiles < 40 ? 16 : tiles <= 160 ? 8 : tiles <= 320 ? 4 : std::min(8LL, (9000 + tiles - 1) / tiles);
             D.agroups = steps <= 16 ? 2 : (int)std::min((steps + 7) / 8 * 2LL, fill);
@@ -522,6 +522,8 @@ int Plan::build_geometry(int flags, Tables& G) const
             L.amax[grp] = std::max(L.amax[grp], D.agroups);
             L.fitems[grp] += fitems;
             L.frows[grp] += rows;
+            L.fgroups[grp] += quads * D.fgroups;
+            L.agroups[grp] += tiles * D.agroups;
             L.asteps += tiles * D.ncanon * elems;
             // (byte offsets into a sinogram that is read directly are 32-bit)
             if ((double)g.np * g.prjWidth * 4.0 >= 2147483648.0) L.asteps = LLONG_MAX / 2;
@@ -865,14 +867,15 @@ constexpr long long kFewItems = 256;    // forward items that get a compute unit
 // Forward launches, by the rows of four-view work-groups in them (us):
 //   many (kViewRows): k_forward_views; 512^2 fan (71e3) 71.5, as four waves on one view's rows
 //   80; 512^2 parallel (142e3) 69.5 / 78; 16 x 192^2 (174e3) 140 / 158; 4 x 224^2 fan (54e3)
-//   69 / 70; 8 x 256^2 (74e3) 79 / 83; 16 x 93^2 of 536 views (100e3) 104 / 119; 100 x 64^2
+//   69 / 70; 384^2 fan (42e3) 54 / 50; 8 x 256^2 (74e3) 79 / 83; 16 x 93^2 of 536 views (100e3) 104 / 119; 100 x 64^2
 //   fan (63e3) 63 / 65; below: 256^2 (9.3e3) 25 / 21, 16 x 64^2 (24e3) 29 / 27.
 //     A work-group takes every group (level -1) where work-groups and rows per work-group say
 //     that the partial sums cost more than a longer last round: 200 x 128^2 (4800 work-groups)
 //     440, as groups 486; 100 x 128^2 odd 352 / 400; 8 x 512^2 odd (4416) 740 / 690; 32 x
 //     512^2 (8864) 2400 / 2350, less than the second launch with the spectrum costs.  It takes
 //     one segment (level 0) where they are few and long: 1024^2 fan (276) 183, as groups 246;
-//     769^2 odd (972) 247 / 267; 2 x 1024^2 (552) 326 / 385; 16 x 224^2 fan (960) 217 / 189.
+//     769^2 odd (972) 247 / 267; 2 x 1024^2 (552) 326 / 385; 16 x 224^2 fan (960) 217 / 189; by
+//     the groups, as slices of a ragged plan differ in them: four 8-fold ones 142 / 174.
 //     Between, a group, or two, four, ... of them while 8000 work-groups are left: 64 x 256^2
 //     two 427, one 442.
 //   fewer: four waves on one view's rows, one work-group per group; or the groups together in
@@ -889,8 +892,8 @@ Plan::Shape Plan::fwd_shape(const ctprj_tune& t, int items, const Tables& G, int
     } else if (sh.views) {
         const long long rows = L.frows[g] / quads;  // of a work-group, padding included
         sh.seg = 4;
-        sh.level = quads >= std::max(2500LL, 15 * rows) ? -1 : 10 * most * quads < 52 * rows ? 0 : 1;
-        while (sh.level > 0 && 2 * sh.level <= most && quads * most >= 16000LL * sh.level) sh.level *= 2;
+        sh.level = quads >= std::max(2500LL, 15 * rows) ? -1 : L.fgroups[g] < 8 * rows ? 0 : 1;
+        while (sh.level > 0 && 2 * sh.level <= most && L.fgroups[g] >= 16000LL * sh.level) sh.level *= 2;
         sh.split = sh.level < 0 ? 1 : sh.level == 0 ? 4 * (int)most : (int)most;
     } else if (L.fmin[g] == most && (most == 2 || (most == 4 && L.fitems[g] <= kFewItems))) {
         sh.seg = 4 * (int)most;
@@ -908,16 +911,20 @@ Plan::Shape Plan::fwd_shape(const ctprj_tune& t, int items, const Tables& G, int
     return sh;
 }
 
-// Adjoint launches: one work-group per group while there are few items, then one per tile,
-// which goes through the groups: 64 x 192^2 (4992 items) 186 / 168 us, 8 x 512^2 fan (4488) 309 /
-// 314, 100 x 160^2 (7800) 235 / 217, 200 x 128^2 (7200) 296 / 259.
+// Adjoint launches: one work-group per group up to kTileGroups of them, then one per tile,
+// which goes through the groups (us, per group / per tile): 2 x 1024^2 fan (21e3) 304 / 315, four
+// ragged 4-fold slices (24e3) 142 / 153, seven 8-fold ones (30e3) 177 / 166, 8 x 512^2 fan (36e3)
+// 309 / 314, 64 x 192^2 (40e3) 186 / 168, 100 x 160^2 (47e3) 235 / 217, 64 x 256^2 (52e3) 302 / 263.
+constexpr long long kTileGroups = 28000;
+
 Plan::Shape Plan::adj_shape(const ctprj_tune& t, int items, const Tables& G, int c, int g) const
 {
     const Loads& L = G.loads[c];
     Shape sh{t.adj_seg, t.adj_split, false, 0, t.adj_seg == 8 && t.adj_split == 1, items, 0};
     if (sh.capped && !(L.amin[g] == 2 && L.amax[g] == 2 && items < 2000)) {
         sh.seg = 4;
-        sh.split = items >= 4600 ? 1 : L.amax[g];
+        const bool room = (size_t)items * L.amax[g] * 512 <= kSplitMaxFloats;
+        sh.split = room && L.agroups[g] < kTileGroups ? L.amax[g] : 1;
     }
     sh.part = sh.split > 1 ? (size_t)items * sh.split * 512 : 0;
     return sh;

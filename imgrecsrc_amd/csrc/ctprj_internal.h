@@ -68,12 +68,14 @@ struct Tables {
     };
     std::vector<Segments> symf, syma;
     // what a launch of chunk c and group g goes by: the slices' least and largest
-    // fgroups and agroups, forward items and rows of four-view work-groups; (whole chunk) the adjoint's steps, a
-    // step being a tile's bins of one canonical view under one element
+    // fgroups and agroups, forward items, rows and groups of four-view work-groups, adjoint
+    // groups; (whole chunk) the adjoint's steps, a step being a tile's bins of one canonical
+    // view under one element
     struct Loads {
         int fmin[4] = {16, 16, 16, 16}, fmax[4] = {1, 1, 1, 1};
         int amin[4] = {16, 16, 16, 16}, amax[4] = {1, 1, 1, 1};
-        long long fitems[4] = {0, 0, 0, 0}, frows[4] = {0, 0, 0, 0}, asteps = 0;
+        long long fitems[4] = {0, 0, 0, 0}, frows[4] = {0, 0, 0, 0}, fgroups[4] = {0, 0, 0, 0};
+        long long agroups[4] = {0, 0, 0, 0}, asteps = 0;
     };
     std::vector<Loads> loads;
     int chunks() const { return (int)orb_start.size() - 1; }

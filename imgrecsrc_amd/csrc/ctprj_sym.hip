@@ -402,7 +402,7 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
                 if (N < 8 || regular) {
                     // one pixel of slack; a row that no lane meets takes any column, so that
                     // its load stays inside
-                    c0 = min(max(__builtin_amdgcn_readlane((int)lo, edge) - 1, -H), H);
+                    c0 = min(max(__builtin_amdgcn_readlane((int)fminf(lo, fH), edge) - 1, -H), H);
                 } else {
                     const bool any = lo <= hi;
                     wave_range_i32(any ? (int)lo : INT_MAX, any ? (int)hi : INT_MIN, c0, last);
@@ -702,8 +702,9 @@ __device__ __forceinline__ void fwd_view_rows(const SliceDesc& S, const Ray& r, 
                     const float hi = fminf(fmaf(fv, r1, r0), fH);
                     const float rowd = COLS ? 0.0f : fmaf(fv, r.sinR, -r.dc);
                     const float rowq = FAN && !COLS ? fmaf(-fv, qc, 1.0f) : 0.0f;
-                    // (the byte offset of the pixel is kept, not its index: one add a pixel less)
-                    int at = ((int)lo - now) * (O::kPlane * 4) + (int)((const char*)row - (const char*)st);
+                    // (the byte offset of the pixel is kept, not its index: one add a pixel less; lanes
+                    // without pixels may have any)
+                    int at = ((int)fminf(lo, fH) - now) * (O::kPlane * 4) + (int)((const char*)row - (const char*)st);
                     for (float fu = lo; fu <= hi; fu += 1.0f, at += O::kPlane * 4) {
                         const char* px = (const char*)st + at;
                         float q[N];
