@@ -87,9 +87,12 @@ int prj_get_geom(ctprj_geom* out);
  * current HIP device, including the FP64 reduction partials of the beam-hardening calls
  * (ctprj_bhc_grad_alpha, _alpha_rays, _grad_ie, ctprj_ie_solve), which therefore never
  * allocate and can be captured in a HIP graph from their first call.  The calls of one
- * plan share its workspace (the transposed image, the filtered sinogram, partial sums):
- * calls on one plan that overlap on different streams race; use one stream per plan, or
- * one plan per stream. */
+ * plan share its workspace, whichever way they go: the symmetric slices' orbit image
+ * (forward; about 4 times the images' size) and orbit sinogram (adjoint), both at most 4
+ * GiB unless one slice needs more, the transposed image of the others, the filtered
+ * sinogram, and the partial sums of either direction.  Calls on one plan that overlap on
+ * different streams race, a forward and an adjoint too; use one stream per plan, or one
+ * plan per stream. */
 int ctprj_plan_create(const ctprj_geom* geoms, int nslices, ctprj_plan** plan);
 int ctprj_plan_destroy(ctprj_plan* plan);
 
@@ -317,10 +320,14 @@ int ctprj_wavelet_l1(ctprj_wavelet* w, const float* d_x, double* l1, void* strea
  * (scaled by ||a||, adaptive penalty rho, stopping when both the change of the split
  * variable and the residual are at most min(relTol, 1e-3), or after maxItr + 1
  * iterations); d_init (may be NULL: a) starts the split variable.  *iterations gets the
- * iteration count (innerSearch).  The loop state stays on the device; three iterations
- * are one HIP graph (captured on the context's own stream at the first call, again
- * after new masks) and the host reads the state once per three iterations.  Calls on one
- * context share its buffers: they must not overlap on different streams. */
+ * iteration count (innerSearch).  The loop state stays on the device, and the host waits
+ * for it, so a stream that is being captured is refused (an error; the capture goes on).
+ * With two taps and up to 6 levels an iteration is one launch and the host reads the
+ * state once per eight, with the next eight already queued: those past the stop do
+ * nothing and end before d_out is written.  Otherwise three iterations are one HIP graph
+ * (captured on the context's own stream at the first call, again after new masks) and the
+ * host reads the state once per three.  Calls on one context share its buffers: they must
+ * not overlap on different streams. */
 int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, double u, double relTol,
                             int maxItr, const float* d_init, float* d_out, int* iterations,
                             void* stream);
@@ -344,7 +351,10 @@ int ctprj_tv_value(ctprj_tv* w, const float* d_x, double* tv, void* stream);
  * maxIter iterations or when ||D - Dold|| / ||D|| < epsilon five times in a row; the
  * dual starts at zero (TV.denoise does not forward its init).  Norms and the stopping
  * test run over all images of the context together.  *iterations gets the count.
- * The loop state stays on the device; the host reads it once per eight iterations. */
+ * The loop state stays on the device; the host reads it once per eight iterations, with
+ * the next eight already queued (those past the stop do nothing and end before d_out is
+ * written).  A stream that is being captured is refused (an error; the capture goes on).
+ * Calls on one context share its buffers: they must not overlap on different streams. */
 int ctprj_tv_denoise(ctprj_tv* w, const float* d_a, double lambda, double epsilon,
                      int maxIter, float* d_out, int* iterations, void* stream);
 
