@@ -234,6 +234,22 @@ def _summary(tag, suffix):
         return json.load(f)
 
 
+def call_launches(tag, tune):
+    """Kernels of one operator call, in launch order, from its counter summary
+    (profiles/<tag>_valu.json) if that was taken at these shapes, else None."""
+    s = _summary(tag, "valu")
+    return list(s["per_kernel"]) if s is not None and s.get("tune") == tune else None
+
+
+def dominant_kernel(tag, tune):
+    """The longest of those kernels, or None."""
+    names = call_launches(tag, tune)
+    if not names:
+        return None
+    per = _summary(tag, "valu")["per_kernel"]
+    return max(names, key=lambda k: per[k].get("GRBM_GUI_ACTIVE", 0.0))
+
+
 def roofline_entry(tag, kernel, kernel_ms, launches, nnz, tune, other_ms):
     """The dominant call against the ceiling that binds it.  The symmetric kernels reuse
     every loaded value for 2-8 updates and move little HBM traffic; their counters
@@ -672,21 +688,14 @@ def main():
     reps = max(5, min(args.steps, 50))
     t_fwd = timed(lambda: P.forward(img, out=sino), reps, stream)
     t_adj = timed(lambda: P.adjoint(sino, out=back), reps, stream)
-    sfx = "_sym" if P.modes()[0] != 0 else ""
-    # each call also runs the pass that lays out its orbit array (a few microseconds)
-    dom_name, dom_ms = (f"k_adjoint{sfx}", t_adj) if t_adj >= t_fwd else (f"k_forward{sfx}", t_fwd)
-    # 8 waves with one work-group stand for the plan's own shape: four views a work-group
-    # and split items at this size
-    own = (tune["fwd_seg"], tune["fwd_split"]) == (8, 1)
-    adj_parts = tune["adj_split"] > 1 or tune["adj_seg"] == 8
-    launches = (["k_orbit_sino", "k_adjoint_sym"] + (["k_adjoint_sym_combine"] if adj_parts else [])
-                if dom_name.startswith("k_adjoint") else
-                ["k_orbit_image",
-                 "k_forward_views" if own or tune["fwd_seg"] == 4 else "k_forward_sym"] +
-                (["k_forward_sym_combine"] if own or tune["fwd_split"] > 1 else []))
-    tag = f"{'adjoint' if dom_name.startswith('k_adjoint') else 'forward'}_{args.workload}"
-    roofline = roofline_entry(tag, dom_name, dom_ms, launches, nnz, tune,
-                              t_fwd if dom_name.startswith("k_adjoint") else t_adj)
+    # the launches of a call are those its counters were taken of (at the same shapes; the
+    # plan's rules pick kernels by size, which is not restated here)
+    launches = {d: call_launches(f"{d}_{args.workload}", tune) for d in ("forward", "adjoint")}
+    dom, dom_ms, other_ms = (("adjoint", t_adj, t_fwd) if t_adj >= t_fwd else
+                             ("forward", t_fwd, t_adj))
+    dom_name = dominant_kernel(f"{dom}_{args.workload}", tune) or f"{dom} call"
+    roofline = roofline_entry(f"{dom}_{args.workload}", dom_name, dom_ms, launches[dom], nnz, tune,
+                              other_ms)
 
     # the pair replayed as one HIP graph next to the same pair launched eagerly: what
     # the call's launches (orbit pass, forward, its combine, the same of the adjoint) cost
@@ -696,7 +705,8 @@ def main():
     t_pair = timed(step, reps, stream)
     t_pair_graph, _, pair_graph = graph_timed(step, reps, stream)
     pair_replay = {"eager_ms": round(t_pair, 4), "graph_ms": round(t_pair_graph, 4),
-                   "launches_per_pair": 4 + (own or tune["fwd_split"] > 1) + adj_parts,
+                   "launches_per_pair": sum(map(len, launches.values()))
+                   if all(launches.values()) else None,
                    "replay_equals_eager": bool(torch.equal(back, back_eager))}
     del pair_graph
     log(f"pair eager {t_pair:.4f} ms, graph replay {t_pair_graph:.4f} ms")
