@@ -1211,8 +1211,8 @@ extern "C" int ctprj_plan_autotune(ctprj_plan* p, int reps, const char* cache_pa
     hipStream_t st = (hipStream_t)stream;
     char arch[64] = "gfx950";
     ctprj_device_arch(arch, sizeof(arch));
-    // "k2": shapes found for other kernels (entries without it) are not those of these
-    const std::string key = tune_key(p, arch) + "|k2|f" + std::to_string(p->tune.flags & 7);
+    // "k3": shapes found for other kernels (entries without it) are not those of these
+    const std::string key = tune_key(p, arch) + "|k3|f" + std::to_string(p->tune.flags & 7);
     if (cache_path) {
         std::ifstream f(cache_path);
         std::string line;
