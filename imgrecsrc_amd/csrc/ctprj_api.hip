@@ -264,10 +264,10 @@ static int grow(float** p, long long* cap, long long floats, const char* what)
 // every slice is split over the queues, in contiguous eighths (adjoint tiles, which cost
 // the same and share bins with their neighbours) or dealt one by one with a turn per round
 // (`deal`: forward items, in view order, whose cost grows with the view's steepness and
-// falls towards the detector's ends), which balances the XCDs whatever the per-slice cost.  Otherwise only slices above a quarter of one XCD's
-// share are split and the others go whole to the least loaded queue, so each XCD's L2
-// serves whole slices (uniform stacks).  Shorter queues are padded with empty items
-// (slice = -1).
+// falls towards the detector's ends), which balances the XCDs whatever the per-slice cost.
+// Otherwise only slices above a quarter of one XCD's share are split and the others go whole
+// to the least loaded queue, so each XCD's L2 serves whole slices (uniform stacks).  Shorter
+// queues are padded with empty items (slice = -1).
 template <class Item>
 static std::vector<Item> batch_order(const std::vector<Item>& in,
                                      const std::vector<ctprj_geom>& geoms, bool spread, bool deal)
@@ -867,15 +867,16 @@ constexpr long long kFewItems = 256;    // forward items that get a compute unit
 // Forward launches, by the rows of four-view work-groups in them (us):
 //   many (kViewRows): k_forward_views; 512^2 fan (71e3) 71.5, as four waves on one view's rows
 //   80; 512^2 parallel (142e3) 69.5 / 78; 16 x 192^2 (174e3) 140 / 158; 4 x 224^2 fan (54e3)
-//   69 / 70; 384^2 fan (42e3) 54 / 50; 8 x 256^2 (74e3) 79 / 83; 16 x 93^2 of 536 views (100e3) 104 / 119; 100 x 64^2
-//   fan (63e3) 63 / 65; below: 256^2 (9.3e3) 25 / 21, 16 x 64^2 (24e3) 29 / 27.
+//   69 / 70; 8 x 256^2 (74e3) 79 / 83; 16 x 93^2 of 536 views (100e3) 104 / 119; 100 x 64^2 fan
+//   (63e3) 63 / 65; below: 384^2 fan (42e3) 54 / 50, 16 x 64^2 (24e3) 29 / 27, 256^2 (9.3e3) 25 /
+//   21.
 //     A work-group takes every group (level -1) where work-groups and rows per work-group say
 //     that the partial sums cost more than a longer last round: 200 x 128^2 (4800 work-groups)
 //     440, as groups 486; 100 x 128^2 odd 352 / 400; 8 x 512^2 odd (4416) 740 / 690; 32 x
-//     512^2 (8864) 2400 / 2350, less than the second launch with the spectrum costs.  It takes
-//     one segment (level 0) where they are few and long: 1024^2 fan (276) 183, as groups 246;
-//     769^2 odd (972) 247 / 267; 2 x 1024^2 (552) 326 / 385; 16 x 224^2 fan (960) 217 / 189; by
-//     the groups, as slices of a ragged plan differ in them: four 8-fold ones 142 / 174.
+//     512^2 (8864) 2475 / 2590 (its groups' sums need two pieces).  It takes one segment
+//     (level 0) where they are few and long: 1024^2 fan (276) 183, as groups 246; 769^2 odd
+//     (972) 247 / 267; 2 x 1024^2 (552) 326 / 385; 16 x 224^2 fan (960) 217 / 189; by the
+//     groups, as slices of a ragged plan differ in them: four 8-fold ones 142 / 174.
 //     Between, a group, or two, four, ... of them while 8000 work-groups are left: 64 x 256^2
 //     two 427, one 442.
 //   fewer: four waves on one view's rows, one work-group per group; or the groups together in
@@ -1011,6 +1012,7 @@ int Plan::launch_adjoint(const float* d_sino, float* d_img, hipStream_t st, bool
 
 int Plan::launch_fbp(const float* d_sino, float* d_img, hipStream_t st)
 {
+    // (a limit of the entry point: detectors of up to 13653 bins; the filter itself has none)
     if (sizeof(float) * 3 * (size_t)max_W > 160 * 1024)
         return fail(CTPRJ_EINVAL, "FBP: prjWidth %d too large", max_W);
     launch_fbp_filter(n_fbp_items, max_W, d_desc, d_fbp_items, d_fbp_kern, d_fbp_kern_off,

@@ -219,7 +219,7 @@ __device__ __forceinline__ const float* orbit_row(const SliceDesc& S, const floa
 // One 32 x 32 tile of the orbit image per work-group: item (slice, first stored row, first
 // column; pad = 1: columns mode).  Images whose u runs along image columns are read
 // straight, the others through an LDS transpose, so every read and write is coalesced.
-// Bound by its writes (16 n^2 bytes): one extra pass over a small array, 5-6 us at 1024^2.
+// Bound by its writes (16 n^2 bytes): one extra pass over a small array, 11 us at 1024^2.
 template <int GRP, bool COLS>
 __device__ __forceinline__ void orbit_tile(const SliceDesc& S, int r0, int u0,
                                            const float* __restrict__ img,
@@ -547,8 +547,8 @@ __device__ __forceinline__ void fwd_sym_rows(const SliceDesc& S, const Ray& r, f
 // Staging per wave, the vector memory unit (three 16-byte loads a row under D4, about 16
 // cycles each), LDS (three writes and the reads) and VALU were each busy two thirds of the
 // time; a row now takes one load and one write a wave, and VALU issue bounds the walk.
-// Forward of 32 x 512^2 parallel 3350 -> 2340 us, 769^2 fan of odd views 352 -> 251, 1024^2
-// fan 175 -> 158, 16 ragged slices 1230 -> 985.  Five waves per SIMD under D4 (96 VGPRs, 4
+// Forward of 32 x 512^2 parallel 3350 -> 2420 us, 769^2 fan of odd views 352 -> 247, 1024^2
+// fan 175 -> 155, 16 ragged slices 1230 -> 985.  Five waves per SIMD under D4 (96 VGPRs, 4
 // spilled outside the pixel loop) against four: 8 x 512^2 607 us against 667; 1024^2 fan 183
 // against 203, which is why the sums' LDS is kept below the sixth granule step (kLdsSums).
 template <int GRP>

@@ -27,8 +27,10 @@ namespace ctprj {
 constexpr int kTvBlock = 256;
 // Work-groups of an iteration, at most: every one of them reads all the partial sums (32 B
 // each), which 1024 keep at 32 MB a launch from L2; larger images give a group several runs
-// of kTvBlock pixels.  24 iterations at 512^2, 800^2 and 2048^2: 392, 600 and 2357 us with
-// 1024, 401, 728 and 3489 with 512, 452, 1051 and 5868 with 256.
+// of kTvBlock pixels.  24 iterations at 512^2, 800^2 and 2048^2: 310, 434 and 1949 us with
+// 1024, 262, 409 and 1950 with 512, 250, 439 and 1999 with 256.  (The line was drawn when the
+// sums took three times the shuffles and few groups lost: 392, 600, 2357 with 1024 against 401,
+// 728, 3489 with 512.)
 constexpr long long kTvGroups = 1024;
 
 // Sum of four values over the work-group, the same in every thread: each wave's lanes by
@@ -191,8 +193,9 @@ __device__ __forceinline__ double tv_primal(double x, double r1, double r1u, dou
 // iteration's, whose partial sums are in part0.  Group 0 keeps the new state in c1.
 // Bound by the chain state -> partial sums -> pixels -> partial sums at small images, by the
 // 88 B a pixel moves at large ones; so a group's first pixels are requested before the sums
-// are added: 24 iterations with their launches took 358 us at 512^2 and 2.04 ms at 2048^2, 398
-// and 2.36 ms without that, and 586 and 2.65 ms as primal, dual and control launches.
+// are added: 24 iterations with their launches take 300 us at 512^2 and 1.95 ms at 2048^2, and
+// took 595 and 2.6 as primal, dual and control launches; without the early request 40 us more
+// at 512^2.
 __global__ __launch_bounds__(kTvBlock) void k_tv_iter(
     const double* __restrict__ X, double* __restrict__ D, double* __restrict__ P1,
     double* __restrict__ P2, const double* __restrict__ R1, const double* __restrict__ R2,
@@ -443,7 +446,7 @@ extern "C" int ctprj_tv_denoise(ctprj_tv* w, const float* d_x, double lambda, do
     // Iterations in batches of kTvBatch.  The host waits for a batch's state only when the
     // next batch (or the output) is queued: with a wait between them the GPU stood still for
     // about 30 us a batch, more than the launches of a batch past the stop take (8 x 2.5 us).
-    // 24 iterations at 512^2: 360 -> 328 us.
+    // 24 iterations at 512^2: 32 us less.
     constexpr int kTvBatch = 8;
     int it = 0, batches = 0;
     auto queue = [&]() -> int {

@@ -749,7 +749,7 @@ __device__ __forceinline__ void haar_analyse(const HaarTaps& T, const double x[4
 
 // Sums of two values over a work-group of NT threads, in thread 0: the lower half of a wave's
 // lanes goes on with the first value, the upper with the second (12 shuffled words, not 24);
-// with haar_total2, 13 iterations at 512^2 192 -> 166 us.
+// with haar_total2, 13 iterations at 512^2 take 26 us less.
 template <int NT>
 __device__ __forceinline__ void haar_sum2(double& a, double& b)
 {
@@ -1449,7 +1449,7 @@ int admm_graph(ctprj_wavelet* w)
 // The two-tap prox: batches of kHaarBatch iterations, one launch each.  The host waits for a
 // batch's state only when the next batch (or the output) is queued: with a wait between them
 // the GPU stood still for about 30 us a batch, more than the launches of a batch past the stop
-// take (8 x 2.5 us).  13 iterations of 6 levels at 512^2: 206 -> 192 us.
+// take (8 x 2.5 us).  13 iterations of 6 levels at 512^2: 13 us less.
 template <int S>
 int haar_admm(ctprj_wavelet* w, const float* d_a, double u, double relTol, int maxItr,
               const float* d_init, float* d_out, int* iterations, hipStream_t st)
@@ -1552,8 +1552,8 @@ extern "C" int ctprj_prox_wavelet_admm(ctprj_wavelet* w, const float* d_a, doubl
     const unsigned g = grid1(n);
     relTol = std::min(1e-3, relTol);  // npg/admm.m:14
     // taps of length 2 on up to 6 levels: an iteration is one launch (13 iterations of 6 levels
-    // at 512^2: 166 us, 836 by the levels' own launches below; at 96^2 72 and 147 for a call
-    // that stops early)
+    // at 512^2: 166 us, 836 by the levels' own launches below; 5 levels at 96^2 120 and 570, and
+    // 156 and 601 for a call that stops early)
     if (w->T.lh == 2 && w->L <= kHaarMaxLevels)
         return haar_tile(w->L) == 64
                    ? haar_admm<64>(w, d_a, u, relTol, maxItr, d_init, d_out, iterations, st)
