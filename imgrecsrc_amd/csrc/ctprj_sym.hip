@@ -1010,7 +1010,7 @@ void k_forward_views(const SliceDesc* __restrict__ slices,
     constexpr GroupMasks GM = group_masks(GRP);
     const unsigned mask = !active ? 0u : (a0 == 0 || GM.q * a0 == S.P) ? GM.rot : GM.all;
     const int b = min(max(it.bin0 + lane, S.blo), S.fold ? S.pC : S.bhi);
-    // this wave's sums by slot, and, level 2 of several groups, the place of their total
+    // this wave's sums by slot
     float reg[N];
     // (the places are formed anew where they are used: no register holds them over the walk)
     auto here = [&]() {
