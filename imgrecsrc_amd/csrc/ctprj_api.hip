@@ -513,7 +513,11 @@ int Plan::build_geometry(int flags, Tables& G) const
             const int steps = (D.ncanon + 7) / 8 * elems;  // of one of eight waves
             const bool longer = rows < 40000 && g.n * std::max(1.0f, g.dSize) >= 350.0f;
             D.fgroups = g.n <= 48 ? 2 : g.n > 224 && (fitems <= 150 || longer) ? 8 : 4;
-            const long long fill = tiles < 40 ? 16 : tiles <= 160 ? 8 : tiles <= 320 ? 4 : std::min(8LL, (9000 + tiles - 1) / tiles);
+            const int room = grp == kGrpD4 ? 1280 : grp == kGrpV4 ? 1792 : 2048;
+            const long long fill = tiles < 40         ? 16
+                                   : 8 * tiles <= room ? 8
+                                   : 4 * tiles <= room ? 4
+                                                       : std::min(8LL, (9000 + tiles - 1) / tiles);
             D.agroups = steps <= 16 ? 2 : (int)std::min((steps + 7) / 8 * 2LL, fill);
             Tables::Loads& L = G.loads.back();
             L.fmin[grp] = std::min(L.fmin[grp], D.fgroups);
@@ -849,11 +853,12 @@ namespace ctprj {
 // work-groups do that, so a slice has the same bits alone, in any batch and in either work
 // order.
 //
-// agroups.  Sets of a slice's canonical views, as many groups as fill the device in one round
-// (about 1280 work-groups of four waves fit), or, where four already exceed it, up to 8 for a
-// shorter last round.  Adjoint, us, by groups: 512^2 fan 4: 50.7, 8: 48.1; 300^2 4: 18.4, 6:
-// 20.4; 16 x 300^2 152, 160, 8: 165; 224^2 fan 8: 16.1, 16: 18.1; 93^2 of 536 views 8: 14.1,
-// 16: 11.3.  Slices of 16 steps of one of eight waves and fewer (a step being about 0.5 us)
+// agroups.  Sets of a slice's canonical views, 8 or 4 groups if that many work-groups of four
+// waves fit the device at once (D4 1280, V4 1792, Z2 2048), up to 8 for a shorter last round
+// where four already do not, and 16 for the few tiles of a small image.  Adjoint, us, by
+// groups: 512^2 fan 4: 50.7, 8: 48.1; 300^2 4: 18.4, 6: 20.4; 16 x 300^2 4: 152, 6: 160, 8: 165;
+// 224^2 fan 8: 16.1, 16: 18.1; 160^2 of 401 views 4: 25.5, 8: 23.4; 93^2 of 536 views 8: 14.1,
+// 16: 11.4.  Slices of 16 steps of one of eight waves and fewer (a step being about 0.5 us)
 // take two groups, which are one work-group of eight waves: 64^2 fan 11.4 us, without the
 // second launch's 2 us.
 //
