@@ -2,7 +2,7 @@
 
 ``Projector`` owns a ``ctprj_plan``: slices of ragged size and mixed parallel/fan
 geometry are packed back to back (images n_s*n_s each, sinograms np_s*prjWidth_s each)
-and every call runs all slices in one launch on torch's current HIP stream.
+and every call runs all slices together, in a few launches on torch's current HIP stream.
 
 Geometry fields are those of the reference's struct prjConf (prj/prj.h:42-57) and the
 ``conf`` struct that tomography/ConfigCT.m:110-116 passes to the MEX 'config' command:

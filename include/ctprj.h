@@ -146,9 +146,9 @@ int ctprj_plan_set_tune(ctprj_plan* plan, const ctprj_tune* tune);
  * by (geometry, device arch). */
 int ctprj_plan_autotune(ctprj_plan* plan, int reps, const char* cache_path, void* stream);
 
-/* sino = A img  (prj/cpuPrj.c:319-616 semantics), all slices in one launch. */
+/* sino = A img  (prj/cpuPrj.c:319-616 semantics), all slices together. */
 int ctprj_forward(ctprj_plan* plan, const float* d_img, float* d_sino, void* stream);
-/* img = A^T sino (prj/cpuPrj.c:46-317 semantics), all slices in one launch. */
+/* img = A^T sino (prj/cpuPrj.c:46-317 semantics), all slices together. */
 int ctprj_adjoint(ctprj_plan* plan, const float* d_sino, float* d_img, void* stream);
 /* FBP command (prj/cpuPrj.c:718-784): fan pre-weight, ramp filter, weighted adjoint. */
 int ctprj_fbp(ctprj_plan* plan, const float* d_sino, float* d_img, void* stream);
