@@ -854,7 +854,7 @@ namespace ctprj {
 // order.
 //
 // agroups.  Sets of a slice's canonical views, 8 or 4 groups if that many work-groups of four
-// waves fit the device at once (D4 1280, V4 1792, Z2 2048), up to 8 for a shorter last round
+// waves fit the device at once (D4 1280, V4 1792, Z2 2048), up to 8 for a shorter tail
 // where four already do not, and 16 for the few tiles of a small image.  Adjoint, us, by
 // groups: 512^2 fan 4: 50.7, 8: 48.1; 300^2 4: 18.4, 6: 20.4; 16 x 300^2 4: 152, 6: 160, 8: 165;
 // 224^2 fan 8: 16.1, 16: 18.1; 160^2 of 401 views 4: 25.5, 8: 23.4; 93^2 of 536 views 8: 14.1,
@@ -876,7 +876,7 @@ constexpr long long kFewItems = 256;    // forward items that get a compute unit
 //   (63e3) 63 / 65; below: 384^2 fan (42e3) 54 / 50, 16 x 64^2 (24e3) 29 / 27, 256^2 (9.3e3) 25 /
 //   21.
 //     A work-group takes every group (level -1) where work-groups and rows per work-group say
-//     that the partial sums cost more than a longer last round: 200 x 128^2 (4800 work-groups)
+//     that the partial sums cost more than a longer tail: 200 x 128^2 (4800 work-groups)
 //     440, as groups 486; 100 x 128^2 odd 352 / 400; 8 x 512^2 odd (4416) 740 / 690; 32 x
 //     512^2 (8864) 2475 / 2590 (its groups' sums need two pieces).  It takes one segment
 //     (level 0) where they are few and long: 1024^2 fan (276) 183, as groups 246; 769^2 odd
