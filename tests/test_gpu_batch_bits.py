@@ -25,7 +25,9 @@ STACKS = [
     ((128, 185, 90, 180, 1.0, 1.0, 0.0), 260),    # all groups in one work-group
     ((256, 367, 180, 360, 1.0, 1.0, 0.0), 64),    # two groups of eight each
     ((512, 729, 90, 180, 1.0, 1.0, 0.0), 3),      # one segment each
-    ((512, 729, 360, 720, 1.0, 1.0, 0.0), 31),    # more partial sums than fit at once
+    ((512, 729, 360, 720, 1.0, 1.0, 0.0), 31),    # all groups, large slices
+    ((700, 1000, 360, 360, 1.0, 1.0, 2800.0), 48),  # a group each, in two pieces
+    ((64, 99, 536, 1072, 1.0, 1.0, 0.0), 970),    # all groups, in two pieces
     ((300, 427, 91, 182, 1.0, 1.0, 0.0), 20),     # 4-fold
     ((301, 427, 91, 91, 1.0, 1.0, 1300.0), 20),   # 2-fold
 ]
@@ -82,7 +84,8 @@ def test_stack(geo, count):
     _compare([geo] * count, (0, count // 2, count - 1), (1, 9))
 
 
-@pytest.mark.parametrize("geo,count", [STACKS[2], STACKS[3], STACKS[7], (STACKS[4][0], 2)])
+@pytest.mark.parametrize("geo,count", [STACKS[2], STACKS[3], STACKS[6], STACKS[7], STACKS[9],
+                                       (STACKS[4][0], 2)])
 def test_gradient_of_a_stack(geo, count):
     """The ray weights stored by the forward, and so the gradient, do not depend on the
     batch either (the cost is one sum over all slices)."""
